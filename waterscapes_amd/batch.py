@@ -29,7 +29,7 @@ import time as _time
 import numpy as np
 import torch
 
-from . import _lib, amg
+from . import _lib, amg, levels as lv
 from ._lib import check, ptr, MAXF
 from .krylov import (MAXLEV, HierDesc, PrecDesc, SolveStats, SolverConfig, SolverOptions,
                      _pick_lpr, compact_level, set_level_degrees)
@@ -87,19 +87,23 @@ def _i32(a):
 
 
 def pad_levels(levels, cinv, depth):
-    """The levels of one instance extended to `depth`: after its coarsest
-    level come copies of that level joined by identity prolongators, so the
-    V-cycle of the padded hierarchy still ends in the exact coarsest solve
-    (smoothing an exact solution leaves it unchanged)."""
+    """The levels of one instance extended to `depth`: its coarsest level
+    becomes an inner one with no matrix and a zero diagonal inverse (its
+    smoothing steps leave 0 and then the correction untouched, its residual
+    is the right-hand side) and passes everything through identity
+    prolongators to the coarsest solve at the bottom, which therefore may be
+    any operator, not only the exact inverse."""
     levels = [dict(lev) for lev in levels]
     last = levels[-1]
     n = last["n"]
     eye_rp = np.arange(n + 1, dtype=np.int64)
     eye_ci = np.arange(n, dtype=np.int32)
     eye_v = np.ones(n)
+    none = dict(A_rp=np.zeros(n + 1, dtype=np.int64), A_ci=np.zeros(0, dtype=np.int32),
+                A_v=np.zeros(0), dinv=np.zeros(n))
     while len(levels) < depth:
         levels[-1].update(nc=n, P_rp=eye_rp, P_ci=eye_ci, P_v=eye_v, R_rp=eye_rp, R_ci=eye_ci,
-                          R_v=eye_v)
+                          R_v=eye_v, **none)
         levels.append(dict(n=n, nc=0, A_rp=last["A_rp"], A_ci=last["A_ci"], A_v=last["A_v"],
                            dinv=last["dinv"], rho=last["rho"]))
     return levels, cinv
@@ -154,7 +158,7 @@ def pack_hierarchy(hiers, scales, skip_A0=False):
         out.append(d)
     sizes = [p[0][-1]["n"] for p in padded]
     off = _prefix(sizes)
-    inv = np.concatenate([(np.asarray(p[1]) / s[k]).reshape(-1) for k, p in enumerate(padded)])
+    inv = np.concatenate([(lv.host_array(p[1]) / s[k]).reshape(-1) for k, p in enumerate(padded)])
     ioff = _prefix([n * n for n in sizes])
     blk = np.repeat(np.arange(len(sizes), dtype=np.int32), sizes)
     return out, (inv, blk, _i32(off), ioff)
@@ -477,7 +481,12 @@ class MPETBatch:
         sys_ = [e.system for e in self.engines]
         # displacement block: scalar P2 Laplacian hierarchies scaled by mu_k
         mus = [s.mu for s in sys_]
-        ulev, ucoarse = pack_hierarchy([(k.levels, k.cinv) for k in kry], mus, skip_A0=True)
+        # the small end of every hierarchy as one dense operator per instance
+        # (levels.py), all instances' together within the byte limit
+        rows = lv.dense_rows(8 if self.precision == "fp64" else 4,
+                             lv.DENSE_TAIL_BYTES // self.K)
+        cut = [k.dense_tails(rows, 0 if self.precision == "fp64" else 1) for k in kry]
+        ulev, ucoarse = pack_hierarchy([c[0] for c in cut], mus, skip_A0=True)
         lap0 = torch.cat([s.prim_t["Lap"] * s.mu for s in sys_]).to(tdt)
         level0 = (self.pats["22"][0], (torch.cat([s.pat_dev["22"][1].to(torch.int64)
                                                   + int(self.p2_off[k])
@@ -496,7 +505,7 @@ class MPETBatch:
             if c is not None:
                 ulev[0].update(c)
         # pressure blocks: field-major block-diagonal hierarchies, scale 1
-        plev, pcoarse = pack_hierarchy([(k.plevels, k.pcinv) for k in kry], [1.0] * self.K)
+        plev, pcoarse = pack_hierarchy([c[1] for c in cut], [1.0] * self.K)
         pmap = np.concatenate([self.pd_off[k] + (np.arange(s.F)[None, :] * s.nP1
                                                  + np.arange(s.nP1)[:, None]).reshape(-1)
                                for k, s in enumerate(sys_)])

@@ -368,10 +368,21 @@ coarse_blockdiag_kernel(int n, const int* __restrict__ blk, const int* __restric
   T acc[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) acc[c] = 0;
-  for (int k = lane; k < sz; k += 64) {
-    const T a = row[k];
+  // four row entries (and their b values) in flight per lane and trip, as in
+  // coarse_kernel: blocks are up to a few thousand rows
+  for (int k0 = lane; k0 < sz; k0 += 256) {
+    T a[4], bv[4][NC];
 #pragma unroll
-    for (int c = 0; c < NC; ++c) acc[c] += a * b[NC * (o + k) + c];
+    for (int j = 0; j < 4; ++j) {
+      const int k = k0 + 64 * j;
+      const int kc = k < sz ? k : sz - 1;
+      a[j] = k < sz ? row[kc] : (T)0;
+      load_nc<T, NC>(b + (long long)NC * (o + kc), bv[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int c = 0; c < NC; ++c) acc[c] += a[j] * bv[j][c];
   }
 #pragma unroll
   for (int c = 0; c < NC; ++c) {

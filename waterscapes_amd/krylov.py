@@ -16,7 +16,7 @@ import numpy as np
 import scipy.sparse as sp
 import torch
 
-from . import _lib, amg, forms
+from . import _lib, amg, forms, levels as lv
 from .amg import AmgParams
 from ._lib import check, ptr
 
@@ -268,6 +268,7 @@ class KrylovSolver:
         if not create_handle:        # host hierarchies only (packed by a batch)
             return
         L = _bind()
+        self._cut_levels(1 if pc32 else 0)
         self.prec64 = self._prec_desc(0) if not pc32 else None
         self.prec32 = self._prec_desc(1) if pc32 else None
         use_csr = cfg.use_csr if cfg.use_csr is not None else (cfg.mode == "fp64")
@@ -395,6 +396,16 @@ class KrylovSolver:
         return self.tuning
 
     # -- setup ----------------------------------------------------------------
+    @property
+    def cinv(self):
+        """Coarsest displacement operator as a host array."""
+        return lv.host_array(self._coarse_u)
+
+    @property
+    def pcinv(self):
+        """Coarsest pressure operator as a host array."""
+        return lv.host_array(self._coarse_p)
+
     def _build_hierarchy(self):
         s = self.sys
         rp, ci = s.pat_host["22"]
@@ -412,10 +423,91 @@ class KrylovSolver:
         Le = (keep @ L @ keep + sp.diags(m.astype(np.float64))).tocsr()
         Le.sort_indices()
         P0 = amg.p1_embedding(s.space, self.dir_nodes)
-        self.levels, self.cinv = amg.setup_host(Le.indptr, Le.indices, Le.data,
+        self.levels, self._coarse_u = amg.setup_host(Le.indptr, Le.indices, Le.data,
                                                 self.cfg.amg, P0=P0)
         # level 0 on the device is the un-eliminated Lap (output masked)
         self.level_dev = {}
+
+    # -- compact copies of the FP32 hierarchies --------------------------------
+    def _compact_u0(self):
+        """Half-precision copy of the P2 level of the FP32 hierarchy, or None."""
+        if not hasattr(self, "_cu0"):
+            self._cu0 = compact_level(self.sys.pat_host["22"], self.lap0) \
+                if self.cfg.compact_level0 else None
+            if self._cu0 is not None:
+                self.compact = self._cu0
+        return self._cu0
+
+    def _compact_p(self, l):
+        """Half-precision copy of pressure level l of the FP32 hierarchy, or
+        None (the coarser ones only with the finest).  Half keeps 11 bits
+        down to 2^-14: with the largest value near 2^10, diagonals down to
+        2^-22 of it stay normal.  Dirichlet rows of the finest level
+        (identity rows of the eliminated P_f) are stored as zeros and masked:
+        the pressure residual is zero there."""
+        if not self.cfg.compact_plevel0 or (l > 0 and self._compact_p(0) is None):
+            return None
+        cache = self.__dict__.setdefault("_cp", {})
+        if l not in cache:
+            lev = self._plevels_full[l]
+            v = torch.as_tensor(lev["A_v"]).to(self.sys.device)
+            extra = {}
+            if l == 0:
+                n1, F = self.sys.nP1, self.sys.F
+                dm = self.pmask.view(n1, F).t().contiguous().view(-1)
+                rows = np.repeat(np.arange(lev["n"], dtype=np.int64), np.diff(lev["A_rp"]))
+                v = v.clone()
+                v[dm[torch.as_tensor(rows).to(v.device)].bool()] = 0.0
+                extra["mask0"] = dm
+            c = compact_level((lev["A_rp"], lev["A_ci"]), v, 2.0 ** -22)
+            if c is not None:
+                c.update(extra)
+            cache[l] = c
+        return cache[l]
+
+    def _cut_levels(self, dtype):
+        """Replace the small end of both hierarchies by their dense V-cycle
+        operators (levels.py), made from the values this precision's kernels
+        would read."""
+        s = self.sys
+        size = 8 if dtype == 0 else 4
+        rows = lv.dense_rows(size)
+        self._plevels_full = self.plevels
+
+        def u_values(l):
+            if l > 0:
+                return None
+            c = self._compact_u0() if dtype == 1 else None
+            return (*s.pat_host["22"],
+                    self.lap0 if c is None else c["A_v16"].double() * c["vscale"])
+
+        def p_values(l):
+            # every level but the dense coarsest is compact
+            c = self._compact_p(l) if dtype == 1 and l < len(self._plevels_full) - 1 else None
+            lev = self._plevels_full[l]
+            return None if c is None else (lev["A_rp"], lev["A_ci"],
+                                           c["A_v16"].double() * c["vscale"])
+        self.levels, self._coarse_u = lv.with_dense_tail(
+            self.levels, self._coarse_u, rows, self.cfg.amg, s.device, u_values, self.mask0)
+        pm = self._compact_p(0) if dtype == 1 else None
+        self.plevels, self._coarse_p = lv.with_dense_tail(
+            self.plevels, self._coarse_p, rows, self.cfg.pamg, s.device, p_values,
+            pm["mask0"] if pm is not None else None)
+
+    def dense_tails(self, rows, u_first):
+        """((u levels, u coarse), (p levels, p coarse)) cut at the first level
+        of at most `rows` rows with the levels' own FP64 values, the
+        displacement hierarchy at level u_first or later (1 where the P2
+        level runs on half-precision values).  Kept for the last `rows`."""
+        key = (rows, u_first)
+        if getattr(self, "_tails", (None,))[0] != key:
+            s = self.sys
+            u = lv.with_dense_tail(self.levels, self._coarse_u, rows, self.cfg.amg, s.device,
+                                   lambda l: (*s.pat_host["22"], self.lap0) if l == 0 else None,
+                                   self.mask0, u_first)
+            p = lv.with_dense_tail(self.plevels, self._coarse_p, rows, self.cfg.pamg, s.device)
+            self._tails = (key, (u, p))
+        return self._tails[1]
 
     def _upload_levels(self, levels, cinv, dtype, level0=None):
         """Device copies of a host hierarchy; level0 = (rp, ci, v) device
@@ -445,40 +537,21 @@ class KrylovSolver:
             return self.level_dev[dtype]
         s = self.sys
         lap = self.lap0 if dtype == 0 else self.lap0.to(torch.float32)
-        u = self._upload_levels(self.levels, self.cinv, dtype,
+        u = self._upload_levels(self.levels, self._coarse_u, dtype,
                                 level0=(s.pat_dev["22"][0], s.pat_dev["22"][1], lap))
-        if dtype == 1 and self.cfg.compact_level0:
-            c = compact_level(s.pat_host["22"], self.lap0)
+        p = self._upload_levels(self.plevels, self._coarse_p, dtype)
+        if dtype == 1:
+            c = self._compact_u0()
             if c is not None:
                 u[0][0].update(c)
-                self.compact = c
-        p = self._upload_levels(self.plevels, self.pcinv, dtype)
-        if dtype == 1 and self.cfg.compact_plevel0:
-            # half keeps 11 bits down to 2^-14: with the largest value near
-            # 2^10, diagonals down to 2^-22 of it stay normal
-            # (Dirichlet rows, identity rows of the eliminated P_f, are
-            # stored as zeros and masked: the pressure residual is zero there)
-            lev = self.plevels[0]
-            n1, F = self.sys.nP1, self.sys.F
-            dm = self.pmask.view(n1, F).t().contiguous().view(-1)
-            rows = np.repeat(np.arange(lev["n"], dtype=np.int64), np.diff(lev["A_rp"]))
-            v = torch.as_tensor(lev["A_v"]).to(self.sys.device)
-            v[dm[torch.as_tensor(rows).to(v.device)].bool()] = 0.0
-            c = compact_level((lev["A_rp"], lev["A_ci"]), v, 2.0 ** -22)
+            # the pressure levels but the dense coarsest: their SpMMs read as
+            # many bytes per V-cycle as the finest displacement level's
             self.pcompact_levels = []
-            if c is not None:
-                p[0][0].update(c, mask0=dm)
-                self.pcompact_levels.append(0)
-                # the coarser levels but the dense coarsest: their SpMMs
-                # read as many bytes per V-cycle as the finest level's
-                for l in range(1, len(self.plevels) - 1):
-                    lv = self.plevels[l]
-                    cl = compact_level((lv["A_rp"], lv["A_ci"]),
-                                       torch.as_tensor(lv["A_v"]).to(self.sys.device),
-                                       2.0 ** -22)
-                    if cl is not None:
-                        p[0][l].update(cl)
-                        self.pcompact_levels.append(l)
+            for l in range(max(len(self.plevels) - 1, 1)):
+                c = self._compact_p(l)
+                if c is not None:
+                    p[0][l].update(c)
+                    self.pcompact_levels.append(l)
         self.level_dev[dtype] = (u, p)
         return u, p
 
@@ -507,7 +580,7 @@ class KrylovSolver:
         Pp = sp.block_diag(blocks, format="csr")
         Pp.sort_indices()
         self.Pp_host = Pp
-        self.plevels, self.pcinv = amg.setup_host(Pp.indptr, Pp.indices, Pp.data, self.cfg.pamg)
+        self.plevels, self._coarse_p = amg.setup_host(Pp.indptr, Pp.indices, Pp.data, self.cfg.pamg)
 
     def _hier_desc(self, h, levels, levs, cinv, params, scale, mask0, nc):
         h.nlev = len(levels)
