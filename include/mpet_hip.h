@@ -105,6 +105,19 @@ typedef struct {
                                  0: hardware order */
 } MpetOpDesc;
 
+/* Rows of a matrix in slices of 64 (one row per lane, each slice padded to
+ * its longest row with zero values at offset 0): entry j of lane i of slice s
+ * sits at 64 (off[s] + j) + i; its column is base[s] plus its 16-bit offset,
+ * from dc, or (dc NULL, FP32 hierarchies) from the upper half of a 32-bit
+ * value whose lower half is the value in half precision times 1 / A_vscale.
+ * row[64 s + i] is the lane's row (-1: none; any order); ceil(n / 64) slices. */
+typedef struct {
+  const int32_t* off;
+  const int32_t* base;
+  const int32_t* row;
+  const uint16_t* dc;
+} MpetSlices;
+
 /* One level of the displacement-block hierarchy (device arrays, int32
  * CSR).  Values / dinv in the precision of the owning MpetPrecDesc. */
 typedef struct {
@@ -126,6 +139,26 @@ typedef struct {
   /* Batches (NULL otherwise): instance of each row of this level, so that
    * the V-cycle skips the rows of instances whose solve has stopped. */
   const int32_t* grp;
+  /* Fused transfers (all NULL: residual, restriction and prolongation run
+   * one by one).  With one smoothing step, x = c D^-1 b: W = R - c (R A)
+   * D^-1 (nc x n) and Q = P - c D^-1 (A P) (n x nc, values).  With more:
+   * W = [-R A, R] (nc x 2n, acting on [x; b]) and Q on the pattern of A P
+   * with value pairs ((A P)_ij, P_ij).  Columns and rows held at zero (mask0)
+   * have zero entries.  lgW, lgQ: log2 of the lanes per row (three columns:
+   * at least 2); A_nnz: nonzeros of the level operator. */
+  const int32_t* W_rp;
+  const int32_t* W_ci;
+  const void* W_v;
+  const int32_t* Q_rp;
+  const int32_t* Q_ci;
+  const void* Q_v;
+  int32_t lgW, lgQ;
+  int64_t A_nnz;
+  /* Sliced copies (off NULL: none) of the level operator (values A_sv) and
+   * of Q (then Q_rp / Q_ci may be NULL and Q_v holds the sliced values). */
+  MpetSlices A_s;
+  const void* A_sv;
+  MpetSlices Q_s;
 } MpetAmgLevelDesc;
 
 #define MPET_MAXLEV 16
@@ -535,6 +568,15 @@ int mpet_solver_destroy(void* h);
  * Returns MPET_ERR_NOT_CONVERGED (stats filled) when maxit is reached. */
 int mpet_solver_solve(void* h, const double* b, double* x, MpetSolveStats* stats,
                       hipStream_t stream);
+
+/* Values of the product C = X Y of two CSR matrices (sorted columns, FP64)
+ * on a given pattern: out[k] = sum over the entries j of X's row row[k] of
+ * X_v[j] Y(X_ci[j], col[k]), in the row's order (deterministic).  Forms the
+ * fused transfers' R A and A P from the level values; no counterpart in the
+ * reference. */
+int mpet_product_values(int64_t nnz, const int32_t* row, const int32_t* col, const int32_t* X_rp,
+                        const int32_t* X_ci, const double* X_v, const int32_t* Y_rp,
+                        const int32_t* Y_ci, const double* Y_v, double* out, hipStream_t stream);
 
 /* One SpMM of an AMG level as the V-cycle launches it (the autotuner's
  * timing probe): NC = 1 or 3 node-interleaved columns, mode 0 y = A x,

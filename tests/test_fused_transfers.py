@@ -1,0 +1,141 @@
+"""Fused residual / restriction and prolongation / smoothing of the AMG
+levels (waterscapes_amd/levels.py, csrc/amg_cycle.h).
+
+* CPU: W and Q equal the sparse products they stand for, with Dirichlet rows
+  held at zero and with levels that carry no matrix (FP64 round-off); the
+  sliced copies hold exactly the matrix.
+* GPU: the block preconditioner with the fused transfers equals the numpy
+  restatement's separate steps, in FP64 and FP32, on hierarchies of several
+  sparse levels: one row per lane group to many and one thread per row
+  (sliced), degrees 1 to 3, small and ordinary meshes."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+from test_batch_pack import _laplacian
+
+
+def _host_values(rows, cols, X, Y):
+    import torch
+    nm = max(Y[0].numel() - 1, 1)
+
+    def dense(t, m):
+        return sp.csr_matrix((t[2].numpy(), t[1].numpy(), t[0].numpy()),
+                             shape=(t[0].numel() - 1, m)).toarray()
+    C = dense(X, nm) @ dense(Y, int(cols.max()) + 1)
+    return torch.as_tensor(C[rows.numpy(), cols.numpy()])
+
+
+@pytest.mark.parametrize("degree", [1, 3])
+@pytest.mark.parametrize("masked,empty", [(False, False), (True, False), (False, True)])
+def test_products_equal_scipy(degree, masked, empty):
+    import torch
+    from waterscapes_amd import amg, levels as lv
+    A = _laplacian(5, 0.1)
+    n = A.shape[0]
+    mask = np.zeros(n, dtype=bool)
+    if masked:
+        mask[::6] = True
+        free = sp.diags((~mask).astype(float))
+        A = (free @ A @ free + sp.diags(mask.astype(float))).tocsr()
+        A.sort_indices()
+    lev = amg.setup_host(A.indptr, A.indices, A.data, amg.AmgParams(max_coarse=5))[0][0]
+    P = sp.csr_matrix((lev["P_v"], lev["P_ci"], lev["P_rp"]), shape=(n, lev["nc"]))
+    dinv = lev["dinv"].copy()
+    if empty:                                # a padded level: no matrix, P = I
+        A = sp.csr_matrix((n, n))
+        P = sp.identity(n, format="csr")
+        dinv[:] = 0.0
+    R = P.T.tocsr()
+    R.sort_indices()
+
+    def dev(M):
+        return (torch.as_tensor(M.indptr.astype(np.int32)),
+                torch.as_tensor(M.indices.astype(np.int32)), torch.as_tensor(M.data))
+    c0 = 0.7
+    f = lv.fused_transfers(dev(A), dev(P), dev(R), torch.as_tensor(dinv), degree, c0,
+                           torch.as_tensor(mask) if masked else None, values=_host_values)
+    live = sp.diags((~mask).astype(float))
+    AP, RA = live @ (A @ P), (R @ A) @ live
+    nc = P.shape[1]
+
+    def csr(rp, ci, v, shape):
+        return sp.csr_matrix((v, f[ci].numpy(), f[rp].numpy()), shape=shape).toarray()
+    if degree == 1:
+        W = csr("W_rp", "W_ci", f["W_v"].numpy(), (nc, n))
+        Q = csr("Q_rp", "Q_ci", f["Q_v"].numpy(), (n, nc))
+        assert np.abs(W - ((R @ live) - c0 * RA @ sp.diags(dinv)).toarray()).max() <= 1e-13
+        assert np.abs(Q - (live @ P - c0 * sp.diags(dinv) @ AP).toarray()).max() <= 1e-13
+    else:
+        W = csr("W_rp", "W_ci", f["W_v"].numpy(), (nc, 2 * n))
+        assert np.abs(W - np.hstack([-RA.toarray(), (R @ live).toarray()])).max() <= 1e-13
+        q = f["Q_v"].numpy().reshape(-1, 2)
+        assert np.abs(csr("Q_rp", "Q_ci", q[:, 0], (n, nc)) - AP.toarray()).max() <= 1e-13
+        assert np.abs(csr("Q_rp", "Q_ci", q[:, 1], (n, nc)) - (live @ P).toarray()).max() <= 1e-13
+
+
+@pytest.mark.parametrize("n,m,density", [(1, 5, 0.0), (64, 64, 0.05), (65, 3, 1.0),
+                                         (1000, 400, 0.02), (1537, 65536, 0.01)])
+@pytest.mark.parametrize("pair", [False, True])
+def test_slices_hold_the_matrix(n, m, density, pair):
+    import torch
+    from waterscapes_amd import levels as lv
+    M = sp.random(n, m, density, random_state=1, format="csr")
+    M.sort_indices()
+    v = torch.as_tensor(np.stack([M.data, 2 * M.data], 1) if pair else M.data)
+    s = lv.slices(torch.as_tensor(M.indptr), torch.as_tensor(M.indices), v, n)
+    off, base, row, val = (s[k].numpy() for k in ("off", "base", "row", "v"))
+    dc = lv._u16(s["dc"]).numpy().view(np.uint16)
+    assert len(off) == len(base) + 1 == (n + 63) // 64 + 1 and len(row) == 64 * len(base)
+    assert np.array_equal(np.sort(row[row >= 0]), np.arange(n))
+    assert len(val) == len(dc) == 64 * off[-1]
+    got = np.zeros((n, m))
+    for at in np.flatnonzero(row >= 0):
+        sl = at // 64
+        k = 64 * (off[sl] + np.arange(off[sl + 1] - off[sl])) + at % 64
+        assert len(k) == 0 or (base[sl] + dc[k]).max() < m
+        x = val[k, 1] / 2 if pair else val[k]
+        np.add.at(got[row[at]], base[sl] + dc[k], x)
+    assert np.array_equal(got, M.toarray())
+
+
+def test_slices_refuse_wide_columns():
+    import torch
+    from waterscapes_amd import levels as lv
+    rp, ci = torch.tensor([0, 2]), torch.tensor([0, 1 << 16])
+    assert lv.slices(rp, ci, torch.ones(2), 1) is None
+    assert lv.slices(rp, ci - torch.tensor([0, 1]), torch.ones(2), 1) is not None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sliced", [False, True])
+@pytest.mark.parametrize("n,A,degs", [(3, 1, (1,)), (5, 3, (1,)), (5, 2, (2,)), (6, 6, (3, 1)),
+                                      (27, 1, (1,)), (27, 1, (2,))])
+@pytest.mark.parametrize("mode", ["fp64", "mixed"])
+def test_preconditioner_with_fused_transfers(n, A, degs, mode, sliced, monkeypatch):
+    import torch
+    from test_gpu_solver import _ref_precond, _setup
+    from waterscapes_amd import levels as lv
+    from waterscapes_amd.amg import AmgParams
+    monkeypatch.setattr(lv, "DENSE_TAIL_BYTES", 30 * 30 * 8)
+    monkeypatch.setattr(lv, "SLICE_ROWS", 1 if sliced else 1 << 30)
+    big = dict(max_coarse=25) if n < 20 else {}
+    _, _, dev, solver, dofs, _ = _setup(
+        n=n, A=A, mode=mode, compact_plevel0=False, autotune=False,
+        amg=AmgParams(smoother_degree=3, level_degrees=degs, **big), pamg=AmgParams(**big))
+    assert len(solver.levels) >= 3 and len(solver.plevels) >= 2
+    dev_levels = solver._level_arrays(0 if mode == "fp64" else 1)
+    assert all(("A_s" in ld) == sliced and "W_v" in ld for h in dev_levels for ld in h[0][:-1])
+    r = np.random.default_rng(2).standard_normal(dev.n)
+    r[np.concatenate(dofs)] = 0.0
+    dtype = torch.float64 if mode == "fp64" else torch.float32
+    x = torch.tensor(r, device="cuda", dtype=dtype)
+    z = solver.precond(x, 0 if mode == "fp64" else 1).double().cpu().numpy()
+    again = solver.precond(x, 0 if mode == "fp64" else 1).double().cpu().numpy()
+    assert np.array_equal(z, again)
+    ref = _ref_precond(solver, r, compact=mode == "mixed")
+    tol = 1e-12 if mode == "fp64" else 1e-5
+    nu = dev.nu
+    for a, b in ((z[:nu], ref[:nu]), (z[nu:], ref[nu:])):
+        assert np.linalg.norm(a - b) <= tol * np.linalg.norm(b)
+    solver.close()

@@ -11,8 +11,9 @@ one matrix row:
     kernel per P2 node row in {4, 8, 16} and per P1 node row in {8, 16},
     and its XCD run length (0 or 4);
   * every AMG level of both hierarchies: lanes per row of the level
-    operator (timed as the Chebyshev step), of the prolongator and of the
-    restriction (timed as plain products), powers of two up to 64.
+    operator (timed as the Chebyshev step) unless it runs sliced, and of the
+    fused restriction, or of prolongator and restriction where they are
+    separate (timed as plain products), powers of two up to 64.
 
 Each candidate is timed on the device with HIP events on the current
 stream (the mean of `reps` launches, the best of `repeats` such means), in
@@ -37,6 +38,7 @@ import torch
 
 from . import _lib
 from ._lib import check, ptr
+from .levels import _log2_lanes
 
 ARCH = "gfx950"
 LANES_OP = (8, 16, 32)
@@ -242,11 +244,15 @@ def tune_hierarchy(levels_host, levels_dev, nc, dtype, heuristic, mask0=None, ca
         row = [0, 0, 0]
         mats = [("A", ld["A_rp"], ld["A_ci"], ld["A_v"], n, n)]
         if ncols:
-            mats += [("P", ld["P_rp"], ld["P_ci"], ld["P_v"], n, ncols),
-                     ("R", ld["R_rp"], ld["R_ci"], ld["R_v"], ncols, n)]
-        for j, (which, rp, ci, v, rows, cols) in enumerate(mats):
-            if l == len(levels_host) - 1 and which == "A":
-                continue          # the coarsest level is a dense solve
+            if "W_v" in ld:       # fused transfers: the restriction's product
+                mats += [("W", ld["W_rp"], ld["W_ci"], ld["W_v"], ncols, 2 * n)]
+            else:
+                mats += [("P", ld["P_rp"], ld["P_ci"], ld["P_v"], n, ncols),
+                         ("R", ld["R_rp"], ld["R_ci"], ld["R_v"], ncols, n)]
+        for which, rp, ci, v, rows, cols in mats:
+            j = {"A": 0, "P": 1, "R": 2, "W": 2}[which]
+            if which == "A" and (l == len(levels_host) - 1 or "A_s" in ld):
+                continue          # a dense solve / one thread per row
             compact = which == "A" and "A_v16" in ld
             nnz = int(ci.numel())
             key = level_key(dtype, nc, which, rows, cols, nnz, compact)
@@ -260,7 +266,7 @@ def tune_hierarchy(levels_host, levels_dev, nc, dtype, heuristic, mask0=None, ca
             b = torch.ones(nc * rows, device=device, dtype=tdt) if mode == 3 else None
             d = torch.zeros(nc * rows, device=device, dtype=tdt) if mode == 3 else None
             dinv = ld["dinv"] if mode == 3 else None
-            m0 = mask0 if (l == 0 and which != "R") else None
+            m0 = mask0 if (l == 0 and which in "AP") else None
             v16 = ld.get("A_v16") if compact else None
             dci = ld.get("A_dci") if compact else None
             vs = float(ld.get("vscale", 1.0)) if compact else 1.0
@@ -274,8 +280,11 @@ def tune_hierarchy(levels_host, levels_dev, nc, dtype, heuristic, mask0=None, ca
                     0.5, 0.5, ptr(m0) if m0 is not None else None, lpr,
                     ptr(v16) if v16 is not None else None, ptr(dci) if dci is not None else None,
                     vs, _lib.stream_ptr())), reps, repeats)
-            dflt = int(heuristic(l, which))
+            dflt = int(heuristic(l, which)) if which != "W" else \
+                1 << _log2_lanes(nnz / max(rows, 1), rows, nc)
             cands = _lpr_cands(nc, dflt)
+            if which == "W":
+                cands = tuple(c for c in cands if c >= (4 if nc == 3 else 1))
             if dflt not in cands:
                 cands = cands + (dflt,)
             best, _ = _pick(cands, dflt, timer, margin, cache)

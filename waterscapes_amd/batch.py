@@ -457,6 +457,9 @@ class MPETBatch:
                 nnzp = arrs[0][1].numel()
                 L.lprP = _pick_lpr(nnzp / max(lev["n"], 1), nc, lev["n"])
                 L.lprR = _pick_lpr(nnzp / max(lev["nc"], 1), nc, lev["nc"])
+        lv.add_fused(devs, levels, params, 0 if self.precision == "fp64" else 1, mask0)
+        for l, ld in enumerate(devs):
+            lv.describe_fused(h.lev[l], ld, levels[l]["n"], levels[l]["nc"], nc)
         inv, blk, off, ioff = coarse
         cinv = torch.as_tensor(inv).to(dev, tdt)
         cblk = torch.as_tensor(blk).to(dev)

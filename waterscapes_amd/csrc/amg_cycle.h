@@ -78,6 +78,17 @@ static int grid_for(long long items, int per_block, int cap) {
   return (int)(b < cap ? b : cap);
 }
 
+// Where the finest pressure level's result goes: position r (field-major,
+// r = f nP1 + c) to the vectors' node-interleaved DOF F c + f, or through a
+// map; identity when both are off.
+struct OutMap {
+  int nP1 = 0, F = 0;
+  const int* map = nullptr;        // explicit places (batches)
+  __device__ __forceinline__ long long operator()(int r) const {
+    return map ? map[r] : (F ? (long long)(r % nP1) * F + r / nP1 : r);
+  }
+};
+
 // ---------------------------------------------------------------------------
 // AMG level kernels on NC-column node-interleaved vectors (NC = 3 for the
 // displacement block: one scalar matrix, three components; NC = 1 for the
@@ -99,7 +110,7 @@ spmm_kernel(int nrows, const int* __restrict__ rp, const int* __restrict__ ci,
             const T* __restrict__ val, const T* __restrict__ x, const T* __restrict__ b,
             T* __restrict__ y, const T* __restrict__ dinv, T* d, T cd, T cr,
             const uint8_t* __restrict__ mask, Skip sk, const int* __restrict__ grp,
-            T* y2, const __half* __restrict__ val16 = nullptr,
+            T* y2, OutMap om, const __half* __restrict__ val16 = nullptr,
             const int16_t* __restrict__ dci = nullptr, T vscale = (T)1) {
   // COMPACT: values stored as half precision times 1/vscale, columns as
   // signed 16-bit offsets from the row (half the bytes per nonzero)
@@ -185,7 +196,7 @@ spmm_kernel(int nrows, const int* __restrict__ rp, const int* __restrict__ ci,
   } else {
     T dd = m ? (T)0 : cd * pd + cr * pdinv * (pb - mine);
     if (y2) y2[o] = dd;
-    y[o] = m ? (T)0 : px + dd;
+    y[NC == 1 ? om(r) : o] = m ? (T)0 : px + dd;
   }
 }
 
@@ -252,6 +263,382 @@ spmm_row_kernel(int nrows, const int* __restrict__ rp, const int* __restrict__ c
   }
 }
 
+
+// ---------------------------------------------------------------------------
+// Fused transfers.  With k pre-smoothing steps from zero ending in x and the
+// residual r = b - A x, restriction and residual are one product
+//     R r = R b - (R A) x,
+// and prolongation of the coarse correction e and the first post-smoothing
+// step from x' = x + P e are one product as well,
+//     b - A x' = r - (A P) e:  d = cr D^-1 (r - (A P) e),  x'' = x + P e + d,
+// with R A and A P formed at set-up.  On the P2 level A P has 0.28 of A's
+// nonzeros (7.2 against 25.4 M at 48^3): one of the level's two products with
+// A becomes one with A P, the residual, needed by the post-smoothing only,
+// shares its launch with the restriction, and on every level two launches
+// fewer depend on each other.
+//   one smoothing step (x = c D^-1 b):  W = R - c (R A) D^-1 acts on b alone
+//     and Q = P - c D^-1 (A P) on e alone;
+//   more steps: W = [-R A, R] acts on [x; b] (one buffer), Q holds the pairs
+//     ((A P)_ij, P_ij) on the pattern of A P.
+// Lanes per row are run-time powers of two (2^lg).
+// ---------------------------------------------------------------------------
+template <typename T>
+__device__ __forceinline__ T lanes_allsum(T v, int lanes) {
+  for (int off = lanes >> 1; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+
+// This lane's part of row r of a CSR (or compact) matrix times x, in the
+// order k, k + lanes, ..; four nonzeros in flight as in spmm_kernel.
+template <typename T, int NC, bool COMPACT>
+__device__ __forceinline__ void row_part(const int* __restrict__ rp, const int* __restrict__ ci,
+                                         const T* __restrict__ val,
+                                         const __half* __restrict__ val16,
+                                         const int16_t* __restrict__ dci,
+                                         const T* __restrict__ x, int r, int lane, int lanes,
+                                         T (&acc)[NC]) {
+  constexpr int U = 4;
+  const int kb = rp[r], ke = rp[r + 1];
+  for (int k = kb + lane; k < ke; k += U * lanes) {
+    T a[U];
+    long long cc[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      const int kk = k + j * lanes;
+      const int kc = kk < ke ? kk : ke - 1;
+      T v;
+      if constexpr (COMPACT) {
+        v = (T)__half2float(val16[kc]);
+        cc[j] = (long long)NC * (r + (int)dci[kc]);
+      } else {
+        v = val[kc];
+        cc[j] = (long long)NC * ci[kc];
+      }
+      a[j] = kk < ke ? v : (T)0;
+    }
+    T xv[U][NC];
+#pragma unroll
+    for (int j = 0; j < U; ++j) load_nc<T, NC>(x + cc[j], xv[j]);
+#pragma unroll
+    for (int j = 0; j < U; ++j)
+#pragma unroll
+      for (int c = 0; c < NC; ++c) acc[c] += a[j] * xv[j][c];
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Sliced rows (SELL-64): one thread per row and all NC columns, slices of 64
+// rows padded to their longest.  Rows are ordered by length within windows
+// of 512 (the P2 rows alternate between 65 and 17-29 nonzeros: padding 5%
+// instead of 49%), so a slice's rows stay neighbours: at the k-th nonzero
+// the 64 lanes read 64 nearby columns, where lanes sharing a row read 8
+// scattered ones.  Columns are 16-bit offsets from the slice's smallest.
+// Used where one thread per row fills the chip (65,536 rows, levels.py).
+// ---------------------------------------------------------------------------
+// Runs of 16 consecutive blocks (4,096 rows) go to one XCD, so that its L2
+// serves a run's gathered planes (48^3 iteration 490 against 495 us without).
+constexpr int SELL_CHUNK = 16;
+
+template <typename T>
+struct Sell {
+  const int* off = nullptr;        // first entry of each slice / 64 (nslice + 1)
+  const int* base = nullptr;       // smallest column of each slice
+  const int* row = nullptr;        // row of each (slice, lane), -1: none
+  const uint16_t* dc = nullptr;    // column - base; null for packed values
+  const void* v = nullptr;         // T, pairs of T, or packed: half | offset << 16
+};
+enum SellValues { SELL_PLAIN = 0, SELL_PACKED = 1, SELL_PAIR = 2 };
+
+// Sums of one row: s1 (and s2 of the second values of pairs).
+template <typename T, int NC, int VK>
+__device__ __forceinline__ void sell_part(const Sell<T>& M, int slice, int lane,
+                                          const T* __restrict__ x, T (&s1)[NC], T (&s2)[NC]) {
+  const int o = M.off[slice], w = M.off[slice + 1] - o;
+  const T* __restrict__ xb = x + (long long)NC * M.base[slice];
+  constexpr int U = 8;             // entries in flight (4: 495 against 490 us)
+  auto entry = [&](int j, T& a, T& p, int& c) {
+    const long long k = ((long long)(o + j) << 6) + lane;
+    if constexpr (VK == SELL_PACKED) {
+      const uint32_t q = ((const uint32_t*)M.v)[k];
+      const uint16_t h = (uint16_t)(q & 0xffffu);
+      __half hv;
+      __builtin_memcpy(&hv, &h, 2);
+      a = (T)__half2float(hv);
+      p = (T)0;
+      c = (int)(q >> 16);
+    } else if constexpr (VK == SELL_PAIR) {
+      T v[2];
+      load_nc<T, 2>((const T*)M.v + 2 * k, v);
+      a = v[0];
+      p = v[1];
+      c = M.dc[k];
+    } else {
+      a = ((const T*)M.v)[k];
+      p = (T)0;
+      c = M.dc[k];
+    }
+  };
+  for (int j = 0; j < w; j += U) {          // w is the wave's own: no divergence
+    T a[U], p[U], xv[U][NC];
+    int c[U];
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      const int jj = j + i < w ? j + i : w - 1;
+      entry(jj, a[i], p[i], c[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < U; ++i) load_nc<T, NC>(xb + NC * c[i], xv[i]);
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      const T ai = j + i < w ? a[i] : (T)0;
+      const T pi = j + i < w ? p[i] : (T)0;
+#pragma unroll
+      for (int q = 0; q < NC; ++q) {
+        s1[q] += ai * xv[i][q];
+        if constexpr (VK == SELL_PAIR) s2[q] += pi * xv[i][q];
+      }
+    }
+  }
+}
+
+// Vectors of a sliced kernel's epilogue, by mode:
+//   1: y = b - A x      3: d' = cd d + cr Dinv (b - A x), y = x + d', y2 = d'
+//   6: y = xs + cr Dinv b + A x (post_kernel, one step)
+//   7: d' = cr Dinv (b - A x), y = xs + P x + d', y2 = d' (pairs)
+template <typename T>
+struct SellEpi {
+  const T *b, *xs, *dinv, *d;
+  T cd, cr, vscale;
+  T *y, *y2;
+  const uint8_t* mask;
+  OutMap om;
+  const int* grp;
+};
+
+template <typename T, int NC, int VK, int MODE>
+__device__ __forceinline__ void sell_rows(const Sell<T>& M, int nslice, int slice, int lane,
+                                          const T* __restrict__ x, const SellEpi<T>& E,
+                                          const Skip& sk) {
+  if (slice >= nslice) return;
+  const int r = M.row[slice * 64 + lane];
+  T pb[NC], px[NC], pd[NC];
+  const long long o = (long long)NC * (r < 0 ? 0 : r);
+  load_nc<T, NC>(E.b + o, pb);
+  if constexpr (MODE == 3) load_nc<T, NC>(x + o, px);
+  if constexpr (MODE >= 6) load_nc<T, NC>(E.xs + o, px);
+#pragma unroll
+  for (int q = 0; q < NC; ++q) pd[q] = 0;
+  if constexpr (MODE == 3)
+    if (E.cd != (T)0) load_nc<T, NC>(E.d + o, pd);
+  T di = 0;
+  if constexpr (MODE != 1) di = E.cr * E.dinv[r < 0 ? 0 : r];
+  const bool m = r >= 0 && E.mask && E.mask[r] != 0;
+  T s1[NC], s2[NC];
+#pragma unroll
+  for (int q = 0; q < NC; ++q) { s1[q] = 0; s2[q] = 0; }
+  sell_part<T, NC, VK>(M, slice, lane, x, s1, s2);
+  if (r < 0 || row_skipped(sk, E.grp, r)) return;
+  T out[NC], dd[NC];
+#pragma unroll
+  for (int q = 0; q < NC; ++q) {
+    T t = s1[q];
+    if constexpr (VK == SELL_PACKED) t *= E.vscale;
+    dd[q] = 0;
+    if constexpr (MODE == 1) {
+      out[q] = m ? (T)0 : pb[q] - t;
+    } else if constexpr (MODE == 3) {
+      dd[q] = m ? (T)0 : E.cd * pd[q] + di * (pb[q] - t);
+      out[q] = m ? (T)0 : px[q] + dd[q];
+    } else if constexpr (MODE == 6) {
+      out[q] = m ? (T)0 : px[q] + di * pb[q] + t;
+    } else {
+      dd[q] = m ? (T)0 : di * (pb[q] - t);
+      out[q] = m ? (T)0 : px[q] + s2[q] + dd[q];
+    }
+  }
+  if constexpr (MODE == 3 || MODE == 7)
+    if (E.y2) __builtin_memcpy(E.y2 + o, dd, sizeof(T) * NC);
+  __builtin_memcpy(E.y + (NC == 1 ? E.om(r) : o), out, sizeof(T) * NC);
+}
+
+template <typename T, int NC, int VK, int MODE>
+__global__ void __launch_bounds__(NT)
+sell_kernel(Sell<T> M, int nslice, const T* __restrict__ x, SellEpi<T> E, Skip sk) {
+  if (sk.all && *sk.all) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tile = xcd_tile(blockIdx.x, gridDim.x, SELL_CHUNK);
+  sell_rows<T, NC, VK, MODE>(M, nslice, tile * (NT / 64) + wave, threadIdx.x & 63, x, E, sk);
+}
+
+// Arguments of the two halves of transfer_kernel.
+template <typename T>
+struct DownArgs {           // bc = W v; with dinv: d = y2 = cr Dinv bc (the coarse
+  int n, lg;                // level's first Chebyshev step)
+  const int *rp, *ci;
+  const T *val, *v;
+  T* bc;
+  const T* dinv;
+  T cr;
+  T *d, *y2;
+  const int* grp;
+};
+template <typename T>
+struct ResArgs {            // r = b - A x, rows with mask 0
+  int n, lg;
+  const int *rp, *ci;
+  const T* val;
+  const __half* val16;
+  const int16_t* dci;
+  T vscale;
+  const T *x, *b;
+  T* r;
+  const uint8_t* mask;
+  const int* grp;
+};
+
+// One row group of the restriction half.
+template <typename T, int NC>
+__device__ __forceinline__ void down_rows(const DownArgs<T>& w, const Skip& sk) {
+  T acc[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) acc[c] = 0;
+  const long long gid = (long long)blockIdx.x * NT + threadIdx.x;
+  const int r = (int)(gid >> w.lg), lanes = 1 << w.lg;
+  const int lane = (int)(gid & (lanes - 1));
+  if (r >= w.n || row_skipped(sk, w.grp, r)) return;     // whole row groups leave
+  const T di = w.dinv ? w.cr * w.dinv[r] : (T)0;
+  row_part<T, NC, false>(w.rp, w.ci, w.val, nullptr, nullptr, w.v, r, lane, lanes, acc);
+  T mine = 0;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const T v = lanes_allsum(acc[c], lanes);
+    if (lane == c) mine = v;
+  }
+  if (lane >= NC) return;
+  const long long o = (long long)NC * r + lane;
+  w.bc[o] = mine;
+  if (w.dinv) {
+    w.d[o] = di * mine;
+    w.y2[o] = di * mine;
+  }
+}
+
+// Blocks [0, nbw) form the coarse right-hand side, the rest the residual:
+// both read only x and b, so one launch holds both (a launch of its own
+// costs 4-5 us, more than the rows of every level but the finest).
+template <typename T, int NC, bool COMPACT>
+__global__ void __launch_bounds__(NT)
+transfer_kernel(DownArgs<T> w, ResArgs<T> a, int nbw, Skip sk) {
+  if (sk.all && *sk.all) return;
+  if ((int)blockIdx.x < nbw) {
+    down_rows<T, NC>(w, sk);
+    return;
+  }
+  T acc[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) acc[c] = 0;
+  const long long gid = (long long)((int)blockIdx.x - nbw) * NT + threadIdx.x;
+  const int r = (int)(gid >> a.lg), lanes = 1 << a.lg;
+  const int lane = (int)(gid & (lanes - 1));
+  if (r >= a.n || row_skipped(sk, a.grp, r)) return;
+  const long long o = (long long)NC * r + (lane < NC ? lane : NC - 1);
+  const T pb = a.b[o];
+  const int m = a.mask ? (int)a.mask[r] : 0;
+  row_part<T, NC, COMPACT>(a.rp, a.ci, a.val, a.val16, a.dci, a.x, r, lane, lanes, acc);
+  T mine = 0;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const T v = lanes_allsum(acc[c], lanes);
+    if (lane == c) mine = v;
+  }
+  if (lane >= NC) return;
+  if constexpr (COMPACT) mine *= a.vscale;
+  a.r[o] = m ? (T)0 : pb - mine;
+}
+
+// The same with the residual's rows sliced.
+template <typename T, int NC, int VK>
+__global__ void __launch_bounds__(NT)
+transfer_sell_kernel(DownArgs<T> w, Sell<T> M, int nslice, const T* __restrict__ x,
+                     SellEpi<T> E, int nbw, Skip sk) {
+  if (sk.all && *sk.all) return;
+  if ((int)blockIdx.x < nbw) {
+    down_rows<T, NC>(w, sk);
+    return;
+  }
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tile = xcd_tile((int)blockIdx.x - nbw, (int)gridDim.x - nbw, SELL_CHUNK);
+  sell_rows<T, NC, VK, 1>(M, nslice, tile * (NT / 64) + wave, threadIdx.x & 63, x, E, sk);
+}
+
+// Prolongation with the first post-smoothing step.  One step in all
+// (PAIR false): y = x + cr Dinv r + Q e.  More (PAIR): d = cr Dinv (r -
+// (A P) e), y = x + P e + d; d is stored for the next step.
+template <typename T, int NC, bool PAIR>
+__global__ void __launch_bounds__(NT)
+post_kernel(int n, int lg, const int* __restrict__ rp, const int* __restrict__ ci,
+            const T* __restrict__ val, const T* __restrict__ e, const T* x, const T* r_,
+            const T* __restrict__ dinv, T cr, T* y, T* d, const uint8_t* __restrict__ mask,
+            OutMap om, Skip sk, const int* __restrict__ grp) {
+  if (sk.all && *sk.all) return;
+  const long long gid = (long long)blockIdx.x * NT + threadIdx.x;
+  const int r = (int)(gid >> lg), lanes = 1 << lg;
+  const int lane = (int)(gid & (lanes - 1));
+  if (r >= n || row_skipped(sk, grp, r)) return;
+  const long long o = (long long)NC * r + (lane < NC ? lane : NC - 1);
+  const T px = x[o], pr = r_[o], di = cr * dinv[r];
+  const int m = mask ? (int)mask[r] : 0;
+  constexpr int U = 4;
+  const int kb = rp[r], ke = rp[r + 1];
+  T s1[NC], s2[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) { s1[c] = 0; s2[c] = 0; }
+  for (int k = kb + lane; k < ke; k += U * lanes) {
+    T a[U], p[U];
+    long long cc[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      const int kk = k + j * lanes;
+      const int kc = kk < ke ? kk : ke - 1;
+      T v[2];
+      if constexpr (PAIR) load_nc<T, 2>(val + 2ll * kc, v);
+      else { v[0] = val[kc]; v[1] = 0; }
+      cc[j] = (long long)NC * ci[kc];
+      a[j] = kk < ke ? v[0] : (T)0;
+      p[j] = kk < ke ? v[1] : (T)0;
+    }
+    T xv[U][NC];
+#pragma unroll
+    for (int j = 0; j < U; ++j) load_nc<T, NC>(e + cc[j], xv[j]);
+#pragma unroll
+    for (int j = 0; j < U; ++j)
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        s1[c] += a[j] * xv[j][c];
+        if constexpr (PAIR) s2[c] += p[j] * xv[j][c];
+      }
+  }
+  T m1 = 0, m2 = 0;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const T v = lanes_allsum(s1[c], lanes);
+    if (lane == c) m1 = v;
+    if constexpr (PAIR) {
+      const T u = lanes_allsum(s2[c], lanes);
+      if (lane == c) m2 = u;
+    }
+  }
+  if (lane >= NC) return;
+  const long long oo = NC == 1 ? om(r) : o;
+  if constexpr (PAIR) {
+    const T dd = m ? (T)0 : di * (pr - m1);
+    if (d) d[o] = dd;
+    y[oo] = m ? (T)0 : px + m2 + dd;
+  } else {
+    y[oo] = m ? (T)0 : px + di * pr + m1;
+  }
+}
+
 // A MINRES vector update fused into the first kernels of a preconditioner
 // apply that read its input (off when y is null): the input entry i is
 // r[i] = y[i] - (alfa / beta) r2o[i], computed where it is first read and
@@ -292,12 +679,14 @@ cheb0_kernel(int nrows, const T* b, T scale, const T* __restrict__ dinv, T cr,
   y[i] = v;
 }
 
-// Dense coarsest solve x = Cinv b (NC columns), one wave per row; each lane
-// keeps four row entries (and their b values) in flight per trip.
+// Dense coarsest solve x = Cinv (scale b) (NC columns), one wave per row;
+// each lane keeps four row entries (and their b values) in flight per trip.
+// b and x may lie in the vectors' own order (om); with k2 on, b's entries
+// are made by it, and each row's wave stores its own.
 template <typename T, int NC>
 __global__ void __launch_bounds__(NT)
-coarse_kernel(int n, const T* __restrict__ cinv, const T* __restrict__ b, T* __restrict__ x,
-              const int* __restrict__ skip) {
+coarse_kernel(int n, const T* __restrict__ cinv, const T* b, T* __restrict__ x,
+              const int* __restrict__ skip, T scale, OutMap om, K2In<T> k2) {
   if (skip && *skip) return;
   const int r = blockIdx.x * (NT / 64) + threadIdx.x / 64;
   const int lane = threadIdx.x % 64;
@@ -306,6 +695,7 @@ coarse_kernel(int n, const T* __restrict__ cinv, const T* __restrict__ b, T* __r
 #pragma unroll
   for (int c = 0; c < NC; ++c) acc[c] = 0;
   const T* __restrict__ row = cinv + (long long)r * n;
+  const T kc2 = k2.y ? (T)(*k2.alfa / *k2.beta) : (T)0;
   for (int k0 = lane; k0 < n; k0 += 256) {
     T a[4], bv[4][NC];
 #pragma unroll
@@ -313,42 +703,51 @@ coarse_kernel(int n, const T* __restrict__ cinv, const T* __restrict__ b, T* __r
       const int k = k0 + 64 * j;
       const int kc = k < n ? k : n - 1;
       a[j] = k < n ? row[kc] : (T)0;
-      load_nc<T, NC>(b + NC * kc, bv[j]);
+      const long long o = NC == 1 ? om(kc) : (long long)NC * kc;
+      if (k2.y) {
+        T yv[NC], rv[NC];
+        load_nc<T, NC>(k2.y + o, yv);
+        load_nc<T, NC>(k2.r2o + o, rv);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) bv[j][c] = yv[c] - kc2 * rv[c];
+      } else {
+        load_nc<T, NC>(b + o, bv[j]);
+      }
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int c = 0; c < NC; ++c) acc[c] += a[j] * bv[j][c];
   }
+  const long long o = NC == 1 ? om(r) : (long long)NC * r;
+  if (k2.y && lane < NC) k2.make(o + lane);
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     T v = group_allsum<64>(acc[c]);
-    if (lane == c) x[NC * r + c] = v;
+    if (lane == c) x[o + c] = scale * v;
   }
 }
 
-// Pressure vectors: node-interleaved [c][F] <-> field-major [f][c].
+// The gather with the first Chebyshev step of the finest pressure level from
+// zero: b = the gathered entry, x = cr Dinv b (and the direction d when
+// given), each at the entry's place in the hierarchy (field-major, or map).
 template <typename T>
 __global__ void __launch_bounds__(NT)
-p_gather_kernel(int nP1, int F, const T* src, T* __restrict__ dst,
-                const int* __restrict__ skip, K2In<T> k2 = K2In<T>()) {
-  if (skip && *skip) return;
-  long long i = (long long)blockIdx.x * NT + threadIdx.x;
-  if (i >= (long long)F * nP1) return;
-  int c = (int)(i / F), f = (int)(i % F);
-  dst[(long long)f * nP1 + c] = k2.y ? k2.make(i) : src[i];
+p_enter_kernel(long long np, int nP1, int F, const int* __restrict__ map, const T* src,
+               T* __restrict__ b, const T* __restrict__ dinv, T cr, T* __restrict__ d,
+               T* __restrict__ x, const uint8_t* __restrict__ mask, Skip sk,
+               const int* __restrict__ grp, K2In<T> k2) {
+  if (sk.all && *sk.all) return;
+  const long long i = (long long)blockIdx.x * NT + threadIdx.x;
+  if (i >= np) return;
+  const int q = map ? map[i] : (int)((i % F) * nP1 + i / F);
+  if (row_skipped(sk, grp, q)) return;
+  const T bv = k2.y ? k2.make(i) : src[i];
+  b[q] = bv;
+  const T v = (mask && mask[q]) ? (T)0 : cr * dinv[q] * bv;
+  if (d) d[q] = v;
+  x[q] = v;
 }
-template <typename T>
-__global__ void __launch_bounds__(NT)
-p_scatter_kernel(int nP1, int F, const T* __restrict__ src, T* __restrict__ dst,
-                 const int* __restrict__ skip) {
-  if (skip && *skip) return;
-  long long i = (long long)blockIdx.x * NT + threadIdx.x;
-  if (i >= (long long)F * nP1) return;
-  int c = (int)(i / F), f = (int)(i % F);
-  dst[i] = src[(long long)f * nP1 + c];
-}
-
 // Block-diagonal dense coarsest solve (many independent instances): row r
 // lies in block blk[r] spanning rows off[b] .. off[b+1]-1, whose dense
 // inverse is stored row-major at inv + ioff[b].
@@ -389,6 +788,15 @@ coarse_blockdiag_kernel(int n, const int* __restrict__ blk, const int* __restric
     T v = group_allsum<64>(acc[c]);
     if (lane == c) x[NC * r + c] = v;
   }
+}
+
+// inv[map[i]] = i (map a permutation of 0 .. n - 1).  A template, so that the
+// translation units including this header share one instance.
+template <typename I>
+__global__ void __launch_bounds__(NT)
+invert_map_kernel_t(int n, const I* __restrict__ map, I* __restrict__ inv) {
+  const int i = blockIdx.x * NT + threadIdx.x;
+  if (i < n) inv[map[i]] = i;
 }
 
 // Pressure vectors through an explicit map: dst[map[i]] = src[i] (gather
@@ -457,6 +865,14 @@ struct LevelDev {
   int deg = 2;                     // Chebyshev degree of this level's smoother
   double cd[MAXDEG], cr[MAXDEG];
   int lpr = 8, lprP = 4, lprR = 8;
+  // fused transfers (transfer_kernel, post_kernel; null: the separate ones),
+  // log2 lanes per row
+  const int *Wrp = nullptr, *Wci = nullptr, *Qrp = nullptr, *Qci = nullptr;
+  const T *Wv = nullptr, *Qv = nullptr;
+  int lgW = 3, lgQ = 2;
+  long long nnz = 0;               // of the level operator
+  // sliced copies of the level operator and of Q (off null: none)
+  Sell<T> As, Qs;
   T *B = nullptr, *X = nullptr, *R = nullptr, *E = nullptr, *S1 = nullptr, *S2 = nullptr,
     *D = nullptr;
 };
@@ -479,7 +895,7 @@ struct Precond {
   int nP1 = 0, F = 0;
   long long nu = 0;
   const int* pmap = nullptr;           // explicit pressure order (batches)
-  T *pin = nullptr, *pout = nullptr;   // field-major pressure buffers
+  int* pinv = nullptr;                 // its inverse
   // optional second stream: the pressure V-cycle runs beside the
   // displacement one (fork / join through the two events; inside a captured
   // graph these become parallel branches)
@@ -509,7 +925,8 @@ static void free_fork(Precond<T>& P) {
 
 template <typename T, int NC, int MODE>
 static void spmm(const LevelDev<T>& L, int which, const T* x, const T* b, T* y, T* d, T cd,
-                 T cr, Skip sk, hipStream_t s, const T* dinv = nullptr, T* y2 = nullptr) {
+                 T cr, Skip sk, hipStream_t s, const T* dinv = nullptr, T* y2 = nullptr,
+                 OutMap om = OutMap()) {
   // which: 0 level operator, 1 prolongator (rows n), 2 restriction (rows nc);
   // dinv: the diagonal inverse used by the epilogue (default the level's)
   int nrows = which == 2 ? L.nc : L.n;
@@ -517,6 +934,20 @@ static void spmm(const LevelDev<T>& L, int which, const T* x, const T* b, T* y, 
   const int* ci = which == 0 ? L.ci : (which == 1 ? L.Pci : L.Rci);
   const T* v = which == 0 ? L.v : (which == 1 ? L.Pv : L.Rv);
   int lpr = which == 0 ? L.lpr : (which == 1 ? L.lprP : L.lprR);
+  if constexpr (MODE == 1 || MODE == 3) {
+    if (which == 0 && L.As.off) {
+      const int ns = (nrows + 63) / 64, nb = (ns + NT / 64 - 1) / (NT / 64);
+      const SellEpi<T> E{b, nullptr, dinv ? dinv : L.dinv, d, cd, cr, (T)L.vscale, y, y2, L.mask,
+                         om, L.grp};
+      if (L.As.dc)
+        hipLaunchKernelGGL((sell_kernel<T, NC, SELL_PLAIN, MODE>), dim3(nb), dim3(NT), 0, s,
+                           L.As, ns, x, E, sk);
+      else if constexpr (sizeof(T) == 4)
+        hipLaunchKernelGGL((sell_kernel<T, NC, SELL_PACKED, MODE>), dim3(nb), dim3(NT), 0, s,
+                           L.As, ns, x, E, sk);
+      return;
+    }
+  }
   const bool compact = which == 0 && L.v16;
   if (NC > 1 && lpr == 1 && !compact) {     // one thread per row, all columns
     const int blocks1 = (nrows + NT - 1) / NT;
@@ -539,14 +970,14 @@ static void spmm(const LevelDev<T>& L, int which, const T* x, const T* b, T* y, 
   case LP:                                                                                     \
     hipLaunchKernelGGL((spmm_kernel<T, NC, (LP < NC ? 4 : LP), MODE, true>), dim3(blocks),     \
                        dim3(NT), 0, s, nrows, rp, ci, v, x, b, y, dinv, d, cd, cr, mask, sk, grp, \
-                       y2, L.v16, L.dci, (T)L.vscale);                                         \
+                       y2, om, L.v16, L.dci, (T)L.vscale);                                     \
     break;
       switch (lpr) {
         SPMM_CASE(4) SPMM_CASE(8) SPMM_CASE(16) SPMM_CASE(32) SPMM_CASE(64)
         default: hipLaunchKernelGGL((spmm_kernel<T, NC, (NC > 4 ? 8 : 4), MODE, true>),
                                     dim3((unsigned)(((long long)nrows * (NC > 4 ? 8 : 4) + NT - 1) / NT)),
                                     dim3(NT), 0, s, nrows, rp, ci, v, x, b, y, dinv, d, cd, cr,
-                                    mask, sk, grp, y2, L.v16, L.dci, (T)L.vscale);
+                                    mask, sk, grp, y2, om, L.v16, L.dci, (T)L.vscale);
       }
 #undef SPMM_CASE
       return;
@@ -555,7 +986,7 @@ static void spmm(const LevelDev<T>& L, int which, const T* x, const T* b, T* y, 
 #define SPMM_CASE(LP)                                                                          \
   case LP:                                                                                     \
     hipLaunchKernelGGL((spmm_kernel<T, NC, (LP < NC ? 4 : LP), MODE>), dim3(blocks), dim3(NT), \
-                       0, s, nrows, rp, ci, v, x, b, y, dinv, d, cd, cr, mask, sk, grp, y2);  \
+                       0, s, nrows, rp, ci, v, x, b, y, dinv, d, cd, cr, mask, sk, grp, y2, om);  \
     break;
   switch (lpr) {
     SPMM_CASE(1) SPMM_CASE(2) SPMM_CASE(4) SPMM_CASE(8) SPMM_CASE(16) SPMM_CASE(32)
@@ -572,70 +1003,154 @@ static T* first_dst(const LevelDev<T>& L, T* out) {
   return L.deg == 1 ? out : L.S1;
 }
 
-// k Chebyshev steps on level l; from zero (x0 == nullptr, b scaled by
-// bscale and copied to bcopy when given; entered: the first step is already
-// in first_dst, made by the restriction) or from x0; result in out.
+// Chebyshev steps i0 .. of level L from cur, the last one into out (through
+// om); the direction of step i0 - 1 is in L.D when i0 > 0.
 template <typename T, int NC>
-static void smooth(const Hier<T>& H, int l, const T* b, T bscale, T* bcopy, const T* x0,
-                   T* out, Skip sk, hipStream_t s, bool entered = false,
-                   K2In<T> k2 = K2In<T>()) {
-  const LevelDev<T>& L = H.lev[l];
-  const int k = L.deg;
-  const T* cur = x0;
-  int i = 0;
+static void smooth_steps(const LevelDev<T>& L, const T* b, const T* cur, int i0, T* out,
+                         Skip sk, hipStream_t s, OutMap om = OutMap()) {
   T* bufs[2] = {L.S1, L.S2};
-  int flip = 0;
-  const T* bb = b;
-  if (!x0) {
-    T* dst = first_dst(L, out);
-    int blocks = (int)(((long long)NC * L.n + NT - 1) / NT);
-    if (!entered)
-      hipLaunchKernelGGL((cheb0_kernel<T, NC>), dim3(blocks), dim3(NT), 0, s, L.n, b, bscale,
-                         L.dinv, (T)L.cr[0], k == 1 ? nullptr : L.D, dst, bcopy, L.mask, sk,
-                         L.grp, k2);
-    if (bcopy) bb = bcopy;
-    cur = dst;
-    i = 1;
-    flip ^= 1;
-  }
-  for (; i < k; ++i) {
-    T* dst = (i == k - 1) ? out : bufs[flip];
+  int flip = i0 & 1;
+  for (int i = i0; i < L.deg; ++i) {
+    const bool last = i == L.deg - 1;
+    T* dst = last ? out : bufs[flip];
     if (dst == cur) dst = bufs[flip ^ 1];
     // the last step's direction is not needed again
-    spmm<T, NC, 3>(L, 0, cur, bb, dst, L.D, (T)L.cd[i], (T)L.cr[i], sk, s, nullptr,
-                   i == k - 1 ? nullptr : L.D);
+    spmm<T, NC, 3>(L, 0, cur, b, dst, L.D, (T)L.cd[i], (T)L.cr[i], sk, s, nullptr,
+                   last ? nullptr : L.D, last ? om : OutMap());
     cur = dst;
     flip ^= 1;
   }
 }
 
+// Pre-smoothing from zero of level l into L.X; b scaled by bscale and
+// copied to bcopy when given; entered: the first step is already in
+// first_dst (made by the restriction or the pressure gather).
 template <typename T, int NC>
-static void vcycle(const Hier<T>& H, int l, const T* b, T bscale, T* out, Skip sk,
-                   hipStream_t s, bool entered = false, K2In<T> k2 = K2In<T>()) {
-  // k2 (a fused input update) only on a level with a smoother
+static void smooth_from_zero(const LevelDev<T>& L, const T* b, T bscale, T* bcopy, Skip sk,
+                             hipStream_t s, bool entered, K2In<T> k2) {
+  T* dst = first_dst(L, L.X);
+  const int blocks = (int)(((long long)NC * L.n + NT - 1) / NT);
+  if (!entered)
+    hipLaunchKernelGGL((cheb0_kernel<T, NC>), dim3(blocks), dim3(NT), 0, s, L.n, b, bscale,
+                       L.dinv, (T)L.cr[0], L.deg == 1 ? nullptr : L.D, dst, bcopy, L.mask, sk,
+                       L.grp, k2);
+  smooth_steps<T, NC>(L, bcopy ? bcopy : b, dst, 1, L.X, sk, s);
+}
+
+// Fused restriction (into level l + 1's right-hand side and first step) and
+// residual of level l after its pre-smoothing, one launch (res false: the
+// restriction alone).
+template <typename T, int NC>
+static void fused_down(const Hier<T>& H, int l, const T* b, Skip sk, hipStream_t s,
+                       bool res = true) {
   const LevelDev<T>& L = H.lev[l];
-  if (l == H.nlev - 1) {
-    const T* bb = b;
-    if (bscale != (T)1) {   // single-level hierarchy: scale into L.B first
-      int blocks = (int)(((long long)NC * L.n + NT - 1) / NT);
-      hipLaunchKernelGGL((cheb0_kernel<T, NC>), dim3(blocks), dim3(NT), 0, s, L.n, b, bscale,
-                         L.dinv, (T)0, L.D, L.X, L.B, L.mask, sk, L.grp);
-      bb = L.B;
-    }
-    int blocks = (L.n + NT / 64 - 1) / (NT / 64);
-    if (H.cblk)
-      hipLaunchKernelGGL((coarse_blockdiag_kernel<T, NC>), dim3(blocks), dim3(NT), 0, s, L.n,
-                         H.cblk, H.coff, H.cioff, H.cinv, bb, out, sk, L.grp);
-    else
-      hipLaunchKernelGGL((coarse_kernel<T, NC>), dim3(blocks), dim3(NT), 0, s, L.n, H.cinv, bb,
-                         out, sk.all);
+  const LevelDev<T>& C = H.lev[l + 1];
+  const bool enter = l + 1 < H.nlev - 1;
+  const DownArgs<T> w{L.nc, L.lgW, L.Wrp, L.Wci, L.Wv, L.deg == 1 ? b : L.X, C.B,
+                      enter ? C.dinv : nullptr, (T)C.cr[0], C.D,
+                      enter ? first_dst(C, C.X) : nullptr, L.grpc};
+  int lgA = 0;
+  while ((1 << lgA) < L.lpr) ++lgA;
+  if (NC == 3 && lgA < 2) lgA = 2;
+  const ResArgs<T> a{L.n, lgA, L.rp, L.ci, L.v, L.v16, L.dci, (T)L.vscale, L.X, b, L.R,
+                     L.mask, L.grp};
+  const int nbw = (int)((((long long)L.nc << L.lgW) + NT - 1) / NT);
+  const int nba = (int)((((long long)L.n << lgA) + NT - 1) / NT);
+  if (res && L.As.off) {
+    const int ns = (L.n + 63) / 64, nbs = (ns + NT / 64 - 1) / (NT / 64);
+    const SellEpi<T> E{b, nullptr, nullptr, nullptr, 0, 0, (T)L.vscale, L.R, nullptr, L.mask,
+                       OutMap(), L.grp};
+    if (L.As.dc)
+      hipLaunchKernelGGL((transfer_sell_kernel<T, NC, SELL_PLAIN>), dim3(nbw + nbs), dim3(NT),
+                         0, s, w, L.As, ns, (const T*)L.X, E, nbw, sk);
+    else if constexpr (sizeof(T) == 4)
+      hipLaunchKernelGGL((transfer_sell_kernel<T, NC, SELL_PACKED>), dim3(nbw + nbs), dim3(NT),
+                         0, s, w, L.As, ns, (const T*)L.X, E, nbw, sk);
     return;
   }
-  T* bcopy = (bscale != (T)1) ? L.B : nullptr;
-  smooth<T, NC>(H, l, b, bscale, bcopy, nullptr, L.X, sk, s, entered, k2);
+  const dim3 grid(nbw + (res ? nba : 0));
+  if constexpr (sizeof(T) == 4) {
+    if (L.v16) {
+      hipLaunchKernelGGL((transfer_kernel<T, NC, true>), grid, dim3(NT), 0, s, w, a, nbw, sk);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((transfer_kernel<T, NC, false>), grid, dim3(NT), 0, s, w, a, nbw, sk);
+}
+
+// Prolongation of C.E with level l's post-smoothing into out.
+template <typename T, int NC>
+static void fused_up(const Hier<T>& H, int l, const T* b, T* out, Skip sk,
+                     hipStream_t s, OutMap om) {
+  const LevelDev<T>& L = H.lev[l];
+  const T* e = H.lev[l + 1].E;
+  const bool one = L.deg == 1;
+  T* dst = one ? out : L.S1;
+  const OutMap dm = one ? om : OutMap();
+  if (L.Qs.off) {
+    const int ns = (L.n + 63) / 64, nb = (ns + NT / 64 - 1) / (NT / 64);
+    const SellEpi<T> E{L.R, L.X, L.dinv, nullptr, 0, (T)L.cr[0], (T)1, dst, one ? nullptr : L.D,
+                       L.mask, dm, L.grp};
+    if (one)
+      hipLaunchKernelGGL((sell_kernel<T, NC, SELL_PLAIN, 6>), dim3(nb), dim3(NT), 0, s, L.Qs, ns,
+                         e, E, sk);
+    else
+      hipLaunchKernelGGL((sell_kernel<T, NC, SELL_PAIR, 7>), dim3(nb), dim3(NT), 0, s, L.Qs, ns,
+                         e, E, sk);
+  } else {
+    const int blocks = (int)((((long long)L.n << L.lgQ) + NT - 1) / NT);
+    if (one)
+      hipLaunchKernelGGL((post_kernel<T, NC, false>), dim3(blocks), dim3(NT), 0, s, L.n, L.lgQ,
+                         L.Qrp, L.Qci, L.Qv, e, (const T*)L.X, (const T*)L.R, L.dinv,
+                         (T)L.cr[0], dst, (T*)nullptr, L.mask, dm, sk, L.grp);
+    else
+      hipLaunchKernelGGL((post_kernel<T, NC, true>), dim3(blocks), dim3(NT), 0, s, L.n, L.lgQ,
+                         L.Qrp, L.Qci, L.Qv, e, (const T*)L.X, (const T*)L.R, L.dinv,
+                         (T)L.cr[0], dst, L.D, L.mask, dm, sk, L.grp);
+  }
+  if (!one) smooth_steps<T, NC>(L, b, L.S1, 1, out, sk, s, om);
+}
+
+// Copy of a level's right-hand side: where it is scaled, and where the fused
+// restriction reads [x; b] as one buffer.
+template <typename T>
+static T* vcycle_bcopy(const LevelDev<T>& L, const T* b, T bscale) {
+  const bool stacked = L.Wv && L.deg > 1;
+  return (bscale != (T)1 || (stacked && b != L.B)) ? L.B : nullptr;
+}
+
+template <typename T, int NC>
+static void vcycle(const Hier<T>& H, int l, const T* b, T bscale, T* out, Skip sk,
+                   hipStream_t s, bool entered = false, K2In<T> k2 = K2In<T>(),
+                   OutMap om = OutMap()) {
+  const LevelDev<T>& L = H.lev[l];
+  if (l == H.nlev - 1) {
+    const int blocks = (L.n + NT / 64 - 1) / (NT / 64);
+    if (H.cblk && bscale != (T)1) {  // scale into L.B first
+      hipLaunchKernelGGL((cheb0_kernel<T, NC>), dim3((int)(((long long)NC * L.n + NT - 1) / NT)),
+                         dim3(NT), 0, s, L.n, b, bscale, L.dinv, (T)0, L.D, L.X, L.B, L.mask, sk,
+                         L.grp);
+      b = L.B;
+    }
+    if (H.cblk)
+      hipLaunchKernelGGL((coarse_blockdiag_kernel<T, NC>), dim3(blocks), dim3(NT), 0, s, L.n,
+                         H.cblk, H.coff, H.cioff, H.cinv, b, out, sk, L.grp);
+    else
+      hipLaunchKernelGGL((coarse_kernel<T, NC>), dim3(blocks), dim3(NT), 0, s, L.n, H.cinv, b,
+                         out, sk.all, bscale, om, k2);
+    return;
+  }
+  T* bcopy = vcycle_bcopy(L, b, bscale);
+  smooth_from_zero<T, NC>(L, b, bscale, bcopy, sk, s, entered, k2);
   const T* bb = bcopy ? bcopy : b;
-  spmm<T, NC, 1>(L, 0, L.X, bb, L.R, nullptr, 0, 0, sk, s);
   const LevelDev<T>& C = H.lev[l + 1];
+  if (L.Wv) {
+    fused_down<T, NC>(H, l, bb, sk, s);
+    vcycle<T, NC>(H, l + 1, C.B, (T)1, C.E, sk, s, l + 1 < H.nlev - 1);
+    fused_up<T, NC>(H, l, bb, out, sk, s, om);
+    return;
+  }
+  spmm<T, NC, 1>(L, 0, L.X, bb, L.R, nullptr, 0, 0, sk, s);
   if (l + 1 < H.nlev - 1) {
     // restriction fused with the coarse level's first smoothing step (its
     // pre-smoothing writes to C.X)
@@ -647,53 +1162,87 @@ static void vcycle(const Hier<T>& H, int l, const T* b, T bscale, T* out, Skip s
     vcycle<T, NC>(H, l + 1, C.B, (T)1, C.E, sk, s);
   }
   spmm<T, NC, 2>(L, 1, C.E, nullptr, L.X, nullptr, 0, 0, sk, s);
-  smooth<T, NC>(H, l, bb, (T)1, nullptr, L.X, out, sk, s);
+  smooth_steps<T, NC>(L, bb, L.X, 0, out, sk, s, om);
 }
 
-// Whether precond_apply can take a fused input update (k2): the first
-// kernels reading the input are the displacement level-0 smoother and the
-// pressure gather.
+// Whether precond_apply can take a fused input update (k2): single
+// instances, whose first kernels read the input directly.
 template <typename T>
 static bool k2_fusable(const Precond<T>& P) {
-  return P.u.nlev > 1 && !P.pmap;
+  return !P.pmap;
 }
+
+// Pressure block of precond_apply on stream s.
+template <typename T>
+static void precond_pressure(const Precond<T>& P, const T* r, T* z, Skip sk, hipStream_t s,
+                             K2In<T> k2) {
+  const long long np = (long long)P.F * P.nP1;
+  const int eb = (int)((np + NT - 1) / NT);
+  const LevelDev<T>& L0 = P.p.lev[0];
+  OutMap om;
+  if (P.pmap) om.map = P.pinv;
+  else { om.nP1 = P.nP1; om.F = P.F; }
+  if (P.p.nlev > 1) {
+    hipLaunchKernelGGL((p_enter_kernel<T>), dim3(eb), dim3(NT), 0, s, np, P.nP1, P.F, P.pmap,
+                       r + P.nu, L0.B, L0.dinv, (T)L0.cr[0], L0.deg == 1 ? nullptr : L0.D,
+                       first_dst(L0, L0.X), L0.mask, sk, L0.grp, k2);
+    vcycle<T, 1>(P.p, 0, L0.B, (T)1, z + P.nu, sk, s, true, K2In<T>(), om);
+  } else if (!P.p.cblk) {
+    vcycle<T, 1>(P.p, 0, r + P.nu, (T)1, z + P.nu, sk, s, false, k2, om);
+  } else {
+    hipLaunchKernelGGL((p_gather_map_kernel<T>), dim3(eb), dim3(NT), 0, s, np, P.pmap, r + P.nu,
+                       L0.B, sk.all);
+    vcycle<T, 1>(P.p, 0, L0.B, (T)1, L0.X, sk, s);
+    hipLaunchKernelGGL((p_scatter_map_kernel<T>), dim3(eb), dim3(NT), 0, s, np, P.pmap, L0.X,
+                       z + P.nu, sk.all);
+  }
+}
+
+// Nonzeros of the P2 level from which its residual moves to the pressure
+// stream, behind the pressure blocks: the two chains then take about the
+// same time.  Below, kernels are launch-bound and the residual is cheapest
+// inside the restriction's launch.
+constexpr long long LATE_RESIDUAL_NNZ = 4ll << 20;
 
 // z = M^-1 r; with k2 (k2_fusable only) r is first made as k2 describes.
 template <typename T>
 static void precond_apply(const Precond<T>& P, const T* r, T* z, Skip sk, hipStream_t s,
                           const K2In<T>* k2 = nullptr) {
-  const int* skip = sk.all;
-  hipStream_t sp = s;
-  if (P.ps) {                      // pressure blocks on the second stream
-    (void)hipEventRecord(P.ev_fork, s);
-    (void)hipStreamWaitEvent(P.ps, P.ev_fork, 0);
-    sp = P.ps;
-  }
   K2In<T> ku, kp;
   if (k2 && k2->y) {
     ku = *k2;
     kp = K2In<T>{k2->y + P.nu, k2->r2o + P.nu, k2->r + P.nu, k2->alfa, k2->beta};
   }
-  vcycle<T, 3>(P.u, 0, r, (T)(1.0 / P.u.scale), z, sk, s, false, ku);
-  long long np = (long long)P.F * P.nP1;
-  int eb = (int)((np + NT - 1) / NT);
-  if (P.pmap)
-    hipLaunchKernelGGL((p_gather_map_kernel<T>), dim3(eb), dim3(NT), 0, sp, np, P.pmap, r + P.nu,
-                       P.pin, skip);
-  else
-    hipLaunchKernelGGL((p_gather_kernel<T>), dim3(eb), dim3(NT), 0, sp, P.nP1, P.F, r + P.nu,
-                       P.pin, skip, kp);
-  vcycle<T, 1>(P.p, 0, P.pin, (T)1, P.pout, sk, sp);
-  if (P.pmap)
-    hipLaunchKernelGGL((p_scatter_map_kernel<T>), dim3(eb), dim3(NT), 0, sp, np, P.pmap, P.pout,
-                       z + P.nu, skip);
-  else
-    hipLaunchKernelGGL((p_scatter_kernel<T>), dim3(eb), dim3(NT), 0, sp, P.nP1, P.F, P.pout,
-                       z + P.nu, skip);
-  if (P.ps) {
+  const LevelDev<T>& U0 = P.u.lev[0];
+  const T us = (T)(1.0 / P.u.scale);
+  auto fork = [&] {                // pressure blocks on the second stream
+    if (!P.ps) return s;
+    (void)hipEventRecord(P.ev_fork, s);
+    (void)hipStreamWaitEvent(P.ps, P.ev_fork, 0);
+    return P.ps;
+  };
+  auto join = [&] {
+    if (!P.ps) return;
     (void)hipEventRecord(P.ev_join, P.ps);
     (void)hipStreamWaitEvent(s, P.ev_join, 0);
+  };
+  if (P.ps && P.u.nlev > 1 && U0.Wv && U0.nnz >= LATE_RESIDUAL_NNZ) {
+    T* bcopy = vcycle_bcopy(U0, r, us);
+    smooth_from_zero<T, 3>(U0, r, us, bcopy, sk, s, false, ku);
+    const T* bb = bcopy ? bcopy : r;
+    const hipStream_t sp = fork();
+    fused_down<T, 3>(P.u, 0, bb, sk, s, false);
+    vcycle<T, 3>(P.u, 1, P.u.lev[1].B, (T)1, P.u.lev[1].E, sk, s, P.u.nlev > 2);
+    precond_pressure(P, r, z, sk, sp, kp);
+    spmm<T, 3, 1>(U0, 0, U0.X, bb, U0.R, nullptr, 0, 0, sk, sp);
+    join();
+    fused_up<T, 3>(P.u, 0, bb, z, sk, s, OutMap());
+    return;
   }
+  const hipStream_t sp = fork();
+  vcycle<T, 3>(P.u, 0, r, us, z, sk, s, false, ku);
+  precond_pressure(P, r, z, sk, sp, kp);
+  join();
 }
 template <typename T>
 static void precond_apply(const Precond<T>& P, const T* r, T* z, const int* skip,
@@ -719,7 +1268,14 @@ static void set_hier_lpr(Hier<T>& H, const int32_t (*lpr)[3]) {
   for (int l = 0; l < H.nlev && l < MPET_MAXLEV; ++l) {
     if (lpr[l][0] > 0) H.lev[l].lpr = lpr[l][0];
     if (lpr[l][1] > 0) H.lev[l].lprP = lpr[l][1];
-    if (lpr[l][2] > 0) H.lev[l].lprR = lpr[l][2];
+    if (lpr[l][2] > 0) {
+      H.lev[l].lprR = lpr[l][2];
+      // of the fused restriction where there is one (three columns: one lane
+      // per component)
+      int lg = H.NC == 3 ? 2 : 0;
+      while ((1 << lg) < lpr[l][2]) ++lg;
+      H.lev[l].lgW = lg;
+    }
   }
 }
 template <typename T>
@@ -776,11 +1332,35 @@ static int build_hier(std::vector<void*>& allocs, const MpetHierDesc* d, int NC,
     chebyshev(lmax / d->eig_ratio, lmax, L.deg, L.cd, L.cr);
     size_t m = (size_t)NC * L.n;
     int rc;
-    if ((rc = alloc_dev(allocs, &L.B, m)) || (rc = alloc_dev(allocs, &L.X, m)) ||
+    // X and B adjacent: the fused restriction of several smoothing steps
+    // reads them as one vector
+    if ((rc = alloc_dev(allocs, &L.X, 2 * m)) ||
         (rc = alloc_dev(allocs, &L.R, m)) || (rc = alloc_dev(allocs, &L.E, m)) ||
         (rc = alloc_dev(allocs, &L.S1, m)) || (rc = alloc_dev(allocs, &L.S2, m)) ||
         (rc = alloc_dev(allocs, &L.D, m)))
       return rc;
+    L.B = L.X + m;
+    if (ld.A_s.off) {
+      if (!ld.A_s.base || !ld.A_s.row || !ld.A_sv || (!ld.A_s.dc && sizeof(T) != 4)) {
+        mpet_set_error("invalid hierarchy description (sliced level)");
+        return ERR_INVALID;
+      }
+      L.As = Sell<T>{ld.A_s.off, ld.A_s.base, ld.A_s.row, ld.A_s.dc, ld.A_sv};
+    }
+    if (ld.W_v && l + 1 < H.nlev) {
+      if (!ld.W_rp || !ld.W_ci || !ld.Q_v || ld.lgW < 0 || ld.lgW > 6 || ld.lgQ < 0 ||
+          ld.lgQ > 6 || (NC == 3 && (ld.lgW < 2 || ld.lgQ < 2)) ||
+          (ld.Q_s.off ? !ld.Q_s.base || !ld.Q_s.row || !ld.Q_s.dc : !ld.Q_rp || !ld.Q_ci)) {
+        mpet_set_error("invalid hierarchy description (fused transfers)");
+        return ERR_INVALID;
+      }
+      L.Wrp = ld.W_rp; L.Wci = ld.W_ci; L.Wv = (const T*)ld.W_v;
+      L.Qrp = ld.Q_rp; L.Qci = ld.Q_ci; L.Qv = (const T*)ld.Q_v;
+      L.lgW = ld.lgW;
+      L.lgQ = ld.lgQ;
+      L.nnz = ld.A_nnz;
+      if (ld.Q_s.off) L.Qs = Sell<T>{ld.Q_s.off, ld.Q_s.base, ld.Q_s.row, ld.Q_s.dc, ld.Q_v};
+    }
   }
   for (int l = 0; l + 1 < H.nlev; ++l) H.lev[l].grpc = H.lev[l + 1].grp;
   H.cinv = (const T*)d->coarse_inv;
@@ -804,7 +1384,12 @@ static int build_precond(std::vector<void*>& allocs, long long nu, const MpetPre
     mpet_set_error("preconditioner sizes do not match the operator");
     return ERR_INVALID;
   }
-  size_t np = (size_t)P.F * P.nP1;
-  if ((rc = alloc_dev(allocs, &P.pin, np)) || (rc = alloc_dev(allocs, &P.pout, np))) return rc;
+  if (P.pmap) {                    // the batch's pressure order, inverted
+    const int np = P.F * P.nP1;
+    if ((rc = alloc_dev(allocs, &P.pinv, (size_t)np))) return rc;
+    hipLaunchKernelGGL((invert_map_kernel_t<int>), dim3((np + NT - 1) / NT), dim3(NT), 0, 0, np, P.pmap,
+                       P.pinv);
+    HIPCHK(hipDeviceSynchronize());
+  }
   return OK;
 }

@@ -30,7 +30,11 @@ class AmgLevelDesc(C.Structure):
                 ("R_rp", C.c_void_p), ("R_ci", C.c_void_p), ("R_v", C.c_void_p),
                 ("lpr", C.c_int32), ("lprP", C.c_int32), ("lprR", C.c_int32),
                 ("A_v16", C.c_void_p), ("A_dci", C.c_void_p), ("A_vscale", C.c_double),
-                ("grp", C.c_void_p)]
+                ("grp", C.c_void_p),
+                ("W_rp", C.c_void_p), ("W_ci", C.c_void_p), ("W_v", C.c_void_p),
+                ("Q_rp", C.c_void_p), ("Q_ci", C.c_void_p), ("Q_v", C.c_void_p),
+                ("lgW", C.c_int32), ("lgQ", C.c_int32), ("A_nnz", C.c_int64),
+                ("A_s", lv.Slices), ("A_sv", C.c_void_p), ("Q_s", lv.Slices)]
 
 
 class HierDesc(C.Structure):
@@ -552,6 +556,8 @@ class KrylovSolver:
                 if c is not None:
                     p[0][l].update(c)
                     self.pcompact_levels.append(l)
+        lv.add_fused(u[0], self.levels, self.cfg.amg, dtype, self.mask0)
+        lv.add_fused(p[0], self.plevels, self.cfg.pamg, dtype, p[0][0].get("mask0"))
         self.level_dev[dtype] = (u, p)
         return u, p
 
@@ -602,6 +608,7 @@ class KrylovSolver:
                 nnzp = ld["P_ci"].numel()
                 L.lprP = _pick_lpr(nnzp / max(lev["n"], 1), nc, lev["n"])
                 L.lprR = _pick_lpr(nnzp / max(lev["nc"], 1), nc, lev["nc"])
+            lv.describe_fused(L, ld, lev["n"], lev["nc"], nc)
         h.coarse_inv = ptr(cinv)
         h.degree = params.smoother_degree
         set_level_degrees(h, params)

@@ -6,14 +6,29 @@ enough, applying it (one launch) replaces the smoothing, residual, transfer
 and coarse-solve launches of that level and every coarser one (four to nine
 dependent launches per level, each a few microseconds whatever its size).
 M is formed in FP64 from the same level values the V-cycle kernels read.
+
+Fused transfers: on the levels that stay sparse, residual and restriction
+are one product with W and prolongation and the first post-smoothing step
+one product with Q (csrc/amg_cycle.h, "Fused transfers"), formed here from
+R A and A P.
+
 The reference leaves the cycle to hypre
 (mpet/mpettotalpressuresolver.py:448).
 """
 from __future__ import annotations
 
+import ctypes as C
+
 import torch
 
+from . import _lib
+from ._lib import check, ptr
 from .amg import chebyshev_coefficients
+
+class Slices(C.Structure):
+    _fields_ = [("off", C.c_void_p), ("base", C.c_void_p), ("row", C.c_void_p),
+                ("dc", C.c_void_p)]
+
 
 # A dense tail is used up to this many bytes of M.  Streaming it costs bytes
 # / ~4.5 TB/s (64 MiB: 15 us) against about four launches per replaced level
@@ -105,3 +120,242 @@ def with_dense_tail(levels, cinv, rows, params, device, values=None, mask0=None,
     for k in ("P_rp", "P_ci", "P_v", "R_rp", "R_ci", "R_v"):
         last.pop(k, None)
     return list(levels[:start]) + [last], M
+
+
+# ---------------------------------------------------------------------------
+# fused transfers
+# ---------------------------------------------------------------------------
+# products (A row entry, P row entry) expanded at a time: bounds the sort's
+# memory to ~1 GB
+_CHUNK = 1 << 25
+
+
+def _product_keys(A, P, nc):
+    """Sorted unique keys row * nc + column of the patterns of A P and P."""
+    (arp, aci), (prp, pci) = A, P
+    dev = aci.device
+    arp, prp = arp.long(), prp.long()
+    n = arp.numel() - 1
+    plen = prp[1:] - prp[:-1]
+    per_nz = plen[aci.long()]                            # products of each A entry
+    ends = torch.cumsum(per_nz, 0) if per_nz.numel() else per_nz
+    total = int(ends[-1]) if ends.numel() else 0
+    rows = torch.repeat_interleave(torch.arange(n, device=dev), arp[1:] - arp[:-1])
+    prow = torch.repeat_interleave(torch.arange(n, device=dev), plen)
+    keys = [prow * nc + pci.long()]                      # rows of A may be empty
+    at, done = 0, 0
+    while done < total:
+        # whole A entries up to about _CHUNK products
+        stop = int(torch.searchsorted(ends, min(done + _CHUNK, total), right=False)) + 1
+        cnt = per_nz[at:stop]
+        rep = torch.repeat_interleave(torch.arange(at, stop, device=dev), cnt)
+        first = ends[at:stop] - cnt
+        off = torch.arange(done, done + rep.numel(), device=dev) - first[rep - at]
+        cols = pci[prp[aci[rep].long()] + off].long()
+        keys.append(torch.unique(rows[rep] * nc + cols))
+        done += rep.numel()
+        at = stop
+    return torch.unique(torch.cat(keys))
+
+
+def _row_pointers(rows, n):
+    out = torch.zeros(n + 1, dtype=torch.int64, device=rows.device)
+    out[1:] = torch.cumsum(torch.bincount(rows, minlength=n), 0)
+    return out
+
+
+def _csr(rows, n, cols, what):
+    rp = _row_pointers(rows, n)
+    if int(rp[-1]) >= 2**31:
+        raise ValueError(f"{what}: too large for 32-bit row pointers")
+    return rp.to(torch.int32), cols.to(torch.int32)
+
+
+def _values(rows, cols, X, Y):
+    out = torch.empty(rows.numel(), dtype=torch.float64, device=rows.device)
+    r, c = rows.to(torch.int32), cols.to(torch.int32)
+    check(_lib.lib().mpet_product_values(r.numel(), ptr(r), ptr(c), *(ptr(t) for t in X),
+                                         *(ptr(t) for t in Y), ptr(out), _lib.stream_ptr()))
+    return out
+
+
+def fused_transfers(A, P, R, dinv, degree, c0, mask=None, values=_values):
+    """W and Q of one level from its device matrices A, P, R = (rp, ci, FP64
+    values) with sorted int32 columns: dict of W_rp, W_ci, W_v, Q_rp, Q_ci,
+    Q_v (FP64 values; Q_v holds pairs for degree > 1).  dinv: FP64 diagonal
+    inverse, c0: the first Chebyshev coefficient, mask: rows held at zero."""
+    n, nc = A[0].numel() - 1, R[0].numel() - 1
+    key = _product_keys(A[:2], P[:2], max(nc, 1))
+    rows, cols = key // nc, key % nc
+    dead = None if mask is None else mask.bool()
+    # A P and P on the pattern of A P
+    ap = values(rows, cols, A, P)
+    prow = torch.repeat_interleave(torch.arange(n, device=key.device),
+                                   (P[0][1:] - P[0][:-1]).long())
+    p = torch.zeros_like(ap)
+    p[torch.searchsorted(key, prow * nc + P[1].long())] = P[2]
+    if dead is not None:
+        ap[dead[rows]] = 0.0
+        p[dead[rows]] = 0.0
+    q = p - c0 * dinv[rows] * ap if degree == 1 else torch.stack([ap, p], 1).reshape(-1)
+    q_rp, q_ci = _csr(rows, n, cols, "fused prolongation")
+    # R A on the transposed pattern
+    order = torch.argsort(cols * n + rows)
+    wr, wc = cols[order], rows[order]
+    ra = values(wr, wc, R, A)
+    rrow = torch.repeat_interleave(torch.arange(nc, device=key.device),
+                                   (R[0][1:] - R[0][:-1]).long())
+    rcol, rv = R[1].long(), R[2].clone()
+    if dead is not None:
+        ra[dead[wc]] = 0.0
+        rv[dead[rcol]] = 0.0
+    if degree == 1:
+        w = -c0 * dinv[wc] * ra
+        w[torch.searchsorted(wr * n + wc, rrow * n + rcol)] += rv
+    else:
+        # row-wise [-R A, R], the columns of R shifted by n
+        ra_rp, r_rp = _row_pointers(wr, nc), R[0].long()
+        at_ra = torch.arange(wr.numel(), device=key.device) + r_rp[wr]
+        at_r = torch.arange(rrow.numel(), device=key.device) + ra_rp[rrow + 1]
+        total = wr.numel() + rrow.numel()
+        w = torch.empty(total, dtype=torch.float64, device=key.device)
+        col = torch.empty(total, dtype=torch.int64, device=key.device)
+        row = torch.empty(total, dtype=torch.int64, device=key.device)
+        w[at_ra], w[at_r] = -ra, rv
+        col[at_ra], col[at_r] = wc, rcol + n
+        row[at_ra], row[at_r] = wr, rrow
+        wr, wc = row, col
+    w_rp, w_ci = _csr(wr, nc, wc, "fused restriction")
+    return dict(W_rp=w_rp, W_ci=w_ci, W_v=w, Q_rp=q_rp, Q_ci=q_ci, Q_v=q)
+
+
+# ---------------------------------------------------------------------------
+# sliced rows
+# ---------------------------------------------------------------------------
+# Levels of at least this many rows run one thread per row on sliced copies:
+# 65,536 rows are 1,024 waves, four per compute unit; below, several lanes
+# share a row.
+SLICE_ROWS = 1 << 16
+# rows are sorted by length within windows of this many (a multiple of 64)
+WINDOW = 512
+
+
+def slices(rp, ci, values, n):
+    """Sliced copy (include/mpet_hip.h, MpetSlices) of a CSR matrix with n
+    rows on its device: dict of off, base, row, dc and v (values: (nnz,) or
+    (nnz, 2)), or None where the columns of some slice span 2^16 or more."""
+    dev = ci.device
+    rp, ci = rp.long(), ci.long()
+    length = rp[1:] - rp[:-1]
+    at = torch.arange(n, device=dev)
+    longest = int(length.max()) + 1 if n else 1
+    order = torch.argsort((at // WINDOW) * longest + (longest - 1 - length), stable=True)
+    ns = (n + 63) // 64
+    row = torch.full((64 * ns,), -1, dtype=torch.int64, device=dev)
+    row[:n] = order
+    width = torch.zeros(64 * ns, dtype=torch.int64, device=dev)
+    width[:n] = length[order]
+    width = width.view(ns, 64).amax(1)
+    off = torch.zeros(ns + 1, dtype=torch.int64, device=dev)
+    off[1:] = torch.cumsum(width, 0)
+    total = 64 * int(off[-1])
+    place = torch.empty(n, dtype=torch.int64, device=dev)
+    place[order] = at                                    # slot of each row
+    of = torch.repeat_interleave(at, length)             # row of each entry
+    slot = place[of]
+    j = torch.arange(ci.numel(), device=dev) - rp[of]
+    dest = (off[slot // 64] + j) * 64 + slot % 64
+    base = torch.full((ns,), 2**31 - 1, dtype=torch.int64, device=dev)
+    base.scatter_reduce_(0, slot // 64, ci, "amin")
+    base[width == 0] = 0
+    delta = ci - base[slot // 64]
+    if total >= 2**37 or (delta.numel() and int(delta.max()) >= 1 << 16):
+        return None
+    dc = torch.zeros(total, dtype=torch.int32, device=dev)
+    dc[dest] = delta.to(torch.int32)
+    v = torch.zeros((total,) + tuple(values.shape[1:]), dtype=values.dtype, device=dev)
+    v[dest] = values
+    return dict(off=off.to(torch.int32), base=base.to(torch.int32), row=row.to(torch.int32),
+                dc=dc, v=v)
+
+
+def _u16(dc):
+    """int32 offsets below 2^16 as 16-bit words (the bits of uint16)."""
+    return torch.where(dc >= 1 << 15, dc - (1 << 16), dc).to(torch.int16)
+
+
+def add_slices(ld, n):
+    """Sliced copies of a level operator and of its Q, where one thread per
+    row fills the chip."""
+    if n < SLICE_ROWS:
+        return
+    if "A_v16" in ld:
+        s = slices(ld["A_rp"], ld["A_ci"], ld["A_v16"], n)
+        if s is not None:            # half | offset << 16 in one 32-bit word
+            bits = s["v"].view(torch.int16).to(torch.int32) & 0xffff
+            word = bits | (_u16(s["dc"]).to(torch.int32) << 16)
+            ld["A_s"] = dict(s, v=word, dc=None)
+    else:
+        s = slices(ld["A_rp"], ld["A_ci"], ld["A_v"], n)
+        if s is not None:
+            ld["A_s"] = dict(s, dc=_u16(s["dc"]))
+    if "Q_v" in ld:
+        q = ld["Q_v"].view(ld["Q_ci"].numel(), -1)
+        s = slices(ld["Q_rp"], ld["Q_ci"], q, n)
+        if s is not None:
+            ld["Q_s"] = dict(s, dc=_u16(s["dc"]))
+
+
+def _describe_slices(S, s):
+    S.off, S.base, S.row, S.dc = (ptr(s[k]) for k in ("off", "base", "row", "dc"))
+
+
+def add_fused(levs, hosts, params, dtype, mask0=None):
+    """Fused transfers of every level but the coarsest, added to the uploaded
+    level dicts `levs` (values in their precision); hosts: the host levels
+    (rho)."""
+    for l, ld in enumerate(levs[:-1]):
+        if "A_v16" in ld:
+            av = ld["A_v16"].double() * ld["vscale"]
+        else:
+            av = ld["A_v"].double()
+        deg = params.degree(l)
+        lmax = hosts[l]["rho"] * params.eig_safety
+        c0 = float(chebyshev_coefficients(lmax / params.eig_ratio, lmax, deg)[1][0])
+        f = fused_transfers((ld["A_rp"], ld["A_ci"], av),
+                            (ld["P_rp"], ld["P_ci"], ld["P_v"].double()),
+                            (ld["R_rp"], ld["R_ci"], ld["R_v"].double()), ld["dinv"].double(),
+                            deg, c0, mask0 if l == 0 else None)
+        tdt = torch.float64 if dtype == 0 else torch.float32
+        f["W_v"], f["Q_v"] = f["W_v"].to(tdt), f["Q_v"].to(tdt)
+        ld.update(f)
+        add_slices(ld, int(hosts[l]["n"]))
+
+
+def _log2_lanes(avg, rows, nc):
+    """Lanes per row of W and Q (log2): about eight nonzeros a lane, more
+    while the launch would hold fewer than 2^19 lanes; three columns need at
+    least four lanes."""
+    lg = 2 if nc == 3 else 0
+    while (8 << lg) < avg and lg < 6:
+        lg += 1
+    while (rows << lg) < (1 << 19) and (1 << lg) < avg and lg < 6:
+        lg += 1
+    return lg
+
+
+def describe_fused(L, ld, n, ncoarse, nc):
+    """Fill the fused-transfer part of an AmgLevelDesc."""
+    if "W_v" not in ld:
+        return
+    L.W_rp, L.W_ci, L.W_v = ptr(ld["W_rp"]), ptr(ld["W_ci"]), ptr(ld["W_v"])
+    L.Q_rp, L.Q_ci, L.Q_v = ptr(ld["Q_rp"]), ptr(ld["Q_ci"]), ptr(ld["Q_v"])
+    L.lgW = _log2_lanes(ld["W_ci"].numel() / max(ncoarse, 1), ncoarse, nc)
+    L.lgQ = _log2_lanes(ld["Q_ci"].numel() / max(n, 1), n, nc)
+    L.A_nnz = ld["A_ci"].numel()
+    if "A_s" in ld:
+        _describe_slices(L.A_s, ld["A_s"])
+        L.A_sv = ptr(ld["A_s"]["v"])
+    if "Q_s" in ld:
+        _describe_slices(L.Q_s, ld["Q_s"])
+        L.Q_v = ptr(ld["Q_s"]["v"])
