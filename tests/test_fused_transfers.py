@@ -6,8 +6,9 @@ levels (waterscapes_amd/levels.py, csrc/amg_cycle.h).
   sliced copies hold exactly the matrix.
 * GPU: the block preconditioner with the fused transfers equals the numpy
   restatement's separate steps, in FP64 and FP32, on hierarchies of several
-  sparse levels: one row per lane group to many and one thread per row
-  (sliced), degrees 1 to 3, small and ordinary meshes."""
+  sparse levels: joint launches of both cycles (no level sliced), separate
+  ones with the large levels or all of them on one thread per row, degrees 1
+  to 3, small and ordinary meshes."""
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -108,24 +109,26 @@ def test_slices_refuse_wide_columns():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("sliced", [False, True])
+@pytest.mark.parametrize("slice_rows", [1 << 30, 600, 1])
 @pytest.mark.parametrize("n,A,degs", [(3, 1, (1,)), (5, 3, (1,)), (5, 2, (2,)), (6, 6, (3, 1)),
                                       (27, 1, (1,)), (27, 1, (2,))])
 @pytest.mark.parametrize("mode", ["fp64", "mixed"])
-def test_preconditioner_with_fused_transfers(n, A, degs, mode, sliced, monkeypatch):
+def test_preconditioner_with_fused_transfers(n, A, degs, mode, slice_rows, monkeypatch):
     import torch
     from test_gpu_solver import _ref_precond, _setup
     from waterscapes_amd import levels as lv
     from waterscapes_amd.amg import AmgParams
     monkeypatch.setattr(lv, "DENSE_TAIL_BYTES", 30 * 30 * 8)
-    monkeypatch.setattr(lv, "SLICE_ROWS", 1 if sliced else 1 << 30)
+    monkeypatch.setattr(lv, "SLICE_ROWS", slice_rows)
     big = dict(max_coarse=25) if n < 20 else {}
     _, _, dev, solver, dofs, _ = _setup(
         n=n, A=A, mode=mode, compact_plevel0=False, autotune=False,
         amg=AmgParams(smoother_degree=3, level_degrees=degs, **big), pamg=AmgParams(**big))
     assert len(solver.levels) >= 3 and len(solver.plevels) >= 2
     dev_levels = solver._level_arrays(0 if mode == "fp64" else 1)
-    assert all(("A_s" in ld) == sliced and "W_v" in ld for h in dev_levels for ld in h[0][:-1])
+    for (levs, _), host in zip(dev_levels, (solver.levels, solver.plevels)):
+        for ld, lev in zip(levs[:-1], host):
+            assert ("A_s" in ld) == (lev["n"] >= slice_rows) and "W_v" in ld
     r = np.random.default_rng(2).standard_normal(dev.n)
     r[np.concatenate(dofs)] = 0.0
     dtype = torch.float64 if mode == "fp64" else torch.float32

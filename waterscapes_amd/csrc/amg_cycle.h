@@ -498,11 +498,11 @@ struct ResArgs {            // r = b - A x, rows with mask 0
 
 // One row group of the restriction half.
 template <typename T, int NC>
-__device__ __forceinline__ void down_rows(const DownArgs<T>& w, const Skip& sk) {
+__device__ __forceinline__ void down_rows(const DownArgs<T>& w, int block, const Skip& sk) {
   T acc[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) acc[c] = 0;
-  const long long gid = (long long)blockIdx.x * NT + threadIdx.x;
+  const long long gid = (long long)block * NT + threadIdx.x;
   const int r = (int)(gid >> w.lg), lanes = 1 << w.lg;
   const int lane = (int)(gid & (lanes - 1));
   if (r >= w.n || row_skipped(sk, w.grp, r)) return;     // whole row groups leave
@@ -523,21 +523,13 @@ __device__ __forceinline__ void down_rows(const DownArgs<T>& w, const Skip& sk) 
   }
 }
 
-// Blocks [0, nbw) form the coarse right-hand side, the rest the residual:
-// both read only x and b, so one launch holds both (a launch of its own
-// costs 4-5 us, more than the rows of every level but the finest).
+// One row group of the residual half.
 template <typename T, int NC, bool COMPACT>
-__global__ void __launch_bounds__(NT)
-transfer_kernel(DownArgs<T> w, ResArgs<T> a, int nbw, Skip sk) {
-  if (sk.all && *sk.all) return;
-  if ((int)blockIdx.x < nbw) {
-    down_rows<T, NC>(w, sk);
-    return;
-  }
+__device__ __forceinline__ void res_rows(const ResArgs<T>& a, int block, const Skip& sk) {
   T acc[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) acc[c] = 0;
-  const long long gid = (long long)((int)blockIdx.x - nbw) * NT + threadIdx.x;
+  const long long gid = (long long)block * NT + threadIdx.x;
   const int r = (int)(gid >> a.lg), lanes = 1 << a.lg;
   const int lane = (int)(gid & (lanes - 1));
   if (r >= a.n || row_skipped(sk, a.grp, r)) return;
@@ -556,6 +548,17 @@ transfer_kernel(DownArgs<T> w, ResArgs<T> a, int nbw, Skip sk) {
   a.r[o] = m ? (T)0 : pb - mine;
 }
 
+// Blocks [0, nbw) form the coarse right-hand side, the rest the residual:
+// both read only x and b, so one launch holds both (a launch of its own
+// costs 3-5 us, more than the rows of every level but the finest).
+template <typename T, int NC, bool COMPACT>
+__global__ void __launch_bounds__(NT)
+transfer_kernel(DownArgs<T> w, ResArgs<T> a, int nbw, Skip sk) {
+  if (sk.all && *sk.all) return;
+  if ((int)blockIdx.x < nbw) down_rows<T, NC>(w, blockIdx.x, sk);
+  else res_rows<T, NC, COMPACT>(a, (int)blockIdx.x - nbw, sk);
+}
+
 // The same with the residual's rows sliced.
 template <typename T, int NC, int VK>
 __global__ void __launch_bounds__(NT)
@@ -563,7 +566,7 @@ transfer_sell_kernel(DownArgs<T> w, Sell<T> M, int nslice, const T* __restrict__
                      SellEpi<T> E, int nbw, Skip sk) {
   if (sk.all && *sk.all) return;
   if ((int)blockIdx.x < nbw) {
-    down_rows<T, NC>(w, sk);
+    down_rows<T, NC>(w, blockIdx.x, sk);
     return;
   }
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -574,14 +577,29 @@ transfer_sell_kernel(DownArgs<T> w, Sell<T> M, int nslice, const T* __restrict__
 // Prolongation with the first post-smoothing step.  One step in all
 // (PAIR false): y = x + cr Dinv r + Q e.  More (PAIR): d = cr Dinv (r -
 // (A P) e), y = x + P e + d; d is stored for the next step.
+template <typename T>
+struct PostArgs {
+  int n, lg;
+  const int *rp, *ci;
+  const T *val, *e, *x, *r, *dinv;
+  T cr;
+  T *y, *d;
+  const uint8_t* mask;
+  OutMap om;
+  const int* grp;
+};
 template <typename T, int NC, bool PAIR>
-__global__ void __launch_bounds__(NT)
-post_kernel(int n, int lg, const int* __restrict__ rp, const int* __restrict__ ci,
-            const T* __restrict__ val, const T* __restrict__ e, const T* x, const T* r_,
-            const T* __restrict__ dinv, T cr, T* y, T* d, const uint8_t* __restrict__ mask,
-            OutMap om, Skip sk, const int* __restrict__ grp) {
-  if (sk.all && *sk.all) return;
-  const long long gid = (long long)blockIdx.x * NT + threadIdx.x;
+__device__ __forceinline__ void post_rows(const PostArgs<T>& A, int block, const Skip& sk) {
+  const int n = A.n, lg = A.lg;
+  const int *__restrict__ rp = A.rp, *__restrict__ ci = A.ci;
+  const T *__restrict__ val = A.val, *__restrict__ e = A.e;
+  const T *x = A.x, *r_ = A.r, *__restrict__ dinv = A.dinv;
+  const T cr = A.cr;
+  T *y = A.y, *d = A.d;
+  const uint8_t* __restrict__ mask = A.mask;
+  const int* __restrict__ grp = A.grp;
+  const OutMap om = A.om;
+  const long long gid = (long long)block * NT + threadIdx.x;
   const int r = (int)(gid >> lg), lanes = 1 << lg;
   const int lane = (int)(gid & (lanes - 1));
   if (r >= n || row_skipped(sk, grp, r)) return;
@@ -638,6 +656,12 @@ post_kernel(int n, int lg, const int* __restrict__ rp, const int* __restrict__ c
     y[oo] = m ? (T)0 : px + di * pr + m1;
   }
 }
+template <typename T, int NC, bool PAIR>
+__global__ void __launch_bounds__(NT)
+post_kernel(PostArgs<T> A, Skip sk) {
+  if (sk.all && *sk.all) return;
+  post_rows<T, NC, PAIR>(A, blockIdx.x, sk);
+}
 
 // A MINRES vector update fused into the first kernels of a preconditioner
 // apply that read its input (off when y is null): the input entry i is
@@ -662,13 +686,12 @@ struct K2In {
 // only when given); the scaled right-hand side is kept in bcopy when given;
 // with k2 on, b is made by k2 (and b itself is not read).
 template <typename T, int NC>
-__global__ void __launch_bounds__(NT)
-cheb0_kernel(int nrows, const T* b, T scale, const T* __restrict__ dinv, T cr,
-             T* __restrict__ d, T* __restrict__ y, T* __restrict__ bcopy,
-             const uint8_t* __restrict__ mask, Skip sk, const int* __restrict__ grp,
-             K2In<T> k2 = K2In<T>()) {
-  if (sk.all && *sk.all) return;
-  long long i = (long long)blockIdx.x * NT + threadIdx.x;
+__device__ __forceinline__ void cheb0_rows(int block, int nrows, const T* b, T scale,
+                                           const T* __restrict__ dinv, T cr, T* __restrict__ d,
+                                           T* __restrict__ y, T* __restrict__ bcopy,
+                                           const uint8_t* __restrict__ mask, const Skip& sk,
+                                           const int* __restrict__ grp, const K2In<T>& k2) {
+  long long i = (long long)block * NT + threadIdx.x;
   if (i >= (long long)NC * nrows) return;
   int r = (int)(i / NC);
   if (row_skipped(sk, grp, r)) return;
@@ -678,17 +701,25 @@ cheb0_kernel(int nrows, const T* b, T scale, const T* __restrict__ dinv, T cr,
   if (d) d[i] = v;
   y[i] = v;
 }
+template <typename T, int NC>
+__global__ void __launch_bounds__(NT)
+cheb0_kernel(int nrows, const T* b, T scale, const T* __restrict__ dinv, T cr,
+             T* __restrict__ d, T* __restrict__ y, T* __restrict__ bcopy,
+             const uint8_t* __restrict__ mask, Skip sk, const int* __restrict__ grp,
+             K2In<T> k2 = K2In<T>()) {
+  if (sk.all && *sk.all) return;
+  cheb0_rows<T, NC>(blockIdx.x, nrows, b, scale, dinv, cr, d, y, bcopy, mask, sk, grp, k2);
+}
 
 // Dense coarsest solve x = Cinv (scale b) (NC columns), one wave per row;
 // each lane keeps four row entries (and their b values) in flight per trip.
 // b and x may lie in the vectors' own order (om); with k2 on, b's entries
 // are made by it, and each row's wave stores its own.
 template <typename T, int NC>
-__global__ void __launch_bounds__(NT)
-coarse_kernel(int n, const T* __restrict__ cinv, const T* b, T* __restrict__ x,
-              const int* __restrict__ skip, T scale, OutMap om, K2In<T> k2) {
-  if (skip && *skip) return;
-  const int r = blockIdx.x * (NT / 64) + threadIdx.x / 64;
+__device__ __forceinline__ void coarse_rows(int block, int n, const T* __restrict__ cinv,
+                                            const T* b, T* __restrict__ x, T scale,
+                                            const OutMap& om, const K2In<T>& k2) {
+  const int r = block * (NT / 64) + threadIdx.x / 64;
   const int lane = threadIdx.x % 64;
   if (r >= n) return;
   T acc[NC];
@@ -727,38 +758,60 @@ coarse_kernel(int n, const T* __restrict__ cinv, const T* b, T* __restrict__ x,
     if (lane == c) x[o + c] = scale * v;
   }
 }
+template <typename T, int NC>
+__global__ void __launch_bounds__(NT)
+coarse_kernel(int n, const T* __restrict__ cinv, const T* b, T* __restrict__ x,
+              const int* __restrict__ skip, T scale, OutMap om, K2In<T> k2) {
+  if (skip && *skip) return;
+  coarse_rows<T, NC>(blockIdx.x, n, cinv, b, x, scale, om, k2);
+}
 
 // The gather with the first Chebyshev step of the finest pressure level from
 // zero: b = the gathered entry, x = cr Dinv b (and the direction d when
 // given), each at the entry's place in the hierarchy (field-major, or map).
 template <typename T>
+struct EnterArgs {
+  long long np;
+  int nP1, F;
+  const int* map;
+  const T* src;
+  T* b;
+  const T* dinv;
+  T cr;
+  T *d, *x;
+  const uint8_t* mask;
+  const int* grp;
+  K2In<T> k2;
+};
+template <typename T>
+__device__ __forceinline__ void enter_rows(const EnterArgs<T>& E, int block, const Skip& sk) {
+  const long long i = (long long)block * NT + threadIdx.x;
+  if (i >= E.np) return;
+  const int q = E.map ? E.map[i] : (int)((i % E.F) * E.nP1 + i / E.F);
+  if (row_skipped(sk, E.grp, q)) return;
+  const T bv = E.k2.y ? E.k2.make(i) : E.src[i];
+  E.b[q] = bv;
+  const T v = (E.mask && E.mask[q]) ? (T)0 : E.cr * E.dinv[q] * bv;
+  if (E.d) E.d[q] = v;
+  E.x[q] = v;
+}
+template <typename T>
 __global__ void __launch_bounds__(NT)
-p_enter_kernel(long long np, int nP1, int F, const int* __restrict__ map, const T* src,
-               T* __restrict__ b, const T* __restrict__ dinv, T cr, T* __restrict__ d,
-               T* __restrict__ x, const uint8_t* __restrict__ mask, Skip sk,
-               const int* __restrict__ grp, K2In<T> k2) {
+p_enter_kernel(EnterArgs<T> E, Skip sk) {
   if (sk.all && *sk.all) return;
-  const long long i = (long long)blockIdx.x * NT + threadIdx.x;
-  if (i >= np) return;
-  const int q = map ? map[i] : (int)((i % F) * nP1 + i / F);
-  if (row_skipped(sk, grp, q)) return;
-  const T bv = k2.y ? k2.make(i) : src[i];
-  b[q] = bv;
-  const T v = (mask && mask[q]) ? (T)0 : cr * dinv[q] * bv;
-  if (d) d[q] = v;
-  x[q] = v;
+  enter_rows(E, blockIdx.x, sk);
 }
 // Block-diagonal dense coarsest solve (many independent instances): row r
 // lies in block blk[r] spanning rows off[b] .. off[b+1]-1, whose dense
 // inverse is stored row-major at inv + ioff[b].
 template <typename T, int NC>
-__global__ void __launch_bounds__(NT)
-coarse_blockdiag_kernel(int n, const int* __restrict__ blk, const int* __restrict__ off,
-                        const int64_t* __restrict__ ioff, const T* __restrict__ inv,
-                        const T* __restrict__ b, T* __restrict__ x, Skip sk,
-                        const int* __restrict__ grp) {
-  if (sk.all && *sk.all) return;
-  const int r = blockIdx.x * (NT / 64) + threadIdx.x / 64;
+__device__ __forceinline__ void blockdiag_rows(int block, int n, const int* __restrict__ blk,
+                                               const int* __restrict__ off,
+                                               const int64_t* __restrict__ ioff,
+                                               const T* __restrict__ inv,
+                                               const T* __restrict__ b, T* __restrict__ x,
+                                               const Skip& sk, const int* __restrict__ grp) {
+  const int r = block * (NT / 64) + threadIdx.x / 64;
   const int lane = threadIdx.x % 64;
   if (r >= n || row_skipped(sk, grp, r)) return;
   const int bk = blk[r];
@@ -788,6 +841,118 @@ coarse_blockdiag_kernel(int n, const int* __restrict__ blk, const int* __restric
     T v = group_allsum<64>(acc[c]);
     if (lane == c) x[NC * r + c] = v;
   }
+}
+template <typename T, int NC>
+__global__ void __launch_bounds__(NT)
+coarse_blockdiag_kernel(int n, const int* __restrict__ blk, const int* __restrict__ off,
+                        const int64_t* __restrict__ ioff, const T* __restrict__ inv,
+                        const T* __restrict__ b, T* __restrict__ x, Skip sk,
+                        const int* __restrict__ grp) {
+  if (sk.all && *sk.all) return;
+  blockdiag_rows<T, NC>(blockIdx.x, n, blk, off, ioff, inv, b, x, sk, grp);
+}
+
+// ---------------------------------------------------------------------------
+// Joint launches.  On small systems a V-cycle kernel takes 3-5 us whatever
+// its rows, and forking the pressure blocks onto a second stream costs more
+// than it hides (12^3, four networks: 94.7 us per iteration forked, 87.7 in
+// one chain); there the i-th step of the displacement cycle and the i-th of
+// the pressure cycle, which are independent, share a launch.  A step is one
+// of the kernels above, named by its kind; lanes per row at run time.
+// ---------------------------------------------------------------------------
+enum StepKind { STEP_NONE, STEP_FIRST, STEP_ENTER, STEP_CHEB, STEP_DOWN, STEP_POST, STEP_DENSE,
+                STEP_BLOCKS };
+
+template <typename T>
+struct Step {
+  int kind = STEP_NONE, blocks = 0, nbw = 0, n = 0;
+  bool compact = false, pair = false;
+  ResArgs<T> a{};                  // matrix and rows (CHEB, DOWN)
+  DownArgs<T> w{};
+  PostArgs<T> p{};
+  EnterArgs<T> e{};
+  const T *b = nullptr, *dinv = nullptr;
+  T cd = 0, cr = 0, scale = 1;
+  T *d = nullptr, *y = nullptr, *y2 = nullptr, *bcopy = nullptr;
+  OutMap om;
+  K2In<T> k2;
+  const T* cinv = nullptr;
+  const int *blk = nullptr, *off = nullptr;
+  const int64_t* ioff = nullptr;
+};
+
+// Chebyshev step d' = cd d + cr Dinv (b - A x), y = x + d' (spmm_kernel mode
+// 3) of one row group; S.a.x and S.a.b hold x and b.
+template <typename T, int NC, bool COMPACT>
+__device__ __forceinline__ void cheb_rows(const Step<T>& S, int block, const Skip& sk) {
+  const ResArgs<T>& a = S.a;
+  const long long gid = (long long)block * NT + threadIdx.x;
+  const int r = (int)(gid >> a.lg), lanes = 1 << a.lg;
+  const int lane = (int)(gid & (lanes - 1));
+  if (r >= a.n || row_skipped(sk, a.grp, r)) return;
+  const long long o = (long long)NC * r + (lane < NC ? lane : NC - 1);
+  const T pb = a.b[o], px = a.x[o], pd = S.cd != (T)0 ? S.d[o] : (T)0, di = S.dinv[r];
+  const int m = a.mask ? (int)a.mask[r] : 0;
+  T acc[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) acc[c] = 0;
+  row_part<T, NC, COMPACT>(a.rp, a.ci, a.val, a.val16, a.dci, a.x, r, lane, lanes, acc);
+  T mine = 0;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const T v = lanes_allsum(acc[c], lanes);
+    if (lane == c) mine = v;
+  }
+  if (lane >= NC) return;
+  if constexpr (COMPACT) mine *= a.vscale;
+  const T dd = m ? (T)0 : S.cd * pd + S.cr * di * (pb - mine);
+  if (S.y2) S.y2[o] = dd;
+  S.y[NC == 1 ? S.om(r) : o] = m ? (T)0 : px + dd;
+}
+
+template <typename T, int NC>
+__device__ __forceinline__ void run_step(const Step<T>& S, int block, const Skip& sk) {
+  switch (S.kind) {
+    case STEP_FIRST:
+      cheb0_rows<T, NC>(block, S.n, S.b, S.scale, S.dinv, S.cr, S.d, S.y, S.bcopy, S.a.mask, sk,
+                        S.a.grp, S.k2);
+      break;
+    case STEP_ENTER:
+      if constexpr (NC == 1) enter_rows(S.e, block, sk);
+      break;
+    case STEP_CHEB:
+      if constexpr (sizeof(T) == 4) {
+        if (S.compact) { cheb_rows<T, NC, true>(S, block, sk); break; }
+      }
+      cheb_rows<T, NC, false>(S, block, sk);
+      break;
+    case STEP_DOWN:
+      if (block < S.nbw) { down_rows<T, NC>(S.w, block, sk); break; }
+      if constexpr (sizeof(T) == 4) {
+        if (S.compact) { res_rows<T, NC, true>(S.a, block - S.nbw, sk); break; }
+      }
+      res_rows<T, NC, false>(S.a, block - S.nbw, sk);
+      break;
+    case STEP_POST:
+      if (S.pair) post_rows<T, NC, true>(S.p, block, sk);
+      else post_rows<T, NC, false>(S.p, block, sk);
+      break;
+    case STEP_DENSE:
+      coarse_rows<T, NC>(block, S.n, S.cinv, S.b, S.y, S.scale, S.om, S.k2);
+      break;
+    case STEP_BLOCKS:
+      blockdiag_rows<T, NC>(block, S.n, S.blk, S.off, S.ioff, S.cinv, S.b, S.y, sk, S.a.grp);
+      break;
+    default: break;
+  }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(NT)
+joint_kernel(Step<T> u, Step<T> p, Skip sk) {
+  if (sk.all && *sk.all) return;
+  if ((int)blockIdx.x < u.blocks) run_step<T, 3>(u, blockIdx.x, sk);
+  else run_step<T, 1>(p, (int)blockIdx.x - u.blocks, sk);
 }
 
 // inv[map[i]] = i (map a permutation of 0 .. n - 1).  A template, so that the
@@ -896,6 +1061,7 @@ struct Precond {
   long long nu = 0;
   const int* pmap = nullptr;           // explicit pressure order (batches)
   int* pinv = nullptr;                 // its inverse
+  bool joint = false;                  // both cycles in joint launches, no fork
   // optional second stream: the pressure V-cycle runs beside the
   // displacement one (fork / join through the two events; inside a captured
   // graph these become parallel branches)
@@ -906,6 +1072,7 @@ struct Precond {
 // Create the fork stream and events of P (default priority, no timing).
 template <typename T>
 static int make_fork(Precond<T>& P) {
+  if (P.joint) return OK;
   if (hipStreamCreateWithFlags(&P.ps, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreateWithFlags(&P.ev_fork, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&P.ev_join, hipEventDisableTiming) != hipSuccess) {
@@ -1037,6 +1204,32 @@ static void smooth_from_zero(const LevelDev<T>& L, const T* b, T bscale, T* bcop
   smooth_steps<T, NC>(L, bcopy ? bcopy : b, dst, 1, L.X, sk, s);
 }
 
+// Blocks of n rows at 2^lg lanes each.
+static int row_blocks(int n, int lg) {
+  return (int)((((long long)n << lg) + NT - 1) / NT);
+}
+template <typename T>
+static DownArgs<T> down_args(const Hier<T>& H, int l, const T* b) {
+  const LevelDev<T>& L = H.lev[l];
+  const LevelDev<T>& C = H.lev[l + 1];
+  const bool enter = l + 1 < H.nlev - 1;
+  return DownArgs<T>{L.nc, L.lgW, L.Wrp, L.Wci, L.Wv, L.deg == 1 ? b : L.X, C.B,
+                     enter ? C.dinv : nullptr, (T)C.cr[0], C.D,
+                     enter ? first_dst(C, C.X) : nullptr, L.grpc};
+}
+// log2 of a level's lanes per row (three columns: at least 4 lanes).
+template <typename T>
+static int level_lg(const LevelDev<T>& L, int NC) {
+  int lg = NC == 3 ? 2 : 0;
+  while ((1 << lg) < L.lpr) ++lg;
+  return lg;
+}
+template <typename T>
+static ResArgs<T> res_args(const LevelDev<T>& L, const T* b, int NC) {
+  return ResArgs<T>{L.n, level_lg(L, NC), L.rp, L.ci, L.v, L.v16, L.dci, (T)L.vscale, L.X, b,
+                    L.R, L.mask, L.grp};
+}
+
 // Fused restriction (into level l + 1's right-hand side and first step) and
 // residual of level l after its pre-smoothing, one launch (res false: the
 // restriction alone).
@@ -1044,18 +1237,9 @@ template <typename T, int NC>
 static void fused_down(const Hier<T>& H, int l, const T* b, Skip sk, hipStream_t s,
                        bool res = true) {
   const LevelDev<T>& L = H.lev[l];
-  const LevelDev<T>& C = H.lev[l + 1];
-  const bool enter = l + 1 < H.nlev - 1;
-  const DownArgs<T> w{L.nc, L.lgW, L.Wrp, L.Wci, L.Wv, L.deg == 1 ? b : L.X, C.B,
-                      enter ? C.dinv : nullptr, (T)C.cr[0], C.D,
-                      enter ? first_dst(C, C.X) : nullptr, L.grpc};
-  int lgA = 0;
-  while ((1 << lgA) < L.lpr) ++lgA;
-  if (NC == 3 && lgA < 2) lgA = 2;
-  const ResArgs<T> a{L.n, lgA, L.rp, L.ci, L.v, L.v16, L.dci, (T)L.vscale, L.X, b, L.R,
-                     L.mask, L.grp};
-  const int nbw = (int)((((long long)L.nc << L.lgW) + NT - 1) / NT);
-  const int nba = (int)((((long long)L.n << lgA) + NT - 1) / NT);
+  const DownArgs<T> w = down_args(H, l, b);
+  const ResArgs<T> a = res_args(L, b, NC);
+  const int nbw = row_blocks(w.n, w.lg), nba = row_blocks(a.n, a.lg);
   if (res && L.As.off) {
     const int ns = (L.n + 63) / 64, nbs = (ns + NT / 64 - 1) / (NT / 64);
     const SellEpi<T> E{b, nullptr, nullptr, nullptr, 0, 0, (T)L.vscale, L.R, nullptr, L.mask,
@@ -1076,6 +1260,12 @@ static void fused_down(const Hier<T>& H, int l, const T* b, Skip sk, hipStream_t
     }
   }
   hipLaunchKernelGGL((transfer_kernel<T, NC, false>), grid, dim3(NT), 0, s, w, a, nbw, sk);
+}
+
+template <typename T>
+static PostArgs<T> post_args(const LevelDev<T>& L, const T* e, T* y, T* d, OutMap om) {
+  return PostArgs<T>{L.n, L.lgQ, L.Qrp, L.Qci, L.Qv, e, L.X, L.R, L.dinv, (T)L.cr[0], y, d,
+                     L.mask, om, L.grp};
 }
 
 // Prolongation of C.E with level l's post-smoothing into out.
@@ -1099,14 +1289,11 @@ static void fused_up(const Hier<T>& H, int l, const T* b, T* out, Skip sk,
                          e, E, sk);
   } else {
     const int blocks = (int)((((long long)L.n << L.lgQ) + NT - 1) / NT);
+    const PostArgs<T> A = post_args(L, e, dst, one ? nullptr : L.D, dm);
     if (one)
-      hipLaunchKernelGGL((post_kernel<T, NC, false>), dim3(blocks), dim3(NT), 0, s, L.n, L.lgQ,
-                         L.Qrp, L.Qci, L.Qv, e, (const T*)L.X, (const T*)L.R, L.dinv,
-                         (T)L.cr[0], dst, (T*)nullptr, L.mask, dm, sk, L.grp);
+      hipLaunchKernelGGL((post_kernel<T, NC, false>), dim3(blocks), dim3(NT), 0, s, A, sk);
     else
-      hipLaunchKernelGGL((post_kernel<T, NC, true>), dim3(blocks), dim3(NT), 0, s, L.n, L.lgQ,
-                         L.Qrp, L.Qci, L.Qv, e, (const T*)L.X, (const T*)L.R, L.dinv,
-                         (T)L.cr[0], dst, L.D, L.mask, dm, sk, L.grp);
+      hipLaunchKernelGGL((post_kernel<T, NC, true>), dim3(blocks), dim3(NT), 0, s, A, sk);
   }
   if (!one) smooth_steps<T, NC>(L, b, L.S1, 1, out, sk, s, om);
 }
@@ -1172,6 +1359,21 @@ static bool k2_fusable(const Precond<T>& P) {
   return !P.pmap;
 }
 
+template <typename T>
+static EnterArgs<T> enter_args(const Precond<T>& P, const T* r, K2In<T> k2) {
+  const LevelDev<T>& L0 = P.p.lev[0];
+  return EnterArgs<T>{(long long)P.F * P.nP1, P.nP1, P.F, P.pmap, r + P.nu, L0.B, L0.dinv,
+                      (T)L0.cr[0], L0.deg == 1 ? nullptr : L0.D, first_dst(L0, L0.X), L0.mask,
+                      L0.grp, k2};
+}
+template <typename T>
+static OutMap pressure_map(const Precond<T>& P) {
+  OutMap om;
+  if (P.pmap) om.map = P.pinv;
+  else { om.nP1 = P.nP1; om.F = P.F; }
+  return om;
+}
+
 // Pressure block of precond_apply on stream s.
 template <typename T>
 static void precond_pressure(const Precond<T>& P, const T* r, T* z, Skip sk, hipStream_t s,
@@ -1179,13 +1381,9 @@ static void precond_pressure(const Precond<T>& P, const T* r, T* z, Skip sk, hip
   const long long np = (long long)P.F * P.nP1;
   const int eb = (int)((np + NT - 1) / NT);
   const LevelDev<T>& L0 = P.p.lev[0];
-  OutMap om;
-  if (P.pmap) om.map = P.pinv;
-  else { om.nP1 = P.nP1; om.F = P.F; }
+  const OutMap om = pressure_map(P);
   if (P.p.nlev > 1) {
-    hipLaunchKernelGGL((p_enter_kernel<T>), dim3(eb), dim3(NT), 0, s, np, P.nP1, P.F, P.pmap,
-                       r + P.nu, L0.B, L0.dinv, (T)L0.cr[0], L0.deg == 1 ? nullptr : L0.D,
-                       first_dst(L0, L0.X), L0.mask, sk, L0.grp, k2);
+    hipLaunchKernelGGL((p_enter_kernel<T>), dim3(eb), dim3(NT), 0, s, enter_args(P, r, k2), sk);
     vcycle<T, 1>(P.p, 0, L0.B, (T)1, z + P.nu, sk, s, true, K2In<T>(), om);
   } else if (!P.p.cblk) {
     vcycle<T, 1>(P.p, 0, r + P.nu, (T)1, z + P.nu, sk, s, false, k2, om);
@@ -1195,6 +1393,136 @@ static void precond_pressure(const Precond<T>& P, const T* r, T* z, Skip sk, hip
     vcycle<T, 1>(P.p, 0, L0.B, (T)1, L0.X, sk, s);
     hipLaunchKernelGGL((p_scatter_map_kernel<T>), dim3(eb), dim3(NT), 0, s, np, P.pmap, L0.X,
                        z + P.nu, sk.all);
+  }
+}
+
+// The steps of a V-cycle from level l (as vcycle; fused transfers on every
+// level but the coarsest).
+template <typename T, int NC>
+static void cycle_smooth(std::vector<Step<T>>& out, const LevelDev<T>& L, const T* b,
+                         const T* cur, T* dst_last, OutMap om) {
+  T* bufs[2] = {L.S1, L.S2};
+  int flip = 1;
+  for (int i = 1; i < L.deg; ++i) {
+    const bool last = i == L.deg - 1;
+    T* dst = last ? dst_last : bufs[flip];
+    if (dst == cur) dst = bufs[flip ^ 1];
+    Step<T> S;
+    S.kind = STEP_CHEB;
+    S.a = res_args(L, b, NC);
+    S.a.x = cur;
+    S.compact = L.v16 != nullptr;
+    S.blocks = row_blocks(L.n, S.a.lg);
+    S.dinv = L.dinv;
+    S.cd = (T)L.cd[i];
+    S.cr = (T)L.cr[i];
+    S.d = L.D;
+    S.y = dst;
+    S.y2 = last ? nullptr : L.D;
+    if (last) S.om = om;
+    out.push_back(S);
+    cur = dst;
+    flip ^= 1;
+  }
+}
+template <typename T, int NC>
+static void cycle_steps(std::vector<Step<T>>& out, const Hier<T>& H, int l, const T* b, T bscale,
+                        T* z, bool entered, K2In<T> k2, OutMap om) {
+  const LevelDev<T>& L = H.lev[l];
+  Step<T> S;
+  if (l == H.nlev - 1) {
+    S.kind = H.cblk ? STEP_BLOCKS : STEP_DENSE;
+    S.blocks = (L.n + NT / 64 - 1) / (NT / 64);
+    S.n = L.n;
+    S.cinv = H.cinv;
+    S.blk = H.cblk;
+    S.off = H.coff;
+    S.ioff = H.cioff;
+    S.b = b;
+    S.y = z;
+    S.scale = bscale;
+    S.om = om;
+    S.k2 = k2;
+    S.a.grp = L.grp;
+    out.push_back(S);
+    return;
+  }
+  T* bcopy = vcycle_bcopy(L, b, bscale);
+  T* first = first_dst(L, L.X);
+  if (!entered) {
+    S.kind = STEP_FIRST;
+    S.blocks = (int)(((long long)NC * L.n + NT - 1) / NT);
+    S.n = L.n;
+    S.b = b;
+    S.scale = bscale;
+    S.dinv = L.dinv;
+    S.cr = (T)L.cr[0];
+    S.d = L.deg == 1 ? nullptr : L.D;
+    S.y = first;
+    S.bcopy = bcopy;
+    S.a.mask = L.mask;
+    S.a.grp = L.grp;
+    S.k2 = k2;
+    out.push_back(S);
+  }
+  const T* bb = bcopy ? bcopy : b;
+  cycle_smooth<T, NC>(out, L, bb, first, L.X, OutMap());
+  S = Step<T>();
+  S.kind = STEP_DOWN;
+  S.w = down_args(H, l, bb);
+  S.a = res_args(L, bb, NC);
+  S.compact = L.v16 != nullptr;
+  S.nbw = row_blocks(S.w.n, S.w.lg);
+  S.blocks = S.nbw + row_blocks(L.n, S.a.lg);
+  out.push_back(S);
+  const LevelDev<T>& C = H.lev[l + 1];
+  cycle_steps<T, NC>(out, H, l + 1, C.B, (T)1, C.E, l + 1 < H.nlev - 1, K2In<T>(), OutMap());
+  const bool one = L.deg == 1;
+  S = Step<T>();
+  S.kind = STEP_POST;
+  S.pair = !one;
+  S.p = post_args(L, C.E, one ? z : L.S1, one ? nullptr : L.D, one ? om : OutMap());
+  S.blocks = row_blocks(L.n, L.lgQ);
+  out.push_back(S);
+  if (!one) cycle_smooth<T, NC>(out, L, bb, L.S1, z, om);
+}
+
+// Whether both cycles can run as steps, and should: every level below the
+// coarsest has fused transfers and none is sliced (the sliced levels are
+// the large ones, where the second stream pays).
+template <typename T>
+static bool joint_ok(const Precond<T>& P) {
+  for (const Hier<T>* H : {&P.u, &P.p}) {
+    for (int l = 0; l + 1 < H->nlev; ++l)
+      if (!H->lev[l].Wv || H->lev[l].As.off || H->lev[l].Qs.off) return false;
+    if (H->nlev == 1 && H->cblk) return false;
+  }
+  return true;
+}
+
+template <typename T>
+static void precond_joint(const Precond<T>& P, const T* r, T* z, Skip sk, hipStream_t s,
+                          K2In<T> ku, K2In<T> kp) {
+  std::vector<Step<T>> u, p;
+  u.reserve(32);
+  p.reserve(32);
+  cycle_steps<T, 3>(u, P.u, 0, r, (T)(1.0 / P.u.scale), z, false, ku, OutMap());
+  const OutMap om = pressure_map(P);
+  if (P.p.nlev > 1) {
+    Step<T> S;
+    S.kind = STEP_ENTER;
+    S.e = enter_args(P, r, kp);
+    S.blocks = (int)((S.e.np + NT - 1) / NT);
+    p.push_back(S);
+    cycle_steps<T, 1>(p, P.p, 0, P.p.lev[0].B, (T)1, z + P.nu, true, K2In<T>(), om);
+  } else {
+    cycle_steps<T, 1>(p, P.p, 0, r + P.nu, (T)1, z + P.nu, false, kp, om);
+  }
+  const Step<T> none;
+  for (size_t i = 0; i < u.size() || i < p.size(); ++i) {
+    const Step<T>& a = i < u.size() ? u[i] : none;
+    const Step<T>& b = i < p.size() ? p[i] : none;
+    hipLaunchKernelGGL((joint_kernel<T>), dim3(a.blocks + b.blocks), dim3(NT), 0, s, a, b, sk);
   }
 }
 
@@ -1212,6 +1540,10 @@ static void precond_apply(const Precond<T>& P, const T* r, T* z, Skip sk, hipStr
   if (k2 && k2->y) {
     ku = *k2;
     kp = K2In<T>{k2->y + P.nu, k2->r2o + P.nu, k2->r + P.nu, k2->alfa, k2->beta};
+  }
+  if (P.joint) {
+    precond_joint(P, r, z, sk, s, ku, kp);
+    return;
   }
   const LevelDev<T>& U0 = P.u.lev[0];
   const T us = (T)(1.0 / P.u.scale);
@@ -1384,6 +1716,7 @@ static int build_precond(std::vector<void*>& allocs, long long nu, const MpetPre
     mpet_set_error("preconditioner sizes do not match the operator");
     return ERR_INVALID;
   }
+  P.joint = joint_ok(P);
   if (P.pmap) {                    // the batch's pressure order, inverted
     const int np = P.F * P.nP1;
     if ((rc = alloc_dev(allocs, &P.pinv, (size_t)np))) return rc;
