@@ -603,8 +603,8 @@ int mpet_solver_set_tuning(void* h, int dtype, const MpetTuning* t);
 int mpet_solver_set_cell_operator(void* h, const MpetCellOpDesc* op);
 
 /* FP64 residuals b - A x of a solver handle (the refinement's outer
- * residuals in mixed mode, the start residuals in FP64 mode) through the
- * FP64 cell-wise operator (op != NULL, fp64 = 1; the handle allocates its
+ * residuals in mixed mode, the start residuals in FP64 mode), and in mode 0
+ * the MINRES iterations' operator, through the FP64 cell-wise operator (op != NULL, fp64 = 1; the handle allocates its
  * work and keeps a copy of the descriptor, whose arrays must outlive it)
  * or back through the FP64 structured operator (op == NULL).  Not used
  * when the handle's FP64 operator is a CSR matrix.  No counterpart in the

@@ -185,28 +185,29 @@ def tune_operator(sys_, dtype, cache=None, reps=10, repeats=3, margin=0.02):
     return best
 
 
-def cell_key(sys_):
+def cell_key(sys_, fp64=False):
     nz = sys_.nnz
-    return (f"cell|{ARCH}|F{sys_.F}|{sys_.cell_op()['nC']}|{sys_.nP2}|{sys_.nP1}|"
+    return (f"cell{'64' if fp64 else ''}|{ARCH}|F{sys_.F}|{sys_.cell_op()['nC']}|{sys_.nP2}|{sys_.nP1}|"
             f"{nz['11']}")
 
 
-def tune_cell_operator(sys_, cache=None, reps=10, repeats=3, margin=0.02):
+def tune_cell_operator(sys_, cache=None, reps=10, repeats=3, margin=0.02, fp64=False):
     """(lanes_u, lanes_p, xcd_chunk) of the cell-wise operator's row kernel."""
     cache = cache if cache is not None else default_cache()
-    key = cell_key(sys_)
+    key = cell_key(sys_, fp64)
     hit = cache.get(key)
     if hit is not None:
         return tuple(hit)
     L = _lib.lib()
     g = torch.Generator(device=sys_.device).manual_seed(0)
-    x = torch.randn(sys_.n, generator=g, device=sys_.device, dtype=torch.float64).float()
+    x = torch.randn(sys_.n, generator=g, device=sys_.device, dtype=torch.float64)
+    x = x if fp64 else x.float()
     y = torch.empty_like(x)
-    work = torch.empty(sys_.cell_work_floats(), dtype=torch.float32, device=sys_.device)
+    work = torch.empty(sys_.cell_work_floats(), dtype=x.dtype, device=sys_.device)
     default = tuple(sys_.cell_lanes) + (sys_.cell_xcd_chunk,)
 
     def timer(c):
-        d = sys_.cell_op_desc(lanes=(c[0], c[1]), xcd_chunk=c[2])
+        d = sys_.cell_op_desc(lanes=(c[0], c[1]), xcd_chunk=c[2], fp64=fp64)
         return time_launches(lambda: check(L.mpet_cell_op_apply(C.byref(d), ptr(x), None, ptr(y),
                                                                 ptr(work), _lib.stream_ptr())),
                              reps, repeats)

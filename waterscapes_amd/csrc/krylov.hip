@@ -72,14 +72,15 @@ __device__ __forceinline__ void k1_scalars(const MinresState* st, T& s, T& c1) {
 }
 
 // K1 epilogue for the cell-wise operator's row kernel (cellwise.h).
+template <typename T>
 struct CwEpiK1 {
-  EpiK1<float> e;
+  EpiK1<T> e;
   const MinresState* st;
   const int* skip;
-  float s = 0.f, c1 = 0.f;
+  T s = 0, c1 = 0;
   __device__ __forceinline__ bool skipped() const { return *skip != 0; }
   __device__ __forceinline__ void prep() { k1_scalars(st, s, c1); }
-  __device__ __forceinline__ double operator()(long long i, float ax) const {
+  __device__ __forceinline__ double operator()(long long i, T ax) const {
     return e(i, ax, s, c1);
   }
 };
@@ -730,8 +731,15 @@ static void minres_iter(MpetSolver* S, Minres<T>& M, const Precond<T>& P, bool c
   bool cw_done = false;
   if constexpr (sizeof(T) == 4) {
     if (!csr && S->has_cw) {
-      CwEpiK1 cepi{EpiK1<float>{M.y, nullptr, zc, Ra, S->cw.dmask}, M.st, skip};
+      CwEpiK1<float> cepi{EpiK1<float>{M.y, nullptr, zc, Ra, S->cw.dmask}, M.st, skip};
       np = cw_launch(S->cw, zc, cepi, M.partial, skip, s);
+      cw_done = true;
+    }
+  } else {
+    // FP64 MINRES on the assembled operator's cell-wise form
+    if (!csr && S->has_cw64 && S->opt.mode == 0) {
+      CwEpiK1<double> cepi{EpiK1<double>{M.y, nullptr, zc, Ra, S->cw64.dmask}, M.st, skip};
+      np = cw_launch(S->cw64, zc, cepi, M.partial, skip, s);
       cw_done = true;
     }
   }
@@ -1318,9 +1326,9 @@ extern "C" int mpet_solver_set_cell_operator(void* h, const MpetCellOpDesc* op) 
   return OK;
 }
 
-// FP64 residuals through the cell-wise FP64 operator (op != NULL) or back
-// through the structured FP64 operator (op == NULL).  The residuals run
-// outside the captured MINRES graphs, so no graph is dropped.
+// FP64 residuals, and in mode 0 the MINRES iterations, through the cell-wise
+// FP64 operator (op != NULL) or back through the structured FP64 operator
+// (op == NULL).  The captured FP64 graph is dropped.
 extern "C" int mpet_solver_set_cell_operator64(void* h, const MpetCellOpDesc* op) {
   MpetSolver* S = (MpetSolver*)h;
   if (!S || S->csr_only || S->mb) {
@@ -1329,6 +1337,8 @@ extern "C" int mpet_solver_set_cell_operator64(void* h, const MpetCellOpDesc* op
     return ERR_INVALID;
   }
   HIPCHK(hipDeviceSynchronize());
+  if (S->graph64) HIPCHK(hipGraphExecDestroy(S->graph64));
+  S->graph64 = nullptr;
   if (!op) {
     S->has_cw64 = false;
     return OK;

@@ -126,6 +126,7 @@ class MPETSolver(object):
         if p["precision"] == "mixed" and self.up.function_space().nmult:
             raise ValueError("systems with nullspace multipliers are solved in FP64 only")
         return SolverConfig(mode=p["precision"], rtol=float(p["krylov_rtol"]),
+                            use_graphs=True, check_every=10,
                             outer_tol=float(p["outer_tol"]), inner_rtol=float(p["inner_rtol"]),
                             maxit=int(p["maxit"]),
                             amg=AmgParams(smoother_degree=int(p["u_smoother_degree"]),

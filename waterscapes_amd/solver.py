@@ -44,6 +44,11 @@ from .krylov import KrylovSolver, SolverConfig
 from .nullspace import Constraints, has_nullspace, pressure_fields
 from .problem import resolved_params
 
+# Cells from which the direct path's FP64 MINRES runs on the cell-wise
+# operator: below, the CSR product is one launch of the ~4 us a launch costs
+# anyway, against the two of the cell-wise form.
+DIRECT_CELLS = 10000
+
 NEUMANN_MARKER = 1
 ROBIN_MARKER = 2
 
@@ -540,8 +545,13 @@ class MPETTotalPressureSolver(object):
         p = self.params
         if direct or (has_nullspace(self.problem) and p["precision"] != "fp64"):
             # the bordered systems of nullspace multipliers run in FP64 only
+            # iterations from captured chunks; from DIRECT_CELLS cells on the
+            # cell-wise operator (multipliers need the CSR matrix)
+            cells = self.problem.mesh.num_cells() >= DIRECT_CELLS and \
+                not has_nullspace(self.problem)
             return SolverConfig(mode="fp64", rtol=1e-12, maxit=int(p["maxit"]),
-                                p0_weight=p["p0_weight"])
+                                p0_weight=p["p0_weight"], use_csr=not cells, fp64_cells=cells,
+                                use_graphs=True, check_every=10)
         if p["fp64_operator"] not in ("csr", "structured"):
             raise ValueError("fp64_operator must be 'csr' or 'structured'")
         if p["fp32_operator"] not in ("cellwise", "structured"):
