@@ -83,20 +83,36 @@ __device__ __forceinline__ int cw_edge(int j, int k) {
   return lo == 0 ? 6 - hi : (lo == 1 ? 4 - hi : 0);
 }
 
-// Phase 1: one thread per cell.
-// (A template, so that the translation units including this header share
-// one instance.)
-template <int NTB, typename T>
-__global__ void __launch_bounds__(NTB)
-cw_cell_kernel(CellOpT<T> op, const T* __restrict__ x, const int* __restrict__ skip) {
-  static_assert(NTB == CW_NT, "one cell per thread of a CW_NT block");
-  if (skip && *skip) return;
-  __shared__ T su[CW_NT * 30];
-  __shared__ T sp[CW_NT * 4];
+// Phase 1 of one block: one thread per cell.  valid: the block's cells; at:
+// this thread's place in the cell tables (stride nC); p0(v): index in x of
+// the total pressure at node1 entry v.
+// The block's partial lists do not depend on the results, so a thread's
+// first PRE of them are read before the cell's own loads and arithmetic:
+// after the barrier only the slot numbers are still to come (block 256,
+// 48^3: ~790 P2 partials, three to four a thread).
+template <typename T, typename P0>
+__device__ __forceinline__ void cw_cell_block(const CellOpT<T>& op, const T* __restrict__ x,
+                                              int b, int valid, long long at, T mu, P0 p0_of,
+                                              T* su, T* sp) {
+  constexpr int PRE = 4;
   const int t = threadIdx.x;
-  const long long e = (long long)blockIdx.x * CW_NT + t;
-  if (e < op.nC) {
-    const long long nC = op.nC;
+  const int q2b = op.bq2[b], q2e = op.bq2[b + 1], q1b = op.bq1[b], q1e = op.bq1[b + 1];
+  int lb2[PRE], le2[PRE], lb1, le1;
+#pragma unroll
+  for (int i = 0; i < PRE; ++i) {
+    const int q = q2b + t + i * CW_NT;
+    const int qc = q < q2e ? q : q2e - 1;
+    lb2[i] = op.lrp2[qc];
+    le2[i] = q < q2e ? op.lrp2[qc + 1] : lb2[i];
+  }
+  {
+    const int q = q1b + t;
+    const int qc = q < q1e ? q : q1e - 1;
+    lb1 = op.lrp1[qc];
+    le1 = op.lrp1[qc + 1];
+  }
+  if (t < valid) {
+    const long long nC = op.nC, e = at;
     int n2[10], n1[4];
 #pragma unroll
     for (int k = 0; k < 10; ++k) n2[k] = op.node2[k * nC + e];
@@ -108,13 +124,11 @@ cw_cell_kernel(CellOpT<T> op, const T* __restrict__ x, const int* __restrict__ s
     const T vol = op.geom[9 * nC + e];
 #pragma unroll
     for (int m = 0; m < 3; ++m) G[0][m] = -(G[1][m] + G[2][m] + G[3][m]);
-    const int F = op.A + 1;
-    const long long nu = 3ll * op.nP2;
     T u[10][3], p0[4];
 #pragma unroll
     for (int k = 0; k < 10; ++k) load_nc<T, 3>(x + 3ll * n2[k], u[k]);
 #pragma unroll
-    for (int v = 0; v < 4; ++v) p0[v] = x[nu + (long long)F * n1[v]];
+    for (int v = 0; v < 4; ++v) p0[v] = x[p0_of(n1[v])];
     // U = sum_j u_j (x) G_j
     T U[3][3];
 #pragma unroll
@@ -124,7 +138,6 @@ cw_cell_kernel(CellOpT<T> op, const T* __restrict__ x, const int* __restrict__ s
         U[b][d] = u[0][b] * G[0][d] + u[1][b] * G[1][d] + u[2][b] * G[2][d] + u[3][b] * G[3][d];
     // vertex stresses (symmetric: xx yy zz xy xz yz) and divergences
     T s[4][6], tr[4];
-    const T mu = op.mu;
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
       T g[3][3];
@@ -196,10 +209,8 @@ cw_cell_kernel(CellOpT<T> op, const T* __restrict__ x, const int* __restrict__ s
   // slot order, stored at the block's contiguous run of partials (scattered
   // 12-byte stores to node-sorted lists measured 3.7x their bytes in memory
   // writes: lines shared by blocks on different XCDs)
-  const int b = blockIdx.x;
   T* __restrict__ Yu = op.Yu;
-  for (int q = op.bq2[b] + t; q < op.bq2[b + 1]; q += CW_NT) {
-    const int lb = op.lrp2[q], le = op.lrp2[q + 1];
+  auto partial2 = [&](int q, int lb, int le) {
     T a[3] = {(T)0, (T)0, (T)0};
     for (int i = lb; i < le; ++i) {
       const int sl = op.lsl2[i];
@@ -208,17 +219,54 @@ cw_cell_kernel(CellOpT<T> op, const T* __restrict__ x, const int* __restrict__ s
       a[2] += su[3 * sl + 2];
     }
     __builtin_memcpy(Yu + 3ll * q, a, 3 * sizeof(T));
+  };
+#pragma unroll
+  for (int i = 0; i < PRE; ++i) {
+    const int q = q2b + t + i * CW_NT;
+    if (q < q2e) partial2(q, lb2[i], le2[i]);
   }
-  for (int q = op.bq1[b] + t; q < op.bq1[b + 1]; q += CW_NT) {
-    const int lb = op.lrp1[q], le = op.lrp1[q + 1];
+  for (int q = q2b + t + PRE * CW_NT; q < q2e; q += CW_NT)
+    partial2(q, op.lrp2[q], op.lrp2[q + 1]);
+  for (int q = q1b + t; q < q1e; q += CW_NT) {
+    if (q != q1b + t) {
+      lb1 = op.lrp1[q];
+      le1 = op.lrp1[q + 1];
+    }
     T a = (T)0;
-    for (int i = lb; i < le; ++i) a += sp[op.lsl1[i]];
+    for (int i = lb1; i < le1; ++i) a += sp[op.lsl1[i]];
     op.Yp[q] = a;
   }
 }
 
-// Phase-2 epilogue of a plain application: y = A x, or y = b - A x with b;
-// rows with dmask set give 0.
+// (A template, so that the translation units including this header share
+// one instance.)
+template <int NTB, typename T>
+__global__ void __launch_bounds__(NTB)
+cw_cell_kernel(CellOpT<T> op, const T* __restrict__ x, const int* __restrict__ skip) {
+  static_assert(NTB == CW_NT, "one cell per thread of a CW_NT block");
+  if (skip && *skip) return;
+  __shared__ T su[CW_NT * 30];
+  __shared__ T sp[CW_NT * 4];
+  const int b = blockIdx.x, first = b * CW_NT;
+  const int F = op.A + 1;
+  const long long nu = 3ll * op.nP2;
+  cw_cell_block(op, x, b, op.nC - first < CW_NT ? op.nC - first : CW_NT,
+                (long long)first + threadIdx.x, op.mu,
+                [&](int n1) { return nu + (long long)F * n1; }, su, sp);
+}
+
+// Phase-2 epilogues finish N consecutive DOFs from i: load() reads what they
+// need besides the row sums (issued before those are formed, so that the
+// loads do not wait for the sums, nor those of one DOF for the store of the
+// one before), finish() stores and returns the partial of a reduction.
+template <typename T, int N>
+struct CwPre {
+  T r[N], z[N];
+  bool m[N];
+};
+
+// Plain application: y = A x, or y = b - A x with b; rows with dmask set
+// give 0.
 template <typename T>
 struct CwEpiApplyT {
   T* y;
@@ -226,10 +274,21 @@ struct CwEpiApplyT {
   const uint8_t* mask;
   __device__ __forceinline__ bool skipped() const { return false; }
   __device__ __forceinline__ void prep() {}
-  __device__ __forceinline__ double operator()(long long i, T ax) const {
-    T v = b ? b[i] - ax : ax;
-    if (mask && mask[i]) v = (T)0;
-    y[i] = v;
+  template <int N>
+  __device__ __forceinline__ void load(long long i, CwPre<T, N>& p) const {
+#pragma unroll
+    for (int c = 0; c < N; ++c) p.r[c] = (T)0;
+    if (b) load_nc<T, N>(b + i, p.r);
+#pragma unroll
+    for (int c = 0; c < N; ++c) p.m[c] = mask && mask[i + c];
+  }
+  template <int N>
+  __device__ __forceinline__ double finish(long long i, const T (&ax)[N],
+                                           const CwPre<T, N>& p) const {
+    T v[N];
+#pragma unroll
+    for (int c = 0; c < N; ++c) v[c] = p.m[c] ? (T)0 : (b ? p.r[c] - ax[c] : ax[c]);
+    __builtin_memcpy(y + i, v, sizeof(T) * N);
     return 0.0;
   }
 };
@@ -256,6 +315,10 @@ cw_rows_kernel(CellOpT<T> op, const T* __restrict__ x, Epi epi, double* __restri
       const int lane = threadIdx.x % GU;
       const int a = tile * RU + threadIdx.x / GU;
       if (a < op.nP2) {
+        // GU = 1: the thread finishes the node's three rows, else one lane each
+        CwPre<T, (GU == 1 ? 3 : 1)> pre;
+        const long long o = GU == 1 ? 3ll * a : 3ll * a + (lane < 3 ? lane : 2);
+        epi.load(o, pre);
         const int kb = op.inc2_rp[a], ke = op.inc2_rp[a + 1];
         T y0 = (T)0, y1 = (T)0, y2 = (T)0;
         // the node's entries are contiguous: two per lane per trip, loads
@@ -279,19 +342,21 @@ cw_rows_kernel(CellOpT<T> op, const T* __restrict__ x, Epi epi, double* __restri
           y1 += __shfl_xor(y1, off, 64);
           y2 += __shfl_xor(y2, off, 64);
         }
-        if constexpr (GU == 1) {           // one thread per row: all three rows
-          acc += epi(3ll * a, y0);
-          acc += epi(3ll * a + 1, y1);
-          acc += epi(3ll * a + 2, y2);
+        if constexpr (GU == 1) {
+          const T ax[3] = {y0, y1, y2};
+          acc += epi.finish(o, ax, pre);
         } else if (lane < 3) {
-          const T yc = lane == 0 ? y0 : (lane == 1 ? y1 : y2);
-          acc += epi(3ll * a + lane, yc);
+          const T ax[1] = {lane == 0 ? y0 : (lane == 1 ? y1 : y2)};
+          acc += epi.finish(o, ax, pre);
         }
       }
     } else {
       const int lane = threadIdx.x % GP;
       const int c = (tile - ntu) * RP + threadIdx.x / GP;
       if (c < op.nP1) {
+        CwPre<T, 1> pre;
+        const long long o = nu + (long long)F * c + (lane < F ? lane : F - 1);
+        epi.load(o, pre);
         T yd = (T)0;
         const int kb = op.inc1_rp[c], ke = op.inc1_rp[c + 1];
         for (int k = kb + lane; k < ke; k += GP) yd += Yp[op.pe1[k]];
@@ -304,11 +369,9 @@ cw_rows_kernel(CellOpT<T> op, const T* __restrict__ x, Epi epi, double* __restri
           const T* xp = x + nu + (long long)F * op.ci11[k];
           const T mm = op.M1[k];
           T xv[F], st[F];
+          load_nc<T, F>(xp, xv);
 #pragma unroll
-          for (int g = 0; g < F; ++g) {
-            xv[g] = xp[g];
-            st[g] = g >= 1 ? op.St[(g - 1) * n11 + k] : (T)0;
-          }
+          for (int g = 0; g < F; ++g) st[g] = g >= 1 ? op.St[(g - 1) * n11 + k] : (T)0;
 #pragma unroll
           for (int g = 0; g < F; ++g) {
             m[g] += mm * xv[g];
@@ -332,7 +395,8 @@ cw_rows_kernel(CellOpT<T> op, const T* __restrict__ x, Epi epi, double* __restri
         if (lane < F) {
 #pragma unroll
           for (int g = 0; g < F; ++g) mine += op.C[lane * MPET_MAXF + g] * m[g];
-          acc += epi(nu + (long long)F * c + lane, mine);
+          const T ax[1] = {mine};
+          acc += epi.finish(o, ax, pre);
         }
       }
     }

@@ -80,8 +80,25 @@ struct CwEpiK1 {
   T s = 0, c1 = 0;
   __device__ __forceinline__ bool skipped() const { return *skip != 0; }
   __device__ __forceinline__ void prep() { k1_scalars(st, s, c1); }
-  __device__ __forceinline__ double operator()(long long i, T ax) const {
-    return e(i, ax, s, c1);
+  template <int N>
+  __device__ __forceinline__ void load(long long i, CwPre<T, N>& p) const {
+    load_nc<T, N>(e.r1 + i, p.r);
+    load_nc<T, N>(e.z + i, p.z);
+#pragma unroll
+    for (int c = 0; c < N; ++c) p.m[c] = e.mask && e.mask[i + c];
+  }
+  template <int N>
+  __device__ __forceinline__ double finish(long long i, const T (&ax)[N],
+                                           const CwPre<T, N>& p) const {
+    T y[N];
+    double acc = 0.0;
+#pragma unroll
+    for (int c = 0; c < N; ++c) {
+      y[c] = p.m[c] ? (T)0 : s * ax[c] - c1 * p.r[c];
+      acc += (double)(s * p.z[c]) * (double)y[c];
+    }
+    __builtin_memcpy(e.y + i, y, sizeof(T) * N);
+    return acc;
   }
 };
 
