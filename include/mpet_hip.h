@@ -672,6 +672,32 @@ int mpet_batch_create(const MpetBatchOpDesc* op64, const MpetBatchOpDesc* op32,
                       void** handle);
 int mpet_batch_destroy(void* h);
 
+/* The packed operator cell by cell (as MpetCellOpDesc, the tables of all
+ * instances concatenated): every instance's cells padded to whole blocks of
+ * cells_per_block (256), nblk blocks in all; table stride 256 nblk.  node2 =
+ * global P2 node, node1 = packed DOF of the P1 node's p_0; geometry in FP64
+ * and (mixed) FP32; entries, slots and partials numbered through.  mu is a
+ * HOST array of K values, the rest device arrays that must outlive the
+ * handle. */
+typedef struct {
+  int32_t nblk, cells_per_block, npart2, npart1;
+  const int32_t *blk_inst, *blk_cells;     /* instance and cells of a block */
+  const int32_t *node2, *node1;
+  const double* geom64;
+  const float* geom32;
+  const double* mu;
+  const int32_t *bq2, *lrp2, *pe2;
+  const int16_t* lsl2;
+  const int32_t *bq1, *lrp1, *pe1;
+  const int16_t* lsl1;
+  const int32_t *inc2_rp, *inc1_rp;
+} MpetBatchCellDesc;
+
+/* Apply the batch's operator cell by cell from now on, in both precisions
+ * (Kuu, Dv and Dt of its operator descriptors are not read any more and may
+ * have been NULL); once per handle, drops captured graphs. */
+int mpet_batch_set_cell_operator(void* h, const MpetBatchCellDesc* desc);
+
 /* One time step of the instances with active[k] != 0 (NULL: all): for each,
  * the solve of mpet_solver_solve on its part of the packed b and x
  * (packed numbering).  stats: host array of K entries.  Synchronises. */

@@ -59,10 +59,23 @@ class BatchLayout(C.Structure):
                 ("pd_off", C.c_void_p)]
 
 
+class BatchCellDesc(C.Structure):
+    _fields_ = [(k, C.c_int32) for k in ("nblk", "cells_per_block", "npart2", "npart1")] + \
+        [(k, C.c_void_p) for k in ("blk_inst", "blk_cells", "node2", "node1", "geom64", "geom32",
+                                   "mu", "bq2", "lrp2", "pe2", "lsl2", "bq1", "lrp1", "pe1",
+                                   "lsl1", "inc2_rp", "inc1_rp")]
+
+
+# Cells from which a batch's operator runs cell by cell (three launches and a
+# third of the bytes of the packed assembled values, two launches).
+BATCH_CELLS = 20000
+
+
 def _bind():
     L = _lib.lib()
     P = C.c_void_p
-    for name, args in (("mpet_batch_create", [P, P, P, P, P, P, C.POINTER(C.c_void_p)]),
+    for name, args in (("mpet_batch_set_cell_operator", [P, P]),
+                       ("mpet_batch_create", [P, P, P, P, P, P, C.POINTER(C.c_void_p)]),
                        ("mpet_batch_destroy", [P]),
                        ("mpet_batch_solve", [P, P, P, P, P, P]),
                        ("mpet_batch_apply", [P, C.c_int, P, P, P, P]),
@@ -256,6 +269,7 @@ class MPETBatch:
                 raise ValueError("all instances of a batch must be on one device")
         self.engines = build_engines(self.solvers, precision)
         self.keep = []
+        self.cells = sum(e.space.mesh.num_cells() for e in self.engines) >= BATCH_CELLS
         self._layout()
         self._pack_operator()
         self._pack_preconditioner()
@@ -271,6 +285,9 @@ class MPETBatch:
                                   pc if precision == "mixed" else None, C.byref(self.opt),
                                   C.byref(h)))
         self.handle = h
+        if self.cells:
+            self.cell_desc = self._pack_cells()
+            check(L.mpet_batch_set_cell_operator(h, C.byref(self.cell_desc)))
         self._state_views()
         self.stats = None
         self.tuning = None
@@ -384,9 +401,11 @@ class MPETBatch:
         nz = self.nnz_off
         L = _lib.lib()
         sptr = _lib.stream_ptr()
-        vals = {}
-        for name, kind, ncomp in (("Kuu", "22", 9), ("Dv", "21", 3), ("Dt", "12", 3),
-                                  ("M1", "11", 1)):
+        # cell by cell, only the P1 x P1 block is read from assembled values
+        prims = (("M1", "11", 1),) if self.cells else \
+            (("Kuu", "22", 9), ("Dv", "21", 3), ("Dt", "12", 3), ("M1", "11", 1))
+        vals = dict.fromkeys(("Kuu", "Dv", "Dt"))
+        for name, kind, ncomp in prims:
             tot = int(nz[kind][-1])
             out = torch.empty(ncomp * tot, dtype=tdt, device=dev)
             view = out.view(ncomp, tot)
@@ -409,6 +428,57 @@ class MPETBatch:
                            ptr(vals["Kuu"]), ptr(vals["Dv"]), ptr(vals["Dt"]), ptr(vals["M1"]),
                            ptr(vals["St"]), ptr(self.p_inst), ptr(self.p_base),
                            ptr(self.coef_dev), ptr(self.dmask))
+
+    def _pack_cells(self):
+        """The instances' cell-wise tables (DeviceSystem.cell_op) packed into
+        one set (MpetBatchCellDesc)."""
+        dev = self.device
+        sys_ = [e.system for e in self.engines]
+        B = sys_[0].CELLS_PER_BLOCK
+        ops = [s.cell_op() for s in sys_]
+        nblk = [(o["nC"] + B - 1) // B for o in ops]
+        total = B * sum(nblk)
+
+        def tables(kind, width, node_of, inc_len):
+            node = torch.zeros(width, total, dtype=torch.int32, device=dev)
+            out = {k: [] for k in ("bq", "lrp", "pe", "rp", "lsl")}
+            parts = slots = at = 0
+            for k, (s, o) in enumerate(zip(sys_, ops)):
+                t = o[kind]
+                node[:, at:at + o["nC"]] = node_of(k, t["node"].view(width, -1))
+                for name, off in (("bq", parts), ("lrp", slots), ("rp", parts)):
+                    v = t[name].long() + off
+                    out[name].append(v if k == self.K - 1 else v[:-1])
+                out["pe"].append(t["pe"].long() + parts)
+                out["lsl"].append(t["lsl"])
+                parts += t["npart"]
+                slots += t["lsl"].numel()
+                at += nblk[k] * B
+            if max(3 * parts, slots) >= 2**31:
+                raise ValueError("batch too large for 32-bit cell tables")
+            r = {n: torch.cat(v) for n, v in out.items()}
+            r = {n: v if n == "lsl" else v.to(torch.int32) for n, v in r.items()}
+            assert r["rp"].numel() == inc_len + 1
+            return node, r, parts
+        n2, t2, np2 = tables("p2", 10, lambda k, t: t + int(self.p2_off[k]), self.nP2)
+        n1, t1, np1 = tables("p1", 4, lambda k, t: t * sys_[k].F
+                             + int(self.nu + self.pd_off[k]), self.nP1)
+        geom = torch.zeros(10, total, dtype=torch.float64, device=dev)
+        blk_cells, at = [], 0
+        for s, o, nb in zip(sys_, ops, nblk):
+            geom[:, at:at + o["nC"]] = s.cell_geom64().view(10, -1)
+            blk_cells += [min(B, o["nC"] - B * i) for i in range(nb)]
+            at += nb * B
+        geom32 = geom.float() if self.precision == "mixed" else None
+        inst = torch.as_tensor(np.repeat(np.arange(self.K, dtype=np.int32), nblk)).to(dev)
+        cells = torch.as_tensor(np.asarray(blk_cells, dtype=np.int32)).to(dev)
+        mu = np.array([s.mu for s in sys_], dtype=np.float64)
+        self.keep += [n2, n1, t2, t1, geom, geom32, inst, cells, mu]
+        return BatchCellDesc(sum(nblk), B, np2, np1, ptr(inst), ptr(cells), ptr(n2), ptr(n1),
+                             ptr(geom), ptr(geom32), ptr(mu),
+                             *(ptr(t2[k]) for k in ("bq", "lrp", "pe", "lsl")),
+                             *(ptr(t1[k]) for k in ("bq", "lrp", "pe", "lsl")), ptr(t2["rp"]),
+                             ptr(t1["rp"]))
 
     def _upload_hier(self, h, levels, coarse, params, mask0, nc, level0=None):
         dev = self.device

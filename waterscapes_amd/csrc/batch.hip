@@ -16,6 +16,10 @@
 // The AMG hierarchies of the instances are concatenated level by level
 // (block diagonal, amg_cycle.h) with a block-diagonal dense coarsest solve.
 //
+// The operator is applied from the assembled packed values, or (set with
+// mpet_batch_set_cell_operator, the large batches) cell by cell: cellwise.h
+// on the cells of all instances, each instance's cells in blocks of its own.
+//
 // MINRES keeps one state per instance.  Row tiles and vector segments never
 // straddle instances, so every partial sum belongs to one instance and one
 // block per instance finalises its scalars in a fixed order (deterministic).
@@ -23,7 +27,7 @@
 // operator rows, vector segments and preconditioner rows (through the
 // per-level row -> instance maps) are left alone, and the preconditioner
 // launches stop once every instance is inactive.
-#include "amg_cycle.h"
+#include "cellwise.h"
 #include "op_rows.h"
 #include <algorithm>
 #include <vector>
@@ -175,6 +179,176 @@ bop_p_kernel(BOp<T> op, const Tile* __restrict__ tiles, int part_off, const T* _
         if (b) mine = b[o] - mine;
         y[o] = msk ? (T)0 : mine;
       }
+    }
+  }
+  if (k1.st) {
+    const double bs = block_sum(acc);
+    if (threadIdx.x == 0) k1.partial[part_off + t] = bs;
+  }
+}
+
+// Packed cell-wise operator: the tables of cellwise.h with every instance's
+// cells padded to whole blocks (nC: the padded count, the tables' stride),
+// node1 = the packed DOF of the node's p_0, entries and partials of all
+// instances one after the other.
+template <typename T>
+struct BCell {
+  CellOpT<T> op;
+  const int* blk_inst;             // instance of each block
+  const int* blk_cells;            // its cells
+  const T* mu;                     // per instance
+};
+
+// Phase 1 (cw_cell_block) of one block; the blocks of instances that stopped
+// are left alone.
+template <typename T>
+__global__ void __launch_bounds__(CW_NT)
+bcw_cell_kernel(BCell<T> C, const T* __restrict__ x, const State* st, int parity) {
+  const int b = blockIdx.x, inst = C.blk_inst[b];
+  if (st && st[inst].inactive[parity]) return;
+  __shared__ T su[CW_NT * 30];
+  __shared__ T sp[CW_NT * 4];
+  cw_cell_block(C.op, x, b, C.blk_cells[b], (long long)b * CW_NT + threadIdx.x, C.mu[inst],
+                [](int n1) { return (long long)n1; }, su, sp);
+}
+
+// Row epilogue of phase 2 for N consecutive DOFs: plain / residual, or the
+// MINRES step (as bop_u_kernel); loads first, as cellwise.h's epilogues.
+template <typename T, int N>
+__device__ __forceinline__ void brow_load(const K1Args<T>& k1, const T* x, const T* b,
+                                          const uint8_t* dmask, long long o, CwPre<T, N>& p) {
+#pragma unroll
+  for (int c = 0; c < N; ++c) p.r[c] = p.z[c] = (T)0;
+  if (k1.st) {
+    load_nc<T, N>(k1.r1 + o, p.r);
+    load_nc<T, N>(x + o, p.z);
+  } else if (b) {
+    load_nc<T, N>(b + o, p.r);
+  }
+#pragma unroll
+  for (int c = 0; c < N; ++c) p.m[c] = dmask && dmask[o + c];
+}
+template <typename T, int N>
+__device__ __forceinline__ double brow_finish(const K1Args<T>& k1, T s, T c1, const T* b, T* y,
+                                              long long o, const T (&ax)[N],
+                                              const CwPre<T, N>& p) {
+  T out[N], v[N];
+  double acc = 0.0;
+#pragma unroll
+  for (int c = 0; c < N; ++c) {
+    if (k1.st) {
+      out[c] = p.m[c] ? (T)0 : s * ax[c] - c1 * p.r[c];
+      v[c] = s * p.z[c];
+      acc += (double)v[c] * (double)out[c];
+    } else {
+      out[c] = p.m[c] ? (T)0 : (b ? p.r[c] - ax[c] : ax[c]);
+    }
+  }
+  __builtin_memcpy(y + o, out, sizeof(T) * N);
+  if (k1.st) __builtin_memcpy(k1.v + o, v, sizeof(T) * N);
+  return acc;
+}
+
+// Phase 2, u rows: one thread per P2 node (2.3 partials a node), tiles of NT
+// nodes of one instance.
+template <typename T>
+__global__ void __launch_bounds__(NT)
+bcw_u_kernel(BCell<T> C, const Tile* __restrict__ tiles, const T* __restrict__ x,
+             const T* __restrict__ b, T* __restrict__ y, const uint8_t* __restrict__ dmask,
+             K1Args<T> k1) {
+  const int t = blockIdx.x;
+  const Tile tl = tiles[t];
+  T s, c1;
+  const bool active = k1_setup(k1, tl.inst, s, c1);
+  const CellOpT<T>& op = C.op;
+  double acc = 0.0;
+  const int a = tl.begin + threadIdx.x;
+  if (active && a < tl.end) {
+    CwPre<T, 3> pre;
+    brow_load(k1, x, b, dmask, 3ll * a, pre);
+    T ax[3] = {(T)0, (T)0, (T)0};
+    const int kb = op.inc2_rp[a], ke = op.inc2_rp[a + 1];
+    for (int k = kb; k < ke; k += 2) {
+      const int k2 = k + 1 < ke ? k + 1 : k;
+      T av[3], bv[3];
+      load_nc<T, 3>(op.Yu + 3ll * op.pe2[k], av);
+      load_nc<T, 3>(op.Yu + 3ll * op.pe2[k2], bv);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        ax[c] += av[c];
+        ax[c] += k + 1 < ke ? bv[c] : (T)0;
+      }
+    }
+    acc = brow_finish(k1, s, c1, b, y, 3ll * a, ax, pre);
+  }
+  if (k1.st) {
+    const double bs = block_sum(acc);
+    if (threadIdx.x == 0) k1.partial[t] = bs;
+  }
+}
+
+// Phase 2, p rows: GP lanes per P1 node, tiles of NT / GP nodes.
+constexpr int BGP = 8;
+template <typename T>
+__global__ void __launch_bounds__(NT)
+bcw_p_kernel(BOp<T> op, BCell<T> C, const Tile* __restrict__ tiles, int part_off,
+             const T* __restrict__ x, const T* __restrict__ b, T* __restrict__ y, K1Args<T> k1) {
+  const int t = blockIdx.x;
+  const Tile tl = tiles[t];
+  T s, c1;
+  const bool active = k1_setup(k1, tl.inst, s, c1);
+  double acc = 0.0;
+  const int lane = threadIdx.x % BGP;
+  const int c = tl.begin + threadIdx.x / BGP;
+  if (active && c < tl.end) {
+    const MpetBatchCoef& ic = op.coef[tl.inst];
+    const int F = ic.F;
+    CwPre<T, 1> pre;
+    const long long o = (long long)op.p_base[c] + (lane < F ? lane : F - 1);
+    brow_load(k1, x, b, op.dmask, o, pre);
+    T yd = 0;
+    for (int k = C.op.inc1_rp[c] + lane; k < C.op.inc1_rp[c + 1]; k += BGP)
+      yd += C.op.Yp[C.op.pe1[k]];
+    T m[MPET_MAXF], sv[MPET_MAXF];
+#pragma unroll
+    for (int g = 0; g < MPET_MAXF; ++g) { m[g] = 0; sv[g] = 0; }
+    const T* St = op.St + ic.st_base;
+    const long long n11 = ic.nnz11, kbase = ic.k11_base;
+    for (int k = op.rp11[c] + lane; k < op.rp11[c + 1]; k += BGP) {
+      const T* xp = x + op.ci11[k];
+      const T mm = op.M1[k];
+      T xv[MPET_MAXF], st[MPET_MAXF];
+#pragma unroll
+      for (int g = 0; g < MPET_MAXF; ++g) {
+        if (g < F) {
+          xv[g] = xp[g];
+          st[g] = g >= 1 ? St[(g - 1) * n11 + k - kbase] : (T)0;
+        }
+      }
+#pragma unroll
+      for (int g = 0; g < MPET_MAXF; ++g) {
+        if (g < F) {
+          m[g] += mm * xv[g];
+          if (g >= 1) sv[g] += st[g] * xv[g];
+        }
+      }
+    }
+    yd = group_allsum<BGP>(yd);
+    T mine = 0;
+#pragma unroll
+    for (int g = 0; g < MPET_MAXF; ++g) {
+      if (g < F) {
+        m[g] = group_allsum<BGP>(m[g]);
+        const T sg = group_allsum<BGP>(sv[g]);
+        if (lane == g) mine = (g == 0) ? yd : (T)ic.stiff[g] * sg;
+      }
+    }
+    if (lane < F) {
+#pragma unroll
+      for (int g = 0; g < MPET_MAXF; ++g)
+        if (g < F) mine += (T)ic.C[lane * MPET_MAXF + g] * m[g];
+      const T ax[1] = {mine};
+      acc = brow_finish(k1, s, c1, b, y, o, ax, pre);
     }
   }
   if (k1.st) {
@@ -390,6 +564,14 @@ struct Batch {
   Tile *utiles = nullptr, *ptiles = nullptr, *segs = nullptr;
   int nut = 0, npt = 0, nseg = 0;
   int *kr0 = nullptr, *kr1 = nullptr;   // K1 partial ranges per instance
+  // cell-wise operator (both precisions): its tiles and partial ranges
+  bool has_cw = false;
+  BCell<double> cw64;
+  BCell<float> cw32;
+  int ncblk = 0, ncut = 0, ncpt = 0;
+  Tile *cutiles = nullptr, *cptiles = nullptr;
+  int *ckr0 = nullptr, *ckr1 = nullptr;
+  std::vector<int64_t> p2_off, p1_off;
   int *sr0 = nullptr, *sr1 = nullptr;   // segment partial ranges per instance
   double* partial = nullptr;            // max(nut + npt, nseg)
   Precond<double> pc64;
@@ -426,12 +608,30 @@ BOp<T> make_bop(const MpetBatchOpDesc* d) {
 }
 
 template <typename T>
+const BCell<T>& cell_of(const Batch* B);
+
+template <typename T>
 void op_launch(const Batch* B, const BOp<T>& op, const T* x, const T* b, T* y, K1Args<T> k1,
                hipStream_t s) {
+  if (B->has_cw) {
+    const BCell<T>& C = cell_of<T>(B);
+    hipLaunchKernelGGL((bcw_cell_kernel<T>), dim3(B->ncblk), dim3(CW_NT), 0, s, C, x, k1.st,
+                       k1.parity);
+    hipLaunchKernelGGL((bcw_u_kernel<T>), dim3(B->ncut), dim3(NT), 0, s, C, B->cutiles, x, b, y,
+                       op.dmask, k1);
+    hipLaunchKernelGGL((bcw_p_kernel<T>), dim3(B->ncpt), dim3(NT), 0, s, op, C, B->cptiles,
+                       B->ncut, x, b, y, k1);
+    return;
+  }
   hipLaunchKernelGGL((bop_u_kernel<T>), dim3(B->nut), dim3(NT), 0, s, op, B->utiles, x, b, y,
                      k1);
   hipLaunchKernelGGL((bop_p_kernel<T>), dim3(B->npt), dim3(NT), 0, s, op, B->ptiles, B->nut, x,
                      b, y, k1);
+}
+
+template <typename T>
+const BCell<T>& cell_of(const Batch* B) {
+  if constexpr (sizeof(T) == 8) return B->cw64; else return B->cw32;
 }
 
 template <typename T>
@@ -458,8 +658,8 @@ void minres_iter(Batch* B, int i, hipStream_t s) {
   const int cur = i & 1, next = (i + 1) & 1;
   K1Args<T> k1{M.st, M.v, Ra, B->partial, cur};
   op_launch<T>(B, op_of<T>(B), M.z, nullptr, M.y, k1, s);
-  hipLaunchKernelGGL(bk1f_kernel, dim3(B->ninst), dim3(NT), 0, s, B->partial, B->kr0, B->kr1,
-                     M.st, cur);
+  hipLaunchKernelGGL(bk1f_kernel, dim3(B->ninst), dim3(NT), 0, s, B->partial,
+                     B->has_cw ? B->ckr0 : B->kr0, B->has_cw ? B->ckr1 : B->kr1, M.st, cur);
   hipLaunchKernelGGL((bk2_kernel<T>), dim3(B->nseg), dim3(NT), 0, s, B->segs, M.y, Rb, Ra, M.st,
                      cur);
   Skip sk;
@@ -591,6 +791,8 @@ int build_layout(Batch* B, const MpetBatchLayout* lay) {
   sr1[K] = (int)(sg_u.size() + sg_p.size());
   std::vector<Tile> segs = sg_u;
   segs.insert(segs.end(), sg_p.begin(), sg_p.end());
+  B->p2_off.assign(lay->p2_off, lay->p2_off + K + 1);
+  B->p1_off.assign(lay->p1_off, lay->p1_off + K + 1);
   B->nut = (int)ut.size();
   B->npt = (int)pt.size();
   B->nseg = (int)segs.size();
@@ -731,6 +933,89 @@ extern "C" int mpet_batch_create(const MpetBatchOpDesc* op64, const MpetBatchOpD
     return rc;
   }
   *handle = B;
+  return OK;
+}
+
+// Tiles of the cell-wise row kernels and their partial ranges.
+static int build_cell_layout(Batch* B) {
+  const int K = B->ninst;
+  std::vector<Tile> ut, pt;
+  std::vector<int> r0(K + 1), r1(K + 1);
+  for (int k = 0; k < K; ++k) {
+    r0[k] = (int)ut.size();
+    for (long long a = B->p2_off[k]; a < B->p2_off[k + 1]; a += NT)
+      ut.push_back(Tile{(int)a, (int)std::min<long long>(a + NT, B->p2_off[k + 1]), k, 0});
+  }
+  r0[K] = (int)ut.size();
+  for (int k = 0; k < K; ++k) {
+    r1[k] = (int)(ut.size() + pt.size());
+    for (long long c = B->p1_off[k]; c < B->p1_off[k + 1]; c += NT / BGP)
+      pt.push_back(Tile{(int)c, (int)std::min<long long>(c + NT / BGP, B->p1_off[k + 1]), k, 0});
+  }
+  r1[K] = (int)(ut.size() + pt.size());
+  B->ncut = (int)ut.size();
+  B->ncpt = (int)pt.size();
+  int rc;
+  if ((rc = upload(B, ut, &B->cutiles)) || (rc = upload(B, pt, &B->cptiles)) ||
+      (rc = upload(B, r0, &B->ckr0)) || (rc = upload(B, r1, &B->ckr1)))
+    return rc;
+  // fewer tiles than the structured kernels have (larger ones), so B->partial
+  // holds their partials too
+  return B->ncut + B->ncpt <= B->nut + B->npt ? OK : ERR_INVALID;
+}
+
+template <typename T>
+static int bcell_from_desc(Batch* B, const MpetBatchCellDesc* d, BCell<T>& C) {
+  int rc = alloc_n(B, (T**)&C.op.Yu, 3 * (size_t)d->npart2 + (size_t)d->npart1);
+  if (rc) return rc;
+  std::vector<T> mu(B->ninst);
+  for (int k = 0; k < B->ninst; ++k) mu[k] = (T)d->mu[k];
+  T* dmu = nullptr;
+  if ((rc = upload(B, mu, &dmu))) return rc;
+  CellOpT<T>& o = C.op;
+  o.nC = d->nblk * CW_NT;
+  o.nP2 = (int)B->p2_off[B->ninst];
+  o.nP1 = (int)B->p1_off[B->ninst];
+  o.node2 = d->node2;
+  o.node1 = d->node1;
+  o.bq2 = d->bq2; o.lrp2 = d->lrp2; o.pe2 = d->pe2; o.lsl2 = d->lsl2;
+  o.bq1 = d->bq1; o.lrp1 = d->lrp1; o.pe1 = d->pe1; o.lsl1 = d->lsl1;
+  o.inc2_rp = d->inc2_rp;
+  o.inc1_rp = d->inc1_rp;
+  o.npart2 = d->npart2;
+  o.npart1 = d->npart1;
+  o.geom = sizeof(T) == 8 ? (const T*)d->geom64 : (const T*)d->geom32;
+  o.Yp = o.Yu + 3ll * d->npart2;
+  C.blk_inst = d->blk_inst;
+  C.blk_cells = d->blk_cells;
+  C.mu = dmu;
+  return OK;
+}
+
+// The batch's operator cell by cell from now on (FP64, and FP32 in mixed
+// mode); captured graphs are dropped.
+extern "C" int mpet_batch_set_cell_operator(void* h, const MpetBatchCellDesc* d) {
+  Batch* B = (Batch*)h;
+  if (!B || !d || d->nblk < 1 || d->cells_per_block != CW_NT || d->npart2 < 1 ||
+      d->npart1 < 1 || !d->blk_inst || !d->blk_cells || !d->node2 || !d->node1 || !d->geom64 ||
+      (B->has_op32 && !d->geom32) || !d->mu || !d->bq2 || !d->lrp2 || !d->pe2 || !d->lsl2 ||
+      !d->bq1 || !d->lrp1 || !d->pe1 || !d->lsl1 || !d->inc2_rp || !d->inc1_rp || B->has_cw) {
+    mpet_set_error("mpet_batch_set_cell_operator: invalid argument");
+    return ERR_INVALID;
+  }
+  HIPCHK(hipDeviceSynchronize());
+  for (auto& g : B->graph) {
+    if (g) HIPCHK(hipGraphExecDestroy(g));
+    g = nullptr;
+  }
+  int rc;
+  if ((rc = build_cell_layout(B)) || (rc = bcell_from_desc(B, d, B->cw64)) ||
+      (B->has_op32 && (rc = bcell_from_desc(B, d, B->cw32)))) {
+    if (rc == ERR_INVALID) mpet_set_error("mpet_batch_set_cell_operator: invalid layout");
+    return rc;
+  }
+  B->ncblk = d->nblk;
+  B->has_cw = true;
   return OK;
 }
 
