@@ -139,13 +139,13 @@ typedef struct {
   /* Batches (NULL otherwise): instance of each row of this level, so that
    * the V-cycle skips the rows of instances whose solve has stopped. */
   const int32_t* grp;
-  /* Fused transfers (all NULL: residual, restriction and prolongation run
-   * one by one).  With one smoothing step, x = c D^-1 b: W = R - c (R A)
+  /* Fused transfers (W_v NULL: residual and restriction run one by one, Q_v
+   * NULL: prolongation and first post-smoothing step).  With one smoothing step, x = c D^-1 b: W = R - c (R A)
    * D^-1 (nc x n) and Q = P - c D^-1 (A P) (n x nc, values).  With more:
    * W = [-R A, R] (nc x 2n, acting on [x; b]) and Q on the pattern of A P
    * with value pairs ((A P)_ij, P_ij).  Columns and rows held at zero (mask0)
    * have zero entries.  lgW, lgQ: log2 of the lanes per row (three columns:
-   * at least 2); A_nnz: nonzeros of the level operator. */
+   * at least 2).  W and Q are independent of each other. */
   const int32_t* W_rp;
   const int32_t* W_ci;
   const void* W_v;
@@ -153,7 +153,6 @@ typedef struct {
   const int32_t* Q_ci;
   const void* Q_v;
   int32_t lgW, lgQ;
-  int64_t A_nnz;
   /* Sliced copies (off NULL: none) of the level operator (values A_sv) and
    * of Q (then Q_rp / Q_ci may be NULL and Q_v holds the sliced values). */
   MpetSlices A_s;

@@ -109,17 +109,23 @@ def test_slices_refuse_wide_columns():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("slice_rows", [1 << 30, 600, 1])
+@pytest.mark.parametrize("slice_rows,mixed_choice", [(1 << 30, False), (1 << 30, True),
+                                                     (600, True), (1, False), (1, True)])
 @pytest.mark.parametrize("n,A,degs", [(3, 1, (1,)), (5, 3, (1,)), (5, 2, (2,)), (6, 6, (3, 1)),
                                       (27, 1, (1,)), (27, 1, (2,))])
 @pytest.mark.parametrize("mode", ["fp64", "mixed"])
-def test_preconditioner_with_fused_transfers(n, A, degs, mode, slice_rows, monkeypatch):
+def test_preconditioner_with_fused_transfers(n, A, degs, mode, slice_rows, mixed_choice,
+                                              monkeypatch):
     import torch
     from test_gpu_solver import _ref_precond, _setup
     from waterscapes_amd import levels as lv
     from waterscapes_amd.amg import AmgParams
     monkeypatch.setattr(lv, "DENSE_TAIL_BYTES", 30 * 30 * 8)
     monkeypatch.setattr(lv, "SLICE_ROWS", slice_rows)
+    # every combination of the two fused transfers, level by level
+    turn = iter([(True, True), (False, True), (True, False), (False, False)] * 8)
+    monkeypatch.setattr(lv, "worth_fusing",
+                        lambda *a: next(turn) if mixed_choice else (True, True))
     big = dict(max_coarse=25) if n < 20 else {}
     _, _, dev, solver, dofs, _ = _setup(
         n=n, A=A, mode=mode, compact_plevel0=False, autotune=False,
@@ -128,7 +134,8 @@ def test_preconditioner_with_fused_transfers(n, A, degs, mode, slice_rows, monke
     dev_levels = solver._level_arrays(0 if mode == "fp64" else 1)
     for (levs, _), host in zip(dev_levels, (solver.levels, solver.plevels)):
         for ld, lev in zip(levs[:-1], host):
-            assert ("A_s" in ld) == (lev["n"] >= slice_rows) and "W_v" in ld
+            assert ("A_s" in ld) == (lev["n"] >= slice_rows)
+            assert mixed_choice or ("W_v" in ld and "Q_v" in ld)
     r = np.random.default_rng(2).standard_normal(dev.n)
     r[np.concatenate(dofs)] = 0.0
     dtype = torch.float64 if mode == "fp64" else torch.float32
@@ -142,3 +149,25 @@ def test_preconditioner_with_fused_transfers(n, A, degs, mode, slice_rows, monke
     for a, b in ((z[:nu], ref[:nu]), (z[nu:], ref[nu:])):
         assert np.linalg.norm(a - b) <= tol * np.linalg.norm(b)
     solver.close()
+
+
+def test_worth_fusing_by_bytes():
+    """W while it reads less than a launch's bytes more than R, Q while less
+    than a launch's bytes more than P and the level operator."""
+    import torch
+    from waterscapes_amd import levels as lv
+
+    def ld(nnz, compact=False):
+        d = dict(A_ci=torch.zeros(nnz), P_ci=torch.zeros(1000))
+        return dict(d, A_v16=None) if compact else d
+
+    def f(w, q, pair):
+        return dict(W_ci=torch.zeros(w), Q_ci=torch.zeros(q), Q_v=torch.zeros(q * (1 + pair)))
+    launch = int(lv.LAUNCH_BYTES)
+    assert lv.worth_fusing(ld(10**4), f(10**4, 10**4, 1), 4, 1000) == (True, True)
+    w = launch // 8 + 1000                    # 8 bytes an entry in FP32
+    assert lv.worth_fusing(ld(10**4), f(w - 1, 10, 0), 4, 1000)[0]
+    assert not lv.worth_fusing(ld(10**4), f(w + 1, 10, 0), 4, 1000)[0]
+    q = (launch + 8 * 1000 + 4 * 10**6) // 8
+    assert lv.worth_fusing(ld(10**6, True), f(10, q - 1, 0), 4, 1000)[1]
+    assert not lv.worth_fusing(ld(10**6, True), f(10, q + 1, 0), 4, 1000)[1]

@@ -245,11 +245,10 @@ def tune_hierarchy(levels_host, levels_dev, nc, dtype, heuristic, mask0=None, ca
         row = [0, 0, 0]
         mats = [("A", ld["A_rp"], ld["A_ci"], ld["A_v"], n, n)]
         if ncols:
-            if "W_v" in ld:       # fused transfers: the restriction's product
-                mats += [("W", ld["W_rp"], ld["W_ci"], ld["W_v"], ncols, 2 * n)]
-            else:
-                mats += [("P", ld["P_rp"], ld["P_ci"], ld["P_v"], n, ncols),
-                         ("R", ld["R_rp"], ld["R_ci"], ld["R_v"], ncols, n)]
+            if "Q_v" not in ld:
+                mats += [("P", ld["P_rp"], ld["P_ci"], ld["P_v"], n, ncols)]
+            mats += [("W", ld["W_rp"], ld["W_ci"], ld["W_v"], ncols, 2 * n) if "W_v" in ld else
+                     ("R", ld["R_rp"], ld["R_ci"], ld["R_v"], ncols, n)]
         for which, rp, ci, v, rows, cols in mats:
             j = {"A": 0, "P": 1, "R": 2, "W": 2}[which]
             if which == "A" and (l == len(levels_host) - 1 or "A_s" in ld):

@@ -271,11 +271,11 @@ spmm_row_kernel(int nrows, const int* __restrict__ rp, const int* __restrict__ c
 // and prolongation of the coarse correction e and the first post-smoothing
 // step from x' = x + P e are one product as well,
 //     b - A x' = r - (A P) e:  d = cr D^-1 (r - (A P) e),  x'' = x + P e + d,
-// with R A and A P formed at set-up.  On the P2 level A P has 0.28 of A's
-// nonzeros (7.2 against 25.4 M at 48^3): one of the level's two products with
-// A becomes one with A P, the residual, needed by the post-smoothing only,
-// shares its launch with the restriction, and on every level two launches
-// fewer depend on each other.
+// with R A and A P formed at set-up.  Each saves a dependent launch; which
+// level takes which follows from their bytes (levels.py): on the P2 level A P
+// has 0.28 of A's nonzeros (7.2 against 25.4 M at 48^3) and replaces a product
+// with A, while R A would only add to the residual, which the post-smoothing
+// needs anyway.
 //   one smoothing step (x = c D^-1 b):  W = R - c (R A) D^-1 acts on b alone
 //     and Q = P - c D^-1 (A P) on e alone;
 //   more steps: W = [-R A, R] acts on [x; b] (one buffer), Q holds the pairs
@@ -1035,7 +1035,6 @@ struct LevelDev {
   const int *Wrp = nullptr, *Wci = nullptr, *Qrp = nullptr, *Qci = nullptr;
   const T *Wv = nullptr, *Qv = nullptr;
   int lgW = 3, lgQ = 2;
-  long long nnz = 0;               // of the level operator
   // sliced copies of the level operator and of Q (off null: none)
   Sell<T> As, Qs;
   T *B = nullptr, *X = nullptr, *R = nullptr, *E = nullptr, *S1 = nullptr, *S2 = nullptr,
@@ -1231,16 +1230,14 @@ static ResArgs<T> res_args(const LevelDev<T>& L, const T* b, int NC) {
 }
 
 // Fused restriction (into level l + 1's right-hand side and first step) and
-// residual of level l after its pre-smoothing, one launch (res false: the
-// restriction alone).
+// residual of level l after its pre-smoothing, one launch.
 template <typename T, int NC>
-static void fused_down(const Hier<T>& H, int l, const T* b, Skip sk, hipStream_t s,
-                       bool res = true) {
+static void fused_down(const Hier<T>& H, int l, const T* b, Skip sk, hipStream_t s) {
   const LevelDev<T>& L = H.lev[l];
   const DownArgs<T> w = down_args(H, l, b);
   const ResArgs<T> a = res_args(L, b, NC);
   const int nbw = row_blocks(w.n, w.lg), nba = row_blocks(a.n, a.lg);
-  if (res && L.As.off) {
+  if (L.As.off) {
     const int ns = (L.n + 63) / 64, nbs = (ns + NT / 64 - 1) / (NT / 64);
     const SellEpi<T> E{b, nullptr, nullptr, nullptr, 0, 0, (T)L.vscale, L.R, nullptr, L.mask,
                        OutMap(), L.grp};
@@ -1252,7 +1249,7 @@ static void fused_down(const Hier<T>& H, int l, const T* b, Skip sk, hipStream_t
                          0, s, w, L.As, ns, (const T*)L.X, E, nbw, sk);
     return;
   }
-  const dim3 grid(nbw + (res ? nba : 0));
+  const dim3 grid(nbw + nba);
   if constexpr (sizeof(T) == 4) {
     if (L.v16) {
       hipLaunchKernelGGL((transfer_kernel<T, NC, true>), grid, dim3(NT), 0, s, w, a, nbw, sk);
@@ -1331,25 +1328,26 @@ static void vcycle(const Hier<T>& H, int l, const T* b, T bscale, T* out, Skip s
   smooth_from_zero<T, NC>(L, b, bscale, bcopy, sk, s, entered, k2);
   const T* bb = bcopy ? bcopy : b;
   const LevelDev<T>& C = H.lev[l + 1];
+  const bool enter = l + 1 < H.nlev - 1;
   if (L.Wv) {
     fused_down<T, NC>(H, l, bb, sk, s);
-    vcycle<T, NC>(H, l + 1, C.B, (T)1, C.E, sk, s, l + 1 < H.nlev - 1);
-    fused_up<T, NC>(H, l, bb, out, sk, s, om);
-    return;
-  }
-  spmm<T, NC, 1>(L, 0, L.X, bb, L.R, nullptr, 0, 0, sk, s);
-  if (l + 1 < H.nlev - 1) {
-    // restriction fused with the coarse level's first smoothing step (its
-    // pre-smoothing writes to C.X)
-    spmm<T, NC, 4>(L, 2, L.R, nullptr, C.B, C.D, 0, (T)C.cr[0], sk, s, C.dinv,
-                   first_dst(C, C.X));
-    vcycle<T, NC>(H, l + 1, C.B, (T)1, C.E, sk, s, true);
   } else {
-    spmm<T, NC, 0>(L, 2, L.R, nullptr, C.B, nullptr, 0, 0, sk, s);
-    vcycle<T, NC>(H, l + 1, C.B, (T)1, C.E, sk, s);
+    spmm<T, NC, 1>(L, 0, L.X, bb, L.R, nullptr, 0, 0, sk, s);
+    // restriction with the coarse level's first smoothing step (its
+    // pre-smoothing writes to C.X)
+    if (enter)
+      spmm<T, NC, 4>(L, 2, L.R, nullptr, C.B, C.D, 0, (T)C.cr[0], sk, s, C.dinv,
+                     first_dst(C, C.X));
+    else
+      spmm<T, NC, 0>(L, 2, L.R, nullptr, C.B, nullptr, 0, 0, sk, s);
   }
-  spmm<T, NC, 2>(L, 1, C.E, nullptr, L.X, nullptr, 0, 0, sk, s);
-  smooth_steps<T, NC>(L, bb, L.X, 0, out, sk, s, om);
+  vcycle<T, NC>(H, l + 1, C.B, (T)1, C.E, sk, s, enter);
+  if (L.Qv) {
+    fused_up<T, NC>(H, l, bb, out, sk, s, om);
+  } else {
+    spmm<T, NC, 2>(L, 1, C.E, nullptr, L.X, nullptr, 0, 0, sk, s);
+    smooth_steps<T, NC>(L, bb, L.X, 0, out, sk, s, om);
+  }
 }
 
 // Whether precond_apply can take a fused input update (k2): single
@@ -1494,7 +1492,7 @@ template <typename T>
 static bool joint_ok(const Precond<T>& P) {
   for (const Hier<T>* H : {&P.u, &P.p}) {
     for (int l = 0; l + 1 < H->nlev; ++l)
-      if (!H->lev[l].Wv || H->lev[l].As.off || H->lev[l].Qs.off) return false;
+      if (!H->lev[l].Wv || !H->lev[l].Qv || H->lev[l].As.off || H->lev[l].Qs.off) return false;
     if (H->nlev == 1 && H->cblk) return false;
   }
   return true;
@@ -1526,12 +1524,6 @@ static void precond_joint(const Precond<T>& P, const T* r, T* z, Skip sk, hipStr
   }
 }
 
-// Nonzeros of the P2 level from which its residual moves to the pressure
-// stream, behind the pressure blocks: the two chains then take about the
-// same time.  Below, kernels are launch-bound and the residual is cheapest
-// inside the restriction's launch.
-constexpr long long LATE_RESIDUAL_NNZ = 4ll << 20;
-
 // z = M^-1 r; with k2 (k2_fusable only) r is first made as k2 describes.
 template <typename T>
 static void precond_apply(const Precond<T>& P, const T* r, T* z, Skip sk, hipStream_t s,
@@ -1545,36 +1537,18 @@ static void precond_apply(const Precond<T>& P, const T* r, T* z, Skip sk, hipStr
     precond_joint(P, r, z, sk, s, ku, kp);
     return;
   }
-  const LevelDev<T>& U0 = P.u.lev[0];
-  const T us = (T)(1.0 / P.u.scale);
-  auto fork = [&] {                // pressure blocks on the second stream
-    if (!P.ps) return s;
+  hipStream_t sp = s;
+  if (P.ps) {                      // pressure blocks on the second stream
     (void)hipEventRecord(P.ev_fork, s);
     (void)hipStreamWaitEvent(P.ps, P.ev_fork, 0);
-    return P.ps;
-  };
-  auto join = [&] {
-    if (!P.ps) return;
+    sp = P.ps;
+  }
+  vcycle<T, 3>(P.u, 0, r, (T)(1.0 / P.u.scale), z, sk, s, false, ku);
+  precond_pressure(P, r, z, sk, sp, kp);
+  if (P.ps) {
     (void)hipEventRecord(P.ev_join, P.ps);
     (void)hipStreamWaitEvent(s, P.ev_join, 0);
-  };
-  if (P.ps && P.u.nlev > 1 && U0.Wv && U0.nnz >= LATE_RESIDUAL_NNZ) {
-    T* bcopy = vcycle_bcopy(U0, r, us);
-    smooth_from_zero<T, 3>(U0, r, us, bcopy, sk, s, false, ku);
-    const T* bb = bcopy ? bcopy : r;
-    const hipStream_t sp = fork();
-    fused_down<T, 3>(P.u, 0, bb, sk, s, false);
-    vcycle<T, 3>(P.u, 1, P.u.lev[1].B, (T)1, P.u.lev[1].E, sk, s, P.u.nlev > 2);
-    precond_pressure(P, r, z, sk, sp, kp);
-    spmm<T, 3, 1>(U0, 0, U0.X, bb, U0.R, nullptr, 0, 0, sk, sp);
-    join();
-    fused_up<T, 3>(P.u, 0, bb, z, sk, s, OutMap());
-    return;
   }
-  const hipStream_t sp = fork();
-  vcycle<T, 3>(P.u, 0, r, us, z, sk, s, false, ku);
-  precond_pressure(P, r, z, sk, sp, kp);
-  join();
 }
 template <typename T>
 static void precond_apply(const Precond<T>& P, const T* r, T* z, const int* skip,
@@ -1679,10 +1653,11 @@ static int build_hier(std::vector<void*>& allocs, const MpetHierDesc* d, int NC,
       }
       L.As = Sell<T>{ld.A_s.off, ld.A_s.base, ld.A_s.row, ld.A_s.dc, ld.A_sv};
     }
-    if (ld.W_v && l + 1 < H.nlev) {
-      if (!ld.W_rp || !ld.W_ci || !ld.Q_v || ld.lgW < 0 || ld.lgW > 6 || ld.lgQ < 0 ||
-          ld.lgQ > 6 || (NC == 3 && (ld.lgW < 2 || ld.lgQ < 2)) ||
-          (ld.Q_s.off ? !ld.Q_s.base || !ld.Q_s.row || !ld.Q_s.dc : !ld.Q_rp || !ld.Q_ci)) {
+    if (l + 1 < H.nlev && (ld.W_v || ld.Q_v)) {
+      const int lo = NC == 3 ? 2 : 0;
+      if ((ld.W_v && (!ld.W_rp || !ld.W_ci || ld.lgW < lo || ld.lgW > 6)) ||
+          (ld.Q_v && !ld.Q_s.off && (!ld.Q_rp || !ld.Q_ci || ld.lgQ < lo || ld.lgQ > 6)) ||
+          (ld.Q_v && ld.Q_s.off && (!ld.Q_s.base || !ld.Q_s.row || !ld.Q_s.dc))) {
         mpet_set_error("invalid hierarchy description (fused transfers)");
         return ERR_INVALID;
       }
@@ -1690,7 +1665,6 @@ static int build_hier(std::vector<void*>& allocs, const MpetHierDesc* d, int NC,
       L.Qrp = ld.Q_rp; L.Qci = ld.Q_ci; L.Qv = (const T*)ld.Q_v;
       L.lgW = ld.lgW;
       L.lgQ = ld.lgQ;
-      L.nnz = ld.A_nnz;
       if (ld.Q_s.off) L.Qs = Sell<T>{ld.Q_s.off, ld.Q_s.base, ld.Q_s.row, ld.Q_s.dc, ld.Q_v};
     }
   }

@@ -33,7 +33,7 @@ class AmgLevelDesc(C.Structure):
                 ("grp", C.c_void_p),
                 ("W_rp", C.c_void_p), ("W_ci", C.c_void_p), ("W_v", C.c_void_p),
                 ("Q_rp", C.c_void_p), ("Q_ci", C.c_void_p), ("Q_v", C.c_void_p),
-                ("lgW", C.c_int32), ("lgQ", C.c_int32), ("A_nnz", C.c_int64),
+                ("lgW", C.c_int32), ("lgQ", C.c_int32),
                 ("A_s", lv.Slices), ("A_sv", C.c_void_p), ("Q_s", lv.Slices)]
 
 

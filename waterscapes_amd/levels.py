@@ -8,9 +8,9 @@ dependent launches per level, each a few microseconds whatever its size).
 M is formed in FP64 from the same level values the V-cycle kernels read.
 
 Fused transfers: on the levels that stay sparse, residual and restriction
-are one product with W and prolongation and the first post-smoothing step
-one product with Q (csrc/amg_cycle.h, "Fused transfers"), formed here from
-R A and A P.
+are one launch with W and prolongation and the first post-smoothing step
+one with Q (csrc/amg_cycle.h, "Fused transfers"), formed here from R A and
+A P, where their bytes do not cost more than the launch they save.
 
 The reference leaves the cycle to hypre
 (mpet/mpettotalpressuresolver.py:448).
@@ -311,9 +311,9 @@ def _describe_slices(S, s):
 
 
 def add_fused(levs, hosts, params, dtype, mask0=None):
-    """Fused transfers of every level but the coarsest, added to the uploaded
-    level dicts `levs` (values in their precision); hosts: the host levels
-    (rho)."""
+    """Fused transfers of every level but the coarsest that is worth it, and
+    sliced copies, added to the uploaded level dicts `levs` (values in their
+    precision); hosts: the host levels (rho)."""
     for l, ld in enumerate(levs[:-1]):
         if "A_v16" in ld:
             av = ld["A_v16"].double() * ld["vscale"]
@@ -326,10 +326,32 @@ def add_fused(levs, hosts, params, dtype, mask0=None):
                             (ld["P_rp"], ld["P_ci"], ld["P_v"].double()),
                             (ld["R_rp"], ld["R_ci"], ld["R_v"].double()), ld["dinv"].double(),
                             deg, c0, mask0 if l == 0 else None)
+        size = 8 if dtype == 0 else 4
+        use_w, use_q = worth_fusing(ld, f, size, n := int(hosts[l]["n"]))
         tdt = torch.float64 if dtype == 0 else torch.float32
-        f["W_v"], f["Q_v"] = f["W_v"].to(tdt), f["Q_v"].to(tdt)
-        ld.update(f)
-        add_slices(ld, int(hosts[l]["n"]))
+        for k, use in (("W", use_w), ("Q", use_q)):
+            if use:
+                ld.update({f"{k}_rp": f[f"{k}_rp"], f"{k}_ci": f[f"{k}_ci"],
+                           f"{k}_v": f[f"{k}_v"].to(tdt)})
+        add_slices(ld, n)
+
+
+# Bytes that take as long as the launch a fused transfer saves: about 3 us of
+# a kernel that streams at 4.5 TB/s.
+LAUNCH_BYTES = 13.5e6
+
+
+def worth_fusing(ld, f, size, n):
+    """(use W, use Q) of a level: W is read instead of R, in one launch with
+    the residual instead of after it; Q instead of P and the level operator."""
+    def matrix(nnz, value):
+        return nnz * (value + 4)
+    a = ld["A_ci"].numel() * (4 if "A_v16" in ld else (size + 2 if n >= SLICE_ROWS
+                                                       else size + 4))
+    pr = matrix(ld["P_ci"].numel(), size)
+    w = matrix(f["W_ci"].numel(), size)
+    q = f["Q_v"].numel() * size + f["Q_ci"].numel() * (2 if n >= SLICE_ROWS else 4)
+    return w < pr + LAUNCH_BYTES, q < pr + a + LAUNCH_BYTES
 
 
 def _log2_lanes(avg, rows, nc):
@@ -346,13 +368,12 @@ def _log2_lanes(avg, rows, nc):
 
 def describe_fused(L, ld, n, ncoarse, nc):
     """Fill the fused-transfer part of an AmgLevelDesc."""
-    if "W_v" not in ld:
-        return
-    L.W_rp, L.W_ci, L.W_v = ptr(ld["W_rp"]), ptr(ld["W_ci"]), ptr(ld["W_v"])
-    L.Q_rp, L.Q_ci, L.Q_v = ptr(ld["Q_rp"]), ptr(ld["Q_ci"]), ptr(ld["Q_v"])
-    L.lgW = _log2_lanes(ld["W_ci"].numel() / max(ncoarse, 1), ncoarse, nc)
-    L.lgQ = _log2_lanes(ld["Q_ci"].numel() / max(n, 1), n, nc)
-    L.A_nnz = ld["A_ci"].numel()
+    if "W_v" in ld:
+        L.W_rp, L.W_ci, L.W_v = ptr(ld["W_rp"]), ptr(ld["W_ci"]), ptr(ld["W_v"])
+        L.lgW = _log2_lanes(ld["W_ci"].numel() / max(ncoarse, 1), ncoarse, nc)
+    if "Q_v" in ld:
+        L.Q_rp, L.Q_ci, L.Q_v = ptr(ld["Q_rp"]), ptr(ld["Q_ci"]), ptr(ld["Q_v"])
+        L.lgQ = _log2_lanes(ld["Q_ci"].numel() / max(n, 1), n, nc)
     if "A_s" in ld:
         _describe_slices(L.A_s, ld["A_s"])
         L.A_sv = ptr(ld["A_s"]["v"])
