@@ -268,16 +268,16 @@ bcw_u_kernel(BCell<T> C, const Tile* __restrict__ tiles, const T* __restrict__ x
     brow_load(k1, x, b, dmask, 3ll * a, pre);
     T ax[3] = {(T)0, (T)0, (T)0};
     const int kb = op.inc2_rp[a], ke = op.inc2_rp[a + 1];
-    for (int k = kb; k < ke; k += 2) {
-      const int k2 = k + 1 < ke ? k + 1 : k;
-      T av[3], bv[3];
-      load_nc<T, 3>(op.Yu + 3ll * op.pe2[k], av);
-      load_nc<T, 3>(op.Yu + 3ll * op.pe2[k2], bv);
+    // four partials in flight: the nodes of small instances have up to eight
+    for (int k = kb; k < ke; k += 4) {
+      T v[4][3];
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        ax[c] += av[c];
-        ax[c] += k + 1 < ke ? bv[c] : (T)0;
-      }
+      for (int j = 0; j < 4; ++j)
+        load_nc<T, 3>(op.Yu + 3ll * op.pe2[k + j < ke ? k + j : ke - 1], v[j]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) ax[c] += k + j < ke ? v[j][c] : (T)0;
     }
     acc = brow_finish(k1, s, c1, b, y, 3ll * a, ax, pre);
   }
