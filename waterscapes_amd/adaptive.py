@@ -93,6 +93,13 @@ def _const(v, name):
     return float(a)
 
 
+# Meshes from this size on bring the indicators to the host through pinned
+# memory of the estimator's own, one row copied out while the next is on its
+# way.  A whole call with and without: 40^3 x 6 tets (12 MB) 683 / 3088 us,
+# 32^3 (6.3 MB) 377 / 556, 24^3 (2.7 MB) 197 / 228, 14^3 (0.5 MB) 315 / 84.
+STAGED_CELLS = 1 << 16
+
+
 class ErrorEstimator:
     """Indicators of mpet/adaptivempetsolver.py:82-222 for a two-field
     MPETSolver (see the module docstring)."""
@@ -158,6 +165,9 @@ class ErrorEstimator:
         self.cell_f = torch.as_tensor(cell_f).to(dev)
         self.tmp = torch.empty(max(3 * self.nF, 1), dtype=torch.float64, device=dev)
         self.out = torch.empty(4 * d.nC, dtype=torch.float64, device=dev)
+        self.stage = None
+        if d.nC >= STAGED_CELLS:
+            self.stage = torch.empty((4, d.nC), dtype=torch.float64, pin_memory=True)
         self._cache = {}               # device node values of time-independent sources
         # lists of error estimate terms, one for each time (:155-159)
         self.eta_1s, self.eta_2s, self.eta_3s, self.eta_4s = [], [], [], []
@@ -228,8 +238,23 @@ class ErrorEstimator:
         check(_lib.lib().mpet_error_indicators(C.byref(d), ptr(x), ptr(xp), ptr(self.fac),
                                                self.nF, ptr(self.cell_f), ptr(self.tmp),
                                                ptr(self.out), _lib.stream_ptr()))
-        out = self.out.view(4, d.nC).cpu().numpy().copy()     # synchronises
+        out = self._to_host(self.out.view(4, d.nC))
         return out[0], out[1], out[2], out[3]
+
+    def _to_host(self, dev):
+        """A new host array with dev's values; synchronises."""
+        if self.stage is None:
+            return dev.cpu().numpy()
+        out = np.empty(dev.shape)
+        done = []
+        for k in range(4):
+            self.stage[k].copy_(dev[k], non_blocking=True)
+            done.append(torch.cuda.Event())
+            done[k].record()
+        for k in range(4):
+            done[k].synchronize()
+            out[k] = self.stage[k].numpy()
+        return out
 
     # -- reference bookkeeping (:165-222) --------------------------------------
     def estimate_error_at_t(self):

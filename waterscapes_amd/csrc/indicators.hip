@@ -29,15 +29,21 @@ namespace mpet {
 
 struct IGeom {
   double g[4][3];   // grad lambda_k
-  double v0[3];
   double vol, h;
 };
 
-__device__ __forceinline__ void igeom(const double* __restrict__ X, const int* __restrict__ cells,
-                                      int e, IGeom& G) {
-  double v[4][3];
-  for (int k = 0; k < 4; ++k)
-    for (int d = 0; d < 3; ++d) v[k][d] = X[3ll * cells[4 * e + k] + d];
+// Local vertices may be taken in any order p of the cell's own (a facet's
+// first, see ind_facet_kernel): vertex i is the cell's p[i], and the edge node
+// of i and j is found from the cell's own numbering (edges (2,3), (1,3),
+// (1,2), (0,3), (0,2), (0,1) after the four vertices).
+__device__ __forceinline__ int p2_edge(int i, int j) {
+  const int lo = i < j ? i : j, hi = i < j ? j : i;
+  return 4 + (lo == 0 ? 6 - hi : (lo == 1 ? 4 - hi : 0));
+}
+
+// Geometry from four vertices: gradients of the barycentric coordinates,
+// volume and diameter (longest edge).
+__device__ __forceinline__ void igeom(const double v[4][3], IGeom& G) {
   double J[3][3];
   for (int d = 0; d < 3; ++d)
     for (int k = 0; k < 3; ++k) J[d][k] = v[k + 1][d] - v[0][d];
@@ -62,11 +68,12 @@ __device__ __forceinline__ void igeom(const double* __restrict__ X, const int* _
     G.g[2][m] = Ji[1][m];
     G.g[3][m] = Ji[2][m];
     G.g[0][m] = -(Ji[0][m] + Ji[1][m] + Ji[2][m]);
-    G.v0[m] = v[0][m];
   }
   G.vol = fabs(det) / 6.0;
   double h2 = 0.0;
+#pragma unroll
   for (int i = 0; i < 4; ++i)
+#pragma unroll
     for (int j = i + 1; j < 4; ++j) {
       double s = 0.0;
       for (int d = 0; d < 3; ++d) s += (v[i][d] - v[j][d]) * (v[i][d] - v[j][d]);
@@ -75,92 +82,99 @@ __device__ __forceinline__ void igeom(const double* __restrict__ X, const int* _
   G.h = sqrt(h2);
 }
 
-// P2 nodes: vertices 0..3, edges (2,3), (1,3), (1,2), (0,3), (0,2), (0,1).
-// The node loops below are unrolled, so every index into the geometry and
-// the barycentric point is a compile-time constant (no private-memory
-// arrays).
-__device__ constexpr int kEdge[6][2] = {{2, 3}, {1, 3}, {1, 2}, {0, 3}, {0, 2}, {0, 1}};
-
-// grad phi_a at barycentric point l: sum_k dphi_a/dlambda_k grad lambda_k.
-__device__ __forceinline__ void p2_grad(const IGeom& G, const double l[4], int a, double out[3]) {
-  if (a < 4) {
-    const double s = 4.0 * l[a] - 1.0;
-    for (int m = 0; m < 3; ++m) out[m] = s * G.g[a][m];
-  } else {
-    const int i = kEdge[a - 4][0], j = kEdge[a - 4][1];
-    for (int m = 0; m < 3; ++m) out[m] = 4.0 * (l[j] * G.g[i][m] + l[i] * G.g[j][m]);
-  }
-}
-
-// Hessian of phi_a (constant): 4 g_a g_a^T (vertex), 4 (g_i g_j^T + g_j g_i^T) (edge).
-__device__ __forceinline__ void p2_hess(const IGeom& G, int a, double H[3][3]) {
-  for (int m = 0; m < 3; ++m)
-    for (int q = 0; q < 3; ++q) {
-      if (a < 4) {
-        H[m][q] = 4.0 * G.g[a][m] * G.g[a][q];
-      } else {
-        const int i = kEdge[a - 4][0], j = kEdge[a - 4][1];
-        H[m][q] = 4.0 * (G.g[i][m] * G.g[j][q] + G.g[j][m] * G.g[i][q]);
-      }
-    }
-}
-
-// grad u (G[i][j] = d_j u_i) at barycentric point l of cell geometry G.
-__device__ __forceinline__ void grad_u(const IGeom& Gm, const double l[4],
-                                       const double* __restrict__ x, const int* p2,
-                                       double Gu[3][3]) {
+// A P2 gradient is linear on the cell, so everything the indicators need of
+// u follows from grad u at the vertices,
+//   (grad u)_n = 4 u_n G_n - sum_j u_j G_j + 4 sum_{k != n} u_{nk} G_k
+// (G_j = grad lambda_j): div sigma = sum_n sigma_n G_n, the divergence by its
+// vertex values, a facet's tractions at its vertices and their means at the
+// edge midpoints.  (Summing basis gradients and Hessians node by node at
+// every point, and the facets' geometry at every point, took 5 times the
+// arithmetic: see the figures at the kernels.)
+// nd: the cell's ten node numbers in the local order; visit(n, g) with g[i][j]
+// = d_j u_i at vertex n, for the first NV vertices.
+template <int NV, typename V>
+__device__ __forceinline__ void vertex_gradients(const IGeom& G, const double* __restrict__ x,
+                                                 const int nd[10], V visit) {
+  double u[10][3];
+#pragma unroll
+  for (int a = 0; a < 10; ++a)
+    for (int i = 0; i < 3; ++i) u[a][i] = x[3ll * nd[a] + i];
+  double U[3][3];
+#pragma unroll
   for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j) Gu[i][j] = 0.0;
 #pragma unroll
-  for (int a = 0; a < 10; ++a) {
-    double gp[3];
-    p2_grad(Gm, l, a, gp);
-    const long long b = 3ll * p2[a];
-    for (int i = 0; i < 3; ++i) {
-      const double ui = x[b + i];
-      for (int j = 0; j < 3; ++j) Gu[i][j] += ui * gp[j];
-    }
+    for (int j = 0; j < 3; ++j)
+      U[i][j] = (u[0][i] * G.g[0][j] + u[1][i] * G.g[1][j]) +
+                (u[2][i] * G.g[2][j] + u[3][i] * G.g[3][j]);
+#pragma unroll
+  for (int n = 0; n < NV; ++n) {
+    double g[3][3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        double t = u[n][i] * G.g[n][j];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (k != n) t += u[p2_edge(n, k)][i] * G.g[k][j];
+        g[i][j] = 4.0 * t - U[i][j];
+      }
+    visit(n, g);
   }
 }
 
-// div sigma(u) = mu Lap u + (mu + lambda) grad div u (constant on the cell).
-__device__ __forceinline__ void div_sigma(const IGeom& Gm, const double* __restrict__ x,
-                                          const int* p2, double mu, double lm, double out[3]) {
-  out[0] = out[1] = out[2] = 0.0;
-#pragma unroll
-  for (int a = 0; a < 10; ++a) {
-    double H[3][3];
-    p2_hess(Gm, a, H);
-    const double tr = H[0][0] + H[1][1] + H[2][2];
-    const long long b = 3ll * p2[a];
-    for (int i = 0; i < 3; ++i) {
-      double s = mu * tr * x[b + i];
-      for (int j = 0; j < 3; ++j) s += (mu + lm) * H[i][j] * x[b + j];
-      out[i] += s;
-    }
-  }
-}
-
+// One thread per cell; the network count is a template argument so that the
+// pressure loops hold exactly A fields.  Bound by the FP64 arithmetic and the
+// registers it holds (two waves a SIMD): 24 us at 32^3 x 6 tets, A = 2 (both
+// kernels and the gather 79 us of a call's 367, the rest brings 6.3 MB to the
+// host; the call took 880 us with per-point gradients and Hessians and a
+// pageable copy).
+template <int A>
 __global__ void __launch_bounds__(128)
 ind_cell_kernel(MpetIndDesc d, const double* __restrict__ x, const double* __restrict__ xp,
                 double* __restrict__ out) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= d.nC) return;
-  const int A = d.A;
   const long long nu = 3ll * d.nP2;
   IGeom G;
-  igeom(d.coords, d.cells, e, G);
   int p2[10], v[4];
-  for (int a = 0; a < 10; ++a) p2[a] = d.cell_p2[10 * e + a];
   for (int k = 0; k < 4; ++k) v[k] = d.cells[4 * e + k];
-  // constant parts of RK_u, RK_u^-: div sigma(u) - sum_i alpha_i grad p_i
-  double cu[3], cup[3];
-  div_sigma(G, x, p2, d.mu, d.lmbda, cu);
-  div_sigma(G, xp, p2, d.mu, d.lmbda, cup);
+  for (int a = 0; a < 10; ++a) p2[a] = d.cell_p2[10 * e + a];
+  {
+    double X[4][3];
+    for (int k = 0; k < 4; ++k)
+      for (int m = 0; m < 3; ++m) X[k][m] = d.coords[3ll * v[k] + m];
+    igeom(X, G);
+  }
+  // constant parts of RK_u, RK_u^-: div sigma(u) - sum_i alpha_i grad p_i;
+  // div(u - u^-) at the vertices
+  double cu[3], cup[3] = {0, 0, 0}, dv[4] = {0, 0, 0, 0};
+  const double mu = d.mu, lm = d.lmbda;
+  auto add = [&](int n, const double g[3][3], double c[3]) {
+    const double tr = g[0][0] + g[1][1] + g[2][2];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      double s = lm * tr * G.g[n][i];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) s += mu * (g[i][j] + g[j][i]) * G.g[n][j];
+      c[i] += s;
+    }
+    return tr;
+  };
+#pragma unroll 1
+  for (int k = 0; k < 2; ++k) {                // one state's values live at a time
+    for (int i = 0; i < 3; ++i) {
+      cu[i] = cup[i];
+      cup[i] = 0.0;
+    }
+    vertex_gradients<4>(G, k ? xp : x, p2, [&](int n, const double g[3][3]) {
+      const double tr = add(n, g, cup);
+      dv[n] = k ? dv[n] - tr : tr;
+    });
+  }
   double r4 = 0.0;
 #pragma unroll
-  for (int j = 0; j < MPET_MAXF; ++j) {
-    if (j >= A) continue;
+  for (int j = 0; j < A; ++j) {
     double gp[3] = {0, 0, 0}, gpp[3] = {0, 0, 0};
     for (int k = 0; k < 4; ++k) {
       const long long q = nu + (long long)A * v[k] + j;
@@ -176,23 +190,8 @@ ind_cell_kernel(MpetIndDesc d, const double* __restrict__ x, const double* __res
     }
   }
   const double idt = 1.0 / d.dt;
-  // div(u - u^-) is linear on the cell: its values at the four vertices
-  double dv[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const double lk[4] = {k == 0 ? 1.0 : 0.0, k == 1 ? 1.0 : 0.0, k == 2 ? 1.0 : 0.0,
-                          k == 3 ? 1.0 : 0.0};
-    double sdv = 0.0;
-#pragma unroll
-    for (int a = 0; a < 10; ++a) {
-      double gphi[3];
-      p2_grad(G, lk, a, gphi);
-      const long long b = 3ll * p2[a];
-      for (int i = 0; i < 3; ++i) sdv += (x[b + i] - xp[b + i]) * gphi[i];
-    }
-    dv[k] = sdv;
-  }
   double zu = 0.0, zudt = 0.0, zp = 0.0, r4s = 0.0;
+#pragma unroll 1
   for (int q = 0; q < d.nq; ++q) {
     const double* l = d.qbary + 4 * q;
     const double w = d.qw[q];
@@ -217,11 +216,10 @@ ind_cell_kernel(MpetIndDesc d, const double* __restrict__ x, const double* __res
     zudt += w * rd2;
     // div(u - u^-) at the point (linear on the cell)
     const double du = l[0] * dv[0] + l[1] * dv[1] + l[2] * dv[2] + l[3] * dv[3];
-    double pj[MPET_MAXF], ppj[MPET_MAXF];
+    double pj[A], ppj[A];
 #pragma unroll
-    for (int j = 0; j < MPET_MAXF; ++j) {
+    for (int j = 0; j < A; ++j) {
       pj[j] = ppj[j] = 0.0;
-      if (j >= A) continue;
       for (int k = 0; k < 4; ++k) {
         const long long qq = nu + (long long)A * v[k] + j;
         pj[j] += l[k] * x[qq];
@@ -229,20 +227,18 @@ ind_cell_kernel(MpetIndDesc d, const double* __restrict__ x, const double* __res
       }
     }
 #pragma unroll
-    for (int j = 0; j < MPET_MAXF; ++j) {
-      if (j >= A) continue;
+    for (int j = 0; j < A; ++j) {
       double gj = 0.0;
       if (d.g)
         for (int m = 0; m < d.nkg; ++m)
           gj += d.Lg[q * d.nkg + m] * d.g[((long long)e * d.nkg + m) * A + j];
       double r = -gj - d.c[j] * (pj[j] - ppj[j]) * idt - d.alpha[j] * du * idt;
 #pragma unroll
-      for (int i = 0; i < MPET_MAXF; ++i)
-        if (i < A) r -= d.S[i * MPET_MAXF + j] * (pj[j] - pj[i]);
+      for (int i = 0; i < A; ++i) r -= d.S[i * MPET_MAXF + j] * (pj[j] - pj[i]);
       zp += w * r * r;
 #pragma unroll
-      for (int i = 0; i < MPET_MAXF; ++i)
-        if (i < A && d.S[i * MPET_MAXF + j] > 3.0e-16)
+      for (int i = 0; i < A; ++i)
+        if (d.S[i * MPET_MAXF + j] > 3.0e-16)
           r4s += w * d.S[i * MPET_MAXF + j] * ((pj[j] - ppj[j]) - (pj[i] - ppj[i])) *
                  (pj[j] - ppj[j]);
     }
@@ -254,137 +250,115 @@ ind_cell_kernel(MpetIndDesc d, const double* __restrict__ x, const double* __res
   out[3ll * d.nC + e] = r4 + r4s * G.vol;
 }
 
-// Barycentric coordinates of point P in cell geometry G.
-__device__ __forceinline__ void bary_of(const IGeom& G, const double P[3], double l[4]) {
-  double s = 0.0;
-  for (int k = 1; k < 4; ++k) {
-    l[k] = G.g[k][0] * (P[0] - G.v0[0]) + G.g[k][1] * (P[1] - G.v0[1]) +
-           G.g[k][2] * (P[2] - G.v0[2]);
-    s += l[k];
-  }
-  l[0] = 1.0 - s;
-}
-
-__constant__ int c_face[4][3] = {{1, 2, 3}, {0, 2, 3}, {0, 1, 3}, {0, 1, 2}};
-
-// sigma(u) n at barycentric point l of a cell (geometry G, P2 nodes p2).
-__device__ __forceinline__ void traction(const IGeom& G, const double l[4],
-                                         const double* __restrict__ x,
-                                         const int* __restrict__ p2, double mu, double lm,
-                                         const double n[3], double t[3]) {
-  double Gu[3][3];
-  grad_u(G, l, x, p2, Gu);
-  const double tr = Gu[0][0] + Gu[1][1] + Gu[2][2];
-  for (int i = 0; i < 3; ++i) {
-    double s = lm * tr * n[i];
-    for (int j = 0; j < 3; ++j) s += mu * (Gu[i][j] + Gu[j][i]) * n[j];
-    t[i] = s;
-  }
-}
-
-// sum_j alpha_j p_j at barycentric point l of a cell with vertices v.
-__device__ __forceinline__ double alpha_p(const MpetIndDesc& d, const double l[4],
-                                          const double* __restrict__ x,
-                                          const int* __restrict__ v, long long nu) {
-  double s = 0.0;
-#pragma unroll
-  for (int j = 0; j < MPET_MAXF; ++j) {
-    if (j >= d.A) continue;
-    double p = 0.0;
-    for (int k = 0; k < 4; ++k) p += l[k] * x[nu + (long long)d.A * v[k] + j];
-    s += d.alpha[j] * p;
-  }
-  return s;
-}
-
 // One interior facet: fac = (cell a, local face a, cell b, local face b).
 // out_f[0..2][t] = avg(h) int_F |RE_p|^2 (sum over j), |RE_u|^2, |RE_u,dt|^2.
-// The tractions of the two cells are formed one after the other (one
-// displacement gradient live at a time).
+// Each cell's vertices are taken facet first (the three shared ones in cell
+// a's order, found in cell b by their numbers), the opposite one last, so
+// that the tractions at the facet's vertices are the first three of
+// vertex_gradients and every register index is static.  The pressures are
+// continuous: their jump alpha_i (p_i^a - p_i^b) n is zero.  RE_u is linear on
+// the facet; the edge-midpoint rule takes the means of its vertex values.
+// Bound as the cell kernel: 48 us for the 32^3 mesh's 390,000 facets.
+template <int A>
 __global__ void __launch_bounds__(128)
 ind_facet_kernel(MpetIndDesc d, const double* __restrict__ x, const double* __restrict__ xp,
                  const int* __restrict__ fac, int nF, double* __restrict__ out_f) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= nF) return;
-  const int ca = fac[4 * t], la = fac[4 * t + 1], cb = fac[4 * t + 2];
-  const int A = d.A;
+  const int la = fac[4 * t + 1], lb = fac[4 * t + 3];
   const long long nu = 3ll * d.nP2;
-  IGeom Ga, Gb;
-  igeom(d.coords, d.cells, ca, Ga);
-  igeom(d.coords, d.cells, cb, Gb);
-  const int* pa = d.cell_p2 + 10ll * ca;
-  const int* pb = d.cell_p2 + 10ll * cb;
-  const int* va = d.cells + 4ll * ca;
-  const int* vb = d.cells + 4ll * cb;
-  // facet vertices (those of cell a's face la), outward normal of cell a
-  double P[3][3];
-  for (int k = 0; k < 3; ++k)
-    for (int m = 0; m < 3; ++m) P[k][m] = d.coords[3ll * va[c_face[la][k]] + m];
-  double nrm[3];
-  {
-    double e1[3], e2[3];
-    for (int m = 0; m < 3; ++m) {
-      e1[m] = P[1][m] - P[0][m];
-      e2[m] = P[2][m] - P[0][m];
-    }
-    nrm[0] = e1[1] * e2[2] - e1[2] * e2[1];
-    nrm[1] = e1[2] * e2[0] - e1[0] * e2[2];
-    nrm[2] = e1[0] * e2[1] - e1[1] * e2[0];
-  }
-  const double len = sqrt(nrm[0] * nrm[0] + nrm[1] * nrm[1] + nrm[2] * nrm[2]);
-  const double area = 0.5 * len;
-  double opp = 0.0;   // (opposite vertex of a - P0) . n  < 0 for the outward normal
-  for (int m = 0; m < 3; ++m) opp += (d.coords[3ll * va[la] + m] - P[0][m]) * nrm[m];
-  const double sg = opp > 0.0 ? -1.0 / len : 1.0 / len;
-  for (int m = 0; m < 3; ++m) nrm[m] *= sg;
-  const double havg = 0.5 * (Ga.h + Gb.h);
-  const double idt = 1.0 / d.dt;
-  // RE_p,j: constant on the facet
-  double fp = 0.0;
+  double re[3][3], rp[3][3], jn[A];
 #pragma unroll
-  for (int j = 0; j < MPET_MAXF; ++j) {
-    if (j >= A) continue;
-    double jn = 0.0;
-    for (int k = 0; k < 4; ++k) {
-      const double xa = x[nu + (long long)A * va[k] + j], xb = x[nu + (long long)A * vb[k] + j];
-      for (int m = 0; m < 3; ++m) jn += (xa * Ga.g[k][m] - xb * Gb.g[k][m]) * nrm[m];
+  for (int k = 0; k < 3; ++k)
+#pragma unroll
+    for (int i = 0; i < 3; ++i) re[k][i] = rp[k][i] = 0.0;
+#pragma unroll
+  for (int j = 0; j < A; ++j) jn[j] = 0.0;
+  double nrm[3] = {0.0, 0.0, 0.0}, area = 0.0, hsum = 0.0;
+  int fv[3] = {0, 0, 0};
+#pragma unroll 1
+  for (int side = 0; side < 2; ++side) {       // one cell's geometry live at a time
+    const int cell = fac[4 * t + 2 * side], opp = side ? lb : la;
+    const int* __restrict__ cv = d.cells + 4ll * cell;
+    const int* __restrict__ c2 = d.cell_p2 + 10ll * cell;
+    // local order: facet vertices, then the opposite one
+    int p[4];
+    p[0] = opp == 0 ? 1 : 0;
+    p[1] = opp <= 1 ? 2 : 1;
+    p[2] = opp <= 2 ? 3 : 2;
+    p[3] = opp;
+    int g4[4];
+    for (int k = 0; k < 4; ++k) g4[k] = cv[p[k]];
+    if (side) {                                 // cell a's order of the shared three
+      int q[3];
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        q[k] = g4[0] == fv[k] ? p[0] : (g4[1] == fv[k] ? p[1] : p[2]);
+      p[0] = q[0]; p[1] = q[1]; p[2] = q[2];
+      g4[0] = fv[0]; g4[1] = fv[1]; g4[2] = fv[2];
+    } else {
+      fv[0] = g4[0]; fv[1] = g4[1]; fv[2] = g4[2];
     }
-    const double r = -d.K[j] * jn;
-    fp += r * r;
-  }
-  fp *= area;
-  // RE_u = sum_j alpha_j (p_j^a - p_j^b) n - (sigma_a - sigma_b) n, and the
-  // same for the previous state, at the three edge midpoints.  The four
-  // (cell, state) tractions are formed one at a time, each cell's geometry
-  // recomputed, so that only one displacement gradient is live.
-  double fu = 0.0, fud = 0.0;
-#pragma unroll 1
-  for (int q = 0; q < 3; ++q) {
-    double X[3];
-    for (int m = 0; m < 3; ++m)   // midpoint of edge q (static indices into P)
-      X[m] = 0.5 * (q == 0 ? P[0][m] + P[1][m] : (q == 1 ? P[1][m] + P[2][m] : P[2][m] + P[0][m]));
-    double re[3] = {0.0, 0.0, 0.0}, rp[3] = {0.0, 0.0, 0.0};
-#pragma unroll 1
-    for (int c4 = 0; c4 < 4; ++c4) {
-      const int cell = (c4 & 1) ? cb : ca;
-      const double* xs = (c4 & 2) ? xp : x;
-      IGeom G;
-      igeom(d.coords, d.cells, cell, G);
-      double l[4];
-      bary_of(G, X, l);
-      double tt[3];
-      traction(G, l, xs, d.cell_p2 + 10ll * cell, d.mu, d.lmbda, nrm, tt);
-      const double ap = alpha_p(d, l, xs, d.cells + 4ll * cell, nu);
-      const double sg = (c4 & 1) ? 1.0 : -1.0;     // cell a: + p_a n - t_a; cell b: - p_b n + t_b
-      for (int i = 0; i < 3; ++i) {
-        const double c = sg * (tt[i] - ap * nrm[i]);
-        if (c4 & 2) rp[i] += c; else re[i] += c;
+    int nd[10];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) nd[k] = c2[p[k]];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = i + 1; j < 4; ++j) nd[p2_edge(i, j)] = c2[p2_edge(p[i], p[j])];
+    IGeom G;
+    {
+      double X[4][3];
+      for (int k = 0; k < 4; ++k)
+        for (int m = 0; m < 3; ++m) X[k][m] = d.coords[3ll * g4[k] + m];
+      igeom(X, G);
+      if (side == 0) {
+        // outward normal of cell a: -grad lambda of the opposite vertex
+        const double n = sqrt(G.g[3][0] * G.g[3][0] + G.g[3][1] * G.g[3][1] +
+                              G.g[3][2] * G.g[3][2]);
+        for (int m = 0; m < 3; ++m) nrm[m] = -G.g[3][m] / n;
+        area = 3.0 * G.vol * n;                 // |F| = 3 |K| |grad lambda_opp|
       }
     }
+    hsum += G.h;
+    const double sg = side ? 1.0 : -1.0;        // RE_u = -(sigma_a - sigma_b) n
+#pragma unroll
+    for (int j = 0; j < A; ++j) {
+      double s = 0.0;
+      for (int k = 0; k < 4; ++k) {
+        const double gn = G.g[k][0] * nrm[0] + G.g[k][1] * nrm[1] + G.g[k][2] * nrm[2];
+        s += x[nu + (long long)A * g4[k] + j] * gn;
+      }
+      jn[j] -= sg * s;
+    }
+    auto traction = [&](const double g[3][3], double (&r)[3]) {
+      const double tr = g[0][0] + g[1][1] + g[2][2];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        double s = d.lmbda * tr * nrm[i];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) s += d.mu * (g[i][j] + g[j][i]) * nrm[j];
+        r[i] += sg * s;
+      }
+    };
+    vertex_gradients<3>(G, x, nd, [&](int n, const double g[3][3]) { traction(g, re[n]); });
+    vertex_gradients<3>(G, xp, nd, [&](int n, const double g[3][3]) { traction(g, rp[n]); });
+  }
+  const double havg = 0.5 * hsum, idt = 1.0 / d.dt;
+  double fp = 0.0;
+#pragma unroll
+  for (int j = 0; j < A; ++j) fp += d.K[j] * jn[j] * d.K[j] * jn[j];
+  fp *= area;
+  double fu = 0.0, fud = 0.0;
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    const int o = q == 2 ? 0 : q + 1;
     double a2 = 0.0, d2 = 0.0;
+#pragma unroll
     for (int i = 0; i < 3; ++i) {
-      a2 += re[i] * re[i];
-      const double r = (re[i] - rp[i]) * idt;
+      const double m = 0.5 * (re[q][i] + re[o][i]);
+      const double r = (m - 0.5 * (rp[q][i] + rp[o][i])) * idt;
+      a2 += m * m;
       d2 += r * r;
     }
     fu += a2 * (area / 3.0);
@@ -418,11 +392,21 @@ using namespace mpet;
 static int launch_indicators(const MpetIndDesc* d, const double* x, const double* xp,
                              const int* fac, int nF, const int* cell_f, double* tmp,
                              double* out, hipStream_t stream, const char* who) {
-  hipLaunchKernelGGL(ind_cell_kernel, dim3((d->nC + 127) / 128), dim3(128), 0, stream, *d, x, xp,
-                     out);
+#define IND_CASE(N)                                                                            \
+  case N:                                                                                      \
+    hipLaunchKernelGGL((ind_cell_kernel<N>), dim3((d->nC + 127) / 128), dim3(128), 0, stream,  \
+                       *d, x, xp, out);                                                        \
+    if (nF > 0)                                                                                \
+      hipLaunchKernelGGL((ind_facet_kernel<N>), dim3((nF + 127) / 128), dim3(128), 0, stream,  \
+                         *d, x, xp, fac, nF, tmp);                                             \
+    break;
+  switch (d->A) {
+    IND_CASE(1) IND_CASE(2) IND_CASE(3) IND_CASE(4) IND_CASE(5) IND_CASE(6) IND_CASE(7)
+    IND_CASE(8)
+    default: break;
+  }
+#undef IND_CASE
   if (nF > 0) {
-    hipLaunchKernelGGL(ind_facet_kernel, dim3((nF + 127) / 128), dim3(128), 0, stream, *d, x,
-                       xp, fac, nF, tmp);
     hipLaunchKernelGGL(ind_gather_kernel, dim3((d->nC + 255) / 256), dim3(256), 0, stream,
                        d->nC, cell_f, (const double*)tmp, nF, out);
   }
