@@ -214,35 +214,33 @@ bcw_cell_kernel(BCell<T> C, const T* __restrict__ x, const State* st, int parity
 
 // Row epilogue of phase 2 for N consecutive DOFs: plain / residual, or the
 // MINRES step (as bop_u_kernel); loads first, as cellwise.h's epilogues.
+// (One source pointer, chosen before the load, and no conditional writes into
+// the struct: otherwise it ends in memory, 17 instead of 8 us for the u rows.)
 template <typename T, int N>
 __device__ __forceinline__ void brow_load(const K1Args<T>& k1, const T* x, const T* b,
-                                          const uint8_t* dmask, long long o, CwPre<T, N>& p) {
+                                          const uint8_t* dmask, long long o, T (&r)[N],
+                                          T (&z)[N], unsigned& m) {
+  const T* src = k1.st ? k1.r1 : b;
+  load_nc<T, N>((src ? src : x) + o, r);
+  load_nc<T, N>(x + o, z);
+  m = 0;
+  if (dmask)
 #pragma unroll
-  for (int c = 0; c < N; ++c) p.r[c] = p.z[c] = (T)0;
-  if (k1.st) {
-    load_nc<T, N>(k1.r1 + o, p.r);
-    load_nc<T, N>(x + o, p.z);
-  } else if (b) {
-    load_nc<T, N>(b + o, p.r);
-  }
-#pragma unroll
-  for (int c = 0; c < N; ++c) p.m[c] = dmask && dmask[o + c];
+    for (int c = 0; c < N; ++c) m |= dmask[o + c] ? 1u << c : 0u;
 }
 template <typename T, int N>
 __device__ __forceinline__ double brow_finish(const K1Args<T>& k1, T s, T c1, const T* b, T* y,
-                                              long long o, const T (&ax)[N],
-                                              const CwPre<T, N>& p) {
+                                              long long o, const T (&ax)[N], const T (&r)[N],
+                                              const T (&z)[N], unsigned m) {
   T out[N], v[N];
   double acc = 0.0;
 #pragma unroll
   for (int c = 0; c < N; ++c) {
-    if (k1.st) {
-      out[c] = p.m[c] ? (T)0 : s * ax[c] - c1 * p.r[c];
-      v[c] = s * p.z[c];
-      acc += (double)v[c] * (double)out[c];
-    } else {
-      out[c] = p.m[c] ? (T)0 : (b ? p.r[c] - ax[c] : ax[c]);
-    }
+    const bool dead = (m >> c) & 1u;
+    v[c] = s * z[c];
+    const T k = s * ax[c] - c1 * r[c], plain = b ? r[c] - ax[c] : ax[c];
+    out[c] = dead ? (T)0 : (k1.st ? k : plain);
+    acc += (double)v[c] * (double)out[c];
   }
   __builtin_memcpy(y + o, out, sizeof(T) * N);
   if (k1.st) __builtin_memcpy(k1.v + o, v, sizeof(T) * N);
@@ -264,8 +262,9 @@ bcw_u_kernel(BCell<T> C, const Tile* __restrict__ tiles, const T* __restrict__ x
   double acc = 0.0;
   const int a = tl.begin + threadIdx.x;
   if (active && a < tl.end) {
-    CwPre<T, 3> pre;
-    brow_load(k1, x, b, dmask, 3ll * a, pre);
+    T pr[3], pz[3];
+    unsigned pm;
+    brow_load(k1, x, b, dmask, 3ll * a, pr, pz, pm);
     T ax[3] = {(T)0, (T)0, (T)0};
     const int kb = op.inc2_rp[a], ke = op.inc2_rp[a + 1];
     // four partials in flight: the nodes of small instances have up to eight
@@ -279,7 +278,7 @@ bcw_u_kernel(BCell<T> C, const Tile* __restrict__ tiles, const T* __restrict__ x
 #pragma unroll
         for (int c = 0; c < 3; ++c) ax[c] += k + j < ke ? v[j][c] : (T)0;
     }
-    acc = brow_finish(k1, s, c1, b, y, 3ll * a, ax, pre);
+    acc = brow_finish(k1, s, c1, b, y, 3ll * a, ax, pr, pz, pm);
   }
   if (k1.st) {
     const double bs = block_sum(acc);
@@ -303,9 +302,10 @@ bcw_p_kernel(BOp<T> op, BCell<T> C, const Tile* __restrict__ tiles, int part_off
   if (active && c < tl.end) {
     const MpetBatchCoef& ic = op.coef[tl.inst];
     const int F = ic.F;
-    CwPre<T, 1> pre;
+    T pr[1], pz[1];
+    unsigned pm;
     const long long o = (long long)op.p_base[c] + (lane < F ? lane : F - 1);
-    brow_load(k1, x, b, op.dmask, o, pre);
+    brow_load(k1, x, b, op.dmask, o, pr, pz, pm);
     T yd = 0;
     for (int k = C.op.inc1_rp[c] + lane; k < C.op.inc1_rp[c + 1]; k += BGP)
       yd += C.op.Yp[C.op.pe1[k]];
@@ -348,7 +348,7 @@ bcw_p_kernel(BOp<T> op, BCell<T> C, const Tile* __restrict__ tiles, int part_off
       for (int g = 0; g < MPET_MAXF; ++g)
         if (g < F) mine += (T)ic.C[lane * MPET_MAXF + g] * m[g];
       const T ax[1] = {mine};
-      acc = brow_finish(k1, s, c1, b, y, o, ax, pre);
+      acc = brow_finish(k1, s, c1, b, y, o, ax, pr, pz, pm);
     }
   }
   if (k1.st) {
