@@ -445,6 +445,15 @@ int mpet_cell_geometry64(const MpetMeshDesc* mesh, double* geom, hipStream_t str
 int mpet_cell_op_apply(const MpetCellOpDesc* op, const void* x, const void* b, void* y,
                        void* work, hipStream_t stream);
 
+/* The two-field operator cell by cell, FP64 (same values as the which = 0
+ * CSR matrix of mpet_tf_expand_csr up to rounding): op's tables with A = F
+ * pressure fields per P1 node (1 <= A < MPET_MAXF), St: A x nnz11, its coef
+ * unused; y = A x or b - A x with the rows of op->dmask zeroed, work as for
+ * mpet_cell_op_apply. */
+int mpet_two_field_cell_apply(const MpetCellOpDesc* op, const MpetTwoFieldCoef* coef,
+                              const double* x, const double* b, double* y, double* work,
+                              hipStream_t stream);
+
 /* Scalar CSR SpMV (PETSc MatMult on AIJ, :493), int64 rowptr, lpr lanes
  * per row in {4,8,16,32,64}; optional residual b and row mask as above. */
 int mpet_csr_spmv(int dtype, long long nrows, const long long* rp, const int* ci,
@@ -609,6 +618,14 @@ int mpet_solver_set_cell_operator(void* h, const MpetCellOpDesc* op);
  * when the handle's FP64 operator is a CSR matrix.  No counterpart in the
  * reference (PETSc's MatMult on the assembled matrix, :493). */
 int mpet_solver_set_cell_operator64(void* h, const MpetCellOpDesc* op);
+
+/* MINRES iterations of an FP64 two-field solver handle
+ * (mpet_solver_create_csr) cell by cell (op != NULL; the handle allocates the
+ * work values and keeps copies of op and coef, op's arrays must outlive it)
+ * or back on the CSR matrix (op == NULL); residuals stay on the CSR matrix.
+ * The captured FP64 graph is dropped.  No counterpart in the reference. */
+int mpet_solver_set_two_field_cells(void* h, const MpetCellOpDesc* op,
+                                    const MpetTwoFieldCoef* coef);
 
 /* z = P^-1 r with the FP64 (dtype 0) or FP32 (1) preconditioner. */
 int mpet_precond_apply(void* h, int dtype, const void* r, void* z, hipStream_t stream);

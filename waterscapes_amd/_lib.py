@@ -134,6 +134,8 @@ def lib():
         "mpet_cell_op_apply": ([P, P, P, P, P, P], C.c_int),
         "mpet_solver_set_cell_operator": ([P, P], C.c_int),
         "mpet_solver_set_cell_operator64": ([P, P], C.c_int),
+        "mpet_solver_set_two_field_cells": ([P, P, P], C.c_int),
+        "mpet_two_field_cell_apply": ([P, P, P, P, P, P, P], C.c_int),
         "mpet_product_values": ([C.c_int64] + [P] * 10, C.c_int),
         "mpet_csr_spmv": ([C.c_int, C.c_longlong, P, P, P, P, P, P, P, C.c_int, P], C.c_int),
         "mpet_soa_convert": ([C.c_int, P, C.c_int, C.c_longlong, P, P], C.c_int),

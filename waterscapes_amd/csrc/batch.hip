@@ -208,8 +208,8 @@ bcw_cell_kernel(BCell<T> C, const T* __restrict__ x, const State* st, int parity
   if (st && st[inst].inactive[parity]) return;
   __shared__ T su[CW_NT * 30];
   __shared__ T sp[CW_NT * 4];
-  cw_cell_block(C.op, x, b, C.blk_cells[b], (long long)b * CW_NT + threadIdx.x, C.mu[inst],
-                [](int n1) { return (long long)n1; }, su, sp);
+  cw_cell_block<false>(C.op, x, b, C.blk_cells[b], (long long)b * CW_NT + threadIdx.x,
+                       C.mu[inst], [&](int n1) { return x[n1]; }, su, sp);
 }
 
 // Row epilogue of phase 2 for N consecutive DOFs: plain / residual, or the

@@ -35,6 +35,11 @@
 // order, so results are reproducible), plus the assembled P1 x P1 part, and
 // hands the row value to an epilogue (plain apply / masked residual, or the
 // fused MINRES step).  Cell tables are structure-of-arrays ([k * nC + e]).
+//
+// The two-field operator (TF; fields u, p_1..p_F, mpet/mpetsolver.py:196-201)
+// is the same cell by cell: its stress is s = mu (g + g^T) + (lambda tr g -
+// sum_f alpha_f p_f) I, still linear on the cell, and the p_f rows get
+// -alpha_f times the divergence that p0's row gets above.
 #pragma once
 #include "amg_cycle.h"
 
@@ -63,6 +68,7 @@ struct CellOpT {
   T C[MPET_MAXF * MPET_MAXF];
   T stiff[MPET_MAXF];
   T mu;
+  T lmbda, alpha[MPET_MAXF];        // two-field operator only
   const uint8_t* dmask;
   int lanes_u, lanes_p, xcd_chunk;
   int npart2, npart1;     // partials of all blocks (P2, P1)
@@ -75,6 +81,7 @@ using CellOp = CellOpT<float>;
 #define MPET_CW_CELLS 256
 #endif
 constexpr int CW_NT = MPET_CW_CELLS;   // cells per block of the cell kernel
+constexpr int TF_GU = 4, TF_GP = 8;   // lanes per two-field P2 / P1 node row
 
 // Index of the UFC edge joining local vertices j != k.
 __device__ __forceinline__ int cw_edge(int j, int k) {
@@ -84,13 +91,13 @@ __device__ __forceinline__ int cw_edge(int j, int k) {
 }
 
 // Phase 1 of one block: one thread per cell.  valid: the block's cells; at:
-// this thread's place in the cell tables (stride nC); p0(v): index in x of
-// the total pressure at node1 entry v.
+// this thread's place in the cell tables (stride nC); p0_of(v): the total
+// pressure at node1 entry v (TF: the isotropic stress of the pressures).
 // The block's partial lists do not depend on the results, so a thread's
 // first PRE of them are read before the cell's own loads and arithmetic:
 // after the barrier only the slot numbers are still to come (block 256,
 // 48^3: ~790 P2 partials, three to four a thread).
-template <typename T, typename P0>
+template <bool TF, typename T, typename P0>
 __device__ __forceinline__ void cw_cell_block(const CellOpT<T>& op, const T* __restrict__ x,
                                               int b, int valid, long long at, T mu, P0 p0_of,
                                               T* su, T* sp) {
@@ -128,7 +135,7 @@ __device__ __forceinline__ void cw_cell_block(const CellOpT<T>& op, const T* __r
 #pragma unroll
     for (int k = 0; k < 10; ++k) load_nc<T, 3>(x + 3ll * n2[k], u[k]);
 #pragma unroll
-    for (int v = 0; v < 4; ++v) p0[v] = x[p0_of(n1[v])];
+    for (int v = 0; v < 4; ++v) p0[v] = p0_of(n1[v]);
     // U = sum_j u_j (x) G_j
     T U[3][3];
 #pragma unroll
@@ -155,9 +162,10 @@ __device__ __forceinline__ void cw_cell_block(const CellOpT<T>& op, const T* __r
           for (int d = 0; d < 3; ++d) g[b][d] += (T)4 * u[m][b] * G[k][d];
       }
       tr[n] = g[0][0] + g[1][1] + g[2][2];
-      s[n][0] = (T)2 * mu * g[0][0] + p0[n];
-      s[n][1] = (T)2 * mu * g[1][1] + p0[n];
-      s[n][2] = (T)2 * mu * g[2][2] + p0[n];
+      const T iso = TF ? op.lmbda * tr[n] + p0[n] : p0[n];
+      s[n][0] = (T)2 * mu * g[0][0] + iso;
+      s[n][1] = (T)2 * mu * g[1][1] + iso;
+      s[n][2] = (T)2 * mu * g[2][2] + iso;
       s[n][3] = mu * (g[0][1] + g[1][0]);
       s[n][4] = mu * (g[0][2] + g[2][0]);
       s[n][5] = mu * (g[1][2] + g[2][1]);
@@ -240,7 +248,7 @@ __device__ __forceinline__ void cw_cell_block(const CellOpT<T>& op, const T* __r
 
 // (A template, so that the translation units including this header share
 // one instance.)
-template <int NTB, typename T>
+template <int NTB, typename T, bool TF>
 __global__ void __launch_bounds__(NTB)
 cw_cell_kernel(CellOpT<T> op, const T* __restrict__ x, const int* __restrict__ skip) {
   static_assert(NTB == CW_NT, "one cell per thread of a CW_NT block");
@@ -248,11 +256,19 @@ cw_cell_kernel(CellOpT<T> op, const T* __restrict__ x, const int* __restrict__ s
   __shared__ T su[CW_NT * 30];
   __shared__ T sp[CW_NT * 4];
   const int b = blockIdx.x, first = b * CW_NT;
-  const int F = op.A + 1;
-  const long long nu = 3ll * op.nP2;
-  cw_cell_block(op, x, b, op.nC - first < CW_NT ? op.nC - first : CW_NT,
-                (long long)first + threadIdx.x, op.mu,
-                [&](int n1) { return nu + (long long)F * n1; }, su, sp);
+  const int F = op.A + (TF ? 0 : 1);
+  const T* __restrict__ xp = x + 3ll * op.nP2;
+  const int valid = op.nC - first < CW_NT ? op.nC - first : CW_NT;
+  const long long at = (long long)first + threadIdx.x;
+  if constexpr (TF)
+    cw_cell_block<true>(op, x, b, valid, at, op.mu, [&](int n1) {
+      T p = (T)0;
+      for (int f = 0; f < F; ++f) p -= op.alpha[f] * xp[(long long)F * n1 + f];
+      return p;
+    }, su, sp);
+  else
+    cw_cell_block<false>(op, x, b, valid, at, op.mu,
+                         [&](int n1) { return xp[(long long)F * n1]; }, su, sp);
 }
 
 // Phase-2 epilogues finish N consecutive DOFs from i: load() reads what they
@@ -298,7 +314,7 @@ using CwEpiApply = CwEpiApplyT<float>;
 // writes all three rows), GP lanes per P1 node row, grid-stride
 // over row tiles (u tiles first), XCD-aware tile order.  The epilogue's
 // per-row results are summed per block into partial[blockIdx.x] (when given).
-template <int F, int GU, int GP, typename Epi, typename T>
+template <int F, int GU, int GP, bool TF, typename Epi, typename T>
 __global__ void __launch_bounds__(256)
 cw_rows_kernel(CellOpT<T> op, const T* __restrict__ x, Epi epi, double* __restrict__ partial) {
   if (epi.skipped()) return;
@@ -371,11 +387,12 @@ cw_rows_kernel(CellOpT<T> op, const T* __restrict__ x, Epi epi, double* __restri
           T xv[F], st[F];
           load_nc<T, F>(xp, xv);
 #pragma unroll
-          for (int g = 0; g < F; ++g) st[g] = g >= 1 ? op.St[(g - 1) * n11 + k] : (T)0;
+          for (int g = 0; g < F; ++g)
+            st[g] = TF ? op.St[g * n11 + k] : (g >= 1 ? op.St[(g - 1) * n11 + k] : (T)0);
 #pragma unroll
           for (int g = 0; g < F; ++g) {
             m[g] += mm * xv[g];
-            if (g >= 1) sv[g] += st[g] * xv[g];
+            if (TF || g >= 1) sv[g] += st[g] * xv[g];
           }
         }
 #pragma unroll
@@ -390,7 +407,8 @@ cw_rows_kernel(CellOpT<T> op, const T* __restrict__ x, Epi epi, double* __restri
             sg += __shfl_xor(sg, off, 64);
           }
           m[g] = mg;
-          if (lane == g) mine = (g == 0) ? yd : op.stiff[g] * sg;
+          if (lane == g)
+            mine = TF ? op.stiff[g] * sg - op.alpha[g] * yd : (g == 0 ? yd : op.stiff[g] * sg);
         }
         if (lane < F) {
 #pragma unroll
@@ -410,24 +428,24 @@ cw_rows_kernel(CellOpT<T> op, const T* __restrict__ x, Epi epi, double* __restri
 // Launch of phase 2 for F fields and the lane counts of the operator (GU in
 // {4, 8, 16}, GP in {8, 16}; others fall back to 8).  Returns the grid
 // (number of partials written when partial is given).
-template <typename Epi, int F, int GU, typename T>
+template <typename Epi, int F, int GU, bool TF, typename T>
 static void cw_rows_gp(const CellOpT<T>& op, int gp, dim3 grid, hipStream_t s, const T* x,
                        Epi epi, double* partial) {
   if (gp == 16)
-    hipLaunchKernelGGL((cw_rows_kernel<F, GU, 16, Epi, T>), grid, dim3(256), 0, s, op, x, epi,
+    hipLaunchKernelGGL((cw_rows_kernel<F, GU, 16, TF, Epi, T>), grid, dim3(256), 0, s, op, x, epi,
                        partial);
   else
-    hipLaunchKernelGGL((cw_rows_kernel<F, GU, 8, Epi, T>), grid, dim3(256), 0, s, op, x, epi,
+    hipLaunchKernelGGL((cw_rows_kernel<F, GU, 8, TF, Epi, T>), grid, dim3(256), 0, s, op, x, epi,
                        partial);
 }
 template <typename Epi, int F, typename T>
 static void cw_rows_f(const CellOpT<T>& op, dim3 grid, hipStream_t s, const T* x, Epi epi,
                       double* partial) {
   switch (op.lanes_u) {
-    case 1: cw_rows_gp<Epi, F, 1>(op, op.lanes_p, grid, s, x, epi, partial); break;
-    case 4: cw_rows_gp<Epi, F, 4>(op, op.lanes_p, grid, s, x, epi, partial); break;
-    case 16: cw_rows_gp<Epi, F, 16>(op, op.lanes_p, grid, s, x, epi, partial); break;
-    default: cw_rows_gp<Epi, F, 8>(op, op.lanes_p, grid, s, x, epi, partial); break;
+    case 1: cw_rows_gp<Epi, F, 1, false>(op, op.lanes_p, grid, s, x, epi, partial); break;
+    case 4: cw_rows_gp<Epi, F, 4, false>(op, op.lanes_p, grid, s, x, epi, partial); break;
+    case 16: cw_rows_gp<Epi, F, 16, false>(op, op.lanes_p, grid, s, x, epi, partial); break;
+    default: cw_rows_gp<Epi, F, 8, false>(op, op.lanes_p, grid, s, x, epi, partial); break;
   }
 }
 static inline int cw_lanes_u(int g) { return (g == 1 || g == 4 || g == 8 || g == 16) ? g : 8; }
@@ -443,7 +461,7 @@ template <typename Epi, typename T>
 static int cw_launch(const CellOpT<T>& op, const T* x, Epi epi, double* partial,
                      const int* skip, hipStream_t s) {
   const int cb = (op.nC + CW_NT - 1) / CW_NT;
-  hipLaunchKernelGGL((cw_cell_kernel<CW_NT, T>), dim3(cb), dim3(CW_NT), 0, s, op, x, skip);
+  hipLaunchKernelGGL((cw_cell_kernel<CW_NT, T, false>), dim3(cb), dim3(CW_NT), 0, s, op, x, skip);
   const int np = grid_for(cw_row_tiles(op), 1, MAX_PARTIALS);
   const dim3 grid(np);
   switch (op.A + 1) {
@@ -456,6 +474,30 @@ static int cw_launch(const CellOpT<T>& op, const T* x, Epi epi, double* partial,
     case 8: cw_rows_f<Epi, 8>(op, grid, s, x, epi, partial); break;
     default: break;
   }
+  return np;
+}
+
+// Both phases of the two-field operator (FP64): 13.8 + 6.9 us at 18^3 x 6 tets,
+// A = 2 (35,000 cells), against 53.7 us for the rows of its CSR matrix (~100
+// nonzeros per u row, ~215 per p row, 12 bytes each), which read 0.2 GB.  One,
+// four and eight lanes per P2 node measured 118.0, 116.3 and 118.1 us an
+// iteration there (170.4 with four at 24^3, 168.8 and 177.1), so the lanes are
+// not tuned.
+template <typename Epi>
+static int cw_launch_tf(const CellOpT<double>& op, const double* x, Epi epi, double* partial,
+                        const int* skip, hipStream_t s) {
+  const int cb = (op.nC + CW_NT - 1) / CW_NT;
+  hipLaunchKernelGGL((cw_cell_kernel<CW_NT, double, true>), dim3(cb), dim3(CW_NT), 0, s, op, x,
+                     skip);
+  const int np = grid_for((op.nP2 + 256 / TF_GU - 1) / (256 / TF_GU) +
+                              (op.nP1 + 256 / TF_GP - 1) / (256 / TF_GP), 1, MAX_PARTIALS);
+#define CWTF(N)                                                                                \
+  case N:                                                                                      \
+    hipLaunchKernelGGL((cw_rows_kernel<N, TF_GU, TF_GP, true, Epi, double>), dim3(np),         \
+                       dim3(256), 0, s, op, x, epi, partial);                                  \
+    break;
+  switch (op.A) { CWTF(1) CWTF(2) CWTF(3) CWTF(4) CWTF(5) CWTF(6) CWTF(7) default: break; }
+#undef CWTF
   return np;
 }
 
@@ -506,12 +548,34 @@ static int cw_from_desc(const MpetCellOpDesc* d, T* work, CellOpT<T>& op) {
   for (int i = 0; i < MPET_MAXF * MPET_MAXF; ++i) op.C[i] = (T)d->coef.C[i];
   for (int i = 0; i < MPET_MAXF; ++i) op.stiff[i] = (T)d->coef.stiff[i];
   op.mu = (T)d->coef.mu;
+  op.lmbda = (T)0;
+  for (int i = 0; i < MPET_MAXF; ++i) op.alpha[i] = (T)0;
   op.dmask = d->dmask;
   op.lanes_u = cw_lanes_u(d->lanes_u);
   op.lanes_p = cw_lanes_p(d->lanes_p);
   op.xcd_chunk = d->xcd_chunk;
   op.Yu = work;
   op.Yp = work + 3ll * d->npart2;
+  return OK;
+}
+
+// Host: device view of the two-field operator: the descriptor's tables and
+// the two-field coefficients (the descriptor's own coef is not used).
+static inline int cw_from_two_field(const MpetCellOpDesc* d, const MpetTwoFieldCoef* coef,
+                                    double* work, CellOpT<double>& op) {
+  if (!coef) {
+    mpet_set_error("invalid two-field coefficients");
+    return ERR_INVALID;
+  }
+  const int rc = cw_from_desc<double>(d, work, op);
+  if (rc) return rc;
+  for (int i = 0; i < MPET_MAXF * MPET_MAXF; ++i) op.C[i] = coef->C[i];
+  for (int i = 0; i < MPET_MAXF; ++i) {
+    op.stiff[i] = coef->stiff[i];
+    op.alpha[i] = coef->alpha[i];
+  }
+  op.mu = coef->mu;
+  op.lmbda = coef->lmbda;
   return OK;
 }
 

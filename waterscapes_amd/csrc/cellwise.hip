@@ -93,3 +93,19 @@ extern "C" int mpet_cell_op_apply(const MpetCellOpDesc* d, const void* x, const 
   return d->fp64 ? cell_op_apply_t<double>(d, x, b, y, work, stream)
                  : cell_op_apply_t<float>(d, x, b, y, work, stream);
 }
+
+extern "C" int mpet_two_field_cell_apply(const MpetCellOpDesc* d, const MpetTwoFieldCoef* coef,
+                                         const double* x, const double* b, double* y,
+                                         double* work, hipStream_t stream) {
+  CellOpT<double> op;
+  const int rc = cw_from_two_field(d, coef, work, op);
+  if (rc) return rc;
+  if (!x || !y) {
+    mpet_set_error("mpet_two_field_cell_apply: null vector");
+    return ERR_INVALID;
+  }
+  cw_launch_tf(op, x, CwEpiApplyT<double>{y, b, op.dmask}, (double*)nullptr,
+               (const int*)nullptr, stream);
+  HIPCHK(hipGetLastError());
+  return OK;
+}

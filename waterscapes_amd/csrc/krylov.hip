@@ -605,6 +605,9 @@ struct MpetSolver {
   // CSR-only solvers (no structured operator): the operator of every mode
   // is the CSR matrix; mixed mode iterates on its FP32 copy
   bool csr_only = false;
+  // two-field MINRES cell by cell (csr_only, mode 0)
+  bool has_tf = false;
+  CellOpT<double> tf;
   float* csr_v32 = nullptr;
 };
 
@@ -741,6 +744,9 @@ static void minres_iter(MpetSolver* S, Minres<T>& M, const Precond<T>& P, bool c
       hipLaunchKernelGGL(k1bf_kernel, dim3(1), dim3(1024), 0, s, M.partial, bg, S->mb, S->n,
                          (const double*)zc, Ra, (const double*)Rb, M.y, M.v, zn, S->tail_inv,
                          M.st, skip);
+    } else if (csr && S->has_tf) {
+      CwEpiK1<double> cepi{EpiK1<double>{M.y, nullptr, zc, Ra, S->opt_mask64}, M.st, skip};
+      np = cw_launch_tf(S->tf, zc, cepi, M.partial, skip, s);
     } else if (csr) {
       epi.mask = S->opt_mask64;
       int lpr = S->csr_lpr;
@@ -1404,6 +1410,43 @@ extern "C" int mpet_solver_set_cell_operator64(void* h, const MpetCellOpDesc* op
   if (rc) return rc;
   S->cw64 = c;
   S->has_cw64 = true;
+  return OK;
+}
+
+// FP64 MINRES of a two-field solver cell by cell (op != NULL) or back on its
+// CSR matrix (op == NULL).  The captured FP64 graph is dropped.
+extern "C" int mpet_solver_set_two_field_cells(void* h, const MpetCellOpDesc* op,
+                                               const MpetTwoFieldCoef* coef) {
+  MpetSolver* S = (MpetSolver*)h;
+  if (!S || !S->csr_only || S->mb || S->opt.mode != 0) {
+    mpet_set_error("mpet_solver_set_two_field_cells: needs an FP64 solver on a CSR matrix "
+                   "without multipliers");
+    return ERR_INVALID;
+  }
+  HIPCHK(hipDeviceSynchronize());
+  if (S->graph64) HIPCHK(hipGraphExecDestroy(S->graph64));
+  S->graph64 = nullptr;
+  if (!op) {
+    S->has_tf = false;
+    return OK;
+  }
+  if (!op->fp64 || op->nP2 != S->op64.nP2 || op->nP1 != S->op64.nP1 || op->A != S->F ||
+      op->npart2 <= 0 || op->npart1 <= 0) {
+    mpet_set_error("mpet_solver_set_two_field_cells: not an FP64 description of the solver's "
+                   "system");
+    return ERR_INVALID;
+  }
+  const long long need = cw_work_floats(op);
+  if (S->cw64_work_n < need) {
+    int rc = alloc_dev(S->allocs, &S->cw64_work, (size_t)need);
+    if (rc) return rc;
+    S->cw64_work_n = need;
+  }
+  CellOpT<double> c;
+  const int rc = cw_from_two_field(op, coef, S->cw64_work, c);
+  if (rc) return rc;
+  S->tf = c;
+  S->has_tf = true;
   return OK;
 }
 

@@ -290,18 +290,22 @@ class DeviceSystem:
             if self.op32 is None:
                 raise ValueError("the cell-wise operator needs the FP32 structured copy")
             v, geom = self.op32, self.cell_op()["geom"]
+        return self._cell_desc(v, geom, _lib.make_coef(self.Cm, self.Cs, self.mu), self.A,
+                               masked, lanes, xcd_chunk, fp64)
+
+    def _cell_desc(self, v, geom, coef, A, masked, lanes, xcd_chunk, fp64):
         cw = self.cell_op()
         t2, t1 = cw["p2"], cw["p1"]
         lu, lp = lanes or self.cell_lanes
         xc = self.cell_xcd_chunk if xcd_chunk is None else xcd_chunk
         p11 = self.pat_dev["11"]
-        return _lib.CellOpDesc(cw["nC"], self.nP2, self.nP1, self.A, ptr(t2["node"]),
+        return _lib.CellOpDesc(cw["nC"], self.nP2, self.nP1, A, ptr(t2["node"]),
                                ptr(t1["node"]), ptr(geom), self.CELLS_PER_BLOCK,
                                t2["npart"], t1["npart"], ptr(t2["bq"]), ptr(t2["lrp"]),
                                ptr(t2["pe"]), ptr(t2["lsl"]), ptr(t1["bq"]), ptr(t1["lrp"]),
                                ptr(t1["pe"]), ptr(t1["lsl"]), ptr(t2["rp"]), ptr(t1["rp"]),
                                ptr(p11[0]), ptr(p11[1]), self.nnz["11"], ptr(v["M1"]),
-                               ptr(v["St"]), _lib.make_coef(self.Cm, self.Cs, self.mu),
+                               ptr(v["St"]), coef,
                                ptr(self.dmask) if masked else None, lu, lp, xc, int(fp64))
 
     def cell_apply(self, x32, b=None, masked=True, lanes=None):
@@ -421,6 +425,29 @@ class TwoFieldSystem(DeviceSystem):
 
     def op_desc(self, dtype, masked=True, lanes=None):
         raise NotImplementedError("the two-field system is held as scalar CSR only")
+
+    def cells_fit(self):
+        """Whether the cell-wise operator takes this system's field count."""
+        return self.F < _lib.MAXF
+
+    def coef(self):
+        return _lib.make_two_field_coef(self.Cm, self.Cs, self.alpha, self.mu, self.lmbda)
+
+    def cell_op_desc(self, masked=True):
+        """MpetCellOpDesc of the FP64 cell-wise two-field operator (its
+        coefficients go beside it, see coef())."""
+        v = {"M1": self.prim_t["M1"], "St": self.prim_t["St"]}
+        return self._cell_desc(v, self.cell_geom64(), _lib.make_coef(self.Cm, self.Cs, self.mu),
+                               self.F, masked, None, None, True)
+
+    def cell_apply(self, x, b=None, masked=True):
+        """y = A x (or b - A x) cell by cell, FP64."""
+        y = torch.empty_like(x)
+        work = torch.empty(self.cell_work_floats(), dtype=torch.float64, device=self.device)
+        d, coef = self.cell_op_desc(masked), self.coef()
+        check(_lib.lib().mpet_two_field_cell_apply(C.byref(d), C.byref(coef), ptr(x), ptr(b),
+                                                   ptr(y), ptr(work), _lib.stream_ptr()))
+        return y
 
     def row_lengths(self, which):
         rp = {k: np.diff(v[0]) for k, v in self.pat_host.items()}

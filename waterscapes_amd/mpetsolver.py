@@ -28,8 +28,13 @@ import torch
 from .amg import AmgParams
 from .fem import Constant, Function, MixedSpace
 from .krylov import SolverConfig
-from .nullspace import pressure_fields
+from .nullspace import has_nullspace, pressure_fields
 from .solver import DirichletBC, FormDescriptor, Parameters, StepEngine
+
+# Cells from which the FP64 MINRES runs cell by cell.  An iteration on cubes of
+# n^3 x 6 tets, A = 2, CSR / cells: n = 8 55.9 / 61.9 us, 10 73.3 / 78.3, 12
+# (10,368 cells) 74.0 / 74.2, 14 104 / 97, 18 165 / 116, 24 303 / 170.
+TWO_FIELD_CELLS = 12000
 
 
 class MPETSolver(object):
@@ -125,8 +130,10 @@ class MPETSolver(object):
             raise ValueError("precision must be 'fp64' or 'mixed'")
         if p["precision"] == "mixed" and self.up.function_space().nmult:
             raise ValueError("systems with nullspace multipliers are solved in FP64 only")
+        cells = p["precision"] == "fp64" and not has_nullspace(self.problem) and \
+            self.problem.mesh.num_cells() >= TWO_FIELD_CELLS
         return SolverConfig(mode=p["precision"], rtol=float(p["krylov_rtol"]),
-                            use_graphs=True, check_every=10,
+                            fp64_cells=cells, use_graphs=True, check_every=10,
                             outer_tol=float(p["outer_tol"]), inner_rtol=float(p["inner_rtol"]),
                             maxit=int(p["maxit"]),
                             amg=AmgParams(smoother_degree=int(p["u_smoother_degree"]),
