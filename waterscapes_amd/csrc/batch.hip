@@ -214,8 +214,8 @@ bcw_cell_kernel(BCell<T> C, const T* __restrict__ x, const State* st, int parity
 
 // Row epilogue of phase 2 for N consecutive DOFs: plain / residual, or the
 // MINRES step (as bop_u_kernel); loads first, as cellwise.h's epilogues.
-// (One source pointer, chosen before the load, and no conditional writes into
-// the struct: otherwise it ends in memory, 17 instead of 8 us for the u rows.)
+// (One source pointer, chosen before the load, into plain arrays: a struct
+// filled under conditions went to LDS, 17 instead of 7 us for the u rows.)
 template <typename T, int N>
 __device__ __forceinline__ void brow_load(const K1Args<T>& k1, const T* x, const T* b,
                                           const uint8_t* dmask, long long o, T (&r)[N],
@@ -250,11 +250,11 @@ __device__ __forceinline__ double brow_finish(const K1Args<T>& k1, T s, T c1, co
 // Phase 2, u rows: one thread per P2 node (2.3 partials a node), tiles of NT
 // nodes of one instance.
 template <typename T>
-__global__ void __launch_bounds__(NT)
-bcw_u_kernel(BCell<T> C, const Tile* __restrict__ tiles, const T* __restrict__ x,
-             const T* __restrict__ b, T* __restrict__ y, const uint8_t* __restrict__ dmask,
-             K1Args<T> k1) {
-  const int t = blockIdx.x;
+__device__ __forceinline__ void bcw_u_rows(const BCell<T>& C, int t,
+                                           const Tile* __restrict__ tiles,
+                                           const T* __restrict__ x, const T* __restrict__ b,
+                                           T* __restrict__ y, const uint8_t* __restrict__ dmask,
+                                           const K1Args<T>& k1) {
   const Tile tl = tiles[t];
   T s, c1;
   const bool active = k1_setup(k1, tl.inst, s, c1);
@@ -289,10 +289,10 @@ bcw_u_kernel(BCell<T> C, const Tile* __restrict__ tiles, const T* __restrict__ x
 // Phase 2, p rows: GP lanes per P1 node, tiles of NT / GP nodes.
 constexpr int BGP = 8;
 template <typename T>
-__global__ void __launch_bounds__(NT)
-bcw_p_kernel(BOp<T> op, BCell<T> C, const Tile* __restrict__ tiles, int part_off,
-             const T* __restrict__ x, const T* __restrict__ b, T* __restrict__ y, K1Args<T> k1) {
-  const int t = blockIdx.x;
+__device__ __forceinline__ void bcw_p_rows(const BOp<T>& op, const BCell<T>& C, int t,
+                                           const Tile* __restrict__ tiles, int part_off,
+                                           const T* __restrict__ x, const T* __restrict__ b,
+                                           T* __restrict__ y, const K1Args<T>& k1) {
   const Tile tl = tiles[t];
   T s, c1;
   const bool active = k1_setup(k1, tl.inst, s, c1);
@@ -355,6 +355,20 @@ bcw_p_kernel(BOp<T> op, BCell<T> C, const Tile* __restrict__ tiles, int part_off
     const double bs = block_sum(acc);
     if (threadIdx.x == 0) k1.partial[part_off + t] = bs;
   }
+}
+
+// The two kinds of rows in one launch (the first nu blocks are u tiles): at
+// six small instances either takes a launch's ~4 us alone.  With the flags'
+// block in bk5_kernel, a batched step of six: 58.3 -> 56.3 ms.
+template <typename T>
+__global__ void __launch_bounds__(NT)
+bcw_rows_kernel(BOp<T> op, BCell<T> C, const Tile* __restrict__ utiles, int nu,
+                const Tile* __restrict__ ptiles, const T* __restrict__ x,
+                const T* __restrict__ b, T* __restrict__ y, K1Args<T> k1) {
+  if ((int)blockIdx.x < nu)
+    bcw_u_rows(C, blockIdx.x, utiles, x, b, y, op.dmask, k1);
+  else
+    bcw_p_rows(op, C, blockIdx.x - nu, ptiles, nu, x, b, y, k1);
 }
 
 // Sum of instance k's partials: ranges [r0[k], r0[k+1]) and [r1[k], r1[k+1])
@@ -442,8 +456,8 @@ bk4f_kernel(const double* __restrict__ partial, const int* __restrict__ r0,
 
 // all[p] = 1 when every instance is inactive for parity p; iflag[p][k] =
 // instance k inactive for parity p (read by the preconditioner kernels).
-__global__ void __launch_bounds__(NT)
-ball_kernel(const State* st, int ninst, int p, int* all, int* iflag) {
+__device__ __forceinline__ void ball_block(const State* st, int ninst, int p, int* all,
+                                           int* iflag) {
   __shared__ int any;
   if (threadIdx.x == 0) any = 0;
   __syncthreads();
@@ -455,13 +469,24 @@ ball_kernel(const State* st, int ninst, int p, int* all, int* iflag) {
   __syncthreads();
   if (threadIdx.x == 0) all[p] = any ? 0 : 1;
 }
+__global__ void __launch_bounds__(NT)
+ball_kernel(const State* st, int ninst, int p, int* all, int* iflag) {
+  ball_block(st, ninst, p, all, iflag);
+}
 
 // w_new = (v - oldeps w1 - delta w2) / gamma; x += phi w_new  (w1 <- w_new).
+// Block 0 sets the next iteration's flags (ball_block), which neither reads
+// nor is read by the other blocks.
 template <typename T>
 __global__ void __launch_bounds__(NT)
 bk5_kernel(const Tile* __restrict__ segs, const T* __restrict__ v, T* __restrict__ w1,
-           const T* __restrict__ w2, T* __restrict__ x, const State* st, int parity) {
-  const Tile sg = segs[blockIdx.x];
+           const T* __restrict__ w2, T* __restrict__ x, const State* st, int parity, int ninst,
+           int* all, int* iflag) {
+  if (blockIdx.x == 0) {
+    ball_block(st, ninst, parity ^ 1, all, iflag);
+    return;
+  }
+  const Tile sg = segs[blockIdx.x - 1];
   const State& S = st[sg.inst];
   if (S.inactive[parity]) return;
   const T oe = (T)S.oldeps, de = (T)S.delta, ig = (T)(1.0 / S.gamma), ph = (T)S.phi;
@@ -617,10 +642,8 @@ void op_launch(const Batch* B, const BOp<T>& op, const T* x, const T* b, T* y, K
     const BCell<T>& C = cell_of<T>(B);
     hipLaunchKernelGGL((bcw_cell_kernel<T>), dim3(B->ncblk), dim3(CW_NT), 0, s, C, x, k1.st,
                        k1.parity);
-    hipLaunchKernelGGL((bcw_u_kernel<T>), dim3(B->ncut), dim3(NT), 0, s, C, B->cutiles, x, b, y,
-                       op.dmask, k1);
-    hipLaunchKernelGGL((bcw_p_kernel<T>), dim3(B->ncpt), dim3(NT), 0, s, op, C, B->cptiles,
-                       B->ncut, x, b, y, k1);
+    hipLaunchKernelGGL((bcw_rows_kernel<T>), dim3(B->ncut + B->ncpt), dim3(NT), 0, s, op, C,
+                       B->cutiles, B->ncut, B->cptiles, x, b, y, k1);
     return;
   }
   hipLaunchKernelGGL((bop_u_kernel<T>), dim3(B->nut), dim3(NT), 0, s, op, B->utiles, x, b, y,
@@ -670,10 +693,8 @@ void minres_iter(Batch* B, int i, hipStream_t s) {
                      (const State*)M.st, cur, B->partial);
   hipLaunchKernelGGL(bk4f_kernel, dim3(B->ninst), dim3(NT), 0, s, B->partial, B->sr0, B->sr1,
                      M.st, cur, next);
-  hipLaunchKernelGGL(ball_kernel, dim3(1), dim3(NT), 0, s, M.st, B->ninst, next, M.all,
-                     M.iflag);
-  hipLaunchKernelGGL((bk5_kernel<T>), dim3(B->nseg), dim3(NT), 0, s, B->segs, M.v, Wa, Wb, M.x,
-                     M.st, cur);
+  hipLaunchKernelGGL((bk5_kernel<T>), dim3(1 + B->nseg), dim3(NT), 0, s, B->segs, M.v, Wa, Wb,
+                     M.x, M.st, cur, B->ninst, M.all, M.iflag);
 }
 
 // r1 = r2 = b, z = M^-1 b, beta1 per instance; instances with keep == 0

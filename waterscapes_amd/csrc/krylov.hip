@@ -230,41 +230,70 @@ dot_kernel(long long n, const T* __restrict__ a, const T* __restrict__ b,
   if (threadIdx.x == 0) partial[blockIdx.x] = bs;
 }
 
-// K4 finalize: beta = sqrt(r2 . z) and the Givens update; decides whether
-// iteration i + 1 runs (writes inactive[next]).
+// The Givens update from tot = r2 . z (one thread): beta = sqrt(tot); decides
+// whether iteration i + 1 runs (writes inactive[next]).
+__device__ __forceinline__ void k4_update(double tot, MinresState* st, int next) {
+  MinresState s = *st;
+  s.oldb = s.beta;
+  // fmax(NaN, c) is c: test the raw sum and the rotation for NaN / inf
+  // before clamping, so a breakdown is reported instead of read as 0
+  const bool bad_in = !(tot == tot) || isinf(tot);
+  s.beta = sqrt(fmax(tot, 0.0));
+  s.oldeps = s.epsln;
+  s.delta = s.cs * s.dbar + s.sn * s.alfa;
+  double gbar = s.sn * s.dbar - s.cs * s.alfa;
+  s.epsln = s.sn * s.beta;
+  s.dbar = -s.cs * s.beta;
+  const double hg = hypot(gbar, s.beta);
+  s.gamma = fmax(hg, 1e-300);
+  s.cs = gbar / s.gamma;
+  s.sn = s.beta / s.gamma;
+  s.phi = s.cs * s.phibar;
+  s.phibar = s.sn * s.phibar;
+  s.it += 1;
+  bool bad = bad_in || !(hg == hg) || !(s.phibar == s.phibar) || isinf(s.phibar);
+  s.nan = bad ? 1 : 0;
+  int conv = (bad || s.phibar <= s.tol || s.beta == 0.0 || s.it >= s.maxit) ? 1 : 0;
+  s.done = conv;
+  s.inactive[next] = conv;
+  *st = s;
+}
+
+// K4 finalize: tot from the dot kernel's partials.
 __global__ void __launch_bounds__(NT)
 k4f_kernel(const double* __restrict__ partial, int np, MinresState* st, int cur, int next) {
   if (st->inactive[cur]) {
     if (threadIdx.x == 0) st->inactive[next] = 1;
     return;
   }
-  double tot = sum_partials(partial, np);
-  if (threadIdx.x == 0) {
-    MinresState s = *st;
-    s.oldb = s.beta;
-    // fmax(NaN, c) is c: test the raw sum and the rotation for NaN / inf
-    // before clamping, so a breakdown is reported instead of read as 0
-    const bool bad_in = !(tot == tot) || isinf(tot);
-    s.beta = sqrt(fmax(tot, 0.0));
-    s.oldeps = s.epsln;
-    s.delta = s.cs * s.dbar + s.sn * s.alfa;
-    double gbar = s.sn * s.dbar - s.cs * s.alfa;
-    s.epsln = s.sn * s.beta;
-    s.dbar = -s.cs * s.beta;
-    const double hg = hypot(gbar, s.beta);
-    s.gamma = fmax(hg, 1e-300);
-    s.cs = gbar / s.gamma;
-    s.sn = s.beta / s.gamma;
-    s.phi = s.cs * s.phibar;
-    s.phibar = s.sn * s.phibar;
-    s.it += 1;
-    bool bad = bad_in || !(hg == hg) || !(s.phibar == s.phibar) || isinf(s.phibar);
-    s.nan = bad ? 1 : 0;
-    int conv = (bad || s.phibar <= s.tol || s.beta == 0.0 || s.it >= s.maxit) ? 1 : 0;
-    s.done = conv;
-    s.inactive[next] = conv;
-    *st = s;
+  const double tot = sum_partials(partial, np);
+  if (threadIdx.x == 0) k4_update(tot, st, next);
+}
+
+// Both steps in one block of 1,024 threads for up to ONE_BLOCK_DOT rows, where
+// a launch fewer is worth more than the chip's other CUs.  Two direct steps
+// with two launches / one block: 4^3 x 6 tets (2,600 rows) 7.64 / 7.29 ms, 6^3
+// (8,000) 14.8 / 15.0, 10^3 (32,000) 22.4 / 24.1.
+constexpr long long ONE_BLOCK_DOT = 4096;
+template <typename T>
+__global__ void __launch_bounds__(1024)
+dot_k4f_kernel(int n, const T* __restrict__ a, const T* __restrict__ b, MinresState* st, int cur,
+               int next) {
+  if (st->inactive[cur]) {
+    if (threadIdx.x == 0) st->inactive[next] = 1;
+    return;
   }
+  double acc = 0.0;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < n; i += 1024) acc += (double)a[i] * (double)b[i];
+  __shared__ double sums[16];
+  const double w = wave_sum(acc);
+  if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6] = w;
+  __syncthreads();
+  if (threadIdx.x) return;
+  double tot = 0.0;
+  for (int k = 0; k < 16; ++k) tot += sums[k];
+  k4_update(tot, st, next);
 }
 
 // K5: w = (v - oldeps w1 - delta w2) / gamma (written over w1); x += phi w.
@@ -284,17 +313,45 @@ k5_kernel(long long n, const T* __restrict__ v, T* __restrict__ w1, const T* __r
 // K5 with v = s z formed here from this iteration's z (s = 1 / oldb: the
 // 1 / beta that K1 scaled z with, bit for bit), so that K1 need not store v.
 template <typename T>
-__global__ void __launch_bounds__(NT)
-k5z_kernel(long long n, const T* __restrict__ z, T* __restrict__ w1, const T* __restrict__ w2,
-           T* __restrict__ x, const MinresState* st, const int* __restrict__ skip) {
-  if (*skip) return;
-  long long i = (long long)blockIdx.x * NT + threadIdx.x;
+__device__ __forceinline__ void k5z_rows(int block, long long n, const T* __restrict__ z,
+                                         T* __restrict__ w1, const T* __restrict__ w2,
+                                         T* __restrict__ x, const MinresState* st) {
+  long long i = (long long)block * NT + threadIdx.x;
   if (i >= n) return;
   const T sv = (T)(1.0 / st->oldb);
   const T oe = (T)st->oldeps, de = (T)st->delta, ig = (T)(1.0 / st->gamma), ph = (T)st->phi;
   T w = (sv * z[i] - oe * w1[i] - de * w2[i]) * ig;
   w1[i] = w;
   x[i] += ph * w;
+}
+template <typename T>
+__global__ void __launch_bounds__(NT)
+k5z_kernel(long long n, const T* __restrict__ z, T* __restrict__ w1, const T* __restrict__ w2,
+           T* __restrict__ x, const MinresState* st, const int* __restrict__ skip) {
+  if (*skip) return;
+  k5z_rows<T>(blockIdx.x, n, z, w1, w2, x, st);
+}
+
+// alfa of one iteration (block 0) and K5 of the one before (the others, which
+// read none of what block 0 writes): nothing between the two launches that
+// this replaces needs x or w, so K5 costs no launch of its own but the last
+// of a chunk.  A small system's launch takes ~4 us whatever it does: two steps
+// 8.18 -> 7.64 ms at 4^3 x 6 tets (direct), 22.1 -> 21.4 at 8^3, 46.9 -> 45.2
+// two-field at 18^3.
+template <typename T>
+__global__ void __launch_bounds__(NT)
+k1f_k5z_kernel(const double* __restrict__ partial, int np, MinresState* st,
+               const int* __restrict__ skip, long long n, const T* __restrict__ z,
+               T* __restrict__ w1, const T* __restrict__ w2, T* __restrict__ x,
+               const int* __restrict__ skip5) {
+  if (blockIdx.x == 0) {
+    if (*skip) return;
+    const double s = sum_partials(partial, np);
+    if (threadIdx.x == 0) st->alfa = s;
+  } else {
+    if (*skip5) return;
+    k5z_rows<T>(blockIdx.x - 1, n, z, w1, w2, x, st);
+  }
 }
 
 // init: r1 = r2 = b, w1 = w2 = x = 0.
@@ -714,7 +771,7 @@ static void launch_k1_op(int F, int gu, int gp, dim3 grid, hipStream_t s, const 
 // One MINRES iteration i (i selects the buffer rotation and skip flag).
 template <typename T>
 static void minres_iter(MpetSolver* S, Minres<T>& M, const Precond<T>& P, bool csr, int i,
-                        hipStream_t s) {
+                        bool last, hipStream_t s) {
   T* Ra = M.R[i & 1];
   T* Rb = M.R[(i + 1) & 1];
   T* Wa = M.W[i & 1];
@@ -802,8 +859,13 @@ static void minres_iter(MpetSolver* S, Minres<T>& M, const Precond<T>& P, bool c
     np = grid_for(ntiles, 1, MAX_PARTIALS);
     launch_k1_op<T>(S->F, gu, gp, dim3(np), s, *op, zc, epi, M.st, skip, M.partial);
   }
-  if (!(csr && S->mb))
-    hipLaunchKernelGGL(k1f_kernel, dim3(1), dim3(NT), 0, s, M.partial, np, M.st, skip);
+  if (!keep_v) {
+    if (i > 0)                      // with the previous iteration's K5
+      hipLaunchKernelGGL((k1f_k5z_kernel<T>), dim3(1 + eb), dim3(NT), 0, s, M.partial, np, M.st,
+                         skip, n, (const T*)zn, Wb, Wa, M.x, &M.st->inactive[next]);
+    else
+      hipLaunchKernelGGL(k1f_kernel, dim3(1), dim3(NT), 0, s, M.partial, np, M.st, skip);
+  }
   if (k2_direct(S, P)) {
     // K2 made by the preconditioner's first kernels (one vector pass and
     // one launch fewer on the iteration's critical path)
@@ -815,13 +877,18 @@ static void minres_iter(MpetSolver* S, Minres<T>& M, const Precond<T>& P, bool c
     hipLaunchKernelGGL((k2_kernel<T>), dim3(eb), dim3(NT), 0, s, n, M.y, Rb, Ra, M.st, skip);
     apply_M(S, P, Ra, zn, skip, s);
   }
-  int dg = dot_grid(n);
-  hipLaunchKernelGGL((dot_kernel<T>), dim3(dg), dim3(NT), 0, s, n, Ra, zn, skip, M.partial);
-  hipLaunchKernelGGL(k4f_kernel, dim3(1), dim3(NT), 0, s, M.partial, dg, M.st, cur, next);
+  if (n <= ONE_BLOCK_DOT) {
+    hipLaunchKernelGGL((dot_k4f_kernel<T>), dim3(1), dim3(1024), 0, s, (int)n, (const T*)Ra,
+                       (const T*)zn, M.st, cur, next);
+  } else {
+    const int dg = dot_grid(n);
+    hipLaunchKernelGGL((dot_kernel<T>), dim3(dg), dim3(NT), 0, s, n, Ra, zn, skip, M.partial);
+    hipLaunchKernelGGL(k4f_kernel, dim3(1), dim3(NT), 0, s, M.partial, dg, M.st, cur, next);
+  }
   if (keep_v)
     hipLaunchKernelGGL((k5_kernel<T>), dim3(eb), dim3(NT), 0, s, n, M.v, Wa, Wb, M.x, M.st,
                        skip);
-  else
+  else if (last)
     hipLaunchKernelGGL((k5z_kernel<T>), dim3(eb), dim3(NT), 0, s, n, (const T*)zc, Wa, Wb, M.x,
                        M.st, skip);
 }
@@ -864,13 +931,13 @@ static int minres_continue(MpetSolver* S, Minres<T>& M, const Precond<T>& P, boo
       hipStream_t cs = S->graph_stream;
       hipGraph_t g;
       HIPCHK(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-      for (int i = 0; i < check; ++i) minres_iter(S, M, P, csr, i, cs);
+      for (int i = 0; i < check; ++i) minres_iter(S, M, P, csr, i, i + 1 == check, cs);
       HIPCHK(hipStreamEndCapture(cs, &g));
       HIPCHK(hipGraphInstantiate(graph, g, nullptr, nullptr, 0));
       HIPCHK(hipGraphDestroy(g));
       HIPCHK(hipGraphLaunch(*graph, s));
     } else {
-      for (int i = 0; i < check; ++i) minres_iter(S, M, P, csr, i, s);
+      for (int i = 0; i < check; ++i) minres_iter(S, M, P, csr, i, i + 1 == check, s);
     }
     done_iters += check;
     HIPCHK(hipMemcpyAsync(M.st_host, M.st, sizeof(MinresState), hipMemcpyDeviceToHost, s));
