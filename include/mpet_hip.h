@@ -179,6 +179,9 @@ typedef struct {
   const int32_t* coarse_off;
   const int64_t* coarse_ioff;
   int32_t level_degree[MPET_MAXLEV];  /* per-level Chebyshev degree (0: degree) */
+  /* One dense block only: row r of coarse_inv is zero outside the columns
+   * coarse_rng[2r] .. coarse_rng[2r+1]-1 (device; NULL: whole rows). */
+  const int32_t* coarse_rng;
 } MpetHierDesc;
 
 /* Block-diagonal preconditioner of prec (:279-283) with Dirichlet rows and

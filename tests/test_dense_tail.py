@@ -52,3 +52,21 @@ def test_first_level_limit_and_rows():
     one, same = lv.with_dense_tail(levels[-1:], cinv, 10**6, prm, "cpu", first=1)
     assert one == levels[-1:] and same is cinv
     assert lv.dense_rows(4, 64 << 20) == 4096 and lv.dense_rows(8, 64 << 20) == 2896
+
+
+def test_column_ranges():
+    """First and one past the last nonzero column of every row, zero rows
+    empty: what the dense pressure kernels read of each row."""
+    import torch
+    from waterscapes_amd import levels as lv
+    rng = np.random.default_rng(3)
+    M = np.zeros((9, 9))
+    M[:4, :4] = rng.standard_normal((4, 4))
+    M[4:, 4:] = rng.standard_normal((5, 5))
+    M[2] = 0.0
+    M[6, 4] = M[7, 8] = 0.0
+    got = lv.column_ranges(torch.as_tensor(M)).numpy()
+    for r in range(9):
+        nz = np.nonzero(M[r])[0]
+        want = (nz[0], nz[-1] + 1) if nz.size else (0, 0)
+        assert tuple(got[r]) == want

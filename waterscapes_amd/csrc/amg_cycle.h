@@ -756,16 +756,22 @@ __device__ __forceinline__ void dense_part(const T* __restrict__ row, const T* _
   }
 }
 
-// Dense coarsest solve x = Cinv (scale b) (NC columns), one wave per row.
+// Dense coarsest solve x = Cinv (scale b) (NC columns), one wave per row over
+// the row's nonzero columns rng (null: all): the pressure fields do not couple
+// in the preconditioner, so a row of F fields has 1 / F of them.  The 64 MiB
+// this can be are read once an apply: whole rows / ranges 75.7 / 68.7 us for
+// the FP64 preconditioner at 16^3 (A = 2), 186 / 182 us FP32 at 36^3 (A = 4).
 // b and x may lie in the vectors' own order (om); with k2 on, b's entries
 // are made by it, and each row's wave stores its own.
 template <typename T, int NC>
 __device__ __forceinline__ void coarse_rows(int block, int n, const T* __restrict__ cinv,
-                                            const T* b, T* __restrict__ x, T scale,
-                                            const OutMap& om, const K2In<T>& k2) {
+                                            const int* __restrict__ rng, const T* b,
+                                            T* __restrict__ x, T scale, const OutMap& om,
+                                            const K2In<T>& k2) {
   const int r = block * (NT / 64) + threadIdx.x / 64;
   const int lane = threadIdx.x % 64;
   if (r >= n) return;
+  const int c0 = rng ? rng[2 * r] : 0, c1 = rng ? rng[2 * r + 1] : n;
   T acc[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) acc[c] = 0;
@@ -773,17 +779,18 @@ __device__ __forceinline__ void coarse_rows(int block, int n, const T* __restric
   const bool own = om.F || om.map;
   const T kc2 = k2.y ? (T)(*k2.alfa / *k2.beta) : (T)0;
   if (!own && k2.y) {
-    dense_part<T, NC, true>(row, k2.y, n, lane, acc, k2.r2o, kc2);
+    dense_part<T, NC, true>(row + c0, k2.y + (long long)NC * c0, c1 - c0, lane, acc,
+                            k2.r2o + (long long)NC * c0, kc2);
   } else if (!own) {
-    dense_part<T, NC>(row, b, n, lane, acc);
+    dense_part<T, NC>(row + c0, b + (long long)NC * c0, c1 - c0, lane, acc);
   } else {
-    for (int k0 = lane; k0 < n; k0 += 256) {
+    for (int k0 = c0 + lane; k0 < c1; k0 += 256) {
       T a[4], bv[4][NC];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int k = k0 + 64 * j;
-        const int kc = k < n ? k : n - 1;
-        a[j] = k < n ? row[kc] : (T)0;
+        const int kc = k < c1 ? k : c1 - 1;
+        a[j] = k < c1 ? row[kc] : (T)0;
         const long long o = NC == 1 ? om(kc) : (long long)NC * kc;
         if (k2.y) {
           T yv[NC], rv[NC];
@@ -811,10 +818,10 @@ __device__ __forceinline__ void coarse_rows(int block, int n, const T* __restric
 }
 template <typename T, int NC>
 __global__ void __launch_bounds__(NT)
-coarse_kernel(int n, const T* __restrict__ cinv, const T* b, T* __restrict__ x,
-              const int* __restrict__ skip, T scale, OutMap om, K2In<T> k2) {
+coarse_kernel(int n, const T* __restrict__ cinv, const int* __restrict__ rng, const T* b,
+              T* __restrict__ x, const int* __restrict__ skip, T scale, OutMap om, K2In<T> k2) {
   if (skip && *skip) return;
-  coarse_rows<T, NC>(blockIdx.x, n, cinv, b, x, scale, om, k2);
+  coarse_rows<T, NC>(blockIdx.x, n, cinv, rng, b, x, scale, om, k2);
 }
 
 // The gather with the first Chebyshev step of the finest pressure level from
@@ -974,7 +981,7 @@ __device__ __forceinline__ void run_step(const Step<T>& S, int block, const Skip
       else post_rows<T, NC, false>(S.p, block, sk);
       break;
     case STEP_DENSE:
-      coarse_rows<T, NC>(block, S.n, S.cinv, S.b, S.y, S.scale, S.om, S.k2);
+      coarse_rows<T, NC>(block, S.n, S.cinv, S.off, S.b, S.y, S.scale, S.om, S.k2);
       break;
     case STEP_BLOCKS:
       blockdiag_rows<T, NC>(block, S.n, S.blk, S.off, S.ioff, S.cinv, S.b, S.y, sk, S.a.grp);
@@ -1083,7 +1090,8 @@ struct Hier {
   int nlev = 0, deg = 2, NC = 1;
   LevelDev<T> lev[MAXLEV];
   const T* cinv = nullptr;
-  // block-diagonal coarsest level (batched instances); null: one dense block
+  // block-diagonal coarsest level (batched instances); cblk null: one dense
+  // block, coff its rows' column ranges (null: whole rows)
   const int *cblk = nullptr, *coff = nullptr;
   const int64_t* cioff = nullptr;
   double scale = 1.0;      // the V-cycle approximates (scale * A0)^-1
@@ -1356,8 +1364,8 @@ static void vcycle(const Hier<T>& H, int l, const T* b, T bscale, T* out, Skip s
       hipLaunchKernelGGL((coarse_blockdiag_kernel<T, NC>), dim3(blocks), dim3(NT), 0, s, L.n,
                          H.cblk, H.coff, H.cioff, H.cinv, b, out, sk, L.grp);
     else
-      hipLaunchKernelGGL((coarse_kernel<T, NC>), dim3(blocks), dim3(NT), 0, s, L.n, H.cinv, b,
-                         out, sk.all, bscale, om, k2);
+      hipLaunchKernelGGL((coarse_kernel<T, NC>), dim3(blocks), dim3(NT), 0, s, L.n, H.cinv,
+                         H.coff, b, out, sk.all, bscale, om, k2);
     return;
   }
   T* bcopy = vcycle_bcopy(L, b, bscale);
@@ -1707,7 +1715,7 @@ static int build_hier(std::vector<void*>& allocs, const MpetHierDesc* d, int NC,
   for (int l = 0; l + 1 < H.nlev; ++l) H.lev[l].grpc = H.lev[l + 1].grp;
   H.cinv = (const T*)d->coarse_inv;
   H.cblk = d->coarse_blk;
-  H.coff = d->coarse_off;
+  H.coff = d->coarse_blk ? d->coarse_off : d->coarse_rng;
   H.cioff = d->coarse_ioff;
   return OK;
 }

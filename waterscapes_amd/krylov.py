@@ -42,7 +42,7 @@ class HierDesc(C.Structure):
                 ("degree", C.c_int32), ("eig_ratio", C.c_double), ("eig_safety", C.c_double),
                 ("scale", C.c_double), ("mask0", C.c_void_p), ("coarse_blk", C.c_void_p),
                 ("coarse_off", C.c_void_p), ("coarse_ioff", C.c_void_p),
-                ("level_degree", C.c_int32 * MAXLEV)]
+                ("level_degree", C.c_int32 * MAXLEV), ("coarse_rng", C.c_void_p)]
 
 
 class PrecDesc(C.Structure):
@@ -633,6 +633,10 @@ class KrylovSolver:
                 L.lprR = _pick_lpr(nnzp / max(lev["nc"], 1), nc, lev["nc"])
             lv.describe_fused(L, ld, lev["n"], lev["nc"], nc)
         h.coarse_inv = ptr(cinv)
+        if nc == 1:                # the fields are blocks of the dense operator
+            rng = lv.column_ranges(cinv)
+            self.keep.append(rng)
+            h.coarse_rng = ptr(rng)
         h.degree = params.smoother_degree
         set_level_degrees(h, params)
         h.eig_ratio = params.eig_ratio

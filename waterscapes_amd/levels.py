@@ -100,6 +100,17 @@ def dense_tail(levels, cinv, start, params, device, values=None, mask0=None):
     return M
 
 
+def column_ranges(M):
+    """(n, 2) int32: the first and one past the last nonzero column of every
+    row of M (0, 0 for a zero row)."""
+    nz = (M != 0).to(torch.uint8)
+    n = M.shape[1]
+    some = nz.any(dim=1)
+    lo = nz.argmax(dim=1)
+    hi = n - nz.flip(1).argmax(dim=1)
+    return (torch.stack([lo, hi], dim=1) * some[:, None]).to(torch.int32).contiguous()
+
+
 def tail_start(levels, rows):
     """The finest level of at most `rows` rows (the coarsest if none is)."""
     for l, lev in enumerate(levels):
