@@ -136,13 +136,16 @@ def _mat_bytes(nnz, rows, s, compact=False):
     return nnz * (4 if compact else s + 4) + (rows + 1) * 4
 
 
-def vcycle_bytes(levels, amgp, NC, s, compact=(), scaled=False):
+def vcycle_bytes(levels, amgp, NC, s, compact=(), scaled=False, nfields=1):
     """Algorithmic HBM bytes of one V-cycle (amg_cycle.h: vcycle / smooth /
     spmm modes), each array read once per launch: matrices, the gathered
     vector once, the epilogue vectors; levels = the host hierarchy dicts,
     compact = the levels stored as half values with 16-bit offsets.  The
     Chebyshev direction is not read by the first step from x and not written
-    by a sequence's last step."""
+    by a sequence's last step.  Counted step by step: a level whose transfers
+    are fused with its smoothing reads other matrices (levels.py, kept where
+    they are no larger), and a pressure field's rows of the dense coarsest
+    operator hold only that field's columns."""
     nl = len(levels)
     tot = 0
 
@@ -158,7 +161,8 @@ def vcycle_bytes(levels, amgp, NC, s, compact=(), scaled=False):
         lev = levels[l]
         n = lev["n"]
         if l == nl - 1:
-            tot += n * n * s + 2 * NC * n * s      # dense coarsest solve
+            # dense coarsest solve (NC = 1: the fields' blocks only)
+            tot += n * n * s // (nfields if NC == 1 else 1) + 2 * NC * n * s
             return
         nnz = len(lev["A_ci"])
         cmp = l in compact
@@ -211,7 +215,7 @@ def iteration_bytes(eng, mixed):
     else:
         k1 = csr_bytes(sysm) + n * s
     vu = vcycle_bytes(kr.levels, kr.cfg.amg, 3, s, compact=_compact_u(kr, mixed), scaled=True)
-    vp = vcycle_bytes(kr.plevels, kr.cfg.pamg, 1, s,
+    vp = vcycle_bytes(kr.plevels, kr.cfg.pamg, 1, s, nfields=sysm.F,
                       compact=_compact_p(kr, mixed)) + 4 * sysm.F * sysm.nP1 * s
     blas = 10 * n * s
     parts = {"k1": int(k1), "vcycle_u": int(vu), "vcycle_p": int(vp), "blas1": int(blas)}
@@ -234,7 +238,7 @@ def step_bytes(eng, mixed, inner, outer):
     else:
         op64 = op_bytes(sysm, 0) if (mixed or kr.csr_desc is None) else csr_bytes(sysm)
     pc = vcycle_bytes(kr.levels, kr.cfg.amg, 3, s, compact=_compact_u(kr, mixed),
-                      scaled=True) + vcycle_bytes(kr.plevels, kr.cfg.pamg, 1, s,
+                      scaled=True) + vcycle_bytes(kr.plevels, kr.cfg.pamg, 1, s, nfields=sysm.F,
                                                   compact=_compact_p(kr, mixed))
     starts = 2 + (outer if mixed else 0)
     solve_overhead = starts * (op64 + n * 8 + pc + 2 * n * s)
@@ -641,8 +645,9 @@ def two_field_cpu_baseline(n_sample, steps, budget_s=20.0):
 
 def main_two_field(args):
     """Two-field MPETSolver (mpet/mpetsolver.py) steps/s: the reference's
-    direct path (MUMPS LU) realised as FP64 MINRES to 1e-12 on the device
-    CSR system with the block AMG preconditioner of prec."""
+    direct path (MUMPS LU) realised as FP64 MINRES to 1e-12 with the block AMG
+    preconditioner of prec, the operator cell by cell (small systems and
+    residuals: the device CSR matrix)."""
     import torch
     from waterscapes_amd import _lib
     n = args.tf_n
@@ -679,7 +684,8 @@ def main_two_field(args):
                       "precision": args.tf_precision},
            "dof_per_s": round(sysd.n * K / total, 1), "iterations": its,
            "setup_s": round(setup, 2),
-           "roofline": {"bound": "hbm", "kernel": f"csr_spmv_kernel<double,{lpr}> (two-field A)",
+           "roofline": {"bound": "hbm", "kernel": f"csr_spmv_kernel<double,{lpr}> (two-field A, "
+                        "the residuals; the FP64 iterations run cell by cell)",
                         "achieved": round(ach, 1), "peak": 8000.0, "unit": "GB/s",
                         "frac": round(ach / 8000.0, 4), "traffic": None,
                         "bytes_per_launch": int(nbytes), "ms_per_launch": round(ms, 4)}}
@@ -1200,10 +1206,11 @@ def main():
             "achieved": round(ach_s, 1), "frac": round(ach_s / 8000.0, 4),
             "traffic": traffic_of("op_apply_48cube_A4_traffic.json"),
             "bytes_per_launch": int(bytes_s), "ms_per_launch": round(ms_s, 4)}
-    # the finest displacement level's Chebyshev step (the top kernel by time
-    # in the V-cycles): half values and 16-bit offsets, three columns, the
-    # solver's tuned lanes; bytes as vcycle_bytes counts a middle step
-    # (direction read and written)
+    # a Chebyshev step with the finest displacement level's CSR matrix, half
+    # values and 16-bit offsets, three columns: the form that reads the level
+    # row by row.  (The V-cycle itself reads this level in slices and fuses the
+    # step with the prolongation where that saves bytes.)  Bytes as
+    # vcycle_bytes counts a middle step (direction read and written)
     kr = eng.krylov
     if getattr(kr, "compact", None) is not None:
         from waterscapes_amd import autotune as at
@@ -1225,8 +1232,9 @@ def main():
         bytes_v = nnz0 * 4 + (n0 + 1) * 4 + 3 * n0 * 4 + 4 * 3 * n0 * 4 + n0 * 4
         ach_v = bytes_v / (ms_v * 1e-3) / 1e9
         out["roofline_vcycle_level0"] = {
-            "kernel": f"spmm_kernel<float,3,{lpr0},3,true> (P2-level Chebyshev step of the "
-                      f"displacement V-cycle, half values, {nnz0} nonzeros x 3 columns)",
+            "kernel": f"spmm_kernel<float,3,{lpr0},3,true> (Chebyshev step with the P2 level's "
+                      f"CSR matrix, half values, {nnz0} nonzeros x 3 columns; the V-cycle reads "
+                      f"the level in slices)",
             "achieved": round(ach_v, 1), "frac": round(ach_v / 8000.0, 4),
             "bytes_per_launch": int(bytes_v), "ms_per_launch": round(ms_v, 4)}
     if not args.no_cpu_baseline and fp64_res is not None:

@@ -7,8 +7,8 @@ one matrix row:
   * the structured operator (fused MINRES step and mpet_op_apply): lanes
     per P2 node row (u rows) and per P1 node row (p rows) in {8, 16, 32},
     and the run length of row tiles dealt to one XCD (xcd_chunk, 0 or 4);
-  * the cell-wise FP32 operator (mpet_cell_op_apply): lanes of its row
-    kernel per P2 node row in {4, 8, 16} and per P1 node row in {8, 16},
+  * the cell-wise operator (mpet_cell_op_apply; FP32, or FP64 on the direct
+    path): lanes of its row kernel per P2 node row in {1, 4, 8, 16} and per P1 node row in {8, 16},
     and its XCD run length (0 or 4);
   * every AMG level of both hierarchies: lanes per row of the level
     operator (timed as the Chebyshev step) unless it runs sliced, and of the

@@ -9,12 +9,13 @@ step for every active instance in one set of kernel launches:
   * each instance keeps its own device-resident system (assembled
     primitives, Dirichlet data, right-hand-side kernels) and its own host
     AMG setup, exactly as a single solver would;
-  * the operator of all instances is packed into one block-diagonal
-    structured operator (u rows of all instances first, then the pressure
-    rows), and the hierarchies are concatenated level by level (instances
+  * the operator of all instances is applied cell by cell, in blocks that hold
+    one instance's cells, or in small batches (BATCH_CELLS) packed into one
+    block-diagonal structured operator (u rows of all instances first, then
+    the pressure rows), and the hierarchies are concatenated level by level (instances
     with fewer levels are padded with identity-prolongation levels ending in
-    their own coarsest matrix; the coarsest level is a block-diagonal dense
-    solve);
+    their own coarsest matrix; the small ends are dense operators, one
+    block per instance);
   * MINRES keeps one state per instance (each instance converges to its own
     tolerance with its own iteration count; finished instances are skipped).
 

@@ -12,7 +12,8 @@
 //       blocks in field-major order: aggregation never couples fields, so
 //       all A+1 blocks share every launch).
 //   Chebyshev smoothing (degree k on [rho/ratio, safety*rho] of D^-1 A),
-//   dense inverse on the coarsest level.
+//   one dense operator for the small end of each hierarchy.  Large systems
+//   run the two V-cycles on two streams, small ones in joint launches.
 //
 // MINRES (Paige & Saunders 1975) keeps its scalar recurrences on the device.
 // Dot products write one partial per block; a one-block finalize kernel
