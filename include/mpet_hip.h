@@ -180,7 +180,8 @@ typedef struct {
   const int64_t* coarse_ioff;
   int32_t level_degree[MPET_MAXLEV];  /* per-level Chebyshev degree (0: degree) */
   /* One dense block only: row r of coarse_inv is zero outside the columns
-   * coarse_rng[2r] .. coarse_rng[2r+1]-1 (device; NULL: whole rows). */
+   * coarse_rng[4r] .. coarse_rng[4r+1]-1 and coarse_rng[4r+2] ..
+   * coarse_rng[4r+3]-1 (device; NULL: whole rows). */
   const int32_t* coarse_rng;
 } MpetHierDesc;
 

@@ -55,18 +55,23 @@ def test_first_level_limit_and_rows():
 
 
 def test_column_ranges():
-    """First and one past the last nonzero column of every row, zero rows
-    empty: what the dense pressure kernels read of each row."""
+    """The two column runs the dense pressure kernels read of each row: all
+    nonzeros, without the longest run of zeros between two of them."""
     import torch
     from waterscapes_amd import levels as lv
     rng = np.random.default_rng(3)
-    M = np.zeros((9, 9))
+    M = np.zeros((12, 12))
     M[:4, :4] = rng.standard_normal((4, 4))
-    M[4:, 4:] = rng.standard_normal((5, 5))
+    M[4:, 4:] = rng.standard_normal((8, 8))
     M[2] = 0.0
-    M[6, 4] = M[7, 8] = 0.0
+    M[0, 10] = 1.0                       # a second run
+    M[6, 4] = M[7, 11] = M[8, 6] = 0.0   # shorter, and an inner zero
     got = lv.column_ranges(torch.as_tensor(M)).numpy()
-    for r in range(9):
-        nz = np.nonzero(M[r])[0]
-        want = (nz[0], nz[-1] + 1) if nz.size else (0, 0)
-        assert tuple(got[r]) == want
+    want = np.tile([4, 12, 12, 12], (12, 1))
+    want[:4] = (0, 4, 4, 4)
+    want[0] = (0, 4, 10, 11)
+    want[2] = 0
+    want[6, 0] = 5
+    want[7, 1:] = 11
+    want[8] = (4, 6, 7, 12)
+    assert np.array_equal(got, want)

@@ -757,12 +757,12 @@ __device__ __forceinline__ void dense_part(const T* __restrict__ row, const T* _
 }
 
 // Dense coarsest solve x = Cinv (scale b) (NC columns), one wave per row over
-// the row's nonzero columns rng (null: all): the pressure fields do not couple
-// in the preconditioner, so a row of F fields has 1 / F of them.  The 64 MiB
-// this can be are read once an apply: whole rows / ranges 75.7 / 68.7 us for
-// the FP64 preconditioner at 16^3 (A = 2), 186 / 182 us FP32 at 36^3 (A = 4).
-// b and x may lie in the vectors' own order (om); with k2 on, b's entries
-// are made by it, and each row's wave stores its own.
+// the row's nonzero columns rng (two runs; null: all): the pressure fields do
+// not couple in the preconditioner, so a row of F fields has 1 / F of them,
+// its field's columns and, further on, those of aggregates formed last.  The 64 MiB
+// this can be are read once an apply.  Whole rows / runs, us per iteration:
+// mixed 8^3 (A = 4, 3,645 rows) 76.3 / 47.8, 6^3 48.6 / 39.3, direct 8^3 (A =
+// 2) 60.7 / 48.8; the FP64 preconditioner at 16^3 75.7 / 68.7 us an apply.
 template <typename T, int NC>
 __device__ __forceinline__ void coarse_rows(int block, int n, const T* __restrict__ cinv,
                                             const int* __restrict__ rng, const T* b,
@@ -771,41 +771,46 @@ __device__ __forceinline__ void coarse_rows(int block, int n, const T* __restric
   const int r = block * (NT / 64) + threadIdx.x / 64;
   const int lane = threadIdx.x % 64;
   if (r >= n) return;
-  const int c0 = rng ? rng[2 * r] : 0, c1 = rng ? rng[2 * r + 1] : n;
   T acc[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) acc[c] = 0;
   const T* __restrict__ row = cinv + (long long)r * n;
   const bool own = om.F || om.map;
   const T kc2 = k2.y ? (T)(*k2.alfa / *k2.beta) : (T)0;
-  if (!own && k2.y) {
-    dense_part<T, NC, true>(row + c0, k2.y + (long long)NC * c0, c1 - c0, lane, acc,
-                            k2.r2o + (long long)NC * c0, kc2);
-  } else if (!own) {
-    dense_part<T, NC>(row + c0, b + (long long)NC * c0, c1 - c0, lane, acc);
-  } else {
-    for (int k0 = c0 + lane; k0 < c1; k0 += 256) {
-      T a[4], bv[4][NC];
+  const int runs = rng ? 2 : 1;
+#pragma unroll 1
+  for (int run = 0; run < runs; ++run) {
+    const int c0 = rng ? rng[4 * r + 2 * run] : 0, c1 = rng ? rng[4 * r + 2 * run + 1] : n;
+    if (c0 >= c1) continue;
+    if (!own && k2.y) {
+      dense_part<T, NC, true>(row + c0, k2.y + (long long)NC * c0, c1 - c0, lane, acc,
+                              k2.r2o + (long long)NC * c0, kc2);
+    } else if (!own) {
+      dense_part<T, NC>(row + c0, b + (long long)NC * c0, c1 - c0, lane, acc);
+    } else {
+      for (int k0 = c0 + lane; k0 < c1; k0 += 256) {
+        T a[4], bv[4][NC];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int k = k0 + 64 * j;
-        const int kc = k < c1 ? k : c1 - 1;
-        a[j] = k < c1 ? row[kc] : (T)0;
-        const long long o = NC == 1 ? om(kc) : (long long)NC * kc;
-        if (k2.y) {
-          T yv[NC], rv[NC];
-          load_nc<T, NC>(k2.y + o, yv);
-          load_nc<T, NC>(k2.r2o + o, rv);
+        for (int j = 0; j < 4; ++j) {
+          const int k = k0 + 64 * j;
+          const int kc = k < c1 ? k : c1 - 1;
+          a[j] = k < c1 ? row[kc] : (T)0;
+          const long long o = NC == 1 ? om(kc) : (long long)NC * kc;
+          if (k2.y) {
+            T yv[NC], rv[NC];
+            load_nc<T, NC>(k2.y + o, yv);
+            load_nc<T, NC>(k2.r2o + o, rv);
 #pragma unroll
-          for (int c = 0; c < NC; ++c) bv[j][c] = yv[c] - kc2 * rv[c];
-        } else {
-          load_nc<T, NC>(b + o, bv[j]);
+            for (int c = 0; c < NC; ++c) bv[j][c] = yv[c] - kc2 * rv[c];
+          } else {
+            load_nc<T, NC>(b + o, bv[j]);
+          }
         }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int c = 0; c < NC; ++c) acc[c] += a[j] * bv[j][c];
       }
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int c = 0; c < NC; ++c) acc[c] += a[j] * bv[j][c];
     }
   }
   const long long o = NC == 1 ? om(r) : (long long)NC * r;

@@ -101,14 +101,21 @@ def dense_tail(levels, cinv, start, params, device, values=None, mask0=None):
 
 
 def column_ranges(M):
-    """(n, 2) int32: the first and one past the last nonzero column of every
-    row of M (0, 0 for a zero row)."""
-    nz = (M != 0).to(torch.uint8)
+    """(n, 4) int32: two column runs [c0, c1), [c2, c3) of every row of M that
+    hold its nonzeros: the first to the last nonzero without the row's
+    longest inner run of zeros (empty runs for a zero row)."""
     n = M.shape[1]
+    j = torch.arange(n, dtype=torch.int32, device=M.device)
+    nz = M != 0
+    last = torch.where(nz, j, -1).cummax(dim=1).values      # last nonzero up to j
+    prev = torch.nn.functional.pad(last[:, :-1], (1, 0), value=-1)
+    gap, c2 = torch.where(nz & (prev >= 0), j - prev - 1, 0).max(dim=1)
+    c0 = torch.where(nz, j, n).amin(dim=1)
+    c3 = last[:, -1] + 1
+    c2 = torch.where(gap > 0, c2.to(torch.int32), c3)
     some = nz.any(dim=1)
-    lo = nz.argmax(dim=1)
-    hi = n - nz.flip(1).argmax(dim=1)
-    return (torch.stack([lo, hi], dim=1) * some[:, None]).to(torch.int32).contiguous()
+    out = torch.stack([c0, c2 - gap, c2, c3], dim=1) * some[:, None]
+    return out.to(torch.int32).contiguous()
 
 
 def tail_start(levels, rows):
