@@ -1,5 +1,5 @@
 """Error indicators for one, three and seven networks, with and without the
-staged copy to the host (GPU): random states on a box mesh vs the oracle.
+staged copy to the host and the sources read through LDS (GPU): random states on a box mesh vs the oracle.
 Every value is a sum of at most ~1e4 FP64 products of the same sign class
 (1e4 eps = 2e-12): 1e-11 of the largest, as for two networks."""
 import numpy as np
@@ -13,8 +13,8 @@ pytestmark = pytest.mark.gpu
 TOL = 1e-11
 
 
-@pytest.mark.parametrize("A,staged", [(1, False), (3, True), (7, True)])
-def test_network_counts(A, staged, monkeypatch):
+@pytest.mark.parametrize("A,staged,deg", [(1, False, 2), (3, True, 3), (7, True, 2)])
+def test_network_counts(A, staged, deg, monkeypatch):
     import torch
     from waterscapes_amd import MPETProblem, MPETSolver, Constant, Expression, BoxMesh
     from waterscapes_amd import adaptive
@@ -27,8 +27,9 @@ def test_network_counts(A, staged, monkeypatch):
                   S=tuple(tuple(r) for r in S))
     mesh = BoxMesh((0.0, 0.0, 0.0), (1.0, 1.5, 0.7), 2, 3, 2)
     problem = MPETProblem(mesh, Constant(0.4), params=dict(params))
-    f_ = Expression(("x[0]*x[1]", "x[2]", "x[1]"), degree=2)
-    problem.f = Expression(("x[0]*x[1]", "x[2]", "x[0]*x[0]"), degree=2)
+    # degree 2: the cell kernel reads the sources through LDS, degree 3: directly
+    f_ = Expression(("x[0]*x[1]", "x[2]", "x[1]"), degree=deg)
+    problem.f = Expression(("x[0]*x[1]", "x[2]", "x[0]*x[0]"), degree=deg)
     problem.g = [Expression("x[1]", degree=1) for _ in range(A)]
     solver = MPETSolver(problem, dict(dt=0.05, theta=1.0, T=0.1))
     n = solver.up.function_space().dim()
@@ -42,7 +43,7 @@ def test_network_counts(A, staged, monkeypatch):
         oracle_mesh(solver.up.function_space()), params, x, xp, 0.05,
         f=lambda X, t: np.stack([X[:, 0] * X[:, 1], X[:, 2], X[:, 0] ** 2], 1),
         fp=lambda X, t: np.stack([X[:, 0] * X[:, 1], X[:, 2], X[:, 1]], 1),
-        g=lambda X, t: np.stack([X[:, 1]] * A, 1), f_degree=2, g_degree=1, t=0.4)
+        g=lambda X, t: np.stack([X[:, 1]] * A, 1), f_degree=deg, g_degree=1, t=0.4)
     for a, b, c in zip(*got, ref):
         assert np.array_equal(a, b)
         assert np.abs(a - c).max() <= TOL * np.abs(c).max()

@@ -129,12 +129,54 @@ __device__ __forceinline__ void vertex_gradients(const IGeom& G, const double* _
 // kernels and the gather 79 us of a call's 367, the rest brings 6.3 MB to the
 // host; the call took 880 us with per-point gradients and Hessians and a
 // pageable copy).
-template <int A>
-__global__ void __launch_bounds__(128)
+// The sources' nodal values are 3 nkf (f, f^-) and A nkg (g) consecutive
+// doubles a cell, read again at every quadrature point.  A thread reading its
+// own cell's has 64 lines a load: 398 us at degree 2 with 15 points, 32^3 x 6
+// tets.  STAGE brings a block's into LDS first (one run in memory; rows of odd
+// length, so that a wave's reads spread over the banks): 128 us there.  Rows
+// past 64 KB a block (degree 3 for both f and f^-) are read directly.
+static inline __host__ __device__ int ind_row(const double* p, int w) { return p ? w | 1 : 0; }
+constexpr int IND_STAGE_ROW = 127;   // doubles a cell: at most 64 KB per 64 cells
+template <int A, bool STAGE>
+__global__ void __launch_bounds__(STAGE ? 64 : 128)
 ind_cell_kernel(MpetIndDesc d, const double* __restrict__ x, const double* __restrict__ xp,
                 double* __restrict__ out) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  constexpr int NTI = STAGE ? 64 : 128;
+  extern __shared__ double ind_lds[];
+  const int e = blockIdx.x * NTI + threadIdx.x;
+  const int wf = 3 * d.nkf, wg = A * d.nkg;
+  const int Wf = ind_row(d.f, wf), Wp = ind_row(d.fp, wf), Wg = ind_row(d.g, wg);
+  const double* sf = ind_lds;
+  const double* sp = ind_lds + NTI * Wf;
+  const double* sg = ind_lds + NTI * (Wf + Wp);
+  if constexpr (STAGE) {
+    const int first = blockIdx.x * NTI;
+    const int cnt = d.nC - first < NTI ? d.nC - first : NTI;
+    auto bring = [&](const double* __restrict__ src, int w, int W, double* dst) {
+      if (!src) return;
+      const double* __restrict__ p = src + (long long)first * w;
+      int row = threadIdx.x / w, col = threadIdx.x % w;
+      for (int i = threadIdx.x; i < cnt * w; i += NTI) {
+        dst[row * W + col] = p[i];
+        col += NTI % w;
+        row += NTI / w;
+        if (col >= w) {
+          col -= w;
+          ++row;
+        }
+      }
+    };
+    bring(d.f, wf, Wf, ind_lds);
+    bring(d.fp, wf, Wp, ind_lds + NTI * Wf);
+    bring(d.g, wg, Wg, ind_lds + NTI * (Wf + Wp));
+    __syncthreads();
+  }
   if (e >= d.nC) return;
+  auto f_at = [&](int k) { return STAGE ? sf[threadIdx.x * Wf + k] : d.f[(long long)e * wf + k]; };
+  auto fp_at = [&](int k) {
+    return STAGE ? sp[threadIdx.x * Wp + k] : d.fp[(long long)e * wf + k];
+  };
+  auto g_at = [&](int k) { return STAGE ? sg[threadIdx.x * Wg + k] : d.g[(long long)e * wg + k]; };
   const long long nu = 3ll * d.nP2;
   IGeom G;
   int p2[10], v[4];
@@ -199,12 +241,12 @@ ind_cell_kernel(MpetIndDesc d, const double* __restrict__ x, const double* __res
     if (d.f)
       for (int m = 0; m < d.nkf; ++m) {
         const double L = d.Lf[q * d.nkf + m];
-        for (int i = 0; i < 3; ++i) fq[i] += L * d.f[(3ll * (long long)e * d.nkf) + 3 * m + i];
+        for (int i = 0; i < 3; ++i) fq[i] += L * f_at(3 * m + i);
       }
     if (d.fp)
       for (int m = 0; m < d.nkf; ++m) {
         const double L = d.Lf[q * d.nkf + m];
-        for (int i = 0; i < 3; ++i) fpq[i] += L * d.fp[(3ll * (long long)e * d.nkf) + 3 * m + i];
+        for (int i = 0; i < 3; ++i) fpq[i] += L * fp_at(3 * m + i);
       }
     double ru2 = 0.0, rd2 = 0.0;
     for (int i = 0; i < 3; ++i) {
@@ -231,7 +273,7 @@ ind_cell_kernel(MpetIndDesc d, const double* __restrict__ x, const double* __res
       double gj = 0.0;
       if (d.g)
         for (int m = 0; m < d.nkg; ++m)
-          gj += d.Lg[q * d.nkg + m] * d.g[((long long)e * d.nkg + m) * A + j];
+          gj += d.Lg[q * d.nkg + m] * g_at(m * A + j);
       double r = -gj - d.c[j] * (pj[j] - ppj[j]) * idt - d.alpha[j] * du * idt;
 #pragma unroll
       for (int i = 0; i < A; ++i) r -= d.S[i * MPET_MAXF + j] * (pj[j] - pj[i]);
@@ -392,10 +434,17 @@ using namespace mpet;
 static int launch_indicators(const MpetIndDesc* d, const double* x, const double* xp,
                              const int* fac, int nF, const int* cell_f, double* tmp,
                              double* out, hipStream_t stream, const char* who) {
+  const int row = ind_row(d->f, 3 * d->nkf) + ind_row(d->fp, 3 * d->nkf) +
+                  ind_row(d->g, d->A * d->nkg);
+  const bool stage = row > 0 && row <= IND_STAGE_ROW;
 #define IND_CASE(N)                                                                            \
   case N:                                                                                      \
-    hipLaunchKernelGGL((ind_cell_kernel<N>), dim3((d->nC + 127) / 128), dim3(128), 0, stream,  \
-                       *d, x, xp, out);                                                        \
+    if (stage)                                                                                 \
+      hipLaunchKernelGGL((ind_cell_kernel<N, true>), dim3((d->nC + 63) / 64), dim3(64),        \
+                         64 * row * sizeof(double), stream, *d, x, xp, out);                   \
+    else                                                                                       \
+      hipLaunchKernelGGL((ind_cell_kernel<N, false>), dim3((d->nC + 127) / 128), dim3(128), 0, \
+                         stream, *d, x, xp, out);                                              \
     if (nF > 0)                                                                                \
       hipLaunchKernelGGL((ind_facet_kernel<N>), dim3((nF + 127) / 128), dim3(128), 0, stream,  \
                          *d, x, xp, fac, nF, tmp);                                             \
