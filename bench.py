@@ -136,7 +136,7 @@ def _mat_bytes(nnz, rows, s, compact=False):
     return nnz * (4 if compact else s + 4) + (rows + 1) * 4
 
 
-def vcycle_bytes(levels, amgp, NC, s, compact=(), scaled=False, nfields=1):
+def vcycle_bytes(levels, amgp, NC, s, compact=(), scaled=False, dense=None):
     """Algorithmic HBM bytes of one V-cycle (amg_cycle.h: vcycle / smooth /
     spmm modes), each array read once per launch: matrices, the gathered
     vector once, the epilogue vectors; levels = the host hierarchy dicts,
@@ -144,8 +144,8 @@ def vcycle_bytes(levels, amgp, NC, s, compact=(), scaled=False, nfields=1):
     Chebyshev direction is not read by the first step from x and not written
     by a sequence's last step.  Counted step by step: a level whose transfers
     are fused with its smoothing reads other matrices (levels.py, kept where
-    they are no larger), and a pressure field's rows of the dense coarsest
-    operator hold only that field's columns."""
+    they are no larger).  dense: the values read of the dense coarsest operator
+    (all of them unless given)."""
     nl = len(levels)
     tot = 0
 
@@ -161,8 +161,7 @@ def vcycle_bytes(levels, amgp, NC, s, compact=(), scaled=False, nfields=1):
         lev = levels[l]
         n = lev["n"]
         if l == nl - 1:
-            # dense coarsest solve (NC = 1: the fields' blocks only)
-            tot += n * n * s // (nfields if NC == 1 else 1) + 2 * NC * n * s
+            tot += (n * n if dense is None else dense) * s + 2 * NC * n * s   # dense end
             return
         nnz = len(lev["A_ci"])
         cmp = l in compact
@@ -196,6 +195,14 @@ def _compact_p(kr, mixed):
     return tuple(getattr(kr, "pcompact_levels", ())) if mixed else ()
 
 
+def _dense_p(kr):
+    """Values the pressure hierarchy's dense end reads: each row's runs."""
+    import torch
+    from waterscapes_amd import levels as lv
+    r = lv.column_ranges(torch.as_tensor(kr._coarse_p)).long()
+    return int((r[:, 1] - r[:, 0] + r[:, 3] - r[:, 2]).sum())
+
+
 def iteration_bytes(eng, mixed):
     """Algorithmic HBM bytes of one MINRES iteration of the engine's solve
     (krylov.hip minres_iter): K1 (operator apply with the fused MINRES step:
@@ -215,7 +222,7 @@ def iteration_bytes(eng, mixed):
     else:
         k1 = csr_bytes(sysm) + n * s
     vu = vcycle_bytes(kr.levels, kr.cfg.amg, 3, s, compact=_compact_u(kr, mixed), scaled=True)
-    vp = vcycle_bytes(kr.plevels, kr.cfg.pamg, 1, s, nfields=sysm.F,
+    vp = vcycle_bytes(kr.plevels, kr.cfg.pamg, 1, s, dense=_dense_p(kr),
                       compact=_compact_p(kr, mixed)) + 4 * sysm.F * sysm.nP1 * s
     blas = 10 * n * s
     parts = {"k1": int(k1), "vcycle_u": int(vu), "vcycle_p": int(vp), "blas1": int(blas)}
@@ -238,7 +245,7 @@ def step_bytes(eng, mixed, inner, outer):
     else:
         op64 = op_bytes(sysm, 0) if (mixed or kr.csr_desc is None) else csr_bytes(sysm)
     pc = vcycle_bytes(kr.levels, kr.cfg.amg, 3, s, compact=_compact_u(kr, mixed),
-                      scaled=True) + vcycle_bytes(kr.plevels, kr.cfg.pamg, 1, s, nfields=sysm.F,
+                      scaled=True) + vcycle_bytes(kr.plevels, kr.cfg.pamg, 1, s, dense=_dense_p(kr),
                                                   compact=_compact_p(kr, mixed))
     starts = 2 + (outer if mixed else 0)
     solve_overhead = starts * (op64 + n * 8 + pc + 2 * n * s)
