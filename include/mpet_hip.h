@@ -110,12 +110,15 @@ typedef struct {
  * sits at 64 (off[s] + j) + i; its column is base[s] plus its 16-bit offset,
  * from dc, or (dc NULL, FP32 hierarchies) from the upper half of a 32-bit
  * value whose lower half is the value in half precision times 1 / A_vscale.
- * row[64 s + i] is the lane's row (-1: none; any order); ceil(n / 64) slices. */
+ * row[64 s + i] is the lane's row (-1: none; any order).  count: the slices
+ * (0: ceil(n / 64)).  A padding entry reads its slice's smallest column, so in
+ * a batch a slice holds rows of one instance only. */
 typedef struct {
   const int32_t* off;
   const int32_t* base;
   const int32_t* row;
   const uint16_t* dc;
+  int32_t count;
 } MpetSlices;
 
 /* One level of the displacement-block hierarchy (device arrays, int32

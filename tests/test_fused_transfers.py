@@ -100,6 +100,41 @@ def test_slices_hold_the_matrix(n, m, density, pair):
     assert np.array_equal(got, M.toarray())
 
 
+@pytest.mark.parametrize("sizes", [(700, 900), (64, 1, 513), (27, 30, 5, 700)])
+@pytest.mark.parametrize("broken", [0, 1])
+def test_slices_stay_inside_an_instance(sizes, broken):
+    """Rows of a packed level's other instances do not read an instance whose
+    vector is NaN, padding entries and rows without entries included; each
+    row's sum is its matrix row's."""
+    import torch
+    from waterscapes_amd import levels as lv
+    blocks = [sp.random(k, k, 0.02, random_state=i, format="lil") for i, k in enumerate(sizes)]
+    for b in blocks:
+        b[b.shape[0] // 2] = 0.0                     # a row without entries
+    blocks[-1][:] = 0.0                              # a padded level: no matrix
+    blocks[-2][::3, :] = 1.0                         # padding beside long rows
+    M = sp.block_diag(blocks, format="csr")
+    M.eliminate_zeros()
+    M.sort_indices()
+    n = M.shape[0]
+    grp = np.repeat(np.arange(len(sizes), dtype=np.int32), sizes)
+    s = lv.slices(torch.as_tensor(M.indptr), torch.as_tensor(M.indices),
+                  torch.as_tensor(M.data), n, torch.as_tensor(grp))
+    off, base, row, dc, v = (s[k].numpy() for k in ("off", "base", "row", "dc", "v"))
+    assert np.array_equal(np.sort(row[row >= 0]), np.arange(n))
+    x = np.random.default_rng(0).standard_normal(n)
+    ref = M @ x
+    x[grp == broken] = np.nan
+    y = np.full(n, np.nan)
+    for at in np.flatnonzero(row >= 0):              # as sell_part: padding multiplies too
+        k = 64 * np.arange(off[at // 64], off[at // 64 + 1]) + at % 64
+        y[row[at]] = (v[k] * x[base[at // 64] + dc[k]]).sum()
+    others = grp != broken
+    assert not np.isnan(y[others]).any()
+    assert np.abs(y[others] - ref[others]).max() <= 1e-13 * np.abs(ref).max()
+    assert len(base) == sum((k + 63) // 64 for k in sizes) == len(off) - 1
+
+
 def test_slices_refuse_wide_columns():
     import torch
     from waterscapes_amd import levels as lv

@@ -50,12 +50,25 @@ def test_nan_in_state_reports_nan(precision, extra):
     assert ei.value.code == 4
 
 
-def test_batch_nan_instance_reports_and_others_match_alone():
+def _sliced(monkeypatch):
+    """Every level sliced, both copies (A and Q), and dense ends small enough
+    for sparse levels to remain."""
+    from waterscapes_amd import levels as lv
+    monkeypatch.setattr(lv, "SLICE_ROWS", 1)
+    monkeypatch.setattr(lv, "DENSE_TAIL_BYTES", 3 * 20 * 20 * 4)
+
+
+@pytest.mark.parametrize("sliced", [False, True])
+def test_batch_nan_instance_reports_and_others_match_alone(sliced, monkeypatch):
     """A NaN in instance 0's state: the batch reports MPET_ERR_NAN, and the
     other instances' first steps equal their solo runs."""
     from waterscapes_amd._lib import MpetError
+    if sliced:
+        _sliced(monkeypatch)
     items = _make([0, 1, 2])
     batch = _batch(items, "mixed")
+    levels = batch.hier_levels["u"][1] + batch.hier_levels["p"][1]
+    assert any("A_s" in ld for ld in levels) == any("Q_s" in ld for ld in levels) == sliced
     s0 = batch.solvers[0]
     dm = batch.engines[0].system.dmask.cpu().numpy().astype(bool)
     free = np.nonzero(~dm)[0]
@@ -73,6 +86,14 @@ def test_batch_nan_instance_reports_and_others_match_alone():
         errs = field_errors(space, got, ref)
         assert max(errs) <= ISOLATION_RTOL, (k, errs)
     batch.close()
+
+
+def test_batch_isolation_sliced(monkeypatch):
+    """Each instance gives the same fields alone and in the mix, with every
+    level on one thread per row."""
+    import test_gpu_batch
+    _sliced(monkeypatch)
+    test_gpu_batch.test_batch_isolation()
 
 
 def test_batch_maxit_reports_not_converged():

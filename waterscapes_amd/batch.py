@@ -504,7 +504,7 @@ class MPETBatch:
             dinv = torch.as_tensor(lev["dinv"]).to(dev, tdt)
             grp = torch.as_tensor(_i32(lev["grp"])).to(dev)
             keep += [rp, ci, v, dinv, grp]
-            ld.update(A_rp=rp, A_ci=ci, A_v=v, dinv=dinv)
+            ld.update(A_rp=rp, A_ci=ci, A_v=v, dinv=dinv, grp=grp)
             L.A_rp, L.A_ci, L.A_v, L.dinv = ptr(rp), ptr(ci), ptr(v), ptr(dinv)
             L.grp = ptr(grp)
             if "A_v16" in lev:

@@ -27,7 +27,7 @@ from .amg import chebyshev_coefficients
 
 class Slices(C.Structure):
     _fields_ = [("off", C.c_void_p), ("base", C.c_void_p), ("row", C.c_void_p),
-                ("dc", C.c_void_p)]
+                ("dc", C.c_void_p), ("count", C.c_int32)]
 
 
 # A dense tail is used up to this many bytes of M.  Streaming it costs bytes
@@ -258,27 +258,42 @@ SLICE_ROWS = 1 << 16
 WINDOW = 512
 
 
-def slices(rp, ci, values, n):
+def slices(rp, ci, values, n, grp=None):
     """Sliced copy (include/mpet_hip.h, MpetSlices) of a CSR matrix with n
     rows on its device: dict of off, base, row, dc and v (values: (nnz,) or
-    (nnz, 2)), or None where the columns of some slice span 2^16 or more."""
+    (nnz, 2)), or None where the columns of some slice span 2^16 or more.
+
+    grp: the instance of each row of a packed level, not decreasing.  Windows
+    and slices hold rows of one instance only: a padding entry multiplies a
+    column of its slice by zero, and 0 x NaN from an instance that broke down
+    must not reach another one's rows."""
     dev = ci.device
     rp, ci = rp.long(), ci.long()
     length = rp[1:] - rp[:-1]
     at = torch.arange(n, device=dev)
+    grp = torch.zeros_like(at) if grp is None else grp.to(dev).long()
+    rows = torch.bincount(grp) if n else at              # of each instance
+    mine = at - (torch.cumsum(rows, 0) - rows)[grp]      # row within the instance
+
+    def chunks(size):                    # of an instance's rows, and its first
+        cnt = (rows + size - 1) // size
+        return int(cnt.sum()), (torch.cumsum(cnt, 0) - cnt)[grp]
+    ns, first_slice = chunks(64)
+    _, first_window = chunks(WINDOW)
     longest = int(length.max()) + 1 if n else 1
-    order = torch.argsort((at // WINDOW) * longest + (longest - 1 - length), stable=True)
-    ns = (n + 63) // 64
+    order = torch.argsort((first_window + mine // WINDOW) * longest + (longest - 1 - length),
+                          stable=True)
+    # instances stay in place, so sorted position i is of instance grp[i]
+    place = torch.empty(n, dtype=torch.int64, device=dev)
+    place[order] = 64 * first_slice + mine               # slot of each row
     row = torch.full((64 * ns,), -1, dtype=torch.int64, device=dev)
-    row[:n] = order
+    row[place] = at
     width = torch.zeros(64 * ns, dtype=torch.int64, device=dev)
-    width[:n] = length[order]
+    width[place] = length
     width = width.view(ns, 64).amax(1)
     off = torch.zeros(ns + 1, dtype=torch.int64, device=dev)
     off[1:] = torch.cumsum(width, 0)
     total = 64 * int(off[-1])
-    place = torch.empty(n, dtype=torch.int64, device=dev)
-    place[order] = at                                    # slot of each row
     of = torch.repeat_interleave(at, length)             # row of each entry
     slot = place[of]
     j = torch.arange(ci.numel(), device=dev) - rp[of]
@@ -307,25 +322,27 @@ def add_slices(ld, n):
     row fills the chip."""
     if n < SLICE_ROWS:
         return
+    grp = ld.get("grp")
     if "A_v16" in ld:
-        s = slices(ld["A_rp"], ld["A_ci"], ld["A_v16"], n)
+        s = slices(ld["A_rp"], ld["A_ci"], ld["A_v16"], n, grp)
         if s is not None:            # half | offset << 16 in one 32-bit word
             bits = s["v"].view(torch.int16).to(torch.int32) & 0xffff
             word = bits | (_u16(s["dc"]).to(torch.int32) << 16)
             ld["A_s"] = dict(s, v=word, dc=None)
     else:
-        s = slices(ld["A_rp"], ld["A_ci"], ld["A_v"], n)
+        s = slices(ld["A_rp"], ld["A_ci"], ld["A_v"], n, grp)
         if s is not None:
             ld["A_s"] = dict(s, dc=_u16(s["dc"]))
     if "Q_v" in ld:
         q = ld["Q_v"].view(ld["Q_ci"].numel(), -1)
-        s = slices(ld["Q_rp"], ld["Q_ci"], q, n)
+        s = slices(ld["Q_rp"], ld["Q_ci"], q, n, grp)
         if s is not None:
             ld["Q_s"] = dict(s, dc=_u16(s["dc"]))
 
 
 def _describe_slices(S, s):
     S.off, S.base, S.row, S.dc = (ptr(s[k]) for k in ("off", "base", "row", "dc"))
+    S.count = s["base"].numel()
 
 
 def add_fused(levs, hosts, params, dtype, mask0=None):
