@@ -718,7 +718,8 @@ typedef struct {
 
 /* Apply the batch's operator cell by cell from now on, in both precisions
  * (Kuu, Dv and Dt of its operator descriptors are not read any more and may
- * have been NULL); once per handle, drops captured graphs. */
+ * have been NULL: until then such a handle's solves and applications return
+ * MPET_ERR_INVALID); once per handle, drops captured graphs. */
 int mpet_batch_set_cell_operator(void* h, const MpetBatchCellDesc* desc);
 
 /* One time step of the instances with active[k] != 0 (NULL: all): for each,

@@ -55,3 +55,26 @@ def test_fp32_operator_and_residual():
                 scale = y64[i].abs().max().item()
                 assert (y32[i].double() - y64[i]).abs().max().item() <= FP32_RTOL * scale
     batch.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_no_operator_is_refused(precision, monkeypatch):
+    """A handle made without packed values, whose cell-wise operator was
+    refused, returns an error from solves and applications (no launch)."""
+    import torch
+    from waterscapes_amd import _lib, batch as B
+    monkeypatch.setattr(B.MPETBatch, "_pack_cells", lambda self: B.BatchCellDesc())
+    b = B.MPETBatch.__new__(B.MPETBatch)
+    with pytest.raises(_lib.MpetError) as ei:
+        b.__init__([it[2] for it in base._make([0, 2])], precision=precision)
+    invalid = ei.value.code
+    x = torch.ones(b.n, dtype=torch.float64, device="cuda")
+    for dtype in (0,) if precision == "fp64" else (0, 1):
+        with pytest.raises(_lib.MpetError) as ei:
+            b.apply(x if dtype == 0 else x.float(), dtype=dtype)
+        assert ei.value.code == invalid
+    y, stats = torch.zeros_like(x), (B.SolveStats * b.K)()
+    rc = B._bind().mpet_batch_solve(b.handle, _lib.ptr(x), _lib.ptr(y), None, stats,
+                                    _lib.stream_ptr())
+    assert rc == invalid and not y.any()
+    b.close()

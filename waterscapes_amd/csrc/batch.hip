@@ -957,6 +957,15 @@ extern "C" int mpet_batch_create(const MpetBatchOpDesc* op64, const MpetBatchOpD
   return OK;
 }
 
+// The operator of one precision can be applied: cell by cell, or from packed
+// values, which a handle created for the cell-wise operator may not have.
+template <typename T>
+static bool op_ready(const Batch* B, const BOp<T>& op) {
+  if (B->has_cw || (op.Kuu && op.Dv && op.Dt)) return true;
+  mpet_set_error("batch operator: neither packed values nor a cell-wise operator");
+  return false;
+}
+
 // Tiles of the cell-wise row kernels and their partial ranges.
 static int build_cell_layout(Batch* B) {
   const int K = B->ninst;
@@ -1049,6 +1058,7 @@ extern "C" int mpet_batch_apply(void* h, int dtype, const void* x, const void* b
     mpet_set_error("mpet_batch_apply: invalid argument");
     return ERR_INVALID;
   }
+  if (dtype == 0 ? !op_ready(B, B->op64) : !op_ready(B, B->op32)) return ERR_INVALID;
   if (dtype == 0)
     op_launch<double>(B, B->op64, (const double*)x, (const double*)b, (double*)y,
                       K1Args<double>{nullptr, nullptr, nullptr, nullptr, 0}, s);
@@ -1106,6 +1116,7 @@ extern "C" int mpet_batch_solve(void* h, const double* b, double* x, const int32
     mpet_set_error("mpet_batch_solve: invalid argument");
     return ERR_INVALID;
   }
+  if (!op_ready(B, B->op64) || (B->opt.mode == 1 && !op_ready(B, B->op32))) return ERR_INVALID;
   const int K = B->ninst;
   const int eb = (int)((B->n + NT - 1) / NT);
   std::vector<int> want(K), outer(K, 0), inner(K, 0), conv(K, 0), bad(K, 0);
