@@ -129,3 +129,27 @@ def test_batch_inactive_instances_untouched():
     assert batch.t[1] == t0[1] and batch.t[0] == pytest.approx(t0[0] + 0.05)
     assert not torch.equal(batch.solvers[0].up.data, before[0])
     batch.close()
+
+
+def test_repack_keeps_dense_tails(monkeypatch):
+    """A re-pack with another number of instances (another row limit, the same
+    cuts) forms no dense tail again and gives the same preconditioner."""
+    import torch
+    from waterscapes_amd import levels as lv
+    made = []
+    form = lv.dense_tail
+    monkeypatch.setattr(lv, "dense_tail", lambda *a, **k: made.append(1) or form(*a, **k))
+    items = _make([0, 1, 2])
+    r = torch.linspace(-1.0, 1.0, 50000, dtype=torch.float64, device="cuda")
+
+    def first_two(batch):
+        z = batch.unpack(batch.precond(batch.pack(r[:batch.n]))).cpu().numpy()
+        batch.close()
+        return z[:int(batch.n_off[2])]
+    z3 = first_two(_batch(items, "fp64"))
+    count = len(made)
+    assert count > 0
+    z2 = first_two(_batch(items[:2], "fp64"))
+    assert len(made) == count
+    assert np.array_equal(z2, z3)
+    assert np.array_equal(first_two(_batch(items, "fp64")), z3)

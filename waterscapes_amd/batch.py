@@ -138,7 +138,8 @@ def csr_blockdiag(blocks):
 
 
 def pack_hierarchy(hiers, scales, skip_A0=False):
-    """Concatenate instance hierarchies level by level (host arrays).
+    """Concatenate instance hierarchies level by level (host arrays; the dense
+    coarsest operators stay on the device where all of them are there).
 
     hiers: list of (levels, cinv) as returned by amg.setup_host; scales:
     per-instance factor s_k (the packed hierarchy approximates
@@ -172,7 +173,11 @@ def pack_hierarchy(hiers, scales, skip_A0=False):
         out.append(d)
     sizes = [p[0][-1]["n"] for p in padded]
     off = _prefix(sizes)
-    inv = np.concatenate([(lv.host_array(p[1]) / s[k]).reshape(-1) for k, p in enumerate(padded)])
+    if all(torch.is_tensor(p[1]) for p in padded):
+        inv = torch.cat([(p[1] / s[k]).reshape(-1) for k, p in enumerate(padded)])
+    else:
+        inv = np.concatenate([(lv.host_array(p[1]) / s[k]).reshape(-1)
+                              for k, p in enumerate(padded)])
     ioff = _prefix([n * n for n in sizes])
     blk = np.repeat(np.arange(len(sizes), dtype=np.int32), sizes)
     return out, (inv, blk, _i32(off), ioff)

@@ -525,16 +525,23 @@ class KrylovSolver:
         """((u levels, u coarse), (p levels, p coarse)) cut at the first level
         of at most `rows` rows with the levels' own FP64 values, the
         displacement hierarchy at level u_first or later (1 where the P2
-        level runs on half-precision values).  Kept for the last `rows`."""
-        key = (rows, u_first)
-        if getattr(self, "_tails", (None,))[0] != key:
-            s = self.sys
-            u = lv.with_dense_tail(self.levels, self._coarse_u, rows, self.cfg.amg, s.device,
-                                   lambda l: (*s.pat_host["22"], self.lap0) if l == 0 else None,
-                                   self.mask0, u_first)
-            p = lv.with_dense_tail(self.plevels, self._coarse_p, rows, self.cfg.pamg, s.device)
-            self._tails = (key, (u, p))
-        return self._tails[1]
+        level runs on half-precision values); the dense operators on the
+        device.  Kept for the last cut of each hierarchy: a batch's limit
+        follows its number of instances, the cut changes with it rarely."""
+        s = self.sys
+        kept = self.__dict__.setdefault("_tails", {})
+
+        def cut(name, levels, coarse, params, first, *more):
+            start = lv.tail_start(levels, rows, first)
+            if kept.get(name, (None,))[0] != start:
+                levels, coarse = lv.with_dense_tail(levels, coarse, rows, params, s.device, *more,
+                                                    first=first)
+                kept[name] = (start, levels,
+                              torch.as_tensor(coarse).to(s.device, torch.float64))
+            return kept[name][1:]
+        return (cut("u", self.levels, self._coarse_u, self.cfg.amg, u_first,
+                    lambda l: (*s.pat_host["22"], self.lap0) if l == 0 else None, self.mask0),
+                cut("p", self.plevels, self._coarse_p, self.cfg.pamg, 0))
 
     def _upload_levels(self, levels, cinv, dtype, level0=None):
         """Device copies of a host hierarchy; level0 = (rp, ci, v) device

@@ -118,19 +118,20 @@ def column_ranges(M):
     return out.to(torch.int32).contiguous()
 
 
-def tail_start(levels, rows):
-    """The finest level of at most `rows` rows (the coarsest if none is)."""
+def tail_start(levels, rows, first=0):
+    """The finest level of at most `rows` rows, not before level `first` (the
+    coarsest if none is)."""
     for l, lev in enumerate(levels):
-        if lev["n"] <= rows:
+        if l >= first and lev["n"] <= rows:
             return l
     return len(levels) - 1
 
 
 def with_dense_tail(levels, cinv, rows, params, device, values=None, mask0=None, first=0):
-    """(levels, cinv) of the hierarchy cut at its finest level of at most
-    `rows` rows (not before level `first`), whose coarsest operator (device
-    FP64 tensor) is the V-cycle that began there."""
-    start = max(tail_start(levels, rows), min(first, len(levels) - 1))
+    """(levels, cinv) of the hierarchy cut at tail_start(levels, rows, first),
+    whose coarsest operator (device FP64 tensor) is the V-cycle that began
+    there."""
+    start = tail_start(levels, rows, first)
     if start == len(levels) - 1:
         return levels, cinv
     M = dense_tail(levels, cinv, start, params, device, values, mask0)
