@@ -75,6 +75,43 @@ def test_products_equal_scipy(degree, masked, empty):
         assert np.abs(csr("Q_rp", "Q_ci", q[:, 1], (n, nc)) - (live @ P).toarray()).max() <= 1e-13
 
 
+@pytest.mark.parametrize("degree", [1, 2])
+@pytest.mark.parametrize("choice", [(True, False), (False, True), (False, False)])
+def test_only_the_chosen_products_are_formed(degree, choice, monkeypatch):
+    """The choice is made from the sizes the products would have; the other
+    product's values are not formed, and a sliced Q replaces its CSR form."""
+    import torch
+    from waterscapes_amd import amg, levels as lv
+    A = _laplacian(5, 0.1)
+    lev = amg.setup_host(A.indptr, A.indices, A.data, amg.AmgParams(max_coarse=5))[0][0]
+    formed = []
+
+    def values(*a):
+        formed.append(a[0].numel())
+        return _host_values(*a)
+
+    def csr(k):
+        return tuple(torch.as_tensor(lev[k + e]).to(torch.float64 if e == "_v" else torch.int32)
+                     for e in ("_rp", "_ci", "_v"))
+    args = csr("A"), csr("P"), csr("R"), torch.as_tensor(lev["dinv"]), degree, 0.7
+    full = lv.fused_transfers(*args, values=values)
+    formed.clear()
+    sizes = {}
+    got = lv.fused_transfers(*args, values=values,
+                             use=lambda f: sizes.update((k, v.numel()) for k, v in f.items())
+                             or choice)
+    assert sizes == {k: full[k].numel() for k in ("W_ci", "Q_ci", "Q_v")}
+    assert len(formed) == sum(choice)
+    assert set(got) == {k for k in full if choice["WQ".index(k[0])]}
+    assert all(torch.equal(got[k], full[k]) for k in got)
+    ld = dict(got, A_rp=args[0][0], A_ci=args[0][1], A_v=args[0][2])
+    monkeypatch.setattr(lv, "SLICE_ROWS", 1)
+    lv.add_slices(ld, lev["n"])
+    assert ("Q_s" in ld) == ("Q_v" in ld) == choice[1] and "Q_ci" not in ld
+    if choice[1]:
+        assert ld["Q_v"] is ld["Q_s"]["v"]
+
+
 @pytest.mark.parametrize("n,m,density", [(1, 5, 0.0), (64, 64, 0.05), (65, 3, 1.0),
                                          (1000, 400, 0.02), (1537, 65536, 0.01)])
 @pytest.mark.parametrize("pair", [False, True])

@@ -198,16 +198,33 @@ def _values(rows, cols, X, Y):
     return out
 
 
-def fused_transfers(A, P, R, dinv, degree, c0, mask=None, values=_values):
+def fused_transfers(A, P, R, dinv, degree, c0, mask=None, values=_values, use=None):
     """W and Q of one level from its device matrices A, P, R = (rp, ci, FP64
     values) with sorted int32 columns: dict of W_rp, W_ci, W_v, Q_rp, Q_ci,
     Q_v (FP64 values; Q_v holds pairs for degree > 1).  dinv: FP64 diagonal
-    inverse, c0: the first Chebyshev coefficient, mask: rows held at zero."""
+    inverse, c0: the first Chebyshev coefficient, mask: rows held at zero.
+    use(f): (form W, form Q) from their sizes alone, f a dict of W_ci, Q_ci and
+    Q_v without storage (None: both)."""
     n, nc = A[0].numel() - 1, R[0].numel() - 1
     key = _product_keys(A[:2], P[:2], max(nc, 1))
-    rows, cols = key // nc, key % nc
+    use_w = use_q = True
+    if use is not None:
+        nnz, many = key.numel(), degree > 1
+        use_w, use_q = use({k: torch.empty(m, device="meta") for k, m in
+                            (("W_ci", nnz + (R[1].numel() if many else 0)), ("Q_ci", nnz),
+                             ("Q_v", nnz * (1 + many)))})
     dead = None if mask is None else mask.bool()
-    # A P and P on the pattern of A P
+    out = {}
+    if use_q:
+        out.update(_fused_prolongation(A, P, dinv, degree, c0, dead, key, n, nc, values))
+    if use_w:
+        out.update(_fused_restriction(A, R, dinv, degree, c0, dead, key, n, nc, values))
+    return out
+
+
+def _fused_prolongation(A, P, dinv, degree, c0, dead, key, n, nc, values):
+    """A P and P on the pattern of A P."""
+    rows, cols = key // nc, key % nc
     ap = values(rows, cols, A, P)
     prow = torch.repeat_interleave(torch.arange(n, device=key.device),
                                    (P[0][1:] - P[0][:-1]).long())
@@ -218,7 +235,12 @@ def fused_transfers(A, P, R, dinv, degree, c0, mask=None, values=_values):
         p[dead[rows]] = 0.0
     q = p - c0 * dinv[rows] * ap if degree == 1 else torch.stack([ap, p], 1).reshape(-1)
     q_rp, q_ci = _csr(rows, n, cols, "fused prolongation")
-    # R A on the transposed pattern
+    return dict(Q_rp=q_rp, Q_ci=q_ci, Q_v=q)
+
+
+def _fused_restriction(A, R, dinv, degree, c0, dead, key, n, nc, values):
+    """R A on the transposed pattern of A P, with R."""
+    rows, cols = key // nc, key % nc
     order = torch.argsort(cols * n + rows)
     wr, wc = cols[order], rows[order]
     ra = values(wr, wc, R, A)
@@ -245,7 +267,7 @@ def fused_transfers(A, P, R, dinv, degree, c0, mask=None, values=_values):
         row[at_ra], row[at_r] = wr, rrow
         wr, wc = row, col
     w_rp, w_ci = _csr(wr, nc, wc, "fused restriction")
-    return dict(W_rp=w_rp, W_ci=w_ci, W_v=w, Q_rp=q_rp, Q_ci=q_ci, Q_v=q)
+    return dict(W_rp=w_rp, W_ci=w_ci, W_v=w)
 
 
 # ---------------------------------------------------------------------------
@@ -337,8 +359,10 @@ def add_slices(ld, n):
     if "Q_v" in ld:
         q = ld["Q_v"].view(ld["Q_ci"].numel(), -1)
         s = slices(ld["Q_rp"], ld["Q_ci"], q, n, grp)
-        if s is not None:
+        if s is not None:            # instead of the CSR form
             ld["Q_s"] = dict(s, dc=_u16(s["dc"]))
+            ld["Q_v"] = s["v"]
+            del ld["Q_rp"], ld["Q_ci"]
 
 
 def _describe_slices(S, s):
@@ -358,17 +382,14 @@ def add_fused(levs, hosts, params, dtype, mask0=None):
         deg = params.degree(l)
         lmax = hosts[l]["rho"] * params.eig_safety
         c0 = float(chebyshev_coefficients(lmax / params.eig_ratio, lmax, deg)[1][0])
+        size, n = (8 if dtype == 0 else 4), int(hosts[l]["n"])
         f = fused_transfers((ld["A_rp"], ld["A_ci"], av),
                             (ld["P_rp"], ld["P_ci"], ld["P_v"].double()),
                             (ld["R_rp"], ld["R_ci"], ld["R_v"].double()), ld["dinv"].double(),
-                            deg, c0, mask0 if l == 0 else None)
-        size = 8 if dtype == 0 else 4
-        use_w, use_q = worth_fusing(ld, f, size, n := int(hosts[l]["n"]))
+                            deg, c0, mask0 if l == 0 else None,
+                            use=lambda f, ld=ld, n=n: worth_fusing(ld, f, size, n))
         tdt = torch.float64 if dtype == 0 else torch.float32
-        for k, use in (("W", use_w), ("Q", use_q)):
-            if use:
-                ld.update({f"{k}_rp": f[f"{k}_rp"], f"{k}_ci": f[f"{k}_ci"],
-                           f"{k}_v": f[f"{k}_v"].to(tdt)})
+        ld.update({k: v.to(tdt) if k in ("W_v", "Q_v") else v for k, v in f.items()})
         add_slices(ld, n)
 
 
@@ -408,11 +429,12 @@ def describe_fused(L, ld, n, ncoarse, nc):
         L.W_rp, L.W_ci, L.W_v = ptr(ld["W_rp"]), ptr(ld["W_ci"]), ptr(ld["W_v"])
         L.lgW = _log2_lanes(ld["W_ci"].numel() / max(ncoarse, 1), ncoarse, nc)
     if "Q_v" in ld:
-        L.Q_rp, L.Q_ci, L.Q_v = ptr(ld["Q_rp"]), ptr(ld["Q_ci"]), ptr(ld["Q_v"])
-        L.lgQ = _log2_lanes(ld["Q_ci"].numel() / max(n, 1), n, nc)
+        L.Q_v = ptr(ld["Q_v"])
+        if "Q_ci" in ld:
+            L.Q_rp, L.Q_ci = ptr(ld["Q_rp"]), ptr(ld["Q_ci"])
+            L.lgQ = _log2_lanes(ld["Q_ci"].numel() / max(n, 1), n, nc)
     if "A_s" in ld:
         _describe_slices(L.A_s, ld["A_s"])
         L.A_sv = ptr(ld["A_s"]["v"])
     if "Q_s" in ld:
         _describe_slices(L.Q_s, ld["Q_s"])
-        L.Q_v = ptr(ld["Q_s"]["v"])
