@@ -7,6 +7,7 @@ import subprocess
 import sys
 
 import numpy as np
+import pytest
 import scipy.sparse as sp
 
 from waterscapes_amd import amg
@@ -54,3 +55,33 @@ def test_coarse_inverse_independent_of_thread_count():
         outs.append(subprocess.run([sys.executable, "-c", code], env=env, check=True,
                                    capture_output=True).stdout)
     assert len(outs[0]) > 0 and outs[0] == outs[1]
+
+
+@pytest.mark.parametrize("tensors", [False, True])
+def test_compact_level(tensors):
+    """Half values and 16-bit offsets of a level operator, from a pattern of
+    host arrays or tensors; refused where an offset or a diagonal is out of
+    range."""
+    import torch
+    from waterscapes_amd.krylov import compact_level
+    n = 40000
+    rp = np.arange(0, 2 * n + 1, 2, dtype=np.int64)
+    ci = np.stack([np.maximum(np.arange(n) - 32767, 0), np.arange(n)], 1).astype(np.int32)
+    ci[0] = 0, 5
+    v = torch.as_tensor(np.random.default_rng(0).uniform(0.1, 3.0, 2 * n))
+
+    def pattern(c):
+        return (torch.as_tensor(rp.astype(np.int32)), torch.as_tensor(c)) if tensors else (rp, c)
+    c = compact_level(pattern(ci.reshape(-1)), v, 2.0 ** -22)
+    rows = np.repeat(np.arange(n), 2)
+    assert np.array_equal(c["A_dci"].numpy().astype(np.int64) + rows, ci.reshape(-1))
+    assert c["A_dci"].dtype == torch.int16 and c["A_v16"].dtype == torch.float16
+    assert 2.0 ** 9 <= float(c["A_v16"].max()) <= 2.0 ** 10
+    assert torch.equal(c["A_v16"], (v / c["vscale"]).half())
+    tiny = v.clone()
+    tiny[2 * 7 + 1] = 1e-8
+    assert compact_level(pattern(ci.reshape(-1)), tiny, 2.0 ** -22) is None
+    assert compact_level(pattern(ci.reshape(-1)), tiny) is not None
+    assert compact_level(pattern(ci.reshape(-1)), torch.zeros_like(v)) is None
+    ci[n - 1, 0] -= 1
+    assert compact_level(pattern(ci.reshape(-1)), v) is None

@@ -574,13 +574,7 @@ class MPETBatch:
         self.mask0 = torch.cat([k.mask0 for k in kry]).contiguous()
         if self.precision == "mixed" and kry[0].cfg.compact_level0:
             # half-precision finest level, as for one instance
-            rp_h = np.concatenate([s.pat_host["22"][0][:-1].astype(np.int64)
-                                   + int(self.nnz_off["22"][k]) for k, s in enumerate(sys_)]
-                                  + [self.nnz_off["22"][-1:]])
-            ci_h = np.concatenate([s.pat_host["22"][1].astype(np.int64) + int(self.p2_off[k])
-                                   for k, s in enumerate(sys_)])
-            c = compact_level((rp_h, ci_h),
-                              torch.cat([s.prim_t["Lap"] * s.mu for s in sys_]))
+            c = compact_level(level0[:2], torch.cat([s.prim_t["Lap"] * s.mu for s in sys_]))
             if c is not None:
                 ulev[0].update(c)
         # pressure blocks: field-major block-diagonal hierarchies, scale 1

@@ -186,33 +186,37 @@ def _pick_lpr(avg, nc=1, rows=None):
     return lanes
 
 
-def compact_level(pattern_host, values, min_diag_ratio=None):
-    """Half-precision copy of a level operator on a host CSR pattern
-    (rp, ci) with device FP64 values: values * 2^e rounded to half (the
-    largest magnitude mapped near 2^10), columns as int16 offsets from the
+def compact_level(pattern, values, min_diag_ratio=None):
+    """Half-precision copy of a level operator on a CSR pattern (rp, ci), host
+    arrays or tensors, with device FP64 values: values * 2^e rounded to half
+    (the largest magnitude mapped near 2^10), columns as int16 offsets from the
     row.  None if some offset does not fit in 16 bits, or (min_diag_ratio
     given) if some nonzero diagonal entry is smaller than min_diag_ratio
     times the largest value: half is absolutely accurate to 2^-25 (scaled)
     below its normal range, so with every nonzero diagonal normal each
-    row's entries keep half's relative precision measured on the row."""
-    rp, ci = pattern_host
-    rows = np.repeat(np.arange(rp.size - 1, dtype=np.int64), np.diff(rp))
-    off = ci.astype(np.int64) - rows
-    if off.size == 0 or np.abs(off).max() > 32767:
+    row's entries keep half's relative precision measured on the row.
+    Formed on the values' device: on the host the offsets of a packed P2 level
+    were a quarter of a batch's packing time."""
+    dev = values.device
+    rp, ci = (torch.as_tensor(t).to(dev) for t in pattern)
+    rp = rp.long()
+    rows = torch.repeat_interleave(torch.arange(rp.numel() - 1, device=dev), rp[1:] - rp[:-1],
+                                   output_size=ci.numel())
+    off = ci.long() - rows
+    if off.numel() == 0 or int(off.abs().max()) > 32767:
         return None
     mag = values.abs()
     vmax = float(mag.max().item())
     if not vmax > 0:
         return None
     if min_diag_ratio is not None:
-        dg = mag[torch.as_tensor(np.flatnonzero(off == 0)).to(mag.device)]
+        dg = mag[off == 0]
         dg = dg[dg > 0]
         if dg.numel() == 0 or float(dg.min().item()) < min_diag_ratio * vmax:
             return None
     e = 10 - int(np.ceil(np.log2(vmax)))
     v16 = (values * (2.0 ** e)).to(torch.float16)
-    dci = torch.as_tensor(off.astype(np.int16)).to(values.device)
-    return {"A_v16": v16, "A_dci": dci, "vscale": 2.0 ** (-e), "exp": e}
+    return {"A_v16": v16, "A_dci": off.to(torch.int16), "vscale": 2.0 ** (-e), "exp": e}
 
 
 class KrylovSolver:
@@ -459,7 +463,7 @@ class KrylovSolver:
     def _compact_u0(self):
         """Half-precision copy of the P2 level of the FP32 hierarchy, or None."""
         if not hasattr(self, "_cu0"):
-            self._cu0 = compact_level(self.sys.pat_host["22"], self.lap0) \
+            self._cu0 = compact_level(self.sys.pat_dev["22"], self.lap0) \
                 if self.cfg.compact_level0 else None
             if self._cu0 is not None:
                 self.compact = self._cu0
