@@ -7,7 +7,7 @@ with running requests deterministically."""
 import numpy as np
 import pytest
 
-from conftest import CFG1
+from conftest import CFG1, cfg2_params
 from test_gpu_api import build_problem, field_errors
 from test_gpu_batch import P_A1, P_A3
 
@@ -137,6 +137,53 @@ def test_footprint_estimate_bounds_allocation():
     # torch's allocations only (native workspaces are extra): the estimate
     # must cover them and not overshoot grossly
     assert 0.5 * used <= est <= 6.0 * used, (est, used)
+
+
+@pytest.mark.parametrize("n,A,count,precision", [(8, 4, 1, "mixed"), (8, 1, 3, "mixed"),
+                                                 (4, 2, 1, "fp64"), (4, 2, 3, "fp64")])
+def test_footprint_covers_dense_ends(n, A, count, precision):
+    """Small instances alone or few in a batch hold more in the dense ends of
+    their hierarchies than in everything else; the estimate covers torch's
+    allocations to 20%, as the terms it had before do."""
+    import torch
+    from waterscapes_amd.batch import MPETBatch
+    from waterscapes_amd.levels import DENSE_TAIL_BYTES
+    from waterscapes_amd.serve import footprint_bytes, tail_bytes, tail_bytes_all
+    w = torch.ones(64, 64, dtype=torch.float64, device="cuda")
+    w @ w                                        # the BLAS workspace is the process's
+    del w
+    torch.cuda.synchronize()
+    base = torch.cuda.memory_allocated()
+    sol = [build_problem(n, cfg2_params(A), "fp64", False, T=10.0, dt=0.05)[1]
+           for _ in range(count)]
+    b = MPETBatch(sol, precision=precision)
+    b.step()
+    torch.cuda.synchronize()
+    used = torch.cuda.memory_allocated() - base
+    space = sol[0].up_.function_space()
+    tails = min(count * tail_bytes(space, precision), tail_bytes_all(precision))
+    est = count * (footprint_bytes(space, precision) - tail_bytes(space, precision)) + tails
+    b.close()
+    assert used <= 1.2 * est, (used, est)
+    assert tail_bytes(space, precision) <= tail_bytes_all(precision)
+    assert tail_bytes_all(precision) == {"mixed": 6, "fp64": 4}[precision] * DENSE_TAIL_BYTES
+
+
+def test_server_shares_the_dense_ends():
+    """Admission counts the dense ends of many instances once, at most as much
+    as a batch can hold."""
+    from waterscapes_amd.serve import MPETServer, Request, tail_bytes_all
+    cap = tail_bytes_all("mixed")
+    srv = MPETServer(hbm_budget=10e9 + cap, setup_workers=0)
+    reqs = [Request(make_solver=None, steps=1, footprint=int(1e9) + cap // 2, tails=cap // 2)
+            for _ in range(11)]
+    for r in reqs[:10]:
+        assert srv._fits(r)
+        srv._hold(r, 1)
+    assert not srv._fits(reqs[10]) and (srv.used, srv.tails) == (10 * int(1e9), 5 * cap)
+    for r in reqs[:10]:
+        srv._hold(r, -1)
+    assert srv.used == srv.tails == 0
 
 
 def test_setup_threads_overlap_ticks_and_keep_results():

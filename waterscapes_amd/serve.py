@@ -13,8 +13,11 @@ resident until the request completes.  At every scheduling tick it
      threads, each on a stream of its own, while the ticks go on; it joins
      the batch at the first tick after its set-up finished (setup_workers =
      0: set up synchronously inside the tick);
-  2. re-packs the batch when requests were admitted (no assembly or AMG
-     setup is repeated: each instance's device state is reused);
+  2. re-packs the batch when requests were admitted.  No assembly or AMG
+     coarsening is repeated (each instance's device state is reused, the dense
+     ends of its hierarchies while their cut stays); the packed levels' fused
+     transfers and slices are formed anew: 58 ms for 12 instances of 8^3 to
+     18^3 cubes, about one batched step of theirs;
   3. runs one batched step of the unfinished instances the tick policy
      picks (requests that arrived while others were running join
      mid-flight: their steps overlap on the device with the others');
@@ -45,6 +48,7 @@ import numpy as np
 import torch
 
 from .batch import MPETBatch, batch_engine
+from .levels import DENSE_TAIL_BYTES, dense_rows
 
 ERR_BUDGET = 6
 
@@ -72,7 +76,7 @@ class Request:
     steps: int
     arrival: float = 0.0
     rid: object = None
-    footprint: int = 0
+    footprint: int = 0                 # HBM bytes alone (0: estimated)
     # filled by the server
     solver: object = None
     admitted: float = None
@@ -82,14 +86,41 @@ class Request:
     result: np.ndarray = None
     niter: list = field(default_factory=list)
     refused: bool = False
+    tails: int = 0                     # of footprint: dense ends, shared in a batch
     _fp: object = None                 # footprint estimate running on a set-up thread
+
+
+def tail_bytes(space, precision="mixed"):
+    """Bound of the HBM bytes of one instance's dense hierarchy ends alone in a
+    batch (levels.py): the packed copy and the FP64 one kept for re-packs.
+    Levels above the row limit are coarsened by at least 8."""
+    s = 4 if precision == "mixed" else 8
+    most = dense_rows(s)
+
+    def end(rows):
+        while rows > most:
+            rows = -(-rows // 8)
+        return rows * rows
+    # FP64 levels all qualify; in mixed precision the P2 level stays sparse
+    u = space.nP2 if precision != "mixed" and space.nP2 <= most else space.nP1
+    return (8 + s) * (end(u) + end((space.A + 1) * space.nP1))
+
+
+def tail_bytes_all(precision="mixed"):
+    """The same bound for any number of instances: the two packed dense
+    operators of a batch hold DENSE_TAIL_BYTES each whatever their number."""
+    s = 4 if precision == "mixed" else 8
+    return 2 * DENSE_TAIL_BYTES * (8 + s) // s
 
 
 def footprint_bytes(space, precision="mixed", robin=False):
     """Estimated HBM bytes of one resident instance: FP64 primitives, the
     packed FP64 / FP32 operator copies, the AMG hierarchies with their work
-    vectors, and the step / MINRES vectors.  From the node patterns only (no
-    device allocation)."""
+    vectors and dense ends, and the step / MINRES vectors.  From the node
+    patterns only (no device allocation).  A batch that runs cell by cell keeps
+    cell tables instead of the packed operator values, which makes more than
+    room for its fused transfers and slices (32^3 cubes, A = 4: 1.46 GB in
+    use of 2.18 GB estimated)."""
     dm = space.dofmap
     nz = {k: int(dm.pattern(k)[1].size) for k in ("22", "21", "12", "11")}
     A, n, nP2, nP1 = space.A, space.ndofs, space.nP2, space.nP1
@@ -104,7 +135,7 @@ def footprint_bytes(space, precision="mixed", robin=False):
     amg = s * nz["22"] + (s + 4) * (nz["22"] + F * nz["11"]) // 2 \
         + 7 * s * (3 * nP2 + F * nP1) * 2
     vecs = 9 * s * n + 13 * 8 * n
-    return int(prim + ops + amg + vecs)
+    return int(prim + ops + amg + vecs + tail_bytes(space, precision))
 
 
 class MPETServer:
@@ -131,10 +162,12 @@ class MPETServer:
         self._pool = None
         self._local = threading.local()
         self.finished = []
+        # footprints of the resident requests but their dense ends, and those
         self.used = 0
+        self.tails = 0
         self.batch = None
         self.batch_reqs = []       # requests packed in self.batch, in order
-        self.pending_free = 0      # footprint of retired requests still packed
+        self.retired = []          # retired requests still packed
         self.t0 = clock()
         self.steps_run = 0
         self.ticks = 0
@@ -177,8 +210,9 @@ class MPETServer:
                     r.solver = r.make_solver()
                 prob = r.solver.problem
                 robin = any(not getattr(b, "is_zero", lambda: False)() for b in prob.beta)
-                r.footprint = footprint_bytes(r.solver.up_.function_space(), self.precision,
-                                              robin)
+                space = r.solver.up_.function_space()
+                r.tails = tail_bytes(space, self.precision)
+                r.footprint = footprint_bytes(space, self.precision, robin)
             return r.footprint
         return self._on_stream(work, req)
 
@@ -228,12 +262,12 @@ class MPETServer:
                 req.done = now
                 self.finished.append(req)
                 continue
-            if self.used + req.footprint > self.budget and self.pending_free:
+            if not self._fits(req) and self.retired:
                 self._drop_batch()         # release retired instances first
-            if self.used + req.footprint > self.budget:
+            if not self._fits(req):
                 break                      # wait until memory frees up
             self.waiting.pop(0)
-            self.used += req.footprint
+            self._hold(req, 1)
             if self.setup_workers > 0:
                 self.preparing.append((req, self._submit(self._setup, req)))
             else:
@@ -242,6 +276,14 @@ class MPETServer:
                 self.active.append(req)
                 changed = True
         return changed
+
+    def _hold(self, req, sign):
+        self.used += sign * (req.footprint - req.tails)
+        self.tails += sign * req.tails
+
+    def _fits(self, req):
+        tails = min(self.tails + req.tails, tail_bytes_all(self.precision))
+        return self.used + req.footprint - req.tails + tails <= self.budget
 
     def busy(self):
         """Requests waiting, being set up or running."""
@@ -253,8 +295,9 @@ class MPETServer:
             self.batch.close()
             self.batch = None
         self.batch_reqs = []
-        self.used -= self.pending_free
-        self.pending_free = 0
+        for r in self.retired:
+            self._hold(r, -1)
+        self.retired = []
         gc.collect()
 
     def _repack(self):
@@ -270,7 +313,7 @@ class MPETServer:
             if r.steps_done >= r.steps:
                 r.result = r.solver.up.vector().get_local().copy()
                 r.done = now
-                self.pending_free += r.footprint
+                self.retired.append(r)
                 r.solver = None
                 self.finished.append(r)
             else:
