@@ -13,8 +13,9 @@ pytestmark = pytest.mark.gpu
 TOL = 1e-11
 
 
-@pytest.mark.parametrize("A,staged,deg", [(1, False, 2), (3, True, 3), (7, True, 2)])
-def test_network_counts(A, staged, deg, monkeypatch):
+@pytest.mark.parametrize("A,staged,deg,with_g", [(1, False, 2, True), (3, True, 3, True),
+                                                 (7, True, 2, True), (2, False, 3, False)])
+def test_network_counts(A, staged, deg, with_g, monkeypatch):
     import torch
     from waterscapes_amd import MPETProblem, MPETSolver, Constant, Expression, BoxMesh
     from waterscapes_amd import adaptive
@@ -27,10 +28,12 @@ def test_network_counts(A, staged, deg, monkeypatch):
                   S=tuple(tuple(r) for r in S))
     mesh = BoxMesh((0.0, 0.0, 0.0), (1.0, 1.5, 0.7), 2, 3, 2)
     problem = MPETProblem(mesh, Constant(0.4), params=dict(params))
-    # degree 2: the cell kernel reads the sources through LDS, degree 3: directly
+    # degree 2, and degree 3 without g (122 doubles a cell, the longest rows
+    # that fit): the cell kernel reads the sources through LDS; else directly
     f_ = Expression(("x[0]*x[1]", "x[2]", "x[1]"), degree=deg)
     problem.f = Expression(("x[0]*x[1]", "x[2]", "x[0]*x[0]"), degree=deg)
-    problem.g = [Expression("x[1]", degree=1) for _ in range(A)]
+    if with_g:
+        problem.g = [Expression("x[1]", degree=1) for _ in range(A)]
     solver = MPETSolver(problem, dict(dt=0.05, theta=1.0, T=0.1))
     n = solver.up.function_space().dim()
     x, xp = rng.standard_normal(n), rng.standard_normal(n)
@@ -43,7 +46,8 @@ def test_network_counts(A, staged, deg, monkeypatch):
         oracle_mesh(solver.up.function_space()), params, x, xp, 0.05,
         f=lambda X, t: np.stack([X[:, 0] * X[:, 1], X[:, 2], X[:, 0] ** 2], 1),
         fp=lambda X, t: np.stack([X[:, 0] * X[:, 1], X[:, 2], X[:, 1]], 1),
-        g=lambda X, t: np.stack([X[:, 1]] * A, 1), f_degree=deg, g_degree=1, t=0.4)
+        g=(lambda X, t: np.stack([X[:, 1]] * A, 1)) if with_g else None, f_degree=deg,
+        g_degree=1, t=0.4)
     for a, b, c in zip(*got, ref):
         assert np.array_equal(a, b)
         assert np.abs(a - c).max() <= TOL * np.abs(c).max()

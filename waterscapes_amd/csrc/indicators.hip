@@ -133,8 +133,11 @@ __device__ __forceinline__ void vertex_gradients(const IGeom& G, const double* _
 // doubles a cell, read again at every quadrature point.  A thread reading its
 // own cell's has 64 lines a load: 398 us at degree 2 with 15 points, 32^3 x 6
 // tets.  STAGE brings a block's into LDS first (one run in memory; rows of odd
-// length, so that a wave's reads spread over the banks): 128 us there.  Rows
-// past 64 KB a block (degree 3 for both f and f^-) are read directly.
+// length, so that a wave's reads spread over the banks): 128 us there.  Up to
+// 64 KB a block: degree 3 for both f and f^- takes 62,464 bytes (two waves a CU,
+// and still the faster: a call 0.89 against 2.57 ms read directly at 32^3, 117
+// against 223 us at 8^3); rows past 127 doubles, such as those with a g beside
+// them, are read directly.
 static inline __host__ __device__ int ind_row(const double* p, int w) { return p ? w | 1 : 0; }
 constexpr int IND_STAGE_ROW = 127;   // doubles a cell: at most 64 KB per 64 cells
 template <int A, bool STAGE>
