@@ -67,8 +67,12 @@ class BatchCellDesc(C.Structure):
                                    "lsl1", "inc2_rp", "inc1_rp")]
 
 
-# Cells from which a batch's operator runs cell by cell (three launches and a
-# third of the bytes of the packed assembled values, two launches).
+# Cells from which a batch's operator runs cell by cell: two launches either
+# way, but a third of the bytes of the packed assembled values and more work a
+# cell.  An iteration cell by cell / packed, us: four instances of 5,400 cells in
+# all 82.9 / 78.3, 12,576 82.0 / 82.1, 17,820 94.2 / 92.5, 24,360 96.5 / 99.6,
+# 41,904 134.6 / 146.7; 12 of 16,200 98.7 / 96.6, of 25,452 101.0 / 104.9; 32 of
+# 20,736 126.6 / 122.2.
 BATCH_CELLS = 20000
 
 

@@ -275,7 +275,14 @@ def _fused_restriction(A, R, dinv, degree, c0, dead, key, n, nc, values):
 # ---------------------------------------------------------------------------
 # Levels of at least this many rows run one thread per row on sliced copies:
 # 65,536 rows are 1,024 waves, four per compute unit; below, several lanes
-# share a row.
+# share a row.  The line also decides between the two branches of a captured
+# graph (a sliced level) and joint launches of both V-cycles (none, amg_cycle.h
+# joint_ok), and lies where neither wins clearly.  An iteration sliced and forked
+# / not sliced, us: direct A = 2 at 16^3 (35,937 P2 rows) 115 / 106, 18^3 126 /
+# 124, 20^3 (68,921) 122 / 122, 22^3 132 / 132; mixed A = 4 at 16^3 100 / 101,
+# 20^3 106 / 110, 22^3 134 / 122, 24^3 140 / 134, 28^3 157 / 149 (forked either
+# way there); mixed A = 1 at 16^3 93 / 88, 20^3 104 / 97, 24^3 116 / 116, 28^3
+# (185,193) 133 / 140; at 48^3 (912,673) joint launches cost 474, slices 425.
 SLICE_ROWS = 1 << 16
 # rows are sorted by length within windows of this many (a multiple of 64)
 WINDOW = 512
