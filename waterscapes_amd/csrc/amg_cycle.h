@@ -348,7 +348,6 @@ struct Sell {
   const int* row = nullptr;        // row of each (slice, lane), -1: none
   const uint16_t* dc = nullptr;    // column - base; null for packed values
   const void* v = nullptr;         // T, pairs of T, or packed: half | offset << 16
-  int n = 0;                       // slices
 };
 enum SellValues { SELL_PLAIN = 0, SELL_PACKED = 1, SELL_PAIR = 2 };
 
@@ -1086,8 +1085,9 @@ struct LevelDev {
   const int *Wrp = nullptr, *Wci = nullptr, *Qrp = nullptr, *Qci = nullptr;
   const T *Wv = nullptr, *Qv = nullptr;
   int lgW = 3, lgQ = 2;
-  // sliced copies of the level operator and of Q (off null: none)
+  // sliced copies of the level operator and of Q (off null: none), their slices
   Sell<T> As, Qs;
+  int nAs = 0, nQs = 0;
   T *B = nullptr, *X = nullptr, *R = nullptr, *E = nullptr, *S1 = nullptr, *S2 = nullptr,
     *D = nullptr;
 };
@@ -1154,7 +1154,7 @@ static void spmm(const LevelDev<T>& L, int which, const T* x, const T* b, T* y, 
   int lpr = which == 0 ? L.lpr : (which == 1 ? L.lprP : L.lprR);
   if constexpr (MODE == 1 || MODE == 3) {
     if (which == 0 && L.As.off) {
-      const int ns = L.As.n, nb = (ns + NT / 64 - 1) / (NT / 64);
+      const int ns = L.nAs, nb = (ns + NT / 64 - 1) / (NT / 64);
       const SellEpi<T> E{b, nullptr, dinv ? dinv : L.dinv, d, cd, cr, (T)L.vscale, y, y2, L.mask,
                          om, L.grp};
       if (L.As.dc)
@@ -1290,7 +1290,7 @@ static void fused_down(const Hier<T>& H, int l, const T* b, Skip sk, hipStream_t
   const ResArgs<T> a = res_args(L, b, NC);
   const int nbw = row_blocks(w.n, w.lg), nba = row_blocks(a.n, a.lg);
   if (L.As.off) {
-    const int ns = L.As.n, nbs = (ns + NT / 64 - 1) / (NT / 64);
+    const int ns = L.nAs, nbs = (ns + NT / 64 - 1) / (NT / 64);
     const SellEpi<T> E{b, nullptr, nullptr, nullptr, 0, 0, (T)L.vscale, L.R, nullptr, L.mask,
                        OutMap(), L.grp};
     if (L.As.dc)
@@ -1327,7 +1327,7 @@ static void fused_up(const Hier<T>& H, int l, const T* b, T* out, Skip sk,
   T* dst = one ? out : L.S1;
   const OutMap dm = one ? om : OutMap();
   if (L.Qs.off) {
-    const int ns = L.Qs.n, nb = (ns + NT / 64 - 1) / (NT / 64);
+    const int ns = L.nQs, nb = (ns + NT / 64 - 1) / (NT / 64);
     const SellEpi<T> E{L.R, L.X, L.dinv, nullptr, 0, (T)L.cr[0], (T)1, dst, one ? nullptr : L.D,
                        L.mask, dm, L.grp};
     if (one)
@@ -1707,8 +1707,8 @@ static int build_hier(std::vector<void*>& allocs, const MpetHierDesc* d, int NC,
         mpet_set_error("invalid hierarchy description (sliced level)");
         return ERR_INVALID;
       }
-      L.As = Sell<T>{ld.A_s.off, ld.A_s.base, ld.A_s.row, ld.A_s.dc, ld.A_sv,
-                     slice_count(ld.A_s, L.n)};
+      L.As = Sell<T>{ld.A_s.off, ld.A_s.base, ld.A_s.row, ld.A_s.dc, ld.A_sv};
+      L.nAs = slice_count(ld.A_s, L.n);
     }
     if (l + 1 < H.nlev && (ld.W_v || ld.Q_v)) {
       const int lo = NC == 3 ? 2 : 0;
@@ -1722,9 +1722,10 @@ static int build_hier(std::vector<void*>& allocs, const MpetHierDesc* d, int NC,
       L.Qrp = ld.Q_rp; L.Qci = ld.Q_ci; L.Qv = (const T*)ld.Q_v;
       L.lgW = ld.lgW;
       L.lgQ = ld.lgQ;
-      if (ld.Q_s.off)
-        L.Qs = Sell<T>{ld.Q_s.off, ld.Q_s.base, ld.Q_s.row, ld.Q_s.dc, ld.Q_v,
-                       slice_count(ld.Q_s, L.n)};
+      if (ld.Q_s.off) {
+        L.Qs = Sell<T>{ld.Q_s.off, ld.Q_s.base, ld.Q_s.row, ld.Q_s.dc, ld.Q_v};
+        L.nQs = slice_count(ld.Q_s, L.n);
+      }
     }
   }
   for (int l = 0; l + 1 < H.nlev; ++l) H.lev[l].grpc = H.lev[l + 1].grp;
