@@ -1,5 +1,6 @@
-"""Error indicators for one, three and seven networks, with and without the
-staged copy to the host and the sources read through LDS (GPU): random states on a box mesh vs the oracle.
+"""Error indicators for one to seven networks, with and without the staged copy
+to the host and the sources read through LDS (GPU): random states on a box mesh
+vs the oracle.
 Every value is a sum of at most ~1e4 FP64 products of the same sign class
 (1e4 eps = 2e-12): 1e-11 of the largest, as for two networks."""
 import numpy as np
