@@ -139,16 +139,18 @@ def test_footprint_estimate_bounds_allocation():
     assert 0.5 * used <= est <= 6.0 * used, (est, used)
 
 
-@pytest.mark.parametrize("n,A,count,precision", [(8, 4, 1, "mixed"), (8, 1, 3, "mixed"),
-                                                 (4, 2, 1, "fp64"), (4, 2, 3, "fp64")])
-def test_footprint_covers_dense_ends(n, A, count, precision):
-    """Small instances alone or few in a batch hold more in the dense ends of
-    their hierarchies than in everything else; the estimate covers torch's
-    allocations to 20%, as the terms it had before do."""
+@pytest.mark.parametrize("n,A,count,precision,limit", [
+    (8, 4, 1, "mixed", None), (8, 4, 1, "mixed", 1 << 20), (8, 1, 3, "mixed", 1 << 23),
+    (4, 2, 1, "fp64", None), (4, 2, 3, "fp64", 1 << 18), (4, 2, 2, "fp64", 0)])
+def test_dense_ends_stay_within_their_limit(n, A, count, precision, limit):
+    """Small instances alone or few in a batch would hold more in the dense
+    ends of their hierarchies than in everything else: torch's allocations
+    stay within the footprints (to 20%, as without dense ends) and the bound
+    of the ends."""
     import torch
     from waterscapes_amd.batch import MPETBatch
     from waterscapes_amd.levels import DENSE_TAIL_BYTES
-    from waterscapes_amd.serve import footprint_bytes, tail_bytes, tail_bytes_all
+    from waterscapes_amd.serve import dense_held, footprint_bytes
     w = torch.ones(64, 64, dtype=torch.float64, device="cuda")
     w @ w                                        # the BLAS workspace is the process's
     del w
@@ -156,34 +158,36 @@ def test_footprint_covers_dense_ends(n, A, count, precision):
     base = torch.cuda.memory_allocated()
     sol = [build_problem(n, cfg2_params(A), "fp64", False, T=10.0, dt=0.05)[1]
            for _ in range(count)]
-    b = MPETBatch(sol, precision=precision)
-    b.step()
+    b = MPETBatch(sol, precision=precision, dense_bytes=limit)
+    st = b.step()
+    assert all(s.converged for s in st)
     torch.cuda.synchronize()
     used = torch.cuda.memory_allocated() - base
-    space = sol[0].up_.function_space()
-    tails = min(count * tail_bytes(space, precision), tail_bytes_all(precision))
-    est = count * (footprint_bytes(space, precision) - tail_bytes(space, precision)) + tails
+    est = 1.2 * count * footprint_bytes(sol[0].up_.function_space(), precision)
     b.close()
-    assert used <= 1.2 * est, (used, est)
-    assert tail_bytes(space, precision) <= tail_bytes_all(precision)
-    assert tail_bytes_all(precision) == {"mixed": 6, "fp64": 4}[precision] * DENSE_TAIL_BYTES
+    assert used <= est + dense_held(DENSE_TAIL_BYTES if limit is None else limit, precision)
 
 
-def test_server_shares_the_dense_ends():
-    """Admission counts the dense ends of many instances once, at most as much
-    as a batch can hold."""
-    from waterscapes_amd.serve import MPETServer, Request, tail_bytes_all
-    cap = tail_bytes_all("mixed")
-    srv = MPETServer(hbm_budget=10e9 + cap, setup_workers=0)
-    reqs = [Request(make_solver=None, steps=1, footprint=int(1e9) + cap // 2, tails=cap // 2)
-            for _ in range(11)]
-    for r in reqs[:10]:
-        assert srv._fits(r)
-        srv._hold(r, 1)
-    assert not srv._fits(reqs[10]) and (srv.used, srv.tails) == (10 * int(1e9), 5 * cap)
-    for r in reqs[:10]:
-        srv._hold(r, -1)
-    assert srv.used == srv.tails == 0
+def test_dense_ends_take_what_the_budget_leaves():
+    """A tight budget admits what it admitted without dense ends; they take
+    what is left."""
+    from waterscapes_amd import levels as lv
+    from waterscapes_amd.serve import MPETServer, dense_held, footprint_bytes
+    reqs = _requests([2])
+    one = footprint_bytes(reqs[0].make_solver().up_.function_space(), "mixed")
+    limits = []
+    for budget in (float(one), one + 6e5, 1e9):
+        srv = MPETServer(hbm_budget=budget, precision="mixed", outer_tol=1e-11,
+                         setup_workers=0)
+        r = _requests([2])[0]
+        r.arrival = 0.0
+        srv.submit(r)
+        srv.tick()
+        limits.append(srv.batch.dense_bytes)
+        assert srv.used + dense_held(limits[-1]) <= budget
+        srv.run()
+        assert not r.refused and r.steps_done == r.steps
+    assert limits == [0, 100000, lv.DENSE_TAIL_BYTES]
 
 
 def test_setup_threads_overlap_ticks_and_keep_results():

@@ -143,7 +143,7 @@ def csr_blockdiag(blocks):
 
 def pack_hierarchy(hiers, scales, skip_A0=False):
     """Concatenate instance hierarchies level by level (host arrays; the dense
-    coarsest operators stay on the device where all of them are there).
+    coarsest operators on the device where one of them is there).
 
     hiers: list of (levels, cinv) as returned by amg.setup_host; scales:
     per-instance factor s_k (the packed hierarchy approximates
@@ -177,10 +177,12 @@ def pack_hierarchy(hiers, scales, skip_A0=False):
         out.append(d)
     sizes = [p[0][-1]["n"] for p in padded]
     off = _prefix(sizes)
-    if all(torch.is_tensor(p[1]) for p in padded):
-        inv = torch.cat([(p[1] / s[k]).reshape(-1) for k, p in enumerate(padded)])
+    dev = next((p[1].device for p in padded if torch.is_tensor(p[1])), None)
+    if dev is not None:
+        inv = torch.cat([(torch.as_tensor(p[1]).to(dev, torch.float64) / s[k]).reshape(-1)
+                         for k, p in enumerate(padded)])
     else:
-        inv = np.concatenate([(lv.host_array(p[1]) / s[k]).reshape(-1)
+        inv = np.concatenate([(np.asarray(p[1]) / s[k]).reshape(-1)
                               for k, p in enumerate(padded)])
     ioff = _prefix([n * n for n in sizes])
     blk = np.repeat(np.arange(len(sizes), dtype=np.int32), sizes)
@@ -252,12 +254,14 @@ class MPETBatch:
     params); their "precision" is overridden by `precision` ("mixed" or
     "fp64").  The solvers' up_ / up become views into the batch's packed
     state, so initial conditions set on them before construction are kept
-    and results are read from them as usual.
+    and results are read from them as usual.  dense_bytes: most bytes of the
+    dense ends of each of the two packed hierarchies (default
+    levels.DENSE_TAIL_BYTES).
     """
 
     def __init__(self, solvers, precision="mixed", rtol=1e-10, outer_tol=3e-11,
                  inner_rtol=1e-6, maxit=5000, max_outer=30, check_every=10, use_graphs=True,
-                 extrapolate=None, extrapolate_order=4, autotune=False):
+                 extrapolate=None, extrapolate_order=4, autotune=False, dense_bytes=None):
         if not torch.cuda.is_available():
             raise RuntimeError("MPETBatch needs a GPU (no CPU fallback)")
         if precision not in ("mixed", "fp64"):
@@ -278,6 +282,8 @@ class MPETBatch:
             if str(torch.device(s.params["device"])) != str(dev):
                 raise ValueError("all instances of a batch must be on one device")
         self.engines = build_engines(self.solvers, precision)
+        # bytes of the packed dense ends of each of the two hierarchies
+        self.dense_bytes = lv.DENSE_TAIL_BYTES if dense_bytes is None else int(dense_bytes)
         self.keep = []
         self.cells = sum(e.space.mesh.num_cells() for e in self.engines) >= BATCH_CELLS
         self._layout()
@@ -567,7 +573,7 @@ class MPETBatch:
         # the small end of every hierarchy as one dense operator per instance
         # (levels.py), all instances' together within the byte limit
         rows = lv.dense_rows(8 if self.precision == "fp64" else 4,
-                             lv.DENSE_TAIL_BYTES // self.K)
+                             self.dense_bytes // self.K)
         cut = [k.dense_tails(rows, 0 if self.precision == "fp64" else 1) for k in kry]
         ulev, ucoarse = pack_hierarchy([c[0] for c in cut], mus, skip_A0=True)
         lap0 = torch.cat([s.prim_t["Lap"] * s.mu for s in sys_]).to(tdt)

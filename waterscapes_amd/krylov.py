@@ -529,19 +529,18 @@ class KrylovSolver:
         """((u levels, u coarse), (p levels, p coarse)) cut at the first level
         of at most `rows` rows with the levels' own FP64 values, the
         displacement hierarchy at level u_first or later (1 where the P2
-        level runs on half-precision values); the dense operators on the
-        device.  Kept for the last cut of each hierarchy: a batch's limit
-        follows its number of instances, the cut changes with it rarely."""
+        level runs on half-precision values); the dense operators formed here
+        are on the device.  Kept for the last cut of each hierarchy: a batch's
+        limit follows its number of instances, the cut changes with it
+        rarely."""
         s = self.sys
         kept = self.__dict__.setdefault("_tails", {})
 
         def cut(name, levels, coarse, params, first, *more):
             start = lv.tail_start(levels, rows, first)
             if kept.get(name, (None,))[0] != start:
-                levels, coarse = lv.with_dense_tail(levels, coarse, rows, params, s.device, *more,
-                                                    first=first)
-                kept[name] = (start, levels,
-                              torch.as_tensor(coarse).to(s.device, torch.float64))
+                kept[name] = (start, *lv.with_dense_tail(levels, coarse, rows, params, s.device,
+                                                         *more, first=first))
             return kept[name][1:]
         return (cut("u", self.levels, self._coarse_u, self.cfg.amg, u_first,
                     lambda l: (*s.pat_host["22"], self.lap0) if l == 0 else None, self.mask0),

@@ -17,7 +17,9 @@ resident until the request completes.  At every scheduling tick it
      coarsening is repeated (each instance's device state is reused, the dense
      ends of its hierarchies while their cut stays); the packed levels' fused
      transfers and slices are formed anew: 58 ms for 12 instances of 8^3 to
-     18^3 cubes, about one batched step of theirs;
+     18^3 cubes, about one batched step of theirs.  The dense ends take what
+     the budget leaves beside the footprints, at most what a batch takes by
+     itself;
   3. runs one batched step of the unfinished instances the tick policy
      picks (requests that arrived while others were running join
      mid-flight: their steps overlap on the device with the others');
@@ -47,8 +49,9 @@ from dataclasses import dataclass, field
 import numpy as np
 import torch
 
+from . import levels as lv
+from .amg import AmgParams
 from .batch import MPETBatch, batch_engine
-from .levels import DENSE_TAIL_BYTES, dense_rows
 
 ERR_BUDGET = 6
 
@@ -76,7 +79,7 @@ class Request:
     steps: int
     arrival: float = 0.0
     rid: object = None
-    footprint: int = 0                 # HBM bytes alone (0: estimated)
+    footprint: int = 0
     # filled by the server
     solver: object = None
     admitted: float = None
@@ -86,41 +89,18 @@ class Request:
     result: np.ndarray = None
     niter: list = field(default_factory=list)
     refused: bool = False
-    tails: int = 0                     # of footprint: dense ends, shared in a batch
     _fp: object = None                 # footprint estimate running on a set-up thread
-
-
-def tail_bytes(space, precision="mixed"):
-    """Bound of the HBM bytes of one instance's dense hierarchy ends alone in a
-    batch (levels.py): the packed copy and the FP64 one kept for re-packs.
-    Levels above the row limit are coarsened by at least 8."""
-    s = 4 if precision == "mixed" else 8
-    most = dense_rows(s)
-
-    def end(rows):
-        while rows > most:
-            rows = -(-rows // 8)
-        return rows * rows
-    # FP64 levels all qualify; in mixed precision the P2 level stays sparse
-    u = space.nP2 if precision != "mixed" and space.nP2 <= most else space.nP1
-    return (8 + s) * (end(u) + end((space.A + 1) * space.nP1))
-
-
-def tail_bytes_all(precision="mixed"):
-    """The same bound for any number of instances: the two packed dense
-    operators of a batch hold DENSE_TAIL_BYTES each whatever their number."""
-    s = 4 if precision == "mixed" else 8
-    return 2 * DENSE_TAIL_BYTES * (8 + s) // s
 
 
 def footprint_bytes(space, precision="mixed", robin=False):
     """Estimated HBM bytes of one resident instance: FP64 primitives, the
     packed FP64 / FP32 operator copies, the AMG hierarchies with their work
-    vectors and dense ends, and the step / MINRES vectors.  From the node
-    patterns only (no device allocation).  A batch that runs cell by cell keeps
-    cell tables instead of the packed operator values, which makes more than
-    room for its fused transfers and slices (32^3 cubes, A = 4: 1.46 GB in
-    use of 2.18 GB estimated)."""
+    vectors, and the step / MINRES vectors, without the dense ends that replace
+    levels of its hierarchies (dense_held).  From the node patterns only (no device
+    allocation).  A batch that runs cell by cell keeps cell tables instead of
+    the packed operator values, which makes more than room for its fused
+    transfers and slices (32^3 cubes, A = 4: 1.40 GB in use of 2.18 GB
+    estimated)."""
     dm = space.dofmap
     nz = {k: int(dm.pattern(k)[1].size) for k in ("22", "21", "12", "11")}
     A, n, nP2, nP1 = space.A, space.ndofs, space.nP2, space.nP1
@@ -132,10 +112,21 @@ def footprint_bytes(space, precision="mixed", robin=False):
     ops = 8 * op_vals + (s * op_vals if precision == "mixed" else 0) + 2 * idx
     # hierarchy: level 0 (Laplacian values, its pattern is shared) plus the
     # coarse levels (bounded by ~half of level 0) and 7 work vectors per row
+    # and the coarsest matrices
+    most = AmgParams().max_coarse
     amg = s * nz["22"] + (s + 4) * (nz["22"] + F * nz["11"]) // 2 \
-        + 7 * s * (3 * nP2 + F * nP1) * 2
+        + 7 * s * (3 * nP2 + F * nP1) * 2 \
+        + s * (min(nP1, most) ** 2 + min(F * nP1, most) ** 2)
     vecs = 9 * s * n + 13 * 8 * n
-    return int(prim + ops + amg + vecs + tail_bytes(space, precision))
+    return int(prim + ops + amg + vecs)
+
+
+def dense_held(limit, precision="mixed"):
+    """Bound of the HBM bytes of a batch's dense hierarchy ends, whatever its
+    instances: two packed operators of at most `limit` bytes (levels.py) and
+    the FP64 copies kept for re-packs."""
+    s = 4 if precision == "mixed" else 8
+    return 2 * limit * (8 + s) // s
 
 
 class MPETServer:
@@ -162,12 +153,10 @@ class MPETServer:
         self._pool = None
         self._local = threading.local()
         self.finished = []
-        # footprints of the resident requests but their dense ends, and those
         self.used = 0
-        self.tails = 0
         self.batch = None
         self.batch_reqs = []       # requests packed in self.batch, in order
-        self.retired = []          # retired requests still packed
+        self.pending_free = 0      # footprint of retired requests still packed
         self.t0 = clock()
         self.steps_run = 0
         self.ticks = 0
@@ -210,9 +199,8 @@ class MPETServer:
                     r.solver = r.make_solver()
                 prob = r.solver.problem
                 robin = any(not getattr(b, "is_zero", lambda: False)() for b in prob.beta)
-                space = r.solver.up_.function_space()
-                r.tails = tail_bytes(space, self.precision)
-                r.footprint = footprint_bytes(space, self.precision, robin)
+                r.footprint = footprint_bytes(r.solver.up_.function_space(), self.precision,
+                                              robin)
             return r.footprint
         return self._on_stream(work, req)
 
@@ -262,12 +250,12 @@ class MPETServer:
                 req.done = now
                 self.finished.append(req)
                 continue
-            if not self._fits(req) and self.retired:
+            if self.used + req.footprint > self.budget and self.pending_free:
                 self._drop_batch()         # release retired instances first
-            if not self._fits(req):
+            if self.used + req.footprint > self.budget:
                 break                      # wait until memory frees up
             self.waiting.pop(0)
-            self._hold(req, 1)
+            self.used += req.footprint
             if self.setup_workers > 0:
                 self.preparing.append((req, self._submit(self._setup, req)))
             else:
@@ -276,14 +264,6 @@ class MPETServer:
                 self.active.append(req)
                 changed = True
         return changed
-
-    def _hold(self, req, sign):
-        self.used += sign * (req.footprint - req.tails)
-        self.tails += sign * req.tails
-
-    def _fits(self, req):
-        tails = min(self.tails + req.tails, tail_bytes_all(self.precision))
-        return self.used + req.footprint - req.tails + tails <= self.budget
 
     def busy(self):
         """Requests waiting, being set up or running."""
@@ -295,16 +275,17 @@ class MPETServer:
             self.batch.close()
             self.batch = None
         self.batch_reqs = []
-        for r in self.retired:
-            self._hold(r, -1)
-        self.retired = []
+        self.used -= self.pending_free
+        self.pending_free = 0
         gc.collect()
 
     def _repack(self):
         self._drop_batch()
         if self.active:
+            spare = max(0.0, self.budget - self.used)
+            limit = int(min(lv.DENSE_TAIL_BYTES, spare / dense_held(1, self.precision)))
             self.batch = MPETBatch([r.solver for r in self.active], precision=self.precision,
-                                   **self.tol)
+                                   dense_bytes=limit, **self.tol)
             self.batch_reqs = list(self.active)
 
     def _retire(self, now):
@@ -313,7 +294,7 @@ class MPETServer:
             if r.steps_done >= r.steps:
                 r.result = r.solver.up.vector().get_local().copy()
                 r.done = now
-                self.retired.append(r)
+                self.pending_free += r.footprint
                 r.solver = None
                 self.finished.append(r)
             else:
